@@ -76,8 +76,11 @@ Launch plan_launch(const pda_ctx* ctx, int pass, bool population, uint64_t units
     uint64_t batch = uint64_t(kWave) * ctx->shape.batch_tiles;
     if (ctx->shape.batch_tiles == 0) {
         // about six grabs per wave: small batches keep the grid's tail
-        // short (a wave that grabs last still walks a whole batch)
-        batch = (units / (max_grid * 6u) + kWave - 1) / kWave * kWave;
+        // short (a wave that grabs last still walks a whole batch); a
+        // population's batches differ in cost by more than the waves do in
+        // speed: about 32 grabs per wave
+        const uint64_t grabs = population ? 32u : 6u;
+        batch = (units / (max_grid * grabs) + kWave - 1) / kWave * kWave;
         batch = std::min<uint64_t>(std::max<uint64_t>(batch, kWave), 4096);
     }
     const uint64_t batches = (units + batch - 1) / batch;

@@ -351,8 +351,13 @@ __device__ __forceinline__ void flush_hist(int32_t* h, int32_t* __restrict__ his
 
 // Work is a flat list of batches: set s owns batches [s * bps, (s + 1) * bps),
 // each covering up to a.batch consecutive units of that set; the list is
-// split into a.queues contiguous ranges with a counter each, as in
-// walk_kernel.  A wave's lanes may be walking units of two sets at once: the
+// dealt out to the a.queues work counters in turn (counter q hands out
+// batches q, q + queues, ...).  Sets differ in their dwell windows per unit by
+// up to two orders of magnitude: contiguous shares of the list gave whole
+// sets to a counter, whose waves (only they take from it) were still walking
+// when the others had ended (64 sets of fast dynamics: 3.6 of 7 waves per
+// SIMD busy over the launch; dealt out: 6.6).  A wave's lanes may be walking
+// units of two sets at once: the
 // workgroup keeps two LDS model slots with an LDS histogram each, and a wave
 // moves to a third set only after the older slot's lanes have finished, so it
 // never drains to change sets.
@@ -377,8 +382,7 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(
     const uint32_t seed = ctl->seed, set_base = ctl->set_base, set_stride = ctl->set_stride;
     const uint32_t queue = blockIdx.x % a.queues;
     const uint32_t nb = a.nsets * a.bps;
-    const uint32_t q_begin = uint32_t(uint64_t(nb) * queue / a.queues);
-    const uint32_t q_end = uint32_t(uint64_t(nb) * (queue + 1u) / a.queues);
+    const uint32_t q_len = nb > queue ? (nb - queue + a.queues - 1u) / a.queues : 0u;
     const uint32_t xrow = blockIdx.x & 7u;
     int set0 = -1, set1 = -1;    // wave-uniform: the set each LDS slot holds
     uint32_t cur = 0;            // slot that receives new units
@@ -399,11 +403,11 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(
                 uint32_t k = 0;
                 if (lane == 0) k = atomicAdd(&work[queue * kCounterStride], 1u);
                 k = __shfl(k, 0);
-                if (k >= q_end - q_begin) {
+                if (k >= q_len) {
                     drained = true;
                     break;
                 }
-                k += q_begin;
+                k = k * a.queues + queue;
                 pool_set = k / a.bps;
                 pool_next = (k - pool_set * a.bps) * a.batch;
                 pool_end = pool_next + a.batch < a.nunits ? pool_next + a.batch : a.nunits;
