@@ -68,7 +68,7 @@ void range_of(const pda_ctx* ctx, const Slot& s, int64_t* b0, int64_t* b1) {
 Launch plan_launch(const pda_ctx* ctx, int pass, bool population, uint64_t units) {
     int per_cu = 0;
     hipError_t e = population ? pop_walk_occupancy(pass, ctx->B, &per_cu)
-                              : walk_occupancy(pass, &per_cu);
+                              : walk_occupancy(pass, ctx->B, &per_cu);
     if (e != hipSuccess || per_cu < 1) per_cu = 1;
     if (ctx->shape.waves_per_cu > 0 && int(ctx->shape.waves_per_cu) < per_cu)
         per_cu = int(ctx->shape.waves_per_cu);
@@ -90,6 +90,14 @@ Launch plan_launch(const pda_ctx* ctx, int pass, bool population, uint64_t units
     const uint32_t q = ctx->shape.queues ? ctx->shape.queues : kDefaultQueues;
     L.queues = std::min<uint32_t>(q, L.grid);
     return L;
+}
+
+void plan_args(RunArgs& a, uint64_t items, uint32_t align) {
+    const UnitDiv q = make_unit_div(a.R);
+    a.div_m = q.m;
+    a.div_sh = q.sh;
+    const uint64_t share = (items + a.queues - 1u) / a.queues;
+    a.q_share = uint32_t(std::max<uint64_t>(1, (share + align - 1u) / align * align));
 }
 
 }  // namespace pda
@@ -178,6 +186,7 @@ int upload_model(Slot& s) {
     s.h_blob->m = M;
     build_binom_table(M, s.h_blob->tab);
     s.any_v = M.any_v != 0;
+    s.quick_rates = M.quick_rates != 0;
     HIP_TRY(hipMemcpyAsync(s.d_blob, s.h_blob, sizeof(ModelBlob), hipMemcpyHostToDevice, s.stream));
     HIP_TRY(hipEventRecord(s.model_copied, s.stream));
     if (!s.any_v) HIP_TRY(launch_guide(s.d_blob, 1, M.n, s.d_thr, s.d_guide, s.stream));
@@ -431,6 +440,7 @@ int pda_run(pda_ctx* ctx, int sid, int R, uint32_t seed, uint32_t set_id, int fl
     a.queues = L.queues;
     a.nsets = 1;
     a.bps = 0;
+    plan_args(a, uint64_t(nunits), kWave);
 
     float* outE = nullptr;
     int32_t* outAcc = nullptr;
@@ -470,8 +480,9 @@ int pda_run(pda_ctx* ctx, int sid, int R, uint32_t seed, uint32_t set_id, int fl
     a.replay_cap = uint32_t(s->replay_cap);
     HIP_TRY(hipEventRecord(s->ev0, s->stream));
     const BinomGuide guide{s->d_thr, s->d_guide};
+    const FastArgs fa = fast_args(s->n, s->quick_rates, a.clk_p);
     HIP_TRY(launch_walk(pass, grid, ctx->d_bursts, ctx->d_ticks, ctx->d_links, s->d_blob, guide, a,
-                        s->d_hist_acc, s->d_replay, s->d_replay_count, s->d_work, outE, outAcc,
+                        fa, s->d_hist_acc, s->d_replay, s->d_replay_count, s->d_work, outE, outAcc,
                         outF, s->stream));
     HIP_TRY(hipEventRecord(s->ev_mid, s->stream));
     if (pass == kPassFast && nunits > 0) {
@@ -479,12 +490,12 @@ int pda_run(pda_ctx* ctx, int sid, int R, uint32_t seed, uint32_t set_id, int fl
         // grid is sized for the worst case and its unneeded workgroups exit
         // at once
         int per_cu = 0;
-        if (walk_occupancy(kPassReplay, &per_cu) != hipSuccess || per_cu < 1) per_cu = 1;
+        if (walk_occupancy(kPassReplay, ctx->B, &per_cu) != hipSuccess || per_cu < 1) per_cu = 1;
         const uint64_t want = (uint64_t(nunits) + kWave - 1) / kWave;
         const uint32_t rgrid =
             uint32_t(std::max<uint64_t>(1, std::min<uint64_t>(want, uint64_t(ctx->num_cu) * per_cu)));
         HIP_TRY(launch_walk(kPassReplay, rgrid, ctx->d_bursts, ctx->d_ticks, ctx->d_links,
-                            s->d_blob, guide, a, s->d_hist_acc, s->d_replay, s->d_replay_count,
+                            s->d_blob, guide, a, fa, s->d_hist_acc, s->d_replay, s->d_replay_count,
                             s->d_work,
                             outE, outAcc, outF, s->stream));
     }

@@ -15,6 +15,7 @@
 #include "../../include/gsmfretda_pda.h"
 #include "pda_layout.h"
 #include "pda_types.h"
+#include "pda_walk.h"
 
 namespace pda {
 
@@ -51,9 +52,10 @@ struct PopGraphKey {
     uint64_t data_gen = 0;
     const void* obs = nullptr;
     // binomial threshold rows: whether the walk reads them, the guide
-    // kernel's state count and the table's buffer
+    // kernel's state count (also the walk's) and the table's buffer
     bool guided = false;
     int max_states = 0;
+    bool quick_rates = false;
     const void* thr = nullptr;
     bool operator==(const PopGraphKey& o) const;
 };
@@ -64,6 +66,7 @@ struct Population {
     std::vector<float> args;         // packed args of every set
     std::vector<int64_t> off;        // start of set s in args
     bool any_v = false;
+    bool quick_rates = false;        // of every set
     size_t cap_sets = 0;             // allocated sets
     uint8_t* h_in = nullptr;         // pinned: PopControl + ModelBlob[cap_sets]
     uint8_t* d_in = nullptr;
@@ -152,6 +155,7 @@ struct RbState {
 };
 
 struct Slot {
+    bool quick_rates = false;     // every rate of the set is in quotient()'s range
     hipStream_t stream = nullptr;
     ModelBlob* h_blob = nullptr;  // pinned staging of the model tables
     ModelBlob* d_blob = nullptr;
@@ -252,13 +256,17 @@ struct Launch {
     uint32_t grid = 1, batch = kWave, queues = 1;
 };
 Launch plan_launch(const pda_ctx* ctx, int pass, bool population, uint64_t units);
+// The fields of a walk's arguments that follow from the others: R's
+// multiply-shift divisor, and the `items` (units, or a population's batches)
+// each of the a.queues work counters hands out, in whole waves of units.
+void plan_args(RunArgs& a, uint64_t items, uint32_t align);
 
 // kernels (pda_kernels.hip)
-hipError_t walk_occupancy(int pass, int* blocks_per_cu);
+hipError_t walk_occupancy(int pass, int B, int* blocks_per_cu);
 hipError_t pop_walk_occupancy(int pass, int B, int* blocks_per_cu);
 hipError_t launch_walk(int pass, uint32_t grid, const BurstDesc* bursts, const uint32_t* ticks,
                        const uint2* links, const ModelBlob* blob, const BinomGuide& guide,
-                       const RunArgs& a, int32_t* hist_acc, uint32_t* replay,
+                       const RunArgs& a, const FastArgs& fa, int32_t* hist_acc, uint32_t* replay,
                        uint32_t* replay_count, uint32_t* work, float* outE, int32_t* outAcc,
                        float* outF, hipStream_t stream);
 hipError_t launch_guide(const ModelBlob* blobs, int nsets, int max_states, ThrPair* thr,
@@ -270,8 +278,8 @@ hipError_t launch_finish(const RunArgs& a, const float* obs, int32_t* hist_acc,
 hipError_t launch_pop_walk(int pass, uint32_t grid, const BurstDesc* bursts,
                            const uint32_t* ticks, const uint2* links, const PopControl* ctl,
                            const ModelBlob* blobs, const BinomGuide& guide, const RunArgs& a,
-                           int32_t* hist_acc, uint64_t* replay, uint32_t* replay_count,
-                           uint32_t* work, hipStream_t stream);
+                           const FastArgs& fa, int32_t* hist_acc, uint64_t* replay,
+                           uint32_t* replay_count, uint32_t* work, hipStream_t stream);
 hipError_t launch_pop_replay(const BurstDesc* bursts, const uint32_t* ticks, const uint2* links,
                              const PopControl* ctl, const ModelBlob* blobs, const RunArgs& a,
                              int32_t* hist_acc, const uint64_t* replay,
@@ -298,8 +306,9 @@ hipError_t rb_walk_occupancy(bool scores, int n, int* per_cu);
 // abandoned (replay_grid workgroups; those beyond the list's need exit)
 hipError_t launch_rb_walk(bool scores, int n, uint32_t grid, uint32_t replay_grid,
                           const BurstDesc* bursts, const uint32_t* ticks, const uint2* links,
-                          const ModelBlob* blob, const RbModel* rbm, const RunArgs& a, uint2* cnt,
-                          float* F, float* S, uint32_t* work, uint32_t* big, uint32_t* huge,
+                          const ModelBlob* blob, const RbModel* rbm, const RunArgs& a,
+                          const FastArgs& fa, uint2* cnt, float* F, float* S, uint32_t* work,
+                          uint32_t* big, uint32_t* huge,
                           uint32_t* big_count, uint32_t* replay, uint32_t* replay_count,
                           hipStream_t stream);
 // dynamic LDS bytes (mode: 0 forward, 1 adjoint, 2 Jacobian)

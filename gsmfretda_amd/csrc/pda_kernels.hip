@@ -1,6 +1,6 @@
 // pda_kernels.hip -- gfx950 kernels of the Monte-Carlo PDA hot path.
 //
-// walk_kernel + finish_kernel replace gSMFRETda's mc_kernel (src/mc.cu:83-197)
+// fast_walk_kernel, walk_kernel and finish_kernel replace gSMFRETda's mc_kernel (src/mc.cu:83-197)
 // together with the host histogram and chi2 of src/streamWorker.cpp:184-206:
 //   * one-wave workgroups; every lane streams through (burst, resample)
 //     units taken from per-XCD work counters, advancing one dwell window
@@ -12,9 +12,9 @@
 //     (seed, set, window, sub-stream, resample, burst) -- no RNG state in
 //     memory, nothing to initialise (replaces setup_kernel,
 //     src/gen_rand.cuh:7-25);
-//   * the common case runs in a lean form (at most 72 VGPRs); the rare units
-//     that need BTPE draws, inversion restarts or large background means are
-//     listed and replayed in full by the same kernel in its general form
+//   * the common case runs in a lean form (fast_walk_kernel, at most 72
+//     VGPRs); the rare units that need BTPE draws, inversion restarts or
+//     large background means are listed and replayed in full by walk_kernel
 //     over the whole grid; finish_kernel then reduces the LDS histograms of
 //     all workgroups and computes chi2 on the device.
 #include <hip/hip_runtime.h>
@@ -38,52 +38,271 @@ enum Pass : int {
 constexpr uint32_t kReplayQueues = 8;
 static_assert(kReplayQueues <= kAuxQueues, "replay counters live on the auxiliary lines");
 
-// The per-unit outputs outE / outAcc / outF are requested together (all
-// null or all set), so one test covers the three stores.
-__device__ __forceinline__ void tally(int32_t* s_hist, const RunArgs& a, const WalkOut& o,
-                                      uint32_t u, float* outE, int32_t* outAcc, float* outF) {
-    const float E = o.F > 0.0f ? o.acc / o.F : 0.0f;
+// Contiguous share of a run's work items (units or batches) that one work
+// counter hands out.
+struct QueueRange {
+    uint32_t begin, end;
+};
+__device__ __forceinline__ QueueRange queue_range(uint32_t queue, uint32_t share, uint32_t n) {
+    const uint64_t b = uint64_t(queue) * share;
+    const uint32_t begin = b < n ? uint32_t(b) : n;
+    return QueueRange{begin, n - begin < share ? n : begin + share};
+}
+
+// Batches of a population that a work counter hands out: every queues-th of
+// the flat list (set 0's batches, set 1's, ...), the first being `queue`.  A
+// set's units take a multiple of another's under faster dynamics; dealt out
+// like this every queue has its share of every set, where contiguous shares
+// gave whole sets to a queue, whose waves (only they take from it) ended
+// long after the others'.
+__device__ __forceinline__ uint32_t pop_queue_length(uint32_t batches, uint32_t queue,
+                                                     uint32_t queues) {
+    return batches > queue ? (batches - queue + queues - 1u) / queues : 0u;
+}
+
+// Lanes of the mask below this one.
+__device__ __forceinline__ uint32_t lanes_below(uint64_t mask) {
+    return __builtin_amdgcn_mbcnt_hi(uint32_t(mask >> 32),
+                                     __builtin_amdgcn_mbcnt_lo(uint32_t(mask), 0u));
+}
+
+// Orders the LDS accesses of the wave's lanes: what a lane wrote before is
+// visible to every lane's reads after it (one-wave workgroups, no barrier).
+__device__ __forceinline__ void wave_lds_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+}
+
+// A unit's efficiency into the LDS histogram.
+__device__ __forceinline__ void tally(int32_t* h, int B, float acc, float F) {
+    const float E = F > 0.0f ? acc / F : 0.0f;
     if (E >= 0.0f && E < 1.0f) {
-        const int bin = int(floor(double(E) * double(a.B)));
-        if (bin < a.B) atomicAdd(&s_hist[bin], 1);
-    }
-    if (outE) {
-        outE[u] = E;
-        outAcc[u] = int32_t(o.acc);
-        outF[u] = o.F;
+        const int bin = int(floor(double(E) * double(B)));
+        if (bin < B) atomicAdd(&h[bin], 1);
     }
 }
 
-// The walk over every unit of the run (kPassFast, kPassGeneral), or over the
-// units the fast pass abandoned (kPassReplay, launched right after it on the
-// same stream, so the replay list and its count are final).  Each one-wave
-// workgroup keeps an LDS histogram and adds it to its XCD's accumulator row
-// at the end (workgroups are dispatched to the 8 XCDs round-robin, so the
-// atomics of a launch spread over 8 x B addresses).  No completion ticket
-// and no fence: the finish kernel, launched behind on the same stream, reads
-// the rows.
-// The fast forms are held to a register count that keeps many waves
-// resident: their window loop waits on dependent loads, and each more
-// resident wave per SIMD hides more of that latency than the registers it
-// gives up cost.  The single-set walk fits 64 VGPRs (8 waves per SIMD, no
-// spill to scratch; -2 % walk time against 7 waves on the 3-state
-// workload, the LDS of 32 workgroups exactly 160 KB); the population walk
-// keeps 72 (7 waves), where 64 would spill.
+// The per-unit outputs of a run that keeps samples.
+__device__ __forceinline__ void store_sample(uint32_t u, float acc, float F, float* outE,
+                                             int32_t* outAcc, float* outF) {
+    outE[u] = F > 0.0f ? acc / F : 0.0f;
+    outAcc[u] = int32_t(acc);
+    outF[u] = F;
+}
+
+// Adds an LDS histogram to an accumulator row and clears it.
+__device__ __forceinline__ void flush_hist(int32_t* h, int32_t* __restrict__ row, int B,
+                                           uint32_t lane) {
+    for (uint32_t i = lane; i < uint32_t(B); i += kWave) {
+        const int32_t v = h[i];
+        if (v) {
+            atomicAdd(&row[i], v);
+            h[i] = 0;
+        }
+    }
+}
+
+// ---- walk in the fast form --------------------------------------------------------
+//
+// The fast form of a run (one parameter set) or of a population's generation.
+// One-wave workgroups; every lane streams through units: one loop pass
+// advances each busy lane by a dwell window, and lanes whose unit ended take
+// another, so neither lanes nor waves wait for the longest unit.  Work is
+// handed out as in walk_kernel (population: pop_walk_kernel).
+// kPop: population (two LDS model slots with a histogram each); kGuided:
+// binomial draws from the threshold rows (else by the inversion loop, for
+// populations too large for a table of rows); kSamples: per-unit outputs.
+//
+// Bound by VALU issue (at or above 95 % of the cycles), so what counts is the
+// instructions of fast_window: the window's arithmetic without the cases its
+// arguments cannot have, correctly rounded quotients from reciprocals kept
+// per model, and the launch's divisions done on the host (unit / R, the
+// queues' shares) took a 3-state evaluation of 100,000 bursts x 100 from 459
+// to 407 us and the 256-set generation from 16.7 to 14.7 ms.  The register
+// limit keeps 8 waves on a SIMD (single set) or 7 (population, where 64 VGPRs
+// would spill): the window loop waits on dependent loads, which the other
+// waves hide.  (Starting 64 units at a time and queueing in LDS those that
+// outlast their first window was slower: 14 % more instructions, the first
+// window's close running for half of the lanes.)
 constexpr int kFastWavesPerEU = 8;
 constexpr int kPopFastWavesPerEU = 7;
 
-template <int kPass>
+struct FastIO {
+    const BurstDesc* bursts;
+    const uint32_t* ticks;
+    const uint2* links;
+    const ModelBlob* blobs;    // [1], or the population's sets
+    const PopControl* ctl;     // population: the sets' stream keys
+    BinomGuide guide;
+    int32_t* hist_acc;
+    void* replay;              // uint32 units; population: (set << 32 | unit)
+    uint32_t* replay_count;
+    uint32_t* work;
+    float* outE;
+    int32_t* outAcc;
+    float* outF;
+};
+
+template <bool kPop, bool kGuided, bool kSamples>
 __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(
-    kPass == kPassFast ? kFastWavesPerEU : 1))) void walk_kernel(
+    kPop ? kPopFastWavesPerEU : kFastWavesPerEU))) void fast_walk_kernel(const FastIO io,
+                                                                         const RunArgs a,
+                                                                         const FastArgs fa) {
+    constexpr int kSlots = kPop ? 2 : 1;
+    __shared__ Model sM[kSlots];
+    extern __shared__ int32_t s_hist[];  // [kSlots][a.B]
+    const uint32_t lane = threadIdx.x;
+    for (uint32_t i = lane; i < uint32_t(kSlots) * uint32_t(a.B); i += kWave) s_hist[i] = 0;
+    if (!kPop) {
+        const uint32_t* src = reinterpret_cast<const uint32_t*>(&io.blobs->m);
+        uint32_t* dst = reinterpret_cast<uint32_t*>(&sM[0]);
+        for (uint32_t i = lane; i < sizeof(Model) / 4; i += kWave) dst[i] = src[i];
+    }
+    wave_lds_sync();
+
+    const uint32_t queue = blockIdx.x % a.queues;
+    // this queue's work: a contiguous share of the units, or every
+    // a.queues-th batch of the generation
+    const QueueRange q = queue_range(queue, a.q_share, kPop ? 0u : a.nunits);
+    const uint32_t q_len = kPop ? pop_queue_length(a.nsets * a.bps, queue, a.queues)
+                                : q.end - q.begin;
+    const uint32_t xrow = blockIdx.x & 7u;
+    const UnitDiv divR{a.div_m, a.div_sh};
+    int set0 = kPop ? -1 : 0, set1 = -1;  // the set each LDS slot holds
+    uint32_t cur = 0;                     // slot that receives new units
+    uint32_t pool_set = 0, pool_next = 0, pool_end = 0;
+    bool drained = false;
+    bool busy = false;
+    uint32_t slot = 0;
+    WalkState<true> st{};
+    UnitKey key{kPop ? io.ctl->seed : a.seed, a.set, 0u, 0u};
+    BurstDesc d{0u, 0u, 0u, 0.0f};
+    while (true) {
+        bool need = !busy;
+        while (!drained) {
+            const uint64_t want = __ballot(need);
+            if (want == 0) break;
+            if (pool_next >= pool_end) {
+                uint32_t k = 0;
+                if (lane == 0) k = atomicAdd(&io.work[queue * kCounterStride], kPop ? 1u : a.batch);
+                k = __builtin_amdgcn_readfirstlane(k);
+                if (k >= q_len) {
+                    drained = true;
+                    break;
+                }
+                if (kPop) {
+                    k = k * a.queues + queue;
+                    pool_set = k / a.bps;
+                    pool_next = (k - pool_set * a.bps) * a.batch;
+                    pool_end = a.nunits - pool_next < a.batch ? a.nunits : pool_next + a.batch;
+                } else {
+                    pool_next = q.begin + k;
+                    pool_end = q.end - pool_next < a.batch ? q.end : pool_next + a.batch;
+                }
+            }
+            if (kPop && int(pool_set) != (cur ? set1 : set0)) {
+                const uint32_t other = cur ^ 1u;
+                if (__any(busy && slot == other)) break;  // the older set is still walking
+                const int old = other ? set1 : set0;
+                if (old >= 0) {
+                    wave_lds_sync();
+                    flush_hist(s_hist + other * uint32_t(a.B),
+                               io.hist_acc + (size_t(old) * 8u + xrow) * size_t(a.B), a.B, lane);
+                }
+                const uint32_t* src = reinterpret_cast<const uint32_t*>(&io.blobs[pool_set].m);
+                uint32_t* dst = reinterpret_cast<uint32_t*>(&sM[other]);
+                for (uint32_t i = lane; i < sizeof(Model) / 4; i += kWave) dst[i] = src[i];
+                wave_lds_sync();
+                if (other) set1 = int(pool_set);
+                else set0 = int(pool_set);
+                cur = other;
+            }
+            const uint32_t rank = lanes_below(want);
+            const uint32_t avail = pool_end - pool_next;
+            if (need && rank < avail) {
+                const uint32_t u = pool_next + rank;
+                const uint32_t bl = unit_div(u, divR);
+                slot = cur;
+                d = io.bursts[a.begin + bl];
+                if (kPop) key.set = io.ctl->set_base + pool_set * io.ctl->set_stride;
+                key.r = u - bl * a.R;
+                key.b = a.begin + bl;
+                if (begin_unit<true>(sM[kPop ? slot : 0u], key, d.P, d.T, st) == kStepMore) {
+                    busy = true;
+                    need = false;
+                } else {
+                    tally(s_hist + slot * uint32_t(a.B), a.B, 0.0f, 0.0f);
+                    if (kSamples) store_sample(u, 0.0f, 0.0f, io.outE, io.outAcc, io.outF);
+                }
+            }
+            const uint32_t taken = uint32_t(__popcll(want));
+            pool_next += taken < avail ? taken : avail;
+        }
+        if (!__any(busy)) break;
+        if (busy) {
+            const Model& M = sM[kPop ? slot : 0u];
+            const uint32_t set = kPop ? uint32_t(slot ? set1 : set0) : 0u;
+            const uint32_t* ticks = io.ticks + d.off;
+            const uint2* links = io.links + d.off;
+            int r;
+            if (kGuided) {
+                const size_t base = kPop ? size_t(M.guide_base) : 0;
+                const BinomGuide g{io.guide.thr + base * kGuideStatePairs,
+                                   io.guide.guide + base * kBinomTable * kGuideBuckets};
+                r = fast_window<false, BinomGuide>(M, &g, key, d.P, d.stop_rel, d.T, ticks, links,
+                                                   a, fa, st);
+            } else {
+                r = fast_window<false, BinomTable>(M, &io.blobs[set].tab, key, d.P, d.stop_rel,
+                                                   d.T, ticks, links, a, fa, st);
+            }
+            if (r != kStepMore) {
+                busy = false;
+                const uint32_t u = (key.b - a.begin) * a.R + key.r;
+                if (r == kStepReplay) {
+                    const uint32_t i = atomicAdd(io.replay_count, 1u);
+                    if (i < a.replay_cap) {
+                        if (kPop) static_cast<uint64_t*>(io.replay)[i] = (uint64_t(set) << 32) | u;
+                        else static_cast<uint32_t*>(io.replay)[i] = u;
+                    }
+                } else {
+                    tally(s_hist + slot * uint32_t(a.B), a.B, st.acc, st.F);
+                    if (kSamples) store_sample(u, st.acc, st.F, io.outE, io.outAcc, io.outF);
+                }
+            }
+        }
+    }
+    wave_lds_sync();
+    if (kPop) {
+        if (set0 >= 0)
+            flush_hist(s_hist, io.hist_acc + (size_t(set0) * 8u + xrow) * size_t(a.B), a.B, lane);
+        if (set1 >= 0)
+            flush_hist(s_hist + uint32_t(a.B),
+                       io.hist_acc + (size_t(set1) * 8u + xrow) * size_t(a.B), a.B, lane);
+    } else {
+        flush_hist(s_hist, io.hist_acc + size_t(xrow) * kMaxBins, a.B, lane);
+    }
+}
+
+// ---- walk in the general form ---------------------------------------------------
+//
+// Every unit of the run (kPassGeneral), or the units the fast pass abandoned
+// (kPassReplay, launched right after it on the same stream, so the replay
+// list and its count are final).  Each one-wave workgroup keeps an LDS
+// histogram and adds it to its XCD's accumulator row at the end (workgroups
+// are dispatched to the 8 XCDs round-robin, so the atomics of a launch spread
+// over 8 x B addresses).  No completion ticket and no fence: the finish
+// kernel, launched behind on the same stream, reads the rows.
+template <int kPass>
+__global__ __launch_bounds__(kWave) void walk_kernel(
     const BurstDesc* __restrict__ bursts, const uint32_t* __restrict__ ticks,
-    const uint2* __restrict__ links, const ModelBlob* __restrict__ blob, const BinomGuide guide,
-    const RunArgs a, int32_t* __restrict__ hist_acc, uint32_t* __restrict__ replay,
-    uint32_t* __restrict__ replay_count, uint32_t* __restrict__ work, float* __restrict__ outE,
-    int32_t* __restrict__ outAcc, float* __restrict__ outF) {
-    constexpr bool kFastForm = kPass == kPassFast;
+    const uint2* __restrict__ links, const ModelBlob* __restrict__ blob, const RunArgs a,
+    int32_t* __restrict__ hist_acc, const uint32_t* __restrict__ replay,
+    const uint32_t* __restrict__ replay_count, uint32_t* __restrict__ work,
+    float* __restrict__ outE, int32_t* __restrict__ outAcc, float* __restrict__ outF) {
     constexpr bool kReplay = kPass == kPassReplay;
     // units of this pass, units per grab, queues and their counters
-    uint32_t nunits = a.nunits, batch = a.batch, queues = a.queues;
+    uint32_t nunits = a.nunits, batch = a.batch, queues = a.queues, share = a.q_share;
     uint32_t* counters = work;
     if (kReplay) {
         const uint32_t c = *replay_count;
@@ -95,10 +314,11 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(
         if (blockIdx.x >= alive) return;  // uniform over the workgroup
         batch = kWave;
         queues = alive < kReplayQueues ? alive : kReplayQueues;
+        share = (nunits + queues - 1u) / queues;
         counters = work + size_t(kMaxQueues) * kCounterStride;
     }
     __shared__ Model sM;
-    __shared__ int32_t s_hist[kMaxBins];
+    extern __shared__ int32_t s_hist[];  // [a.B]
     const uint32_t lane = threadIdx.x;
     {
         const uint32_t* src = reinterpret_cast<const uint32_t*>(&blob->m);
@@ -122,16 +342,15 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(
     // whole batch, so the batch sets the grid's tail.  Photons are read
     // through L1/L2.  A replay pass takes its units the same way from the
     // replay list.
-    const uint32_t queue = blockIdx.x % queues;
-    const uint32_t q_begin = uint32_t(uint64_t(nunits) * queue / queues);
-    const uint32_t q_end = uint32_t(uint64_t(nunits) * (queue + 1u) / queues);
+    const QueueRange q = queue_range(blockIdx.x % queues, share, nunits);
+    uint32_t* counter = &counters[(blockIdx.x % queues) * kCounterStride];
     uint32_t pool_next = 0, pool_end = 0;  // the wave's current batch
     bool busy = false;
     uint32_t u = 0;
-    WalkState<kFastForm> st{};
+    WalkState<false> st{};
     UnitKey key{a.seed, a.set, 0u, 0u};
     BurstDesc d{0u, 0u, 0u, 0.0f};
-    const UnitDiv divR = make_unit_div(a.R);
+    const UnitDiv divR{a.div_m, a.div_sh};
     bool drained = false;
     while (true) {
         bool need = !busy;
@@ -140,17 +359,16 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(
             if (want == 0) break;
             if (pool_next >= pool_end) {
                 uint32_t off = 0;
-                if (lane == 0) off = atomicAdd(&counters[queue * kCounterStride], batch);
+                if (lane == 0) off = atomicAdd(counter, batch);
                 off = __shfl(off, 0);
-                if (off >= q_end - q_begin) {
+                if (off >= q.end - q.begin) {
                     drained = true;
                     break;
                 }
-                pool_next = q_begin + off;
-                pool_end = pool_next + batch < q_end ? pool_next + batch : q_end;
+                pool_next = q.begin + off;
+                pool_end = pool_next + batch < q.end ? pool_next + batch : q.end;
             }
-            const uint32_t rank = __builtin_amdgcn_mbcnt_hi(
-                uint32_t(want >> 32), __builtin_amdgcn_mbcnt_lo(uint32_t(want), 0u));
+            const uint32_t rank = lanes_below(want);
             const uint32_t avail = pool_end - pool_next;
             if (need && rank < avail) {
                 u = kReplay ? replay[pool_next + rank] : pool_next + rank;
@@ -159,11 +377,12 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(
                 d = bursts[b];
                 key.r = u - bl * a.R;
                 key.b = b;
-                if (begin_unit<kFastForm>(sM, key, d.P, d.T, st) == kStepMore) {
+                if (begin_unit<false>(sM, key, d.P, d.T, st) == kStepMore) {
                     busy = true;
                     need = false;
                 } else {
-                    tally(s_hist, a, WalkOut{0.0f, 0.0f, false}, u, outE, outAcc, outF);
+                    tally(s_hist, a.B, 0.0f, 0.0f);
+                    if (outE) store_sample(u, 0.0f, 0.0f, outE, outAcc, outF);
                 }
             }
             const uint32_t taken = uint32_t(__popcll(want));
@@ -171,25 +390,17 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(
         }
         if (!__any(busy)) break;
         if (busy) {
-            const int r = step_window<kFastForm, false, BinomGuide>(
-                sM, &guide, key, d.P, d.stop_rel, d.T, ticks + d.off, links + d.off, a, st);
+            const int r = general_window(sM, key, d.P, d.stop_rel, d.T, ticks + d.off,
+                                         links + d.off, a, st);
             if (r != kStepMore) {
-                if (r == kStepReplay) {
-                    const uint32_t slot = atomicAdd(replay_count, 1u);
-                    if (slot < a.replay_cap) replay[slot] = u;
-                } else {
-                    tally(s_hist, a, WalkOut{st.acc, st.F, false}, u, outE, outAcc, outF);
-                }
+                tally(s_hist, a.B, st.acc, st.F);
+                if (outE) store_sample(u, st.acc, st.F, outE, outAcc, outF);
                 busy = false;
             }
         }
     }
     __syncthreads();
-    int32_t* row = hist_acc + size_t(blockIdx.x & 7u) * kMaxBins;
-    for (uint32_t i = lane; i < uint32_t(a.B); i += kWave) {
-        const int32_t v = s_hist[i];
-        if (v) atomicAdd(&row[i], v);
-    }
+    flush_hist(s_hist, hist_acc + size_t(blockIdx.x & 7u) * kMaxBins, a.B, lane);
 }
 
 // Threshold rows of the fast walk's binomial draws, one wave per (state,
@@ -329,48 +540,18 @@ __global__ __launch_bounds__(kWave * kFinishWaves) void finish_kernel(
 // call (src/gpuWorker.cpp:71-80); the units and their random streams are the
 // same as a single-set run with set id set_base + s * set_stride.
 
-__device__ __forceinline__ int e_bin(float acc, float F, int B) {
-    const float E = F > 0.0f ? acc / F : 0.0f;
-    if (!(E >= 0.0f && E < 1.0f)) return -1;
-    const int bin = int(floor(double(E) * double(B)));
-    return bin < B ? bin : -1;
-}
-
-// Adds an LDS histogram to its set's accumulator row of this XCD and clears it.
-__device__ __forceinline__ void flush_hist(int32_t* h, int32_t* __restrict__ hist_acc,
-                                           uint32_t set, uint32_t xrow, int B, uint32_t lane) {
-    int32_t* row = hist_acc + (size_t(set) * 8u + xrow) * size_t(B);
-    for (uint32_t i = lane; i < uint32_t(B); i += kWave) {
-        const int32_t v = h[i];
-        if (v) {
-            atomicAdd(&row[i], v);
-            h[i] = 0;
-        }
-    }
-}
-
-// Work is a flat list of batches: set s owns batches [s * bps, (s + 1) * bps),
-// each covering up to a.batch consecutive units of that set; the list is
-// dealt out to the a.queues work counters in turn (counter q hands out
-// batches q, q + queues, ...).  Sets differ in their dwell windows per unit by
-// up to two orders of magnitude: contiguous shares of the list gave whole
-// sets to a counter, whose waves (only they take from it) were still walking
-// when the others had ended (64 sets of fast dynamics: 3.6 of 7 waves per
-// SIMD busy over the launch; dealt out: 6.6).  A wave's lanes may be walking
-// units of two sets at once: the
-// workgroup keeps two LDS model slots with an LDS histogram each, and a wave
-// moves to a third set only after the older slot's lanes have finished, so it
-// never drains to change sets.
-// kGuided (fast form): binomial draws from the sets' threshold rows (guide),
-// else by the inversion loop from each set's BinomTable.
-template <int kPass, bool kGuided>
-__global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(
-    kPass == kPassFast ? kPopFastWavesPerEU : 1))) void pop_walk_kernel(
+// The general form over every (set, unit) of a population with distance
+// broadening.  Work is a flat list of batches: set s owns batches
+// [s * bps, (s + 1) * bps), each covering up to a.batch consecutive units of
+// that set; the list is dealt out to a.queues counters in turn
+// (pop_queue_length).  A wave's lanes may be walking units of two sets
+// at once: the workgroup keeps two LDS model slots with an LDS histogram
+// each, and a wave moves to a third set only after the older slot's lanes
+// have finished, so it never drains to change sets.
+__global__ __launch_bounds__(kWave) void pop_walk_kernel(
     const BurstDesc* __restrict__ bursts, const uint32_t* __restrict__ ticks,
     const uint2* __restrict__ links, const PopControl* __restrict__ ctl,
-    const ModelBlob* __restrict__ blobs, const BinomGuide guide, const RunArgs a,
-    int32_t* __restrict__ hist_acc,
-    uint64_t* __restrict__ replay, uint32_t* __restrict__ replay_count,
+    const ModelBlob* __restrict__ blobs, const RunArgs a, int32_t* __restrict__ hist_acc,
     uint32_t* __restrict__ work) {
     __shared__ Model sM[2];
     extern __shared__ int32_t s_hist[];  // [2][a.B]
@@ -378,21 +559,19 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(
     for (uint32_t i = lane; i < 2u * uint32_t(a.B); i += kWave) s_hist[i] = 0;
     __syncthreads();
 
-    constexpr bool kFastForm = kPass == kPassFast;
     const uint32_t seed = ctl->seed, set_base = ctl->set_base, set_stride = ctl->set_stride;
     const uint32_t queue = blockIdx.x % a.queues;
-    const uint32_t nb = a.nsets * a.bps;
-    const uint32_t q_len = nb > queue ? (nb - queue + a.queues - 1u) / a.queues : 0u;
+    const uint32_t q_len = pop_queue_length(a.nsets * a.bps, queue, a.queues);
     const uint32_t xrow = blockIdx.x & 7u;
     int set0 = -1, set1 = -1;    // wave-uniform: the set each LDS slot holds
     uint32_t cur = 0;            // slot that receives new units
     uint32_t pool_set = 0, pool_next = 0, pool_end = 0;
     bool busy = false;
-    uint32_t my_slot = 0, my_set = 0, u = 0;
-    WalkState<kFastForm> st{};
+    uint32_t my_slot = 0;
+    WalkState<false> st{};
     UnitKey key{seed, 0u, 0u, 0u};
     BurstDesc d{0u, 0u, 0u, 0.0f};
-    const UnitDiv divR = make_unit_div(a.R);
+    const UnitDiv divR{a.div_m, a.div_sh};
     bool drained = false;
     while (true) {
         bool need = !busy;
@@ -417,8 +596,8 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(
                 if (__any(busy && my_slot == other)) break;  // the older set is still walking
                 const int old = other ? set1 : set0;
                 if (old >= 0)
-                    flush_hist(s_hist + other * uint32_t(a.B), hist_acc, uint32_t(old), xrow,
-                               a.B, lane);
+                    flush_hist(s_hist + other * uint32_t(a.B),
+                               hist_acc + (size_t(old) * 8u + xrow) * size_t(a.B), a.B, lane);
                 const uint32_t* src = reinterpret_cast<const uint32_t*>(&blobs[pool_set].m);
                 uint32_t* dst = reinterpret_cast<uint32_t*>(&sM[other]);
                 for (uint32_t i = lane; i < sizeof(Model) / 4; i += kWave) dst[i] = src[i];
@@ -427,25 +606,22 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(
                 else set0 = int(pool_set);
                 cur = other;
             }
-            const uint32_t rank = __builtin_amdgcn_mbcnt_hi(
-                uint32_t(want >> 32), __builtin_amdgcn_mbcnt_lo(uint32_t(want), 0u));
+            const uint32_t rank = lanes_below(want);
             const uint32_t avail = pool_end - pool_next;
             if (need && rank < avail) {
-                u = pool_next + rank;
+                const uint32_t u = pool_next + rank;
                 my_slot = cur;
-                my_set = pool_set;
                 const uint32_t bl = unit_div(u, divR);
                 const uint32_t b = a.begin + bl;
                 d = bursts[b];
-                key.set = set_base + my_set * set_stride;
+                key.set = set_base + pool_set * set_stride;
                 key.r = u - bl * a.R;
                 key.b = b;
-                if (begin_unit<kFastForm>(sM[my_slot], key, d.P, d.T, st) == kStepMore) {
+                if (begin_unit<false>(sM[my_slot], key, d.P, d.T, st) == kStepMore) {
                     busy = true;
                     need = false;
                 } else {
-                    const int bin = e_bin(0.0f, 0.0f, a.B);
-                    if (bin >= 0) atomicAdd(&s_hist[my_slot * uint32_t(a.B) + uint32_t(bin)], 1);
+                    tally(s_hist + my_slot * uint32_t(a.B), a.B, 0.0f, 0.0f);
                 }
             }
             const uint32_t taken = uint32_t(__popcll(want));
@@ -453,33 +629,20 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(
         }
         if (!__any(busy)) break;
         if (busy) {
-            int r;
-            if (kGuided) {
-                const size_t base = size_t(sM[my_slot].guide_base);
-                const BinomGuide g{guide.thr + base * kGuideStatePairs,
-                                   guide.guide + base * kBinomTable * kGuideBuckets};
-                r = step_window<kFastForm, false, BinomGuide>(sM[my_slot], &g, key, d.P,
-                                                              d.stop_rel, d.T, ticks + d.off,
-                                                              links + d.off, a, st);
-            } else {
-                r = step_window<kFastForm>(sM[my_slot], &blobs[my_set].tab, key, d.P, d.stop_rel,
-                                           d.T, ticks + d.off, links + d.off, a, st);
-            }
+            const int r = general_window(sM[my_slot], key, d.P, d.stop_rel, d.T,
+                                         ticks + d.off, links + d.off, a, st);
             if (r != kStepMore) {
-                if (r == kStepReplay) {
-                    const uint32_t slot = atomicAdd(replay_count, 1u);
-                    if (slot < a.replay_cap) replay[slot] = (uint64_t(my_set) << 32) | u;
-                } else {
-                    const int bin = e_bin(st.acc, st.F, a.B);
-                    if (bin >= 0) atomicAdd(&s_hist[my_slot * uint32_t(a.B) + uint32_t(bin)], 1);
-                }
+                tally(s_hist + my_slot * uint32_t(a.B), a.B, st.acc, st.F);
                 busy = false;
             }
         }
     }
     __syncthreads();
-    if (set0 >= 0) flush_hist(s_hist, hist_acc, uint32_t(set0), xrow, a.B, lane);
-    if (set1 >= 0) flush_hist(s_hist + uint32_t(a.B), hist_acc, uint32_t(set1), xrow, a.B, lane);
+    if (set0 >= 0)
+        flush_hist(s_hist, hist_acc + (size_t(set0) * 8u + xrow) * size_t(a.B), a.B, lane);
+    if (set1 >= 0)
+        flush_hist(s_hist + uint32_t(a.B), hist_acc + (size_t(set1) * 8u + xrow) * size_t(a.B),
+                   a.B, lane);
 }
 
 // Recomputes abandoned (set, unit) pairs in the general form, one per lane,
@@ -500,8 +663,7 @@ __global__ __launch_bounds__(kWave) void pop_replay_kernel(
         const UnitKey key{ctl->seed, ctl->set_base + set * ctl->set_stride, u - bl * a.R, b};
         const WalkOut o = walk_unit<false>(blobs[set].m, nullptr, key, d.P, d.stop_rel, d.T,
                                            ticks + d.off, links + d.off, a);
-        const int bin = e_bin(o.acc, o.F, a.B);
-        if (bin >= 0) atomicAdd(&hist_acc[size_t(set) * 8u * size_t(a.B) + uint32_t(bin)], 1);
+        tally(hist_acc + size_t(set) * 8u * size_t(a.B), a.B, o.acc, o.F);
     }
 }
 
@@ -807,34 +969,42 @@ __global__ __launch_bounds__(kMbThreads) void microbench_kernel(int iters, float
 
 // ---- launchers (called by the C-ABI layer) ---------------------------------
 
-hipError_t walk_occupancy(int pass, int* blocks_per_cu) {
+hipError_t walk_occupancy(int pass, int B, int* blocks_per_cu) {
+    const size_t lds = sizeof(int32_t) * size_t(B);
     if (pass == kPassFast)
-        return hipOccupancyMaxActiveBlocksPerMultiprocessor(blocks_per_cu, walk_kernel<kPassFast>,
-                                                            kWave, 0);
+        return hipOccupancyMaxActiveBlocksPerMultiprocessor(
+            blocks_per_cu, fast_walk_kernel<false, true, false>, kWave, lds);
     if (pass == kPassReplay)
         return hipOccupancyMaxActiveBlocksPerMultiprocessor(blocks_per_cu,
-                                                            walk_kernel<kPassReplay>, kWave, 0);
+                                                            walk_kernel<kPassReplay>, kWave, lds);
     return hipOccupancyMaxActiveBlocksPerMultiprocessor(blocks_per_cu, walk_kernel<kPassGeneral>,
-                                                        kWave, 0);
+                                                        kWave, lds);
 }
 
 hipError_t launch_walk(int pass, uint32_t grid, const BurstDesc* bursts, const uint32_t* ticks,
                        const uint2* links, const ModelBlob* blob, const BinomGuide& guide,
-                       const RunArgs& a, int32_t* hist_acc, uint32_t* replay,
+                       const RunArgs& a, const FastArgs& fa, int32_t* hist_acc, uint32_t* replay,
                        uint32_t* replay_count, uint32_t* work, float* outE, int32_t* outAcc,
                        float* outF, hipStream_t stream) {
-    if (pass == kPassFast)
-        hipLaunchKernelGGL(walk_kernel<kPassFast>, dim3(grid), dim3(kWave), 0, stream, bursts,
-                           ticks, links, blob, guide, a, hist_acc, replay, replay_count, work, outE,
+    const size_t lds = sizeof(int32_t) * size_t(a.B);
+    if (pass == kPassFast) {
+        const FastIO io{bursts, ticks, links, blob, nullptr, guide, hist_acc, replay,
+                        replay_count, work, outE, outAcc, outF};
+        if (outE)
+            hipLaunchKernelGGL((fast_walk_kernel<false, true, true>), dim3(grid), dim3(kWave), lds,
+                               stream, io, a, fa);
+        else
+            hipLaunchKernelGGL((fast_walk_kernel<false, true, false>), dim3(grid), dim3(kWave),
+                               lds, stream, io, a, fa);
+    } else if (pass == kPassReplay) {
+        hipLaunchKernelGGL(walk_kernel<kPassReplay>, dim3(grid), dim3(kWave), lds, stream, bursts,
+                           ticks, links, blob, a, hist_acc, replay, replay_count, work, outE,
                            outAcc, outF);
-    else if (pass == kPassReplay)
-        hipLaunchKernelGGL(walk_kernel<kPassReplay>, dim3(grid), dim3(kWave), 0, stream, bursts,
-                           ticks, links, blob, guide, a, hist_acc, replay, replay_count, work, outE,
+    } else {
+        hipLaunchKernelGGL(walk_kernel<kPassGeneral>, dim3(grid), dim3(kWave), lds, stream, bursts,
+                           ticks, links, blob, a, hist_acc, replay, replay_count, work, outE,
                            outAcc, outF);
-    else
-        hipLaunchKernelGGL(walk_kernel<kPassGeneral>, dim3(grid), dim3(kWave), 0, stream, bursts,
-                           ticks, links, blob, guide, a, hist_acc, replay, replay_count, work, outE,
-                           outAcc, outF);
+    }
     return hipGetLastError();
 }
 
@@ -857,29 +1027,28 @@ hipError_t pop_walk_occupancy(int pass, int B, int* blocks_per_cu) {
     const size_t lds = sizeof(int32_t) * 2u * size_t(B);
     if (pass == kPassFast)
         return hipOccupancyMaxActiveBlocksPerMultiprocessor(
-            blocks_per_cu, pop_walk_kernel<kPassFast, true>, kWave, lds);
-    return hipOccupancyMaxActiveBlocksPerMultiprocessor(
-        blocks_per_cu, pop_walk_kernel<kPassGeneral, false>, kWave, lds);
+            blocks_per_cu, fast_walk_kernel<true, true, false>, kWave, lds);
+    return hipOccupancyMaxActiveBlocksPerMultiprocessor(blocks_per_cu, pop_walk_kernel, kWave,
+                                                        lds);
 }
 
 hipError_t launch_pop_walk(int pass, uint32_t grid, const BurstDesc* bursts,
                            const uint32_t* ticks, const uint2* links, const PopControl* ctl,
                            const ModelBlob* blobs, const BinomGuide& guide, const RunArgs& a,
-                           int32_t* hist_acc, uint64_t* replay, uint32_t* replay_count,
-                           uint32_t* work, hipStream_t stream) {
+                           const FastArgs& fa, int32_t* hist_acc, uint64_t* replay,
+                           uint32_t* replay_count, uint32_t* work, hipStream_t stream) {
     const size_t lds = sizeof(int32_t) * 2u * size_t(a.B);
+    const FastIO io{bursts, ticks, links, blobs, ctl, guide, hist_acc, replay,
+                    replay_count, work, nullptr, nullptr, nullptr};
     if (pass == kPassFast && guide.thr)
-        hipLaunchKernelGGL((pop_walk_kernel<kPassFast, true>), dim3(grid), dim3(kWave), lds,
-                           stream, bursts, ticks, links, ctl, blobs, guide, a, hist_acc, replay,
-                           replay_count, work);
+        hipLaunchKernelGGL((fast_walk_kernel<true, true, false>), dim3(grid), dim3(kWave), lds,
+                           stream, io, a, fa);
     else if (pass == kPassFast)
-        hipLaunchKernelGGL((pop_walk_kernel<kPassFast, false>), dim3(grid), dim3(kWave), lds,
-                           stream, bursts, ticks, links, ctl, blobs, guide, a, hist_acc, replay,
-                           replay_count, work);
+        hipLaunchKernelGGL((fast_walk_kernel<true, false, false>), dim3(grid), dim3(kWave), lds,
+                           stream, io, a, fa);
     else
-        hipLaunchKernelGGL((pop_walk_kernel<kPassGeneral, false>), dim3(grid), dim3(kWave), lds,
-                           stream, bursts, ticks, links, ctl, blobs, guide, a, hist_acc, replay,
-                           replay_count, work);
+        hipLaunchKernelGGL(pop_walk_kernel, dim3(grid), dim3(kWave), lds, stream, bursts, ticks,
+                           links, ctl, blobs, a, hist_acc, work);
     return hipGetLastError();
 }
 

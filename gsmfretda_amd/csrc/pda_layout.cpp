@@ -160,6 +160,7 @@ int build_model(const Photophysics& s, int n, const float* args, int nargs, Mode
     M.gmx = s.gamma - s.crosstalk;
     M.omdd = 1.0f - s.dexdir;
     M.r0 = s.r0;
+    M.quick_rates = 1;
     // P_i2j column s, without the diagonal, as running sums (drawJ_Si2Sj)
     for (int st = 0; st < n; ++st) {
         float sum = 0.0f;
@@ -171,7 +172,14 @@ int build_model(const Photophysics& s, int n, const float* args, int nargs, Mode
             run += K[to + st * n] / sum;
             M.nscum[st][jj] = run;
         }
-        for (int j = 0; j < n; ++j) M.krate[st][j] = K[j + st * n];
+        for (int jj = n - 2; jj < kMaxStates; ++jj) M.nscum[st][jj] = INFINITY;
+        for (int j = 0; j < n; ++j) {
+            const float k = K[j + st * n];
+            M.krate[st][j] = k;
+            M.kdiv[st][j][0] = -k;
+            M.kdiv[st][j][1] = 1.0f / -k;
+            if (j != st && !quotient_range(k)) M.quick_rates = 0;
+        }
     }
     // genMatP's unnormalised inflow (diagonal added then removed), running sums
     float run = 0.0f;

@@ -151,6 +151,49 @@ PDA_HD float flog(float x) {
     return e * 0x1.62ep-1f - ((half_f2 - (s * (half_f2 + R) + e * 0x1.0bfbe8p-15f)) - f);
 }
 
+// flog(uniform24(x)): the same operations on the same values, without the
+// cases a uniform in (0, 1] does not have.  The exponent and the reduced
+// mantissa come from the integer (x >> 8) + 1, whose float is the uniform
+// times 2^24; the carry of the added constant is flog's comparison with
+// sqrt(2).  The division f / (2 + f) is the correctly rounded sequence of the
+// compiler's own, without the scaling it needs outside 2^+-96 (f is 0 or at
+// least 2^-24 in magnitude, 2 + f lies in (1.7, 2.42)).
+PDA_HD float flog_uniform24(uint32_t x) {
+    const uint32_t bits = fbits(float((x >> 8) + 1u)) + (0x3f800000u - 0x3f3504f4u);
+    const float e = float(int32_t(bits >> 23) - (127 + 24));
+    const float f = bitsf((bits & 0x007FFFFFu) + 0x3f3504f4u) - 1.0f;
+    const float b = 2.0f + f;
+#ifdef __HIP_DEVICE_COMPILE__
+    float r = __builtin_amdgcn_rcpf(b);
+    r = fmaf(fmaf(-b, r, 1.0f), r, r);
+    float s = f * r;
+    s = fmaf(fmaf(-b, s, f), r, s);
+    s = fmaf(fmaf(-b, s, f), r, s);
+#else
+    const float s = f / b;
+#endif
+    const float z = s * s;
+    float poly = fmaf(z, 0x1.c71c72p-3f, 0x1.24924ap-2f);
+    poly = fmaf(z, poly, 0x1.99999ap-2f);
+    poly = fmaf(z, poly, 0x1.555556p-1f);
+    const float R = z * poly;
+    const float half_f2 = 0.5f * f * f;
+    return e * 0x1.62ep-1f - ((half_f2 - (s * (half_f2 + R) + e * 0x1.0bfbe8p-15f)) - f);
+}
+
+// a / b, correctly rounded, with rb = 1 / b rounded to float: a first
+// quotient within 2 ulp, a correction that leaves it within one, and the
+// final one, whose remainder is exact and which therefore rounds as the
+// division does (Markstein, "Computation of elementary functions on the IBM
+// RISC System/6000 processor", 1990).  b within quotient_range and a quotient
+// that neither underflows nor overflows; an infinite one comes out NaN.
+PDA_HD float quotient(float a, float b, float rb) {
+    float q = a * rb;
+    q = fmaf(fmaf(-b, q, a), rb, q);
+    return fmaf(fmaf(-b, q, a), rb, q);
+}
+PDA_HD bool quotient_range(float b) { return b >= 0x1p-40f && b <= 0x1p40f; }
+
 PDA_HD float pow2f(int k) { return bitsf(uint32_t(k + 127) << 23); }
 
 PDA_HD float fexp(float x) {
@@ -169,6 +212,26 @@ PDA_HD float fexp(float x) {
     const int k = int(kf);
     const int ka = k / 2;
     return (e * pow2f(ka)) * pow2f(k - ka);
+}
+
+// fexp(-lam) for lam in [0, 64]: one scaling, whose result is normal and
+// therefore the exact multiple that fexp's two scalings give.
+PDA_HD float fexp_minus(float lam) {
+    const float x = -lam;
+    const float kf = floorf(x * 0x1.715476p+0f + 0.5f);
+    const float r = (x - kf * 0x1.62ep-1f) - kf * 0x1.0bfbe8p-15f;
+    float e = fmaf(r, 0x1.a01a02p-13f, 0x1.6c16c2p-10f);
+    e = fmaf(r, e, 0x1.111112p-7f);
+    e = fmaf(r, e, 0x1.555556p-5f);
+    e = fmaf(r, e, 0x1.555556p-3f);
+    e = fmaf(r, e, 0.5f);
+    e = fmaf(r, e, 1.0f);
+    e = fmaf(r, e, 1.0f);
+#ifdef __HIP_DEVICE_COMPILE__
+    return __builtin_amdgcn_ldexpf(e, int(kf));
+#else
+    return e * pow2f(int(kf));
+#endif
 }
 
 PDA_HD double dlog(double x) {

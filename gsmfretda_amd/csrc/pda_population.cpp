@@ -34,7 +34,7 @@ bool PopGraphKey::operator==(const PopGraphKey& o) const {
            queues == o.queues && replay_cap == o.replay_cap && clk_p == o.clk_p &&
            bg_ad == o.bg_ad && bg_dd == o.bg_dd && bursts == o.bursts && ticks == o.ticks &&
            links == o.links && data_gen == o.data_gen && obs == o.obs && guided == o.guided &&
-           max_states == o.max_states && thr == o.thr;
+           max_states == o.max_states && quick_rates == o.quick_rates && thr == o.thr;
 }
 
 void drop_graph(Population& p) {
@@ -145,7 +145,8 @@ int enqueue_population(pda_ctx* ctx, Slot& s, int pass, uint32_t grid, const Run
         guide = BinomGuide{p.d_thr, p.d_guide};
     }
     HIP_TRY(launch_pop_walk(pass, grid, ctx->d_bursts, ctx->d_ticks, ctx->d_links, ctl, blobs,
-                            guide, a, p.d_hist_acc, p.d_replay, p.d_replay_count, p.d_work,
+                            guide, a, fast_args(p.max_states, p.quick_rates, a.clk_p),
+                            p.d_hist_acc, p.d_replay, p.d_replay_count, p.d_work,
                             s.stream));
     if (pass == 0)
         HIP_TRY(launch_pop_replay(ctx->d_bursts, ctx->d_ticks, ctx->d_links, ctl, blobs, a,
@@ -215,6 +216,7 @@ int run_population(pda_ctx* ctx, Slot& s, int R, uint32_t seed, uint32_t set_bas
     a.replay_cap = uint32_t(std::min<size_t>(p.replay_cap, 0xFFFFFFFFu));
     a.nsets = uint32_t(p.nsets);
     a.bps = uint32_t(bps);
+    plan_args(a, bps * uint64_t(p.nsets), 1u);
     const uint32_t grid = units > 0 ? L.grid : 1u;
 
     // the generation's stream keys travel with its models
@@ -250,6 +252,7 @@ int run_population(pda_ctx* ctx, Slot& s, int R, uint32_t seed, uint32_t set_bas
         k.obs = ctx->d_obs;
         k.guided = pass == 0 && p.guided;
         k.max_states = p.max_states;
+        k.quick_rates = p.quick_rates;
         k.thr = p.d_thr;
         if (!p.exec || !(k == p.key)) {
             drop_graph(p);
@@ -318,13 +321,14 @@ int pda_set_population(pda_ctx* ctx, int sid, int nsets, const int32_t* nstates,
     Population& p = s->pop;
     // validate and build every set before touching the slot
     std::vector<Model> models(static_cast<size_t>(nsets));
-    bool any_v = false;
+    bool any_v = false, quick_rates = true;
     for (int i = 0; i < nsets; ++i) {
         std::string err;
         const int n = nstates[i];
         const int rc = build_model(s->ph, n, args + off[size_t(i)], n * (n + 1), models[size_t(i)], err);
         if (rc) return fail(rc, "set %d: %s", i, err.c_str());
         any_v = any_v || models[size_t(i)].any_v != 0;
+        quick_rates = quick_rates && models[size_t(i)].quick_rates != 0;
     }
     HIP_TRY(hipStreamSynchronize(s->stream));
     p.in_flight = false;
@@ -375,6 +379,7 @@ int pda_set_population(pda_ctx* ctx, int sid, int nsets, const int32_t* nstates,
     p.args.assign(args, args + nargs_total);
     p.off = off;
     p.any_v = any_v;
+    p.quick_rates = quick_rates;
     return PDA_OK;
 }
 
@@ -479,7 +484,7 @@ int pda_autotune(pda_ctx* ctx, int sid, int population, int R, int reps, int* ba
     if (rc) return rc;
     int per_cu = 0;
     const int pass = population ? (s->pop.any_v ? 2 : 0) : (s->any_v ? 2 : 0);
-    HIP_TRY(population ? pop_walk_occupancy(pass, ctx->B, &per_cu) : walk_occupancy(pass, &per_cu));
+    HIP_TRY(population ? pop_walk_occupancy(pass, ctx->B, &per_cu) : walk_occupancy(pass, ctx->B, &per_cu));
     if (per_cu < 1) per_cu = 1;
     const LaunchShape saved = ctx->shape;
     auto time_shape = [&](const LaunchShape& sh, float* out) -> int {

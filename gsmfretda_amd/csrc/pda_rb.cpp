@@ -396,6 +396,7 @@ int rb_enqueue_forward(pda_ctx* ctx, Slot& s, RbState& r, const Model& M,
     const uint32_t grid = uint32_t(std::max<uint64_t>(1, std::min(max_grid, (uint64_t(units) + batch - 1) / batch)));
     a.batch = uint32_t(batch);
     a.queues = std::min<uint32_t>(ctx->shape.queues ? ctx->shape.queues : kDefaultQueues, grid);
+    plan_args(a, uint64_t(units), kWave);
     PassShape ps;
     if (int rc = pass_shape(ctx, 0, n, false, a.B, cap, a.nunits, ps)) return rc;
     RunArgs la = a;
@@ -431,7 +432,8 @@ int rb_enqueue_forward(pda_ctx* ctx, Slot& s, RbState& r, const Model& M,
     HIP_TRY(launch_rb_memo(n, d_rbm, r.d_pmf_tab, ML.d_list, ML.nvec, r.d_poolP, s.rb_aux));
     HIP_TRY(hipEventRecord(s.rb_join, s.rb_aux));
     HIP_TRY(launch_rb_walk(scores, n, grid, uint32_t(ctx->num_cu) * 4u, ctx->d_bursts, ctx->d_ticks,
-                           ctx->d_links, d_blob, d_rbm, a, r.d_cnt, r.d_F, r.d_S, r.d_work,
+                           ctx->d_links, d_blob, d_rbm, a,
+                           fast_args(n, M.quick_rates != 0, a.clk_p), r.d_cnt, r.d_F, r.d_S, r.d_work,
                            r.d_big, r.d_huge, r.d_big_count, r.d_replay, r.d_replay_count,
                            s.stream));
     HIP_TRY(hipEventRecord(r.ev_walk, s.stream));

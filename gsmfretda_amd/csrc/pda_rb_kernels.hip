@@ -161,7 +161,8 @@ template <bool kScores, int kN>
 __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(7))) void rb_walk_kernel(
     const BurstDesc* __restrict__ bursts, const uint32_t* __restrict__ ticks,
     const uint2* __restrict__ links, const ModelBlob* __restrict__ blob,
-    const RbModel* __restrict__ rbm, const RunArgs a, uint2* __restrict__ cnt_out,
+    const RbModel* __restrict__ rbm, const RunArgs a, const FastArgs fa,
+    uint2* __restrict__ cnt_out,
     float* __restrict__ F_out, float* __restrict__ S_out, uint32_t* __restrict__ work,
     uint32_t* __restrict__ big, uint32_t* __restrict__ huge, uint32_t* __restrict__ big_count,
     uint32_t* __restrict__ replay, uint32_t* __restrict__ replay_count) {
@@ -180,15 +181,16 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(7))) void
     RbAcc<kN, kScores> acc;
 
     const uint32_t queue = blockIdx.x % a.queues;
-    const uint32_t q_begin = uint32_t(uint64_t(a.nunits) * queue / a.queues);
-    const uint32_t q_end = uint32_t(uint64_t(a.nunits) * (queue + 1u) / a.queues);
+    const uint64_t q_first = uint64_t(queue) * a.q_share;
+    const uint32_t q_begin = q_first < a.nunits ? uint32_t(q_first) : a.nunits;
+    const uint32_t q_end = a.nunits - q_begin < a.q_share ? a.nunits : q_begin + a.q_share;
     uint32_t pool_next = 0, pool_end = 0;
     bool busy = false;
     uint32_t u = 0;
     WalkState<true> st{};
     UnitKey key{a.seed, a.set, 0u, 0u};
     BurstDesc d{0u, 0u, 0u, 0.0f};
-    const UnitDiv divR = make_unit_div(a.R);
+    const UnitDiv divR{a.div_m, a.div_sh};
     bool drained = false;
     while (true) {
         bool need = !busy;
@@ -230,8 +232,8 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(7))) void
         if (!__any(busy)) break;
         if (busy) {
             WindowInfo wi;
-            const int r = step_window<true, true>(sM, nullptr, key, d.P, d.stop_rel, d.T,
-                                                  ticks + d.off, links + d.off, a, st, &wi);
+            const int r = fast_window<true>(sM, nullptr, key, d.P, d.stop_rel, d.T, ticks + d.off,
+                                            links + d.off, a, fa, st, &wi);
             if (r == kStepReplay) {
                 replay[atomicAdd(replay_count, 1u)] = u;
                 busy = false;
@@ -287,8 +289,8 @@ __global__ __launch_bounds__(kWave) void rb_replay_kernel(
             int r = begin_unit<false>(sM, key, d.P, d.T, st);
             while (r == kStepMore) {
                 WindowInfo wi;
-                r = step_window<false, true>(sM, nullptr, key, d.P, d.stop_rel, d.T,
-                                             ticks + d.off, links + d.off, a, st, &wi);
+                r = general_window<true>(sM, key, d.P, d.stop_rel, d.T, ticks + d.off,
+                                         links + d.off, a, st, &wi);
                 acc.absorb(sR, wi);
             }
             acc.store(u, st.F, lane, cnt_out, F_out, S_out, big, huge, big_count);
@@ -1074,12 +1076,12 @@ hipError_t rb_big_occupancy(int mode, bool wide, int dyn_lds, int* per_cu) {
 template <bool kScores, int kN>
 static void launch_rb_walk_n(uint32_t grid, uint32_t replay_grid, const BurstDesc* bursts,
                              const uint32_t* ticks, const uint2* links, const ModelBlob* blob,
-                             const RbModel* rbm, const RunArgs& a, uint2* cnt, float* F, float* S,
-                             uint32_t* work, uint32_t* big, uint32_t* huge, uint32_t* big_count,
+                             const RbModel* rbm, const RunArgs& a, const FastArgs& fa, uint2* cnt,
+                             float* F, float* S, uint32_t* work, uint32_t* big, uint32_t* huge, uint32_t* big_count,
                              uint32_t* replay, uint32_t* replay_count, hipStream_t stream) {
     hipLaunchKernelGGL((rb_walk_kernel<kScores, kN>), dim3(grid), dim3(kWave), 0, stream, bursts,
-                       ticks, links, blob, rbm, a, cnt, F, S, work, big, huge, big_count, replay,
-                       replay_count);
+                       ticks, links, blob, rbm, a, fa, cnt, F, S, work, big, huge, big_count,
+                       replay, replay_count);
     hipLaunchKernelGGL((rb_replay_kernel<kScores, kN>), dim3(replay_grid), dim3(kWave), 0, stream,
                        bursts, ticks, links, blob, rbm, a, cnt, F, S, big, huge, big_count, replay,
                        replay_count);
@@ -1087,13 +1089,13 @@ static void launch_rb_walk_n(uint32_t grid, uint32_t replay_grid, const BurstDes
 
 hipError_t launch_rb_walk(bool scores, int n, uint32_t grid, uint32_t replay_grid,
                           const BurstDesc* bursts, const uint32_t* ticks, const uint2* links,
-                          const ModelBlob* blob, const RbModel* rbm, const RunArgs& a, uint2* cnt,
-                          float* F, float* S, uint32_t* work, uint32_t* big, uint32_t* huge,
-                          uint32_t* big_count, uint32_t* replay, uint32_t* replay_count,
-                          hipStream_t stream) {
+                          const ModelBlob* blob, const RbModel* rbm, const RunArgs& a,
+                          const FastArgs& fa, uint2* cnt, float* F, float* S, uint32_t* work,
+                          uint32_t* big, uint32_t* huge, uint32_t* big_count,
+                          uint32_t* replay, uint32_t* replay_count, hipStream_t stream) {
 #define PDA_RB_WALK(SC, N)                                                                    \
-    launch_rb_walk_n<SC, N>(grid, replay_grid, bursts, ticks, links, blob, rbm, a, cnt, F, S,  \
-                            work, big, huge, big_count, replay, replay_count, stream)
+    launch_rb_walk_n<SC, N>(grid, replay_grid, bursts, ticks, links, blob, rbm, a, fa, cnt, F, \
+                            S, work, big, huge, big_count, replay, replay_count, stream)
     if (n < 2 || n > kRbMaxStates) return hipErrorInvalidValue;
     if (scores) {
         if (n == 2) PDA_RB_WALK(true, 2);

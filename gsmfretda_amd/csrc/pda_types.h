@@ -55,8 +55,14 @@ struct Model {
     int32_t guide_base;
     float pad0;
     float p0cum[kMaxStates];                      // running sums of genMatP's inflow
-    float nscum[kMaxStates][kMaxStates];          // [s][jj] running sums of P_i2j column s
+    // [s][jj] running sums of P_i2j column s; the last of the n - 1 entries,
+    // which every draw past the others takes, and the rest are +inf
+    float nscum[kMaxStates][kMaxStates];
     float krate[kMaxStates][kMaxStates];          // [s][j] = K(j, s), rate s -> j
+    // [s][j]: -K(j, s) and its reciprocal rounded to float (quotient())
+    float kdiv[kMaxStates][kMaxStates][2];
+    int32_t quick_rates;          // every rate within quotient()'s range
+    int32_t pad1;
     float v[kMaxStates];
     float base[kMaxStates];                       // r0 (1/E - 1)^(1/6)
     float ep0[kMaxStates];                        // broadened E when v == 0
@@ -119,6 +125,9 @@ struct RunArgs {
     uint32_t replay_cap; // capacity of the replay list
     uint32_t nsets;      // population runs: parameter sets
     uint32_t bps;        // population runs: work batches per set
+    // derived by plan_args: floor(u / R) as (u div_m) >> div_sh (UnitDiv of
+    // R), and the work items (units; population runs: batches) of a queue
+    uint32_t div_m, div_sh, q_share;
 };
 
 // Device result of one run, followed by int32 hist[B].

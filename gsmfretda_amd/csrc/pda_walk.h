@@ -212,47 +212,30 @@ struct NoDeduce {
 // divisions by 1 and 2 are exact (the identity and a power-of-two scaling),
 // so pk * lam and (pk * lam) * 0.5 round to the loop's values; the loop then
 // continues from k = 3 only for the lanes whose uniform lies beyond the
-// cumulative probability of 2 photons, so a wave no longer runs the loop as
-// often as its longest draw needs.
+// cumulative probability of 2 photons and whose cap allows it, so a wave no
+// longer runs the loop as often as its longest draw needs.  (The cumulative
+// sums do not decrease, so a uniform beyond one is beyond those before; a
+// mean of 0 or less has exp(0) = 1, which no uniform exceeds.)
 PDA_HD float background_single(float lam, float cap, float u_first, float u_cap) {
     if (lam > 64.0f || !(cap < 0x1p30f)) return -1.0f;
-    int32_t k = 0;
-    bool over = false;
-    if (lam > 0.0f) {
-        const float pk0 = fexp(-lam);
-        const float pk1 = pk0 * lam;
-        const float cdf1 = pk0 + pk1;
-        const float pk2 = (pk1 * lam) * 0.5f;
-        const float cdf2 = cdf1 + pk2;
-        float pk = pk0, cdf = pk0;
-        bool go = u_first > pk0;
-        if (go) {  // k = 1
-            k = 1;
-            over = 1.0f > cap;
-            pk = pk1;
-            cdf = cdf1;
-            go = !over && u_first > cdf1;
-        }
-        if (go) {  // k = 2
-            k = 2;
-            over = 2.0f > cap;
-            pk = pk2;
-            cdf = cdf2;
-            go = !over && u_first > cdf2;
-        }
-        while (go) {
-            ++k;
-            if (float(k) > cap) {
-                over = true;
-                break;
-            }
+    lam = fmaxf(lam, 0.0f);
+    const float pk0 = fexp_minus(lam);
+    const float pk1 = pk0 * lam;
+    const float cdf1 = pk0 + pk1;
+    const float pk2 = (pk1 * lam) * 0.5f;
+    const float cdf2 = cdf1 + pk2;
+    int32_t k = (u_first > pk0 ? 1 : 0) + (u_first > cdf1 ? 1 : 0);
+    if (u_first > cdf2) {
+        k = 3;
+        float pk = pk2, cdf = cdf2;
+        while (float(k) <= cap) {
             pk = (pk * lam) / float(k);
             cdf = cdf + pk;
-            go = u_first > cdf;
+            if (!(u_first > cdf)) break;
+            ++k;
         }
     }
-    if (!over && float(k) <= cap) return float(k);
-    return floorf(cap * u_cap);
+    return float(k) <= cap ? float(k) : floorf(cap * u_cap);
 }
 
 // Walk state of one unit between windows.  The fast form keeps the window
@@ -301,18 +284,33 @@ PDA_HD int begin_unit(const Model& M, const UnitKey& key, uint32_t P, float T,
     return kStepMore;
 }
 
-// One dwell window of the walk (one pass of the while loop, src/mc.cu:117-191).
-// tick/link point at the burst's photons in LDS or in global memory.
-// kCounts (general form only): no acceptor draw; the window is described in
-// *wi instead, for the Rao-Blackwellised form that sums the binomial pmf.
-// Tab: BinomTable (inversion loop) or BinomGuide (thresholds) for the fast
-// form's binomial draw; unused by the general form.
-template <bool kFast, bool kCounts = false, class Tab = BinomTable>
-PDA_HD int step_window(const Model& M, const typename NoDeduce<Tab>::type* tab, const UnitKey& key,
-                       uint32_t P,
-                       uint32_t stop_rel, float T, const uint32_t* tick, const uint2* link,
-                       const RunArgs& a, WalkState<kFast>& st, WindowInfo* wi = nullptr) {
-    using Tick = typename WalkState<kFast>::Tick;
+// Where a window that ends at tick w1 closes: the first channel photon at or
+// after w1 (photons in neither channel carry its tick, the links its index),
+// else the last photon.  A bound past the last but one is the last photon
+// whatever its tick; c < last, as a unit whose cursor reaches it ends.
+PDA_HD uint32_t window_close(const uint32_t* tick, const uint2* link, uint32_t c, uint32_t last,
+                             uint32_t w1) {
+    uint32_t lo = c, hi = last;
+    while (lo < hi) {
+        const uint32_t mid = (lo + hi) >> 1;
+        if (tick[mid] < w1) lo = mid + 1u;
+        else hi = mid;
+    }
+    if (lo < last) {
+        const uint32_t f1 = link[lo].x & kIndexMask;
+        if (f1 < last) return f1;
+    }
+    return last;
+}
+
+// One dwell window of the walk (one pass of the while loop, src/mc.cu:117-191)
+// in the general form.  tick/link point at the burst's photons.
+// kCounts: no acceptor draw; the window is described in *wi instead, for the
+// Rao-Blackwellised form that sums the binomial pmf.
+template <bool kCounts = false>
+PDA_HD int general_window(const Model& M, const UnitKey& key, uint32_t P, uint32_t stop_rel,
+                          float T, const uint32_t* tick, const uint2* link, const RunArgs& a,
+                          WalkState<false>& st, WindowInfo* wi = nullptr) {
     const int n = M.n;
     const int s = st.s;
     const uint32_t w = st.w;
@@ -329,35 +327,17 @@ PDA_HD int step_window(const Model& M, const typename NoDeduce<Tab>::type* tab, 
     // dwell at the chosen transition's rate (drawTau, src/mc.cu:122)
     const float tau = flog(uniform24(A.w[1])) / (-M.krate[s][j]);
     const float tsum = st.tsum + tau;
-    Tick w1;
+    int64_t w1;
     uint32_t w1c;
     if (!(tsum < T)) {
-        w1 = Tick(stop_rel);
+        w1 = stop_rel;
         w1c = stop_rel;
     } else {
         const float wf = float(st.w0) + tsum / a.clk_p;  // src/mc.cu:132
-        if (kFast) {
-            if (wf >= 0x1p31f) return kStepReplay;
-            w1 = Tick(uint32_t(wf));
-            w1c = uint32_t(w1);
-        } else {
-            const int64_t w64 = wf >= 0x1p62f ? (int64_t(1) << 62) : int64_t(wf);
-            w1 = Tick(w64);
-            w1c = w64 <= 0 ? 0u : (w64 >= int64_t(kTickSentinel) ? kTickSentinel : uint32_t(w64));
-        }
+        w1 = wf >= 0x1p62f ? (int64_t(1) << 62) : int64_t(wf);
+        w1c = w1 <= 0 ? 0u : (w1 >= int64_t(kTickSentinel) ? kTickSentinel : uint32_t(w1));
     }
-    // window close: first channel photon at or after w1, else the last photon
-    uint32_t lo = st.c, hi = P;
-    while (lo < hi) {
-        const uint32_t mid = (lo + hi) >> 1;
-        if (tick[mid] < w1c) lo = mid + 1u;
-        else hi = mid;
-    }
-    uint32_t close = last;
-    if (lo < P) {
-        const uint32_t f1 = link[lo].x & kIndexMask;
-        if (f1 < close) close = f1;
-    }
+    const uint32_t close = window_close(tick, link, st.c, last, w1c);
     // sticky-flag count over [c, close) (src/mc.cu:171-180)
     const uint2 L = link[st.c];
     const uint32_t f = L.x & kIndexMask;
@@ -370,45 +350,19 @@ PDA_HD int step_window(const Model& M, const typename NoDeduce<Tab>::type* tab, 
     float m;
     if (!a.bg_on) {
         m = floorf(fv + 0.5f);
-    } else {  // background photons (src/mc.cu:153-166)
-        // A window's photons carry one colour, so one of the two capped
-        // draws has a cap of 0 and gives 0 whatever its uniforms are (k = 0,
-        // or past the cap with floor(0 u) = 0): only the other is made, on
-        // its channel's rate and words.  One exponential and one inversion
-        // loop per window instead of two, whose lanes had each waited for
-        // the other channel's (with two draws a 3-state evaluation of
-        // 100,000 bursts x 100 took 434 us and the 256-set generation
-        // 19.9 ms, with one 417 us and 19.1 ms; under a 30 kHz background
-        // 323 and 275 us).  (fv - bgd) - bga is fv - bg then, exactly.
+    } else {  // background photons (src/mc.cu:153-166), one channel's (see fast_window)
         const Block Bk = draw_block(key, w, kSubBackground);
-        float dt;
-        if (kFast) dt = float(int32_t(uint32_t(w1) - uint32_t(st.w0))) * a.clk_p;
-        else dt = float(int64_t(w1) - int64_t(st.w0)) * a.clk_p;
+        const float dt = float(w1 - st.w0) * a.clk_p;
         const bool donor = colour == 1u;
-        const float lam = dt * (donor ? a.bg_dd : a.bg_ad);
-        const float cap = donor ? M.gmx * nd : M.omdd * na;
-        const float u_first = uniform24(donor ? Bk.w[1] : Bk.w[0]);
-        const float u_cap = uniform24(donor ? Bk.w[3] : Bk.w[2]);
-        float bg;
-        if (kFast) {
-            bg = background_single(lam, cap, u_first, u_cap);
-            if (bg < 0.0f) return kStepReplay;
-        } else {
-            bg = background_count(lam, cap, u_first, u_cap, key, w,
-                                  donor ? kSubPoissonD : kSubPoissonA);
-        }
+        const float bg = background_count(
+            dt * (donor ? a.bg_dd : a.bg_ad), donor ? M.gmx * nd : M.omdd * na,
+            uniform24(donor ? Bk.w[1] : Bk.w[0]), uniform24(donor ? Bk.w[3] : Bk.w[2]), key, w,
+            donor ? kSubPoissonD : kSubPoissonA);
         m = floorf((fv - bg) + 0.5f);
     }
-    int64_t x;
+    int64_t x = 0;
     if (kCounts) {
-        x = 0;
-        wi->s = s;
-        wi->j = j;
-        wi->tau = tau;
-        wi->m = int32_t(m);
-    } else if (kFast) {
-        x = binomial_fast(int(m), s, M, *tab, A.w[2], A.w[3]);
-        if (x < 0) return kStepReplay;
+        *wi = WindowInfo{s, j, tau, int32_t(m)};
     } else {
         // broadened efficiency (drawE, src/gen_rand.cuh:63-68)
         float de;
@@ -433,6 +387,102 @@ PDA_HD int step_window(const Model& M, const typename NoDeduce<Tab>::type* tab, 
     return kStepMore;
 }
 
+// What the fast form needs besides the model, the same for every unit of a
+// launch: jumps = the largest state count - 2, the comparisons of the
+// next-state draw; quick: the rates and the tick length are in quotient()'s
+// range; clk_r: 1 / clk_p rounded to float.
+struct FastArgs {
+    int32_t jumps;
+    int32_t quick;
+    float clk_r;
+};
+PDA_HD FastArgs fast_args(int max_states, bool quick_rates, float clk_p) {
+    return FastArgs{max_states - 2, quick_rates && quotient_range(clk_p) ? 1 : 0, 1.0f / clk_p};
+}
+
+// The same window in the fast form (v = 0), the same values from fewer
+// operations; kStepReplay where the window needs the general form.  Tab:
+// BinomTable (inversion loop) or BinomGuide (thresholds) for the acceptor
+// draw.
+template <bool kCounts = false, class Tab = BinomTable>
+PDA_HD int fast_window(const Model& M, const typename NoDeduce<Tab>::type* tab, const UnitKey& key,
+                       uint32_t P, uint32_t stop_rel, float T, const uint32_t* tick,
+                       const uint2* link, const RunArgs& a, const FastArgs& fa,
+                       WalkState<true>& st, WindowInfo* wi = nullptr) {
+    const int s = st.s;
+    const uint32_t w = st.w;
+    const uint32_t last = P - 1u;
+    const Block A = draw_block(key, w, kSubMain);
+    // next state: the running sums do not decrease, so the first one above u
+    // comes after as many as are not above it (a rate sum of 0 makes them
+    // NaN, never above); the entries from n - 2 on are +inf
+    int j = 0;
+    if (fa.jumps > 0) {
+        const float u = uniform24(A.w[0]);
+        j = (M.nscum[s][0] > u ? 0 : 1) + (M.nscum[s][1] > u ? 0 : 1);
+        for (int i = 2; i < fa.jumps; ++i) j += M.nscum[s][i] > u ? 0 : 1;
+    }
+    j += j >= s ? 1 : 0;
+    const float lg = flog_uniform24(A.w[1]);
+    const float mk = M.kdiv[s][j][0];
+    const float tau = fa.quick ? quotient(lg, mk, M.kdiv[s][j][1]) : lg / mk;
+    const float tsum = st.tsum + tau;
+    uint32_t w1 = stop_rel;
+    if (tsum < T) {
+        const float ticks = fa.quick ? quotient(tsum, a.clk_p, fa.clk_r) : tsum / a.clk_p;
+        const float wf = float(st.w0) + ticks;
+        if (!(wf < 0x1p31f)) return kStepReplay;
+        w1 = uint32_t(wf);
+    }
+    const uint32_t close = window_close(tick, link, st.c, last, w1);
+    // the count of the one colour the window has (0 for a photon in both
+    // channels, whose run ends at itself)
+    const uint2 L = link[st.c];
+    const uint32_t f = L.x & kIndexMask;
+    const uint32_t e = L.y < close ? L.y : close;
+    const float cnt = float(e > f ? e - f : 0u);
+    const bool donor = (L.x >> 30) == 1u;
+    const float fv = (donor ? M.gmx : M.omdd) * cnt;
+    float m = fv;
+    if (a.bg_on) {
+        // Background photons (src/mc.cu:153-166).  The window's photons carry
+        // one colour, so one of the two capped draws has a cap of 0 and gives
+        // 0 whatever its uniforms are (k = 0, or past the cap with
+        // floor(0 u) = 0): only the other is made, on its channel's rate and
+        // words (the window leaves the fast form when either mean is above
+        // 64).  One exponential and one inversion
+        // loop per window instead of two, whose lanes had each waited for
+        // the other channel's (with two draws a 3-state evaluation of
+        // 100,000 bursts x 100 took 434 us and the 256-set generation
+        // 19.9 ms, with one 417 us and 19.1 ms; under a 30 kHz background
+        // 323 and 275 us).  (fv - bgd) - bga is fv - bg then, exactly.
+        const Block Bk = draw_block(key, w, kSubBackground);
+        const float dt = float(int32_t(w1 - st.w0)) * a.clk_p;
+        const float lam = dt * (donor ? a.bg_dd : a.bg_ad);
+        if (dt * fmaxf(a.bg_ad, a.bg_dd) > 64.0f) return kStepReplay;
+        const float bg = background_single(lam, fv, uniform24(donor ? Bk.w[1] : Bk.w[0]),
+                                           uniform24(donor ? Bk.w[3] : Bk.w[2]));
+        if (bg < 0.0f) return kStepReplay;
+        m = fv - bg;
+    }
+    m = floorf(m + 0.5f);
+    if (kCounts) {
+        *wi = WindowInfo{s, j, tau, int32_t(m)};
+    } else {
+        const int x = int(binomial_fast(int(m), s, M, *tab, A.w[2], A.w[3]));
+        if (x < 0) return kStepReplay;
+        st.acc += float(x);
+    }
+    st.F += fv;
+    st.tsum = tsum;
+    st.w0 = w1;
+    st.s = j;
+    st.c = close;
+    st.w = w + 1u;
+    if (close == last || !(T > tsum) || st.w >= kMaxWindows) return kStepDone;
+    return kStepMore;
+}
+
 // One (burst, resample) unit: the body of mc_kernel (src/mc.cu:92-196).
 template <bool kFast, class Tab = BinomTable>
 PDA_HD WalkOut walk_unit(const Model& M, const typename NoDeduce<Tab>::type* tab, const UnitKey& key,
@@ -440,8 +490,13 @@ PDA_HD WalkOut walk_unit(const Model& M, const typename NoDeduce<Tab>::type* tab
                          const uint2* link, const RunArgs& a) {
     WalkState<kFast> st;
     int r = begin_unit<kFast>(M, key, P, T, st);
-    while (r == kStepMore)
-        r = step_window<kFast, false, Tab>(M, tab, key, P, stop_rel, T, tick, link, a, st);
+    if constexpr (kFast) {
+        const FastArgs fa = fast_args(M.n, M.quick_rates != 0, a.clk_p);
+        while (r == kStepMore)
+            r = fast_window<false, Tab>(M, tab, key, P, stop_rel, T, tick, link, a, fa, st);
+    } else {
+        while (r == kStepMore) r = general_window(M, key, P, stop_rel, T, tick, link, a, st);
+    }
     return WalkOut{st.acc, st.F, r == kStepReplay};
 }
 
