@@ -432,8 +432,8 @@ int pda_run(pda_ctx* ctx, int sid, int R, uint32_t seed, uint32_t set_id, int fl
     a.bg_ad = ctx->bg_ad;
     a.bg_dd = ctx->bg_dd;
     a.nstates = s->n;
-    // general pass for broadening, else the fast pass and a replay pass
-    const int pass = s->any_v ? kPassGeneral : kPassFast;
+    // the fast form, then the general form over the units it abandoned
+    const int pass = s->any_v ? kPassBroad : kPassGuided;
     const Launch L = plan_launch(ctx, pass, false, uint64_t(nunits));
     const uint32_t grid = L.grid;
     a.batch = L.batch;
@@ -469,7 +469,7 @@ int pda_run(pda_ctx* ctx, int sid, int R, uint32_t seed, uint32_t set_id, int fl
         outAcc = s->d_acc;
         outF = s->d_F;
     }
-    if (pass == kPassFast && size_t(nunits) > s->replay_cap) {
+    if (size_t(nunits) > s->replay_cap) {
         HIP_TRY(hipStreamSynchronize(s->stream));
         (void)hipFree(s->d_replay);
         s->d_replay = nullptr;
@@ -480,12 +480,12 @@ int pda_run(pda_ctx* ctx, int sid, int R, uint32_t seed, uint32_t set_id, int fl
     a.replay_cap = uint32_t(s->replay_cap);
     HIP_TRY(hipEventRecord(s->ev0, s->stream));
     const BinomGuide guide{s->d_thr, s->d_guide};
-    const FastArgs fa = fast_args(s->n, s->quick_rates, a.clk_p);
+    const FastArgs fa = fast_args(s->n, s->quick_rates, a.clk_p, s->ph.r0);
     HIP_TRY(launch_walk(pass, grid, ctx->d_bursts, ctx->d_ticks, ctx->d_links, s->d_blob, guide, a,
                         fa, s->d_hist_acc, s->d_replay, s->d_replay_count, s->d_work, outE, outAcc,
                         outF, s->stream));
     HIP_TRY(hipEventRecord(s->ev_mid, s->stream));
-    if (pass == kPassFast && nunits > 0) {
+    if (nunits > 0) {
         // the abandoned units, in the general form over the whole GPU; the
         // grid is sized for the worst case and its unneeded workgroups exit
         // at once

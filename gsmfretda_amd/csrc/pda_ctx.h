@@ -51,10 +51,10 @@ struct PopGraphKey {
     const void* links = nullptr;
     uint64_t data_gen = 0;
     const void* obs = nullptr;
-    // binomial threshold rows: whether the walk reads them, the guide
-    // kernel's state count (also the walk's) and the table's buffer
-    bool guided = false;
+    // the guide kernel's state count (also the walk's), the table's buffer,
+    // and what else the walk takes from the sets
     int max_states = 0;
+    float r0 = 0.f;
     bool quick_rates = false;
     const void* thr = nullptr;
     bool operator==(const PopGraphKey& o) const;
@@ -67,6 +67,7 @@ struct Population {
     std::vector<int64_t> off;        // start of set s in args
     bool any_v = false;
     bool quick_rates = false;        // of every set
+    float r0 = 0.f;                  // photophysics the sets were built with
     size_t cap_sets = 0;             // allocated sets
     uint8_t* h_in = nullptr;         // pinned: PopControl + ModelBlob[cap_sets]
     uint8_t* d_in = nullptr;
@@ -163,7 +164,7 @@ struct Slot {
     // (guide_kernel, enqueued with every model upload)
     ThrPair* d_thr = nullptr;     // kGuideThrPairs
     uint8_t* d_guide = nullptr;   // kGuideBytes
-    bool any_v = false;           // broadening: the general pass walks every unit
+    bool any_v = false;           // broadening: efficiencies drawn per window
     uint32_t* d_replay = nullptr;  // units the fast pass abandoned
     uint32_t* d_replay_count = nullptr;
     uint32_t* d_work = nullptr;    // kWorkWords: work counters of the run, one per line
@@ -247,10 +248,6 @@ int noalloc_setup(int device);
 void free_rb(RbState& r);
 void free_rb_memo(pda_ctx* ctx);
 
-// Walk passes (pda_kernels.hip): fast form, general form over the replay
-// list, general form over every unit.
-constexpr int kPassFast = 0, kPassReplay = 1, kPassGeneral = 2;
-
 // Grid and batch of a walk launch over `units` work units.
 struct Launch {
     uint32_t grid = 1, batch = kWave, queues = 1;
@@ -274,7 +271,6 @@ hipError_t launch_guide(const ModelBlob* blobs, int nsets, int max_states, ThrPa
 hipError_t launch_finish(const RunArgs& a, const float* obs, int32_t* hist_acc,
                          uint32_t* replay_count, uint32_t* work, ResultHeader* result,
                          hipStream_t stream);
-// guide.thr == nullptr: the fast form draws binomials by the inversion loop
 hipError_t launch_pop_walk(int pass, uint32_t grid, const BurstDesc* bursts,
                            const uint32_t* ticks, const uint2* links, const PopControl* ctl,
                            const ModelBlob* blobs, const BinomGuide& guide, const RunArgs& a,

@@ -26,13 +26,6 @@
 
 namespace pda {
 
-// Which form a walk launch runs.
-enum Pass : int {
-    kPassFast = 0,     // fast form; abandoned units go to the replay list
-    kPassReplay = 1,   // general form over the units of the replay list
-    kPassGeneral = 2,  // general form for every unit (models with broadening)
-};
-
 // Work counters of a replay pass: one per XCD, on the counter lines after the
 // kMaxQueues lines of the walk (kAuxQueues of them).
 constexpr uint32_t kReplayQueues = 8;
@@ -105,14 +98,34 @@ __device__ __forceinline__ void flush_hist(int32_t* h, int32_t* __restrict__ row
 
 // ---- walk in the fast form --------------------------------------------------------
 //
-// The fast form of a run (one parameter set) or of a population's generation.
-// One-wave workgroups; every lane streams through units: one loop pass
-// advances each busy lane by a dwell window, and lanes whose unit ended take
-// another, so neither lanes nor waves wait for the longest unit.  Work is
-// handed out as in walk_kernel (population: pop_walk_kernel).
-// kPop: population (two LDS model slots with a histogram each); kGuided:
-// binomial draws from the threshold rows (else by the inversion loop, for
-// populations too large for a table of rows); kSamples: per-unit outputs.
+// The fast form of a run (one parameter set) or of a population's generation,
+// in one-wave workgroups.
+//
+// Work stealing at two levels.  A wave takes batches of consecutive units
+// from a work counter; its lanes take units from the batch as they need
+// them.  One loop pass advances every busy lane by one window, and a lane
+// whose unit ends starts another in the same pass, so lanes do not wait
+// for the wave's longest unit and waves do not wait for the grid's
+// slowest batch.  The units are split into a.queues contiguous ranges
+// with a counter each, every counter on its own 256-byte line (device-
+// scope atomics to one line serialise); workgroup g draws from queue
+// g % a.queues, so with a multiple of 8 queues each queue is served by
+// one XCD and its bursts stay in that XCD's L2.  Batches are small
+// (about six grabs per wave): the wave that grabs last still walks a
+// whole batch, so the batch sets the grid's tail.  Photons are read
+// through L1/L2.
+//
+// A population's work is a flat list of batches: set s owns batches
+// [s * bps, (s + 1) * bps), each covering up to a.batch consecutive units of
+// that set; the list is dealt out to the counters in turn (pop_queue_length).
+// A wave's lanes may be walking units of two sets at once: the workgroup keeps
+// two LDS model slots with an LDS histogram each, and a wave moves to a third
+// set only after the older slot's lanes have finished, so it never drains to
+// change sets.
+//
+// kPop: population (two LDS model slots with a histogram each); kPass: the
+// acceptor draw (kPassGuided, kPassTable, kPassBroad); kSamples: per-unit
+// outputs.
 //
 // Bound by VALU issue (at or above 95 % of the cycles), so what counts is the
 // instructions of fast_window: the window's arithmetic without the cases its
@@ -125,8 +138,14 @@ __device__ __forceinline__ void flush_hist(int32_t* h, int32_t* __restrict__ row
 // waves hide.  (Starting 64 units at a time and queueing in LDS those that
 // outlast their first window was slower: 14 % more instructions, the first
 // window's close running for half of the lanes.)
-constexpr int kFastWavesPerEU = 8;
-constexpr int kPopFastWavesPerEU = 7;
+// The draw of a broadened efficiency and its binomial (kPassBroad) need up to
+// 77 registers.  They had been the general form's, at 186 registers and two
+// waves per SIMD with logarithms, exponentials and divisions in double per
+// window: 50,000 bursts x 50 of a 3-state model 371 -> 197 us, 64 sets x
+// 20,000 x 16 2.74 -> 1.41 ms.
+constexpr int fast_waves_per_eu(bool pop, int pass) {
+    return pass == kPassBroad ? 6 : pop ? 7 : 8;
+}
 
 struct FastIO {
     const BurstDesc* bursts;
@@ -144,11 +163,10 @@ struct FastIO {
     float* outF;
 };
 
-template <bool kPop, bool kGuided, bool kSamples>
+template <bool kPop, int kPass, bool kSamples>
 __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(
-    kPop ? kPopFastWavesPerEU : kFastWavesPerEU))) void fast_walk_kernel(const FastIO io,
-                                                                         const RunArgs a,
-                                                                         const FastArgs fa) {
+    fast_waves_per_eu(kPop, kPass)))) void fast_walk_kernel(const FastIO io, const RunArgs a,
+                                                            const FastArgs fa) {
     constexpr int kSlots = kPop ? 2 : 1;
     __shared__ Model sM[kSlots];
     extern __shared__ int32_t s_hist[];  // [kSlots][a.B]
@@ -246,7 +264,11 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(
             const uint32_t* ticks = io.ticks + d.off;
             const uint2* links = io.links + d.off;
             int r;
-            if (kGuided) {
+            if (kPass == kPassBroad) {
+                const BroadDraw draw{};
+                r = fast_window<false, BroadDraw>(M, &draw, key, d.P, d.stop_rel, d.T, ticks,
+                                                  links, a, fa, st);
+            } else if (kPass == kPassGuided) {
                 const size_t base = kPop ? size_t(M.guide_base) : 0;
                 const BinomGuide g{io.guide.thr + base * kGuideStatePairs,
                                    io.guide.guide + base * kBinomTable * kGuideBuckets};
@@ -286,37 +308,28 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(
 
 // ---- walk in the general form ---------------------------------------------------
 //
-// Every unit of the run (kPassGeneral), or the units the fast pass abandoned
-// (kPassReplay, launched right after it on the same stream, so the replay
-// list and its count are final).  Each one-wave workgroup keeps an LDS
-// histogram and adds it to its XCD's accumulator row at the end (workgroups
-// are dispatched to the 8 XCDs round-robin, so the atomics of a launch spread
-// over 8 x B addresses).  No completion ticket and no fence: the finish
-// kernel, launched behind on the same stream, reads the rows.
-template <int kPass>
+// The units the fast form abandoned, launched right after it on the same
+// stream, so the replay list and its count are final.  Each one-wave
+// workgroup keeps an LDS histogram and adds it to its XCD's accumulator row
+// at the end (workgroups are dispatched to the 8 XCDs round-robin, so the
+// atomics of a launch spread over 8 x B addresses).  No completion ticket and
+// no fence: the finish kernel, launched behind on the same stream, reads the
+// rows.
 __global__ __launch_bounds__(kWave) void walk_kernel(
     const BurstDesc* __restrict__ bursts, const uint32_t* __restrict__ ticks,
     const uint2* __restrict__ links, const ModelBlob* __restrict__ blob, const RunArgs a,
     int32_t* __restrict__ hist_acc, const uint32_t* __restrict__ replay,
     const uint32_t* __restrict__ replay_count, uint32_t* __restrict__ work,
     float* __restrict__ outE, int32_t* __restrict__ outAcc, float* __restrict__ outF) {
-    constexpr bool kReplay = kPass == kPassReplay;
-    // units of this pass, units per grab, queues and their counters
-    uint32_t nunits = a.nunits, batch = a.batch, queues = a.queues, share = a.q_share;
-    uint32_t* counters = work;
-    if (kReplay) {
-        const uint32_t c = *replay_count;
-        nunits = c < a.replay_cap ? c : a.replay_cap;
-        // as many workgroups as the list needs a wave for, each queue served
-        // by at least one of them
-        const uint32_t need = (nunits + kWave - 1u) / kWave;
-        const uint32_t alive = need < gridDim.x ? need : gridDim.x;
-        if (blockIdx.x >= alive) return;  // uniform over the workgroup
-        batch = kWave;
-        queues = alive < kReplayQueues ? alive : kReplayQueues;
-        share = (nunits + queues - 1u) / queues;
-        counters = work + size_t(kMaxQueues) * kCounterStride;
-    }
+    const uint32_t c = *replay_count;
+    const uint32_t nunits = c < a.replay_cap ? c : a.replay_cap;
+    // as many workgroups as the list needs a wave for, each queue served by
+    // at least one of them
+    const uint32_t waves = (nunits + kWave - 1u) / kWave;
+    const uint32_t alive = waves < gridDim.x ? waves : gridDim.x;
+    if (blockIdx.x >= alive) return;  // uniform over the workgroup
+    const uint32_t queues = alive < kReplayQueues ? alive : kReplayQueues;
+    const uint32_t queue = blockIdx.x % queues;
     __shared__ Model sM;
     extern __shared__ int32_t s_hist[];  // [a.B]
     const uint32_t lane = threadIdx.x;
@@ -328,22 +341,9 @@ __global__ __launch_bounds__(kWave) void walk_kernel(
     }
     __syncthreads();
 
-    // Work stealing at two levels.  A wave takes batches of consecutive units
-    // from a work counter; its lanes take units from the batch as they need
-    // them.  One loop pass advances every busy lane by one window, and a lane
-    // whose unit ends starts another in the same pass, so lanes do not wait
-    // for the wave's longest unit and waves do not wait for the grid's
-    // slowest batch.  The units are split into a.queues contiguous ranges
-    // with a counter each, every counter on its own 256-byte line (device-
-    // scope atomics to one line serialise); workgroup g draws from queue
-    // g % a.queues, so with a multiple of 8 queues each queue is served by
-    // one XCD and its bursts stay in that XCD's L2.  Batches are small
-    // (about six grabs per wave): the wave that grabs last still walks a
-    // whole batch, so the batch sets the grid's tail.  Photons are read
-    // through L1/L2.  A replay pass takes its units the same way from the
-    // replay list.
-    const QueueRange q = queue_range(blockIdx.x % queues, share, nunits);
-    uint32_t* counter = &counters[(blockIdx.x % queues) * kCounterStride];
+    // handed out as in fast_walk_kernel, a wave's worth at a time
+    const QueueRange q = queue_range(queue, (nunits + queues - 1u) / queues, nunits);
+    uint32_t* counter = &work[(kMaxQueues + queue) * kCounterStride];
     uint32_t pool_next = 0, pool_end = 0;  // the wave's current batch
     bool busy = false;
     uint32_t u = 0;
@@ -359,19 +359,19 @@ __global__ __launch_bounds__(kWave) void walk_kernel(
             if (want == 0) break;
             if (pool_next >= pool_end) {
                 uint32_t off = 0;
-                if (lane == 0) off = atomicAdd(counter, batch);
+                if (lane == 0) off = atomicAdd(counter, uint32_t(kWave));
                 off = __shfl(off, 0);
                 if (off >= q.end - q.begin) {
                     drained = true;
                     break;
                 }
                 pool_next = q.begin + off;
-                pool_end = pool_next + batch < q.end ? pool_next + batch : q.end;
+                pool_end = q.end - pool_next < kWave ? q.end : pool_next + kWave;
             }
             const uint32_t rank = lanes_below(want);
             const uint32_t avail = pool_end - pool_next;
             if (need && rank < avail) {
-                u = kReplay ? replay[pool_next + rank] : pool_next + rank;
+                u = replay[pool_next + rank];
                 const uint32_t bl = unit_div(u, divR);
                 const uint32_t b = a.begin + bl;
                 d = bursts[b];
@@ -540,14 +540,8 @@ __global__ __launch_bounds__(kWave * kFinishWaves) void finish_kernel(
 // call (src/gpuWorker.cpp:71-80); the units and their random streams are the
 // same as a single-set run with set id set_base + s * set_stride.
 
-// The general form over every (set, unit) of a population with distance
-// broadening.  Work is a flat list of batches: set s owns batches
-// [s * bps, (s + 1) * bps), each covering up to a.batch consecutive units of
-// that set; the list is dealt out to a.queues counters in turn
-// (pop_queue_length).  A wave's lanes may be walking units of two sets
-// at once: the workgroup keeps two LDS model slots with an LDS histogram
-// each, and a wave moves to a third set only after the older slot's lanes
-// have finished, so it never drains to change sets.
+// The general form over every (set, unit) of a population whose replay list
+// overflowed; work and sets as in fast_walk_kernel.
 __global__ __launch_bounds__(kWave) void pop_walk_kernel(
     const BurstDesc* __restrict__ bursts, const uint32_t* __restrict__ ticks,
     const uint2* __restrict__ links, const PopControl* __restrict__ ctl,
@@ -971,14 +965,20 @@ __global__ __launch_bounds__(kMbThreads) void microbench_kernel(int iters, float
 
 hipError_t walk_occupancy(int pass, int B, int* blocks_per_cu) {
     const size_t lds = sizeof(int32_t) * size_t(B);
-    if (pass == kPassFast)
-        return hipOccupancyMaxActiveBlocksPerMultiprocessor(
-            blocks_per_cu, fast_walk_kernel<false, true, false>, kWave, lds);
     if (pass == kPassReplay)
-        return hipOccupancyMaxActiveBlocksPerMultiprocessor(blocks_per_cu,
-                                                            walk_kernel<kPassReplay>, kWave, lds);
-    return hipOccupancyMaxActiveBlocksPerMultiprocessor(blocks_per_cu, walk_kernel<kPassGeneral>,
-                                                        kWave, lds);
+        return hipOccupancyMaxActiveBlocksPerMultiprocessor(blocks_per_cu, walk_kernel, kWave, lds);
+    if (pass == kPassBroad)
+        return hipOccupancyMaxActiveBlocksPerMultiprocessor(
+            blocks_per_cu, fast_walk_kernel<false, kPassBroad, false>, kWave, lds);
+    return hipOccupancyMaxActiveBlocksPerMultiprocessor(
+        blocks_per_cu, fast_walk_kernel<false, kPassGuided, false>, kWave, lds);
+}
+
+template <bool kPop, int kPass, bool kSamples>
+static void launch_fast(uint32_t grid, size_t lds, const FastIO& io, const RunArgs& a,
+                        const FastArgs& fa, hipStream_t stream) {
+    hipLaunchKernelGGL((fast_walk_kernel<kPop, kPass, kSamples>), dim3(grid), dim3(kWave), lds,
+                       stream, io, a, fa);
 }
 
 hipError_t launch_walk(int pass, uint32_t grid, const BurstDesc* bursts, const uint32_t* ticks,
@@ -987,24 +987,19 @@ hipError_t launch_walk(int pass, uint32_t grid, const BurstDesc* bursts, const u
                        uint32_t* replay_count, uint32_t* work, float* outE, int32_t* outAcc,
                        float* outF, hipStream_t stream) {
     const size_t lds = sizeof(int32_t) * size_t(a.B);
-    if (pass == kPassFast) {
-        const FastIO io{bursts, ticks, links, blob, nullptr, guide, hist_acc, replay,
-                        replay_count, work, outE, outAcc, outF};
-        if (outE)
-            hipLaunchKernelGGL((fast_walk_kernel<false, true, true>), dim3(grid), dim3(kWave), lds,
-                               stream, io, a, fa);
-        else
-            hipLaunchKernelGGL((fast_walk_kernel<false, true, false>), dim3(grid), dim3(kWave),
-                               lds, stream, io, a, fa);
-    } else if (pass == kPassReplay) {
-        hipLaunchKernelGGL(walk_kernel<kPassReplay>, dim3(grid), dim3(kWave), lds, stream, bursts,
-                           ticks, links, blob, a, hist_acc, replay, replay_count, work, outE,
-                           outAcc, outF);
-    } else {
-        hipLaunchKernelGGL(walk_kernel<kPassGeneral>, dim3(grid), dim3(kWave), lds, stream, bursts,
-                           ticks, links, blob, a, hist_acc, replay, replay_count, work, outE,
-                           outAcc, outF);
-    }
+    const FastIO io{bursts, ticks, links, blob, nullptr, guide, hist_acc, replay,
+                    replay_count, work, outE, outAcc, outF};
+    if (pass == kPassReplay)
+        hipLaunchKernelGGL(walk_kernel, dim3(grid), dim3(kWave), lds, stream, bursts, ticks, links,
+                           blob, a, hist_acc, replay, replay_count, work, outE, outAcc, outF);
+    else if (pass == kPassBroad && outE)
+        launch_fast<false, kPassBroad, true>(grid, lds, io, a, fa, stream);
+    else if (pass == kPassBroad)
+        launch_fast<false, kPassBroad, false>(grid, lds, io, a, fa, stream);
+    else if (outE)
+        launch_fast<false, kPassGuided, true>(grid, lds, io, a, fa, stream);
+    else
+        launch_fast<false, kPassGuided, false>(grid, lds, io, a, fa, stream);
     return hipGetLastError();
 }
 
@@ -1025,11 +1020,14 @@ hipError_t launch_finish(const RunArgs& a, const float* obs, int32_t* hist_acc,
 
 hipError_t pop_walk_occupancy(int pass, int B, int* blocks_per_cu) {
     const size_t lds = sizeof(int32_t) * 2u * size_t(B);
-    if (pass == kPassFast)
+    if (pass == kPassGeneral)
+        return hipOccupancyMaxActiveBlocksPerMultiprocessor(blocks_per_cu, pop_walk_kernel, kWave,
+                                                            lds);
+    if (pass == kPassBroad)
         return hipOccupancyMaxActiveBlocksPerMultiprocessor(
-            blocks_per_cu, fast_walk_kernel<true, true, false>, kWave, lds);
-    return hipOccupancyMaxActiveBlocksPerMultiprocessor(blocks_per_cu, pop_walk_kernel, kWave,
-                                                        lds);
+            blocks_per_cu, fast_walk_kernel<true, kPassBroad, false>, kWave, lds);
+    return hipOccupancyMaxActiveBlocksPerMultiprocessor(
+        blocks_per_cu, fast_walk_kernel<true, kPassGuided, false>, kWave, lds);
 }
 
 hipError_t launch_pop_walk(int pass, uint32_t grid, const BurstDesc* bursts,
@@ -1040,15 +1038,15 @@ hipError_t launch_pop_walk(int pass, uint32_t grid, const BurstDesc* bursts,
     const size_t lds = sizeof(int32_t) * 2u * size_t(a.B);
     const FastIO io{bursts, ticks, links, blobs, ctl, guide, hist_acc, replay,
                     replay_count, work, nullptr, nullptr, nullptr};
-    if (pass == kPassFast && guide.thr)
-        hipLaunchKernelGGL((fast_walk_kernel<true, true, false>), dim3(grid), dim3(kWave), lds,
-                           stream, io, a, fa);
-    else if (pass == kPassFast)
-        hipLaunchKernelGGL((fast_walk_kernel<true, false, false>), dim3(grid), dim3(kWave), lds,
-                           stream, io, a, fa);
-    else
+    if (pass == kPassGeneral)
         hipLaunchKernelGGL(pop_walk_kernel, dim3(grid), dim3(kWave), lds, stream, bursts, ticks,
                            links, ctl, blobs, a, hist_acc, work);
+    else if (pass == kPassBroad)
+        launch_fast<true, kPassBroad, false>(grid, lds, io, a, fa, stream);
+    else if (pass == kPassTable)
+        launch_fast<true, kPassTable, false>(grid, lds, io, a, fa, stream);
+    else
+        launch_fast<true, kPassGuided, false>(grid, lds, io, a, fa, stream);
     return hipGetLastError();
 }
 

@@ -330,6 +330,47 @@ PDA_HD float distance_efficiency(float rd, float r0) {
     return 1.0f / (1.0f + (q2 * q2) * q2);
 }
 
+// gauss() for the same words: sqrt(-2 log u) cos(2 pi u') with the log of a
+// 24-bit uniform and the quarter turn selected without branches.
+PDA_HD float gauss_uniform24(uint32_t a, uint32_t b) {
+    const float y = 4.0f * uniform24(b);
+    const float q = floorf(y + 0.5f);
+    const float t = (y - q) * 0x1.921fb6p+0f;
+    const float t2 = t * t;
+    float sp = fmaf(t2, 0x1.71de3ap-19f, -0x1.a01a02p-13f);
+    sp = fmaf(t2, sp, 0x1.111112p-7f);
+    sp = fmaf(t2, sp, -0x1.555556p-3f);
+    const float sn = fmaf(t2, sp, 1.0f) * t;
+    float cp = fmaf(t2, -0x1.27e4fcp-22f, 0x1.a01a02p-16f);
+    cp = fmaf(t2, cp, -0x1.6c16c2p-10f);
+    cp = fmaf(t2, cp, 0x1.555556p-5f);
+    cp = fmaf(t2, cp, -0.5f);
+    const float cs = fmaf(t2, cp, 1.0f);
+    const uint32_t turn = uint32_t(int(q)) & 3u;  // cos, -sin, -cos, sin
+    const float v = (turn & 1u) ? sn : cs;
+    const float c = turn == 1u || turn == 2u ? -v : v;
+    return sqrtf(-2.0f * flog_uniform24(a)) * c;
+}
+
+// distance_efficiency() with 1 / r0 rounded to float (r0 in quotient_range):
+// the quotient and the reciprocal without the division's scaling where their
+// operands are in its range (the reciprocal's sequence is the compiler's own).
+PDA_HD float distance_efficiency_quick(float rd, float r0, float r0_r) {
+    const float ad = fabsf(rd);
+    const float q = ad >= 0x1p-40f && ad <= 0x1p40f ? quotient(rd, r0, r0_r) : rd / r0;
+    const float q2 = q * q;
+    const float b = 1.0f + (q2 * q2) * q2;
+#ifdef __HIP_DEVICE_COMPILE__
+    if (!(b <= 0x1p90f)) return 1.0f / b;
+    float r = __builtin_amdgcn_rcpf(b);
+    r = fmaf(fmaf(-b, r, 1.0f), r, r);
+    float x = fmaf(fmaf(-b, r, 1.0f), r, r);
+    return fmaf(fmaf(-b, x, 1.0f), r, x);
+#else
+    return 1.0f / b;
+#endif
+}
+
 // ---- binomial -------------------------------------------------------------
 // Inversion (src/binom.cuh:135-169) when n < kInversionMaxN or
 // min(p,1-p) n <= 30, BTPE (Kachitvichyanukul & Schmeiser 1988,

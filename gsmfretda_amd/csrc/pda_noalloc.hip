@@ -131,7 +131,7 @@ extern "C" int pda_run_noalloc(pda_ctx* ctx, int sid, int R, uint32_t seed, uint
     a.replay_cap = uint32_t(kReplayCapacity);
     a.nsets = 1;
     a.bps = 0;
-    const int pass = s->any_v ? kPassGeneral : kPassFast;
+    const int pass = s->any_v ? kPassBroad : kPassGuided;
     const Launch L = plan_launch(ctx, pass, false, uint64_t(nunits));
     a.batch = L.batch;
     a.queues = L.queues;
@@ -141,10 +141,10 @@ extern "C" int pda_run_noalloc(pda_ctx* ctx, int sid, int R, uint32_t seed, uint
                        hist_acc);
     HIP_TRY(hipGetLastError());
     const BinomGuide guide{s->d_thr, s->d_guide};
-    const FastArgs fa = fast_args(s->n, s->quick_rates, a.clk_p);
+    const FastArgs fa = fast_args(s->n, s->quick_rates, a.clk_p, s->ph.r0);
     HIP_TRY(launch_walk(pass, L.grid, ctx->d_bursts, ctx->d_ticks, ctx->d_links, s->d_blob, guide,
                         a, fa, hist_acc, replay, count, work, nullptr, nullptr, nullptr, s->stream));
-    if (pass == kPassFast && nunits > 0) {
+    if (nunits > 0) {
         int per_cu = 0;
         if (walk_occupancy(kPassReplay, ctx->B, &per_cu) != hipSuccess || per_cu < 1) per_cu = 1;
         const uint64_t want = (uint64_t(nunits) + kWave - 1) / kWave;

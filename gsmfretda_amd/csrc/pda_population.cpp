@@ -7,7 +7,7 @@
 // generation -- sets of uneven state counts over the same resident bursts --
 // in one launch sequence that is captured once into a hipGraph and replayed:
 //   H2D copy of the generation's model tables and stream keys
-//   -> pop_walk_kernel (persistent grid, fast form)
+//   -> fast_walk_kernel (persistent grid)
 //   -> pop_replay_kernel (abandoned units, general form)
 //   -> pop_finish_kernel (one workgroup per set: histogram and chi2)
 //   -> D2H copy of every set's histogram and chi2.
@@ -33,7 +33,7 @@ bool PopGraphKey::operator==(const PopGraphKey& o) const {
            bg_on == o.bg_on && b0 == o.b0 && b1 == o.b1 && grid == o.grid && batch == o.batch &&
            queues == o.queues && replay_cap == o.replay_cap && clk_p == o.clk_p &&
            bg_ad == o.bg_ad && bg_dd == o.bg_dd && bursts == o.bursts && ticks == o.ticks &&
-           links == o.links && data_gen == o.data_gen && obs == o.obs && guided == o.guided &&
+           links == o.links && data_gen == o.data_gen && obs == o.obs && r0 == o.r0 &&
            max_states == o.max_states && quick_rates == o.quick_rates && thr == o.thr;
 }
 
@@ -140,15 +140,15 @@ int enqueue_population(pda_ctx* ctx, Slot& s, int pass, uint32_t grid, const Run
     HIP_TRY(hipMemcpyAsync(p.d_in, p.h_in, in_bytes(size_t(p.nsets)), hipMemcpyHostToDevice,
                            s.stream));
     BinomGuide guide{nullptr, nullptr};
-    if (pass == 0 && p.guided) {
+    if (pass == kPassGuided) {
         HIP_TRY(launch_guide(blobs, p.nsets, p.max_states, p.d_thr, p.d_guide, s.stream));
         guide = BinomGuide{p.d_thr, p.d_guide};
     }
     HIP_TRY(launch_pop_walk(pass, grid, ctx->d_bursts, ctx->d_ticks, ctx->d_links, ctl, blobs,
-                            guide, a, fast_args(p.max_states, p.quick_rates, a.clk_p),
+                            guide, a, fast_args(p.max_states, p.quick_rates, a.clk_p, p.r0),
                             p.d_hist_acc, p.d_replay, p.d_replay_count, p.d_work,
                             s.stream));
-    if (pass == 0)
+    if (pass != kPassGeneral)
         HIP_TRY(launch_pop_replay(ctx->d_bursts, ctx->d_ticks, ctx->d_links, ctl, blobs, a,
                                   p.d_hist_acc, p.d_replay, p.d_replay_count,
                                   uint32_t(ctx->num_cu) * 4u, s.stream));
@@ -176,7 +176,10 @@ int run_population(pda_ctx* ctx, Slot& s, int R, uint32_t seed, uint32_t set_bas
     if (total > (int64_t(1) << 40)) return fail(PDA_E_ARG, "population too large");
     int rc = ensure_pop_buffers(ctx, s, ctx->B);
     if (rc) return rc;
-    const int pass = (p.any_v || force_general) ? 2 : 0;
+    const int pass = force_general ? kPassGeneral
+                     : p.any_v     ? kPassBroad
+                     : p.guided    ? kPassGuided
+                                   : kPassTable;
     Launch L = plan_launch(ctx, pass, true, uint64_t(total));
     uint64_t bps = units > 0 ? (uint64_t(units) + L.batch - 1) / L.batch : 0;
     if (bps * uint64_t(p.nsets) >= (uint64_t(1) << 31)) {
@@ -189,7 +192,7 @@ int run_population(pda_ctx* ctx, Slot& s, int R, uint32_t seed, uint32_t set_bas
     // general form
     const size_t want_cap = size_t(std::min<int64_t>(
         total, std::max<int64_t>(int64_t(1) << 20, total / 16)));
-    if (pass == 0 && want_cap > p.replay_cap) {
+    if (pass != kPassGeneral && want_cap > p.replay_cap) {
         HIP_TRY(hipStreamSynchronize(s.stream));
         drop_graph(p);
         (void)hipFree(p.d_replay);
@@ -250,9 +253,9 @@ int run_population(pda_ctx* ctx, Slot& s, int R, uint32_t seed, uint32_t set_bas
         k.links = ctx->d_links;
         k.data_gen = ctx->data_gen;
         k.obs = ctx->d_obs;
-        k.guided = pass == 0 && p.guided;
         k.max_states = p.max_states;
         k.quick_rates = p.quick_rates;
+        k.r0 = p.r0;
         k.thr = p.d_thr;
         if (!p.exec || !(k == p.key)) {
             drop_graph(p);
@@ -380,6 +383,7 @@ int pda_set_population(pda_ctx* ctx, int sid, int nsets, const int32_t* nstates,
     p.off = off;
     p.any_v = any_v;
     p.quick_rates = quick_rates;
+    p.r0 = s->ph.r0;
     return PDA_OK;
 }
 
@@ -483,7 +487,7 @@ int pda_autotune(pda_ctx* ctx, int sid, int population, int R, int reps, int* ba
     int rc = sync_all(ctx);
     if (rc) return rc;
     int per_cu = 0;
-    const int pass = population ? (s->pop.any_v ? 2 : 0) : (s->any_v ? 2 : 0);
+    const int pass = (population ? s->pop.any_v : s->any_v) ? kPassBroad : kPassGuided;
     HIP_TRY(population ? pop_walk_occupancy(pass, ctx->B, &per_cu) : walk_occupancy(pass, ctx->B, &per_cu));
     if (per_cu < 1) per_cu = 1;
     const LaunchShape saved = ctx->shape;

@@ -20,6 +20,20 @@ constexpr uint32_t kCounterStride = 64;  // uint32 words between counters
 constexpr uint32_t kAuxQueues = 8;
 constexpr size_t kWorkWords = size_t(kMaxQueues + kAuxQueues) * kCounterStride;
 
+// How a walk launch runs: the fast form with the acceptor draws of models
+// without distance broadening from threshold rows (kPassGuided) or by the
+// inversion loop (kPassTable: populations whose rows would take too much
+// memory), or of models with broadening (kPassBroad); the general form over
+// the units that a fast form abandoned (kPassReplay), or over every unit of a
+// population (kPassGeneral: its replay list overflowed).
+enum WalkPass : int {
+    kPassGuided = 0,
+    kPassTable = 1,
+    kPassBroad = 2,
+    kPassReplay = 3,
+    kPassGeneral = 4,
+};
+
 // One burst, original order (the range [begin, end) of mc::setBurstBd
 // addresses these directly).  16 bytes, one dwordx4 load.
 struct BurstDesc {

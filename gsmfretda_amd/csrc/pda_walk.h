@@ -182,6 +182,66 @@ PDA_HD int64_t binomial_fast(int n, int s, const Model& M, const BinomGuide& g, 
     return binomial_guided(n, s, M, g, hi, lo);
 }
 
+// binomial() for n < kBinomTable trials of any p, or -1 where the uniform lies
+// too near a threshold to tell or the inversion restarts.  As for the rows
+// above, X is a non-decreasing function of the uniform that passes from k to
+// k + 1 where U = S_k + d, |d| <= k 2^-54, S_k the exact sum of the loop's
+// px_0 .. px_k; here C_k, the running sum of products computed with a power
+// instead of exp(n log q) and one reciprocal instead of a division a step,
+// stands for it, and a uniform within kBroadBand = 2^-38 of C_k is left to
+// the general form (about 10^-11 of the draws).  Errors of C_k, all relative
+// to sums of at most 1.0001: the power's 14 and the products' 4 k roundings
+// and the reciprocal's 2^-50, below 800 x 2^-53 + 127 x 2^-50; the loop's own
+// 5 k roundings; its q^n = exp(n log q), whose argument is at most 88.1 in
+// magnitude and within 3 units of 2^-53 relative of the exact one, and
+// exp itself: below 300 x 2^-53.  Together less than 2^-41.
+constexpr double kBroadBand = 0x1p-38;
+PDA_HD int binomial_broad(int n, float p, uint32_t hi, uint32_t lo) {
+    if (n <= 0 || !(p >= 0.0f && p <= 1.0f)) return 0;
+    if (n >= kBinomTable) return -1;
+    const bool flip = p > 0.5f;
+    const double pp = flip ? 1.0 - double(p) : double(p);
+    const double q = 1.0 - pp;
+    double C = 1.0;  // q^n by squaring
+    double sq = q;
+    for (int e = n; e > 0; e >>= 1) {
+        if (e & 1) C *= sq;
+        sq *= sq;
+    }
+#ifdef __HIP_DEVICE_COMPILE__
+    double rq = __builtin_amdgcn_rcp(q);
+    rq = fma(fma(-q, rq, 1.0), rq, rq);
+    rq = fma(fma(-q, rq, 1.0), rq, rq);
+#else
+    const double rq = 1.0 / q;
+#endif
+    const double ratio = pp * rq;
+    const double U = uniform53(hi, lo);
+    double px = C;
+    double left = double(n);  // n - X
+    int X = 0;
+    while (U > C && X < n) {
+        ++X;
+#ifdef __HIP_DEVICE_COMPILE__
+        double inv = __builtin_amdgcn_rcp(double(X));
+        inv = fma(fma(-double(X), inv, 1.0), inv, inv);
+        inv = fma(fma(-double(X), inv, 1.0), inv, inv);
+#else
+        const double inv = 1.0 / double(X);
+#endif
+        px = (px * ratio) * (left * inv);
+        left -= 1.0;
+        if (U < C + kBroadBand) return -1;  // too near the threshold passed
+        C += px;
+    }
+    if (U > C - kBroadBand) return -1;
+    // past the loop's bound, 10 standard deviations above the mean: a restart
+    const double np = double(n) * pp;
+    const double over = double(X) - np;
+    if (over > 0.0 && over * over > 99.0 * (np * q + 1.0)) return -1;
+    return flip ? n - X : X;
+}
+
 // Division of a unit index by the resample count without a divide
 // instruction sequence: for d >= 1, l = ceil(log2 d) and m = ceil(2^(31+l) / d)
 // (< 2^32), floor(u m / 2^(31+l)) = floor(u / d) for every u < 2^31 (m d =
@@ -390,20 +450,26 @@ PDA_HD int general_window(const Model& M, const UnitKey& key, uint32_t P, uint32
 // What the fast form needs besides the model, the same for every unit of a
 // launch: jumps = the largest state count - 2, the comparisons of the
 // next-state draw; quick: the rates and the tick length are in quotient()'s
-// range; clk_r: 1 / clk_p rounded to float.
+// range; clk_r: 1 / clk_p rounded to float; r0_r: 1 / r0, or 0 when r0 is
+// out of that range.
 struct FastArgs {
     int32_t jumps;
     int32_t quick;
-    float clk_r;
+    float clk_r, r0_r;
 };
-PDA_HD FastArgs fast_args(int max_states, bool quick_rates, float clk_p) {
-    return FastArgs{max_states - 2, quick_rates && quotient_range(clk_p) ? 1 : 0, 1.0f / clk_p};
+PDA_HD FastArgs fast_args(int max_states, bool quick_rates, float clk_p, float r0) {
+    return FastArgs{max_states - 2, quick_rates && quotient_range(clk_p) ? 1 : 0, 1.0f / clk_p,
+                    quotient_range(r0) ? 1.0f / r0 : 0.0f};
 }
 
-// The same window in the fast form (v = 0), the same values from fewer
-// operations; kStepReplay where the window needs the general form.  Tab:
-// BinomTable (inversion loop) or BinomGuide (thresholds) for the acceptor
-// draw.
+// Tab of fast_window for models with distance broadening: the efficiency is
+// drawn per window, so there is no table of its binomials.
+struct BroadDraw {};
+
+// The same window in the fast form, the same values from fewer operations;
+// kStepReplay where the window needs the general form.  Tab: BinomGuide
+// (thresholds) or BinomTable (inversion loop) for the acceptor draw of a
+// model without distance broadening, BroadDraw for one with.
 template <bool kCounts = false, class Tab = BinomTable>
 PDA_HD int fast_window(const Model& M, const typename NoDeduce<Tab>::type* tab, const UnitKey& key,
                        uint32_t P, uint32_t stop_rel, float T, const uint32_t* tick,
@@ -469,7 +535,20 @@ PDA_HD int fast_window(const Model& M, const typename NoDeduce<Tab>::type* tab, 
     if (kCounts) {
         *wi = WindowInfo{s, j, tau, int32_t(m)};
     } else {
-        const int x = int(binomial_fast(int(m), s, M, *tab, A.w[2], A.w[3]));
+        int x;
+        if constexpr (std::is_same<Tab, BroadDraw>::value) {
+            // broadened efficiency (drawE, src/gen_rand.cuh:63-68)
+            float de = M.ep0[s];
+            if (M.v[s] != 0.0f) {
+                const Block C = draw_block(key, w, kSubNormal);
+                const float rd = gauss_uniform24(C.w[0], C.w[1]) * M.v[s] + M.base[s];
+                de = fa.r0_r != 0.0f ? distance_efficiency_quick(rd, M.r0, fa.r0_r)
+                                     : distance_efficiency(rd, M.r0);
+            }
+            x = binomial_broad(int(m), de, A.w[2], A.w[3]);
+        } else {
+            x = int(binomial_fast(int(m), s, M, *tab, A.w[2], A.w[3]));
+        }
         if (x < 0) return kStepReplay;
         st.acc += float(x);
     }
@@ -491,7 +570,7 @@ PDA_HD WalkOut walk_unit(const Model& M, const typename NoDeduce<Tab>::type* tab
     WalkState<kFast> st;
     int r = begin_unit<kFast>(M, key, P, T, st);
     if constexpr (kFast) {
-        const FastArgs fa = fast_args(M.n, M.quick_rates != 0, a.clk_p);
+        const FastArgs fa = fast_args(M.n, M.quick_rates != 0, a.clk_p, M.r0);
         while (r == kStepMore)
             r = fast_window<false, Tab>(M, tab, key, P, stop_rel, T, tick, link, a, fa, st);
     } else {
