@@ -203,14 +203,15 @@ struct Slot {
 
 namespace pda {
 // Parameter-independent layout of the RB pmf memo for n states: the count
-// vectors with sum < kRbMemoCap, listed by total (so the lanes of a wave
-// build pmfs of one length), and per vector its offset in the pool and the
-// offsets of its leave-one-out pmfs (the pmfs of the vectors with one trial
+// vectors with sum < kRbMemoCap, in the pool by total, per vector its offset
+// there and the offsets of its leave-one-out pmfs (the pmfs of the vectors with one trial
 // of the 1st..4th counted state removed, which the pool holds too).
 struct RbMemoLayout {
-    uint32_t nvec = 0;
     uint64_t poolP = 0;               // floats
-    uint4* d_list = nullptr;          // list order: counts (x, y), offP, 0
+    // rb_memo_kernel's items: counts of all states but the last (x, y), first
+    // count of the last, number of counts
+    uint4* d_items = nullptr;
+    uint32_t nitems = 0;
     uint32_t* d_rank_offP = nullptr;  // by rb_rank
     uint4* d_rank_offD = nullptr;     // by rb_rank: leave-one-out offsets in the pool
 };
@@ -311,11 +312,10 @@ hipError_t launch_rb_walk(bool scores, int n, uint32_t grid, uint32_t replay_gri
 int rb_unit_threads();
 size_t rb_unit_lds_bytes(int B, int mode, int n);
 size_t rb_big_lds_bytes(int B, int cap, int mode, bool wide);
-size_t rb_memo_lds_bytes(int n);
 hipError_t launch_rb_table(const RbModel* rbm, const double* lf, float* pmf_tab, int n,
                            hipStream_t stream);
-hipError_t launch_rb_memo(int n, const RbModel* rbm, const float* pmf_tab, const uint4* list,
-                          uint32_t nvec, float* poolP, hipStream_t stream);
+hipError_t launch_rb_memo(int n, const float* pmf_tab, const uint4* items, uint32_t nitems,
+                          const uint32_t* rank_offP, float* poolP, hipStream_t stream);
 hipError_t launch_rb_unit(int mode, int n, uint32_t grid, const RbModel* rbm, const RunArgs& a,
                           const uint2* cnt, const float* F, const float* S, const double* Sbar,
                           const double* g, const uint32_t* rank_offP, const uint4* rank_offD,

@@ -59,7 +59,7 @@ void free_rb(RbState& r) {
 
 void free_rb_memo(pda_ctx* ctx) {
     for (RbMemoLayout& L : ctx->rb_memo) {
-        (void)hipFree(L.d_list);
+        (void)hipFree(L.d_items);
         (void)hipFree(L.d_rank_offP);
         (void)hipFree(L.d_rank_offD);
         L = RbMemoLayout();
@@ -156,15 +156,13 @@ void build_rb_model(const Model& M, RbModel& R, bool* rates_positive, bool* p_in
 
 // The memo layout of n states (built once per context and state count):
 // the count vectors with sum < kRbMemoCap in lexicographic order are ranked
-// 0, 1, ... (rb_rank); the build list holds them by total, and the pools
-// follow the list, so that the blocks written by one wave of rb_memo_kernel
-// (64 consecutive list entries) are adjacent: P blocks of Mt + 1 floats in
-// list order.  A vector's leave-one-out pmfs are the blocks of the vectors
+// 0, 1, ... (rb_rank); the pool holds their pmfs (blocks of Mt + 1 floats) by
+// total.  A vector's leave-one-out pmfs are the blocks of the vectors
 // with one trial fewer of each counted state (Mt - 1 < kRbMemoCap: in the
 // pool too); their offsets are kept per vector.
 int ensure_memo_layout(pda_ctx* ctx, int n) {
     RbMemoLayout& L = ctx->rb_memo[n];
-    if (L.d_list) return PDA_OK;
+    if (L.d_items) return PDA_OK;
     const int T = kRbMemoCap - 1;
     struct Vec {
         int m[kRbMaxStates];
@@ -199,15 +197,10 @@ int ensure_memo_layout(pda_ctx* ctx, int n) {
             return fail(PDA_E_STATE, "RB memo: rank of a count vector disagrees with the enumeration");
     std::stable_sort(v.begin(), v.end(), [](const Vec& x, const Vec& y) { return x.Mt < y.Mt; });
     const size_t nv = v.size();
-    std::vector<uint4> list(nv);
     std::vector<uint32_t> rank_offP(nv);
     std::vector<uint4> rank_offD(nv, make_uint4(0u, 0u, 0u, 0u));
     uint64_t offP = 0;
     for (size_t i = 0; i < nv; ++i) {
-        uint32_t cnt[kRbMaxStates];
-        for (int s = 0; s < kRbMaxStates; ++s) cnt[s] = uint32_t(v[i].m[s]);
-        const uint2 c = rb_pack(cnt);
-        list[i] = make_uint4(c.x, c.y, uint32_t(offP), 0u);
         rank_offP[v[i].rank] = uint32_t(offP);
         offP += uint64_t(v[i].Mt) + 1u;
     }
@@ -225,6 +218,18 @@ int ensure_memo_layout(pda_ctx* ctx, int n) {
             d[j++] = rank_offP[rb_rank(mm, n, T)];
         }
     }
+    // the memo kernel's items: per vector with last count 0 the runs of its
+    // last counts
+    std::vector<uint4> items;
+    for (const Vec& e : v) {
+        if (e.m[n - 1] != 0) continue;
+        uint32_t cnt[kRbMaxStates];
+        for (int s = 0; s < kRbMaxStates; ++s) cnt[s] = uint32_t(e.m[s]);
+        const uint2 c = rb_pack(cnt);
+        for (int m = 0; m <= T - e.Mt; m += kRbMemoRun)
+            items.push_back(make_uint4(c.x, c.y, uint32_t(m),
+                                       uint32_t(std::min(kRbMemoRun, T - e.Mt - m + 1))));
+    }
     if (offP >= (uint64_t(1) << 32)) return fail(PDA_E_STATE, "RB memo pool exceeds 2^32 entries");
     auto upload = [&](auto** dst, const auto& src) -> int {
         using T = std::remove_reference_t<decltype(src[0])>;
@@ -233,16 +238,16 @@ int ensure_memo_layout(pda_ctx* ctx, int n) {
         return PDA_OK;
     };
     RbMemoLayout out;
-    int rc = upload(&out.d_list, list);
+    int rc = upload(&out.d_items, items);
     if (!rc) rc = upload(&out.d_rank_offP, rank_offP);
     if (!rc) rc = upload(&out.d_rank_offD, rank_offD);
     if (rc) {
-        (void)hipFree(out.d_list);
+        (void)hipFree(out.d_items);
         (void)hipFree(out.d_rank_offP);
         (void)hipFree(out.d_rank_offD);
         return rc;
     }
-    out.nvec = uint32_t(nv);
+    out.nitems = uint32_t(items.size());
     out.poolP = offP;
     L = out;
     return PDA_OK;
@@ -404,8 +409,6 @@ int rb_enqueue_forward(pda_ctx* ctx, Slot& s, RbState& r, const Model& M,
     // the memo of this set: every count vector's pmf
     if (int rc = ensure_memo_layout(ctx, n)) return rc;
     const RbMemoLayout& ML = ctx->rb_memo[n];
-    if (rb_memo_lds_bytes(n) + 512 > ctx->lds_per_block)
-        return fail(PDA_E_STATE, "the RB memo kernel exceeds the LDS of a workgroup");
     if (ML.poolP > r.cap_poolP) {
         HIP_TRY(hipStreamSynchronize(s.stream));
         (void)hipFree(r.d_poolP);
@@ -429,7 +432,8 @@ int rb_enqueue_forward(pda_ctx* ctx, Slot& s, RbState& r, const Model& M,
     HIP_TRY(hipEventRecord(s.rb_fork, s.stream));
     HIP_TRY(hipStreamWaitEvent(s.rb_aux, s.rb_fork, 0));
     HIP_TRY(launch_rb_table(d_rbm, ctx->d_lf, r.d_pmf_tab, n, s.rb_aux));
-    HIP_TRY(launch_rb_memo(n, d_rbm, r.d_pmf_tab, ML.d_list, ML.nvec, r.d_poolP, s.rb_aux));
+    HIP_TRY(launch_rb_memo(n, r.d_pmf_tab, ML.d_items, ML.nitems, ML.d_rank_offP, r.d_poolP,
+                           s.rb_aux));
     HIP_TRY(hipEventRecord(s.rb_join, s.rb_aux));
     HIP_TRY(launch_rb_walk(scores, n, grid, uint32_t(ctx->num_cu) * 4u, ctx->d_bursts, ctx->d_ticks,
                            ctx->d_links, d_blob, d_rbm, a,

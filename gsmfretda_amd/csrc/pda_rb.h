@@ -108,6 +108,8 @@ PDA_HD int rb_pmf_index(int s, int m, int k) { return s * kRbPmfStride + m * (m 
 // total Mt < kRbMemoCap are computed once per forward and looked up by the
 // units; units with larger totals compute their own.
 constexpr int kRbMemoCap = 48;
+// Counts of the last state that one wave of the memo kernel builds pmfs for.
+constexpr int kRbMemoRun = 8;
 // Units that compute their own pmf are listed in two lists: totals below
 // kRbBigSplit (pmfs of at most kRbBigSplit entries: small LDS buffers, many
 // workgroups per CU) and the rest (buffers for the largest total any burst

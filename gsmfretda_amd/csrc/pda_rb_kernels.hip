@@ -11,9 +11,9 @@
 //   rb_table_kernel      the binomial pmfs of every state, counts < 256
 //   rb_memo_kernel       the pmf (a convolution of one binomial per state)
 //                        of every count vector with a small acceptor total,
-//                        one lane per vector, in a strip of LDS of its own,
-//                        (the derivative passes' leave-one-trial-out pmfs
-//                        are the pmfs of the vectors with one trial fewer)
+//                        a wave per few vectors, lanes over outcomes (the
+//                        derivative passes' leave-one-trial-out pmfs are the
+//                        pmfs of the vectors with one trial fewer)
 //   rb_unit_kernel       every unit with a small total: its pmf from the
 //                        memo spread into the E histogram as 2^-32 fixed
 //                        point (forward), or the cotangent-weighted pmf and
@@ -43,16 +43,8 @@ namespace pda {
 // totals for rb_big_kernel.  The mean Mt is about 6 on the 3-state
 // workloads and 24 on the 4-state fast-dynamics one, where 97 % of the
 // units have Mt < 48.
-//
-// rb_memo_kernel: one lane per count vector, the pmf in a strip of LDS of
-// its own; kRbStride floats between the strips of consecutive lanes (odd,
-// so that lanes reading the same offset hit distinct LDS banks).
-constexpr int kRbStride = kRbMemoCap + 1;
-constexpr int kRbMemoWaves = 1;  // waves per workgroup of rb_memo_kernel
-// Entries per state of the pmf table rb_memo_kernel keeps in LDS: counts
-// m < kRbMemoCap, entry (m, k) at m (m + 1) / 2 + k (the first entries of
-// the state's block of the global table).
-constexpr int kRbMemoTab = kRbMemoCap * (kRbMemoCap + 1) / 2;
+constexpr int kRbMemoWaves = 4;  // waves per workgroup of rb_memo_kernel
+static_assert(kRbMemoCap <= kWave, "a memo pmf fits the lanes of a wave");
 // rb_unit_kernel: waves per workgroup, and its work counters (the
 // kAuxQueues lines after the walk's, workgroup g on counter g % kAuxQueues,
 // each over a contiguous share of the units: one queue per XCD).
@@ -305,20 +297,12 @@ __device__ __forceinline__ double wave_sum(double v) {
     return v;
 }
 
-// Inclusive prefix sum / maximum over the lanes of the wave.
+// Inclusive prefix sum over the lanes of the wave.
 __device__ __forceinline__ int wave_scan_sum(int v, int lane) {
 #pragma unroll
     for (int d = 1; d < kWave; d <<= 1) {
         const int t = __shfl_up(v, d);
         if (lane >= d) v += t;
-    }
-    return v;
-}
-__device__ __forceinline__ int wave_scan_max(int v, int lane) {
-#pragma unroll
-    for (int d = 1; d < kWave; d <<= 1) {
-        const int t = __shfl_up(v, d);
-        if (lane >= d) v = t > v ? t : v;
     }
     return v;
 }
@@ -333,35 +317,6 @@ __device__ __forceinline__ void wave_lds_sync() {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-}
-
-// Spreading the elements of 64 variable-length items over the lanes: item
-// l (owned by lane l) has len_l elements at positions pos_l .. pos_l +
-// len_l - 1 of the wave's concatenation (pos = exclusive prefix sum of len).
-// Window w holds positions 64 w .. 64 w + 63, one per lane; the owner of a
-// lane's position is the last item starting at or before it: each item
-// starting inside the window marks its start slot, and a running maximum
-// over the slots (carried across windows) names the owner.  slot: 64 ints of
-// the wave's LDS.  Calls body(j, owner) for each lane (j >= total: no
-// element), with every lane of the wave present at each call (shuffles may
-// be used); what the caller's lanes wrote to LDS before the call is visible
-// to body, and the body's LDS accesses end before the next window's.
-template <typename Body>
-__device__ __forceinline__ void wave_windows(int len, int pos, int total, int lane, int* slot,
-                                             Body&& body) {
-    int carry = -1;
-    wave_lds_sync();
-    for (int wb = 0; wb < total; wb += kWave) {
-        slot[lane] = -1;
-        wave_lds_sync();
-        if (len > 0 && pos >= wb && pos < wb + kWave) slot[pos - wb] = lane;
-        wave_lds_sync();
-        int own = wave_scan_max(slot[lane], lane);
-        own = own > carry ? own : carry;
-        carry = __shfl(own, kWave - 1);
-        body(wb + lane, own);
-        wave_lds_sync();
-    }
 }
 
 // What the passes compute per unit, with P(a), a = 0..Mt, the unit's pmf
@@ -388,84 +343,68 @@ __device__ __forceinline__ void wave_windows(int len, int pos, int total, int la
 // different bins, so d M_b / d p_s gathers m_s P_s(c) at the unit's bin
 // boundaries; the rate columns add P(a) (S - Sbar) to the row of bin(a).
 
-// Bytes of rb_memo_kernel's dynamic LDS: the n states' pmf tables, then per
-// lane one strip (the pmf).
-__host__ __device__ inline size_t rb_memo_lds(int n) {
-    return sizeof(float) * (size_t(n) * kRbMemoTab + size_t(kRbMemoWaves) * kWave * kRbStride);
-}
+// The memo: the pmf of every count vector of the list's items into poolP.
+// (The derivative passes' leave-one-out pmfs are the pmfs of the vectors with
+// one trial fewer, in the same pool.)  An item is the counts of all states but
+// the last and a run of counts of the last (kRbMemoRun at most); a wave takes
+// it, lane q holding outcome q (Mt < 48 outcomes fit a wave).  The states'
+// binomials are convolved in state order, each output summed k ascending from
+// 0.0f, as the oracle does: z += Y[k] X[q - k], X moving up one lane per step,
+// the lanes below getting 0.  Outcomes outside the overlap add an exact 0, so
+// the result is the oracle's bit for bit; a count of 0 leaves X as it is (its
+// binomial is [1]).  Y's index is the same for all lanes: its loads are scalar.
+// Three instructions a step and no LDS.  With a lane per vector, each walking
+// its own chain of convolutions in a strip of LDS (31 KB a wave: five waves a
+// CU), the 249,900 vectors of four states took 411 us, longer than the walk
+// they are built beside, and the 19,600 of three 101 us; like this 135 and
+// 14 us beside the walk.  The prefix is convolved again for each run:
+// about a tenth of the steps, and every wave independent of every other.
+typedef float Floats8 __attribute__((ext_vector_type(8), aligned(4)));
+static_assert(kRbMemoCap + 8 < kRbPmfTable, "rows of the pmf table follow the memo's");
 
-// The memo: for each count vector of the list (one lane each) its pmf P
-// into poolP at its offP.  (The derivative passes' leave-one-out pmfs are
-// the pmfs of the vectors with one trial fewer, in the same pool.)  The list
-// runs by total, the offsets follow it, and each wave copies its lanes'
-// blocks out of LDS together: adjacent blocks, coalesced writes.
+template <int kN>
 __global__ __launch_bounds__(kWave * kRbMemoWaves) void rb_memo_kernel(
-    const RbModel* __restrict__ rbm, const float* __restrict__ pmf_tab,
-    const uint4* __restrict__ list, uint32_t nvec, float* __restrict__ poolP) {
-    extern __shared__ float s_f[];
-    __shared__ RbModel sR;
-    __shared__ int s_slot[kRbMemoWaves][kWave];
-    __shared__ int s_pos[kRbMemoWaves][kWave];
-    __shared__ uint32_t s_dst[kRbMemoWaves][kWave];
-    const int tid = int(threadIdx.x), lane = tid % kWave, wave = tid / kWave;
-    {
-        const uint32_t* src = reinterpret_cast<const uint32_t*>(rbm);
-        uint32_t* dst = reinterpret_cast<uint32_t*>(&sR);
-        for (uint32_t i = uint32_t(tid); i < sizeof(RbModel) / 4; i += blockDim.x) dst[i] = src[i];
-    }
-    __syncthreads();
-    const int n = sR.n;
-    float* tab = s_f;
-    for (int i = tid; i < n * kRbMemoTab; i += int(blockDim.x)) {
-        const int s = i / kRbMemoTab;
-        tab[i] = pmf_tab[size_t(s) * kRbPmfStride + size_t(i - s * kRbMemoTab)];
-    }
-    __syncthreads();
-    float* strips = tab + n * kRbMemoTab + size_t(wave) * kWave * kRbStride;
-    float* X = strips + lane * kRbStride;
-    const uint32_t v = blockIdx.x * blockDim.x + uint32_t(tid);
-    const bool act = v < nvec;
-    const uint4 e = act ? list[v] : make_uint4(0u, 0u, 0u, 0u);
-    const uint2 c = make_uint2(e.x, e.y);
-    // the pmf in X: the states' binomials convolved in state order, each
-    // output summed k ascending from 0.0f (the oracle's order); outputs
-    // descending, so that each overwrites an entry of X no later output reads
-    int xl = 1;
-    X[0] = 1.0f;
+    const float* __restrict__ pmf_tab, const uint4* __restrict__ items, uint32_t nitems,
+    const uint32_t* __restrict__ rank_offP, float* __restrict__ poolP) {
+    const int q = int(threadIdx.x) % kWave;
+    const uint32_t i = blockIdx.x * uint32_t(kRbMemoWaves) +
+                       uint32_t(__builtin_amdgcn_readfirstlane(int(threadIdx.x) / kWave));
+    if (i >= nitems) return;  // uniform over the wave; no barrier below
+    const uint4 e = items[i];
+    const uint2 c = make_uint2(uint32_t(__builtin_amdgcn_readfirstlane(int(e.x))),
+                               uint32_t(__builtin_amdgcn_readfirstlane(int(e.y))));
+    const int first = __builtin_amdgcn_readfirstlane(int(e.z));
+    const int runs = __builtin_amdgcn_readfirstlane(int(e.w));
+    // X (*) Binomial(m, p_s)
+    auto convolve = [&](float X, int s, int m) {
+        const float* Y = pmf_tab + size_t(s) * kRbPmfStride + m * (m + 1) / 2;
+        float z = 0.0f;
+        for (int k0 = 0; k0 <= m; k0 += 8) {  // entries past m: the next rows', taken as 0
+            const Floats8 y = *reinterpret_cast<const Floats8*>(Y + k0);
 #pragma unroll
-    for (int s = 0; s < kRbMaxStates; ++s) {
-        const int m = s < n ? int(rb_count(c, s)) : 0;
-        if (m == 0) continue;
-        const float* Y = tab + s * kRbMemoTab + m * (m + 1) / 2;
-        if (xl == 1) {
-            for (int k = 0; k <= m; ++k) X[k] = Y[k];
-        } else {
-            for (int q = xl + m - 1; q >= 0; --q) {
-                const int k0 = q - (xl - 1) > 0 ? q - (xl - 1) : 0;
-                const int k1 = q < m ? q : m;
-                float z = 0.0f;
-                for (int k = k0; k <= k1; ++k) z = z + Y[k] * X[q - k];
-                X[q] = z;
+            for (int k = 0; k < 8; ++k) {
+                z = z + (k0 + k <= m ? y[k] : 0.0f) * X;
+                X = bitsf(uint32_t(__builtin_amdgcn_update_dpp(0, int(fbits(X)), 0x138, 0xf, 0xf,
+                                                               true)));  // wave_shr:1
             }
         }
-        xl += m;
+        return z;
+    };
+    float X = q == 0 ? 1.0f : 0.0f;
+    int mm[kRbMaxStates] = {0, 0, 0, 0};
+    int total = 0;
+#pragma unroll
+    for (int s = 0; s < kN - 1; ++s) {
+        mm[s] = int(rb_count(c, s));
+        total += mm[s];
+        if (mm[s] > 0) X = convolve(X, s, mm[s]);
     }
-    int* slot = s_slot[wave];
-    int* spos = s_pos[wave];
-    uint32_t* sdst = s_dst[wave];
-    // copy the wave's pmfs out: lane l's block of xl floats at offP
-    const int len = act ? xl : 0;
-    const int incl = wave_scan_sum(len, lane);
-    const int pos = incl - len;
-    const int total = __shfl(incl, kWave - 1);
-    spos[lane] = pos;
-    sdst[lane] = e.z;
-    wave_windows(len, pos, total, lane, slot, [&](int j, int own) {
-        if (j < total) {
-            const int ai = j - spos[own];
-            poolP[sdst[own] + uint32_t(ai)] = strips[own * kRbStride + ai];
-        }
-    });
+    for (int m = first; m < first + runs; ++m) {
+        const float z = m > 0 ? convolve(X, kN - 1, m) : X;
+        mm[kN - 1] = m;
+        const uint32_t off = rank_offP[rb_rank(mm, kN, kRbMemoCap - 1)];
+        if (q <= total + m) poolP[off + uint32_t(q)] = z;
+    }
 }
 
 // Owner of position j of the wave's concatenation: the last lane l with
@@ -1113,7 +1052,6 @@ hipError_t launch_rb_walk(bool scores, int n, uint32_t grid, uint32_t replay_gri
 int rb_unit_threads() { return kWave * kRbUnitWaves; }
 size_t rb_unit_lds_bytes(int B, int mode, int n) { return rb_unit_lds(B, mode, n); }
 size_t rb_big_lds_bytes(int B, int cap, int mode, bool wide) { return rb_big_lds(B, cap, mode, wide); }
-size_t rb_memo_lds_bytes(int n) { return rb_memo_lds(n); }
 
 hipError_t launch_rb_table(const RbModel* rbm, const double* lf, float* pmf_tab, int n,
                            hipStream_t stream) {
@@ -1123,12 +1061,18 @@ hipError_t launch_rb_table(const RbModel* rbm, const double* lf, float* pmf_tab,
     return hipGetLastError();
 }
 
-hipError_t launch_rb_memo(int n, const RbModel* rbm, const float* pmf_tab, const uint4* list,
-                          uint32_t nvec, float* poolP, hipStream_t stream) {
-    const uint32_t threads = kWave * kRbMemoWaves;
-    const dim3 grid((nvec + threads - 1) / threads);
-    hipLaunchKernelGGL(rb_memo_kernel, grid, dim3(threads), rb_memo_lds(n), stream, rbm, pmf_tab,
-                       list, nvec, poolP);
+hipError_t launch_rb_memo(int n, const float* pmf_tab, const uint4* items, uint32_t nitems,
+                          const uint32_t* rank_offP, float* poolP, hipStream_t stream) {
+    const dim3 grid((nitems + kRbMemoWaves - 1) / kRbMemoWaves), threads(kWave * kRbMemoWaves);
+    if (n == 2)
+        hipLaunchKernelGGL(rb_memo_kernel<2>, grid, threads, 0, stream, pmf_tab, items, nitems,
+                           rank_offP, poolP);
+    else if (n == 3)
+        hipLaunchKernelGGL(rb_memo_kernel<3>, grid, threads, 0, stream, pmf_tab, items, nitems,
+                           rank_offP, poolP);
+    else
+        hipLaunchKernelGGL(rb_memo_kernel<4>, grid, threads, 0, stream, pmf_tab, items, nitems,
+                           rank_offP, poolP);
     return hipGetLastError();
 }
 
