@@ -121,9 +121,11 @@ struct RbState {
     uint8_t* h_res = nullptr;          // pinned
     double* d_g = nullptr;             // cotangent per bin
     double* h_g = nullptr;             // pinned
-    double* d_grad = nullptr;          // n + K
+    double* d_grad = nullptr;          // kRbGradRows rows of n + K, then their sum
     float* d_pmf_tab = nullptr;        // binomial pmfs of the states, counts < 256
-    double* d_jac = nullptr;           // [kMaxBins][n + K] rows of 16
+    // kRbJacRows times [B][n + K] rows of 16, then their sum (capacity in bins)
+    double* d_jac = nullptr;
+    int cap_jac = 0;
     double* h_jac = nullptr;           // pinned
     // units whose acceptor total is too large for the memo, listed by the
     // walk: totals below kRbBigSplit (d_big) and the rest (d_huge), each of
@@ -309,18 +311,21 @@ hipError_t launch_rb_walk(bool scores, int n, uint32_t grid, uint32_t replay_gri
                           uint32_t* big_count, uint32_t* replay, uint32_t* replay_count,
                           hipStream_t stream);
 // dynamic LDS bytes (mode: 0 forward, 1 adjoint, 2 Jacobian)
-int rb_unit_threads();
-size_t rb_unit_lds_bytes(int B, int mode, int n);
+int rb_unit_threads(int mode);
+size_t rb_unit_lds_bytes(int B, int mode, int n, int copies, bool pool);
 size_t rb_big_lds_bytes(int B, int cap, int mode, bool wide);
 hipError_t launch_rb_table(const RbModel* rbm, const double* lf, float* pmf_tab, int n,
                            hipStream_t stream);
 hipError_t launch_rb_memo(int n, const float* pmf_tab, const uint4* items, uint32_t nitems,
                           const uint32_t* rank_offP, float* poolP, hipStream_t stream);
-hipError_t launch_rb_unit(int mode, int n, uint32_t grid, const RbModel* rbm, const RunArgs& a,
-                          const uint2* cnt, const float* F, const float* S, const double* Sbar,
-                          const double* g, const uint32_t* rank_offP, const uint4* rank_offD,
-                          const float* poolP, unsigned long long* hist_acc,
-                          double* grad, uint32_t* work, hipStream_t stream);
+// copies: of the LDS accumulators; tile: units a workgroup takes at a time;
+// pool: the smallest totals' pmfs kept in LDS
+hipError_t launch_rb_unit(int mode, int n, uint32_t grid, int copies, int tile, bool pool,
+                          const RunArgs& a, const uint2* cnt, const float* F, const float* S,
+                          const double* Sbar, const double* g, const uint32_t* rank_offP,
+                          const uint4* rank_offD, const float* poolP,
+                          unsigned long long* hist_acc, double* grad, uint32_t* work,
+                          hipStream_t stream);
 hipError_t launch_rb_big(int mode, bool wide, uint32_t grid, int cap, const RbModel* rbm,
                          const double* lf,
                          const float* pmf_tab, const RunArgs& a, const uint2* cnt, const float* F,
@@ -329,6 +334,8 @@ hipError_t launch_rb_big(int mode, bool wide, uint32_t grid, int cap, const RbMo
                          unsigned long long* hist_acc, double* grad, hipStream_t stream);
 hipError_t launch_rb_score_mean(const RunArgs& a, int K, const float* S, double* Sbar,
                                 int num_cu, hipStream_t stream);
+// out[i] = sum of the nrows rows of n doubles
+hipError_t launch_rb_rows(const double* rows, int n, int nrows, double* out, hipStream_t stream);
 hipError_t launch_rb_finish(const RunArgs& a, const float* obs, unsigned long long* hist_acc,
                             uint32_t* work, void* res, hipStream_t stream);
 

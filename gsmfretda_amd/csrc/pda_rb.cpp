@@ -78,7 +78,7 @@ struct RbResultHeaderH {  // device RbResultHeader
     int32_t B;
 };
 constexpr size_t kRbResBytes = sizeof(RbResultHeaderH) + sizeof(uint64_t) * kMaxBins;
-constexpr int kGradLen = kRbMaxStates + kRbMaxPairs;
+constexpr int kGradLen = kRbGradLen;
 constexpr size_t kRbCounters = kWorkWords;  // queue counters + the pmf pass's
 
 int ensure_rb(pda_ctx* ctx, RbState& r) {
@@ -101,10 +101,10 @@ int ensure_rb(pda_ctx* ctx, RbState& r) {
         if (!r.h_g)
             HIP_TRY(hipHostMalloc(reinterpret_cast<void**>(&r.h_g), sizeof(double) * kMaxBins,
                                   hipHostMallocDefault));
-        if (!r.d_grad) HIP_TRY(hipMalloc(&r.d_grad, sizeof(double) * kGradLen));
+        if (!r.d_grad)
+            HIP_TRY(hipMalloc(&r.d_grad, sizeof(double) * kGradLen * (kRbGradRows + 1)));
         if (!r.d_pmf_tab)
             HIP_TRY(hipMalloc(&r.d_pmf_tab, sizeof(float) * size_t(kRbMaxStates) * kRbPmfStride));
-        if (!r.d_jac) HIP_TRY(hipMalloc(&r.d_jac, sizeof(double) * kGradLen * kMaxBins));
         if (!r.h_jac)
             HIP_TRY(hipHostMalloc(reinterpret_cast<void**>(&r.h_jac),
                                   sizeof(double) * kGradLen * kMaxBins, hipHostMallocDefault));
@@ -248,17 +248,20 @@ int ensure_memo_layout(pda_ctx* ctx, int n) {
         return rc;
     }
     out.nitems = uint32_t(items.size());
-    out.poolP = offP;
+    // four more: the unit passes read four entries at a time
+    out.poolP = offP + 4u;
     L = out;
     return PDA_OK;
 }
 
 // Launch shape of one pmf pass (mode 0 forward, 1 adjoint, 2 Jacobian):
-// rb_unit_kernel on every slot its LDS allows (at most enough workgroups for
-// the units), about eight grabs per wave; rb_big_kernel on every slot its
-// LDS allows (its workgroups beyond the listed units exit at once).
+// rb_unit_kernel on every slot its LDS allows (at most a workgroup per tile);
+// rb_big_kernel on every slot its LDS allows (its workgroups beyond the listed
+// units exit at once).
 struct PassShape {
-    uint32_t unit_grid = 1, batch = kWave, big_grid = 1, huge_grid = 1;
+    uint32_t unit_grid = 1, big_grid = 1, huge_grid = 1;
+    int copies = 1, tile = kWave;
+    bool pool = false;
     int big_cap = 1;    // rb_big_kernel's buffers for the big list (the huge list: the run's cap)
     bool wide = false;  // rb_big_kernel's derivative buffers in double
 };
@@ -266,32 +269,49 @@ int pass_shape(pda_ctx* ctx, int mode, int n, bool wide, int B, int cap, uint32_
                PassShape& ps) {
     static const char* names[] = {"forward", "adjoint", "Jacobian"};
     constexpr size_t kStatic = sizeof(RbModel) + 64;  // the kernels' static LDS
-    const size_t lds = rb_unit_lds_bytes(B, mode, n);
-    if (lds + kStatic > ctx->lds_per_block)
+    // the bins a pass supports: rows of an odd number of doubles and the score
+    // differences of four waves
+    const size_t rows = sizeof(double) * size_t(mode == 2 ? B * ((n * n) | 1) : B);
+    if (rows + (mode ? sizeof(double) * 4u * kWave * size_t(n * (n - 1)) : 0) + kStatic >
+        ctx->lds_per_block)
         return fail(PDA_E_DATA, "%d bins exceed the LDS of the RB %s pass", B, names[mode]);
+    // The adjoint keeps the pool's first floats in LDS (3 states, 6.4e6 units:
+    // 155 us, 174 without), unless the run is too small to repay the copy;
+    // the forward reads each entry once and is faster with the LDS left to
+    // more workgroups (forward 451 us, 470 with), as is the Jacobian with it
+    // left to copies.  Copies: the Jacobian's rows of 3 states take 246 us
+    // with 8, 227 with 16, 215 with 32; the forward's gain nothing past 16.
+    const size_t threads = size_t(rb_unit_threads(mode));
+    const size_t budget = std::min<size_t>(ctx->lds_per_block, mode == 2 ? 131072 : 40960);
+    const int most = mode == 1 ? 1 : mode == 2 ? 32 : 16;
+    ps.pool = mode == 1 && nunits >= 65536u && rb_unit_lds_bytes(B, mode, n, 1, true) <= budget;
+    ps.copies = 1;
+    while (ps.copies < most && rb_unit_lds_bytes(B, mode, n, 2 * ps.copies, ps.pool) <= budget)
+        ps.copies *= 2;
+    const size_t lds = rb_unit_lds_bytes(B, mode, n, ps.copies, ps.pool);
     int per = 0;
     HIP_TRY(rb_unit_occupancy(mode, n, int(lds), &per));
-    const uint64_t threads = uint64_t(rb_unit_threads());
-    const uint64_t g = std::min<uint64_t>(uint64_t(ctx->num_cu) * uint64_t(std::max(per, 1)),
-                                          (uint64_t(nunits) + threads - 1) / threads);
-    ps.unit_grid = uint32_t(std::max<uint64_t>(g, 1));
-    uint64_t bt = uint64_t(nunits) / (uint64_t(ps.unit_grid) * (threads / kWave) * 8u);
-    bt = (bt + kWave - 1) / kWave * kWave;
-    ps.batch = uint32_t(std::min<uint64_t>(std::max<uint64_t>(bt, kWave), 4096));
+    const uint64_t slots = uint64_t(ctx->num_cu) * uint64_t(std::max(per, 1));
+    // tiles of four units per thread, fewer while that leaves slots empty
+    uint64_t tile = threads * 4u;
+    while (tile > 2u * kWave && (uint64_t(nunits) + tile - 1) / tile < slots) tile /= 2;
+    ps.tile = int(tile);
+    ps.unit_grid = uint32_t(std::max<uint64_t>(
+        1, std::min<uint64_t>(slots, (uint64_t(nunits) + tile - 1) / tile)));
+    int per_big = 0;
     // double buffers where asked for and they fit, else float
     ps.wide = wide && rb_big_lds_bytes(B, cap, mode, true) + kStatic <= ctx->lds_per_block;
     const size_t blds = rb_big_lds_bytes(B, cap, mode, ps.wide);
     if (blds + kStatic > ctx->lds_per_block)
         return fail(PDA_E_DATA, "%d bins and bursts needing %d acceptor outcomes exceed the LDS "
                     "of the RB %s pass", B, cap, names[mode]);
-    per = 0;
-    HIP_TRY(rb_big_occupancy(mode, ps.wide, int(blds), &per));
-    ps.huge_grid = uint32_t(std::max(1, ctx->num_cu * std::max(per, 1)));
+    HIP_TRY(rb_big_occupancy(mode, ps.wide, int(blds), &per_big));
+    ps.huge_grid = uint32_t(std::max(1, ctx->num_cu * std::max(per_big, 1)));
     ps.big_cap = std::min(cap, kRbBigSplit);
-    per = 0;
+    per_big = 0;
     HIP_TRY(rb_big_occupancy(mode, ps.wide, int(rb_big_lds_bytes(B, ps.big_cap, mode, ps.wide)),
-                             &per));
-    ps.big_grid = uint32_t(std::max(1, ctx->num_cu * std::max(per, 1)));
+                             &per_big));
+    ps.big_grid = uint32_t(std::max(1, ctx->num_cu * std::max(per_big, 1)));
     return PDA_OK;
 }
 
@@ -404,8 +424,6 @@ int rb_enqueue_forward(pda_ctx* ctx, Slot& s, RbState& r, const Model& M,
     plan_args(a, uint64_t(units), kWave);
     PassShape ps;
     if (int rc = pass_shape(ctx, 0, n, false, a.B, cap, a.nunits, ps)) return rc;
-    RunArgs la = a;
-    la.batch = ps.batch;
     // the memo of this set: every count vector's pmf
     if (int rc = ensure_memo_layout(ctx, n)) return rc;
     const RbMemoLayout& ML = ctx->rb_memo[n];
@@ -442,9 +460,9 @@ int rb_enqueue_forward(pda_ctx* ctx, Slot& s, RbState& r, const Model& M,
                            s.stream));
     HIP_TRY(hipEventRecord(r.ev_walk, s.stream));
     HIP_TRY(hipStreamWaitEvent(s.stream, s.rb_join, 0));
-    HIP_TRY(launch_rb_unit(0, n, ps.unit_grid, d_rbm, la, r.d_cnt, r.d_F, nullptr, nullptr, nullptr,
-                           ML.d_rank_offP, ML.d_rank_offD, r.d_poolP, r.d_hist,
-                           nullptr, r.d_work, s.stream));
+    HIP_TRY(launch_rb_unit(0, n, ps.unit_grid, ps.copies, ps.tile, ps.pool, a, r.d_cnt, r.d_F,
+                           nullptr, nullptr, nullptr, ML.d_rank_offP, ML.d_rank_offD, r.d_poolP,
+                           r.d_hist, nullptr, r.d_work, s.stream));
     HIP_TRY(launch_rb_big(0, false, ps.big_grid, ps.big_cap, d_rbm, ctx->d_lf, r.d_pmf_tab, a, r.d_cnt,
                           r.d_F, nullptr, nullptr, nullptr, r.d_big, r.d_big_count, r.d_hist,
                           nullptr, s.stream));
@@ -552,8 +570,8 @@ int enqueue_derivative(pda_ctx* ctx, Slot& s, RbState& r, int mode, double* out)
     a.nstates = r.n;
     PassShape ps;
     if (int rc = pass_shape(ctx, mode, r.n, r.wide, r.B, r.cap, a.nunits, ps)) return rc;
-    RunArgs la = a;
-    la.batch = ps.batch;
+    a.queues = 1;
+    plan_args(a, a.nunits, kWave);
     const RbModel* d_rbm = static_cast<const RbModel*>(r.d_rbm);
     const RbMemoLayout& ML = ctx->rb_memo[r.n];
     const double* g = mode == 1 ? r.d_g : nullptr;
@@ -563,9 +581,9 @@ int enqueue_derivative(pda_ctx* ctx, Slot& s, RbState& r, int mode, double* out)
         HIP_TRY(launch_rb_score_mean(a, r.K, r.d_S, r.d_Sbar, ctx->num_cu, s.stream));
         r.sbar_valid = true;
     }
-    HIP_TRY(launch_rb_unit(mode, r.n, ps.unit_grid, d_rbm, la, r.d_cnt, r.d_F, r.d_S, r.d_Sbar, g,
-                           ML.d_rank_offP, ML.d_rank_offD, r.d_poolP, nullptr, out,
-                           r.d_work, s.stream));
+    HIP_TRY(launch_rb_unit(mode, r.n, ps.unit_grid, ps.copies, ps.tile, ps.pool, a, r.d_cnt,
+                           r.d_F, r.d_S, r.d_Sbar, g, ML.d_rank_offP, ML.d_rank_offD, r.d_poolP,
+                           nullptr, out, r.d_work, s.stream));
     HIP_TRY(launch_rb_big(mode, ps.wide, ps.big_grid, ps.big_cap, d_rbm, ctx->d_lf, r.d_pmf_tab, a,
                           r.d_cnt, r.d_F, r.d_S, r.d_Sbar, g, r.d_big, r.d_big_count, nullptr, out,
                           s.stream));
@@ -582,11 +600,13 @@ int enqueue_derivative(pda_ctx* ctx, Slot& s, RbState& r, int mode, double* out)
 // stream), its gradient copied to r.h_grad.
 int rb_enqueue_adjoint(pda_ctx* ctx, Slot& s, RbState& r, const double* g) {
     std::memcpy(r.h_g, g, sizeof(double) * size_t(r.B));
-    HIP_TRY(hipMemsetAsync(r.d_grad, 0, sizeof(double) * kGradLen, s.stream));
+    HIP_TRY(hipMemsetAsync(r.d_grad, 0, sizeof(double) * kGradLen * kRbGradRows, s.stream));
     HIP_TRY(hipMemcpyAsync(r.d_g, r.h_g, sizeof(double) * size_t(r.B), hipMemcpyHostToDevice,
                            s.stream));
     if (int rc = enqueue_derivative(ctx, s, r, 1, r.d_grad)) return rc;
-    HIP_TRY(hipMemcpyAsync(r.h_grad, r.d_grad, sizeof(double) * kGradLen, hipMemcpyDeviceToHost,
+    double* sum = r.d_grad + kGradLen * kRbGradRows;
+    HIP_TRY(launch_rb_rows(r.d_grad, kGradLen, kRbGradRows, sum, s.stream));
+    HIP_TRY(hipMemcpyAsync(r.h_grad, sum, sizeof(double) * kGradLen, hipMemcpyDeviceToHost,
                            s.stream));
     HIP_TRY(hipMemsetAsync(r.d_work, 0, sizeof(uint32_t) * kRbCounters, s.stream));
     r.adj_ran = true;
@@ -604,9 +624,18 @@ void rb_collect_adjoint(const RbState& r, double* grad, int nargs) {
 // Enqueues the Jacobian pass of state r's last forward, copied to r.h_jac.
 int rb_enqueue_jacobian(pda_ctx* ctx, Slot& s, RbState& r) {
     const size_t bytes = sizeof(double) * kGradLen * size_t(r.B);
-    HIP_TRY(hipMemsetAsync(r.d_jac, 0, bytes, s.stream));
+    if (r.B > r.cap_jac) {  // the caller waited for the stream
+        (void)hipFree(r.d_jac);
+        r.d_jac = nullptr;
+        r.cap_jac = 0;
+        HIP_TRY(hipMalloc(&r.d_jac, bytes * (kRbJacRows + 1)));
+        r.cap_jac = r.B;
+    }
+    HIP_TRY(hipMemsetAsync(r.d_jac, 0, bytes * kRbJacRows, s.stream));
     if (int rc = enqueue_derivative(ctx, s, r, 2, r.d_jac)) return rc;
-    HIP_TRY(hipMemcpyAsync(r.h_jac, r.d_jac, bytes, hipMemcpyDeviceToHost, s.stream));
+    double* sum = r.d_jac + size_t(kGradLen) * size_t(r.B) * kRbJacRows;
+    HIP_TRY(launch_rb_rows(r.d_jac, kGradLen * r.B, kRbJacRows, sum, s.stream));
+    HIP_TRY(hipMemcpyAsync(r.h_jac, sum, bytes, hipMemcpyDeviceToHost, s.stream));
     HIP_TRY(hipMemsetAsync(r.d_work, 0, sizeof(uint32_t) * kRbCounters, s.stream));
     r.adj_ran = true;
     return PDA_OK;

@@ -167,6 +167,15 @@ PDA_HD uint64_t rb_fixed(float P) {
     return x < 4294967296.0 ? uint64_t(uint32_t(x)) : uint64_t(x);
 }
 
+// Rows that the workgroups of a derivative pass add their sums to (workgroup g
+// to row g mod the rows), summed afterwards: thousands of waves adding to one
+// line of doubles had kept each other waiting longer than the pass itself
+// worked.  The adjoint's gradient (rows of kRbGradLen doubles) and the
+// Jacobian ([B][kRbGradLen]).
+constexpr int kRbGradLen = kRbMaxStates + kRbMaxPairs;
+constexpr int kRbGradRows = 64;
+constexpr int kRbJacRows = 8;
+
 // Summary of one unit's walk: per-state photon counts (16 bits each), F.
 PDA_HD uint2 rb_pack(const uint32_t* cnt) {
     uint2 v;

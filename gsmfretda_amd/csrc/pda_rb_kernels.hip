@@ -18,8 +18,8 @@
 //                        memo spread into the E histogram as 2^-32 fixed
 //                        point (forward), or the cotangent-weighted pmf and
 //                        its derivatives (adjoint), or the derivatives of
-//                        every bin (Jacobian); lanes over the (unit,
-//                        outcome) pairs of 64 units at a time
+//                        every bin (Jacobian); a lane per unit, the units of
+//                        a tile sorted by length
 //   rb_big_kernel        the same for the listed units, one wave per unit,
 //                        lanes over acceptor totals, the pmf built in LDS
 //   rb_score_mean_kernel per burst, the mean score of its R resamples
@@ -45,14 +45,12 @@ namespace pda {
 // units have Mt < 48.
 constexpr int kRbMemoWaves = 4;  // waves per workgroup of rb_memo_kernel
 static_assert(kRbMemoCap <= kWave, "a memo pmf fits the lanes of a wave");
-// rb_unit_kernel: waves per workgroup, and its work counters (the
-// kAuxQueues lines after the walk's, workgroup g on counter g % kAuxQueues,
-// each over a contiguous share of the units: one queue per XCD).
-constexpr int kRbUnitWaves = 4;
+// rb_unit_kernel's work counters: the kAuxQueues lines after the walk's,
+// workgroup g on counter g % kAuxQueues, each over a contiguous share of the
+// units (one queue per XCD).
 constexpr uint32_t kRbUnitCounter = kMaxQueues * kCounterStride;
-// Jacobian rows in global memory, kRbJacCols doubles each: the set's n
-// efficiency columns, then its n (n - 1) rates (rb_big_kernel's LDS rows
-// hold the rates from column kRbMaxStates).
+// rb_big_kernel's LDS rows of the Jacobian hold the rates from column
+// kRbMaxStates.
 constexpr int kRbJacCols = kRbMaxStates + kRbMaxPairs;
 
 constexpr int kRbFwd = 0, kRbGrad = 1, kRbJac = 2;
@@ -359,6 +357,7 @@ __device__ __forceinline__ void wave_lds_sync() {
 // they are built beside, and the 19,600 of three 101 us; like this 135 and
 // 14 us beside the walk.  The prefix is convolved again for each run:
 // about a tenth of the steps, and every wave independent of every other.
+typedef float Floats4 __attribute__((ext_vector_type(4), aligned(4)));
 typedef float Floats8 __attribute__((ext_vector_type(8), aligned(4)));
 static_assert(kRbMemoCap + 8 < kRbPmfTable, "rows of the pmf table follow the memo's");
 
@@ -407,272 +406,320 @@ __global__ __launch_bounds__(kWave * kRbMemoWaves) void rb_memo_kernel(
     }
 }
 
-// Owner of position j of the wave's concatenation: the last lane l with
-// pos_l <= j (pos is nondecreasing over the lanes and pos_0 = 0; a lane with
-// len 0 shares its pos with the next lane, so for j < total the last such
-// lane has len > 0).  Binary search over the lanes with shuffles; *pown
-// gets the owner's pos.
-__device__ __forceinline__ int wave_owner(int pos, int j, int* pown) {
-    int idx = 0, pbest = 0;
-#pragma unroll
-    for (int step = kWave / 2; step > 0; step >>= 1) {
-        const int t = idx + step;
-        const int p = __shfl(pos, t);
-        if (p <= j) {
-            idx = t;
-            pbest = p;
-        }
-    }
-    *pown = pbest;
-    return idx;
+// ---- units with a small acceptor total ---------------------------------------
+//
+// rb_unit_kernel takes every unit with Mt < kRbMemoCap, a lane per unit.  A
+// workgroup takes a tile of consecutive units, sorts them by Mt in LDS
+// (counting sort, longest first), and its waves take 64 of the sorted units at
+// a time, all lanes looping over their unit's outcomes a = 0..Mt together:
+// sorted, the lanes' loops are nearly of one length.  What belongs to a unit
+// (F and its reciprocal, the memo offsets, the scores, the sums over its
+// outcomes) stays in the lane's registers.  The pmfs of the smallest totals
+// (the pool's first floats) are kept in LDS, where 64 lanes read 64 blocks at
+// once; longer units read the pool in memory.
+//   forward: P(a) into the bin of a, 2^-32 fixed point;
+//   adjoint: h and sum_c P_s(c) dG(c) of the unit in registers, the unit's
+//     scores once per unit;
+//   Jacobian: the outcome's n efficiency terms, as m_s (P_s(a - 1) - P_s(a))
+//     at the bin of a (the bin boundaries' terms gathered by bin), and its
+//     n (n - 1) rate terms, into the bin's row.
+// The histogram and the rows are LDS accumulators with atomics.  The lanes of
+// a group tend to the same bins (outcome 0 is bin 0 for all), so there are
+// `copies` of each accumulator, lane l using copy l % copies, copies adjacent:
+// lanes on different copies never meet in a bank.
+// Spreading the concatenated outcomes of 64 units over the lanes instead
+// (each lane finding its outcome's unit by a search over the lanes and
+// fetching the unit's data by shuffles, about 25 LDS instructions per 64
+// outcomes besides the atomics), every wave adding its sums to one line in
+// memory at the end, took, at 3 states, 100,000 bursts x 64, 139 us forward,
+// 667 adjoint and 579 Jacobian; like this it takes 77, 152 and 215.  The
+// adjoint and the Jacobian of 4 states of fast dynamics, 50,000 x 8: 491 and
+// 123 -> 68 and 83 us.
+constexpr int kRbUnitPer = 4;  // units per thread of a full tile
+
+// Totals whose pmfs a workgroup keeps in LDS (the pool begins with them), and
+// their floats: sum over t < totals of C(t + n - 1, n - 1) (t + 1).
+__host__ __device__ constexpr int rb_lds_totals(int n) { return n == 2 ? 24 : n == 3 ? 14 : 10; }
+// Three more, for the reads of four that begin in the last block.
+__host__ __device__ constexpr int rb_lds_floats(int n) {
+    return (n == 2 ? 4900 : n == 3 ? 6020 : 5863) + 3;
+}
+// Accumulators of a workgroup per copy, in 8-byte entries: the forward's bins;
+// the Jacobian's rows of n efficiency and n (n - 1) rate columns.  (The
+// adjoint's cotangent is not an accumulator: one copy, and a 0 for the
+// outcomes outside the histogram.)
+__host__ __device__ inline int rb_unit_acc(int B, int mode, int n) {
+    return mode == kRbJac ? B * n * n : mode == kRbGrad ? B + 1 : B;
+}
+// Dynamic LDS: the accumulators, the pool's first floats, the tile's order
+// and its 64 counters (one per total, one for the group to take next).
+__host__ __device__ inline size_t rb_unit_lds(int B, int mode, int n, int copies, int threads,
+                                              bool pool) {
+    return sizeof(double) * size_t(rb_unit_acc(B, mode, n)) * size_t(copies) +
+           (pool ? sizeof(float) * size_t(rb_lds_floats(n)) : 0) +
+           sizeof(uint16_t) * size_t(threads) * kRbUnitPer + sizeof(uint32_t) * 64u;
 }
 
-// Per-wave LDS of rb_unit_kernel (doubles), derivative passes: S - Sbar per
-// unit and rate pair of the set's n states.
-__host__ __device__ inline int rb_unit_wave_doubles(int mode, int n) {
-    return mode == kRbFwd ? 0 : kWave * n * (n - 1);
-}
-// The Jacobian's LDS row per bin: n efficiency columns, then the n (n - 1)
-// rates, padded to an odd number of doubles (odd rows spread the rows'
-// entries over the banks).
-__host__ __device__ constexpr int rb_unit_jac_row(int n) { return (n + n * (n - 1)) | 1; }
-// Dynamic LDS of rb_unit_kernel: the 8-byte head (the forward's fixed-point
-// histogram, the adjoint's cotangent, the Jacobian's [B][rb_unit_jac_row]
-// rows), rounded to 16 bytes, then the waves' regions.  Sized to the set's
-// states: the 3-state Jacobian fits seven four-wave workgroups per CU.
-__host__ __device__ inline int rb_unit_head(int B, int mode, int n) {
-    return ((mode == kRbJac ? B * rb_unit_jac_row(n) : B) + 1) & ~1;
-}
-__host__ __device__ inline size_t rb_unit_lds(int B, int mode, int n) {
-    return sizeof(double) * (size_t(rb_unit_head(B, mode, n)) +
-                             size_t(kRbUnitWaves) * size_t(rb_unit_wave_doubles(mode, n)));
-}
-
-// One (unit, outcome) element of a window: its unit's lane, outcome, and
-// what the pass reads for it (prefetched one window ahead).
-struct RbElem {
-    bool act;
-    int own, pown, ai, Mi;
-    float F, P;
-    uint32_t cx, cy;
-    float pd[kRbMaxStates];  // P_s(ai) of the unit's counted states (derivative passes)
+// What one unit pass reads and writes, and its shape.
+struct RbUnitArgs {
+    const uint2* cnt;
+    const float* F;
+    const float* S;
+    const double* Sbar;
+    const double* g;
+    const uint32_t* rank_offP;
+    const uint4* rank_offD;
+    const float* poolP;
+    unsigned long long* hist_acc;
+    double* grad;
+    uint32_t* work;
+    int32_t copies;  // accumulator copies, a power of two
+    int32_t tile;    // units a workgroup takes at a time
+    int32_t pool;    // the pool's first floats are kept in LDS
 };
 
-// Every unit u < a.nunits with Mt < kRbMemoCap.  A wave takes a.batch
-// consecutive units per grab and handles them 64 at a time: the units'
-// outcomes a = 0..Mt, concatenated, are spread over the lanes in windows of
-// 64, so each lane handles one (unit, outcome) pair per window whatever the
-// units' lengths.  A lane finds its pair's unit by a binary search over the
-// lanes' start positions and takes the unit's data from that lane by
-// shuffles; the pmf entries come from the memo, each window's loads issued
-// while the previous window is processed.  No barrier after the prologue:
-// each wave adds to the workgroup's LDS accumulators with atomics.
+// rb_bin() for F in quotient_range and its reciprocal rF rounded to float; B
+// for outcomes outside the histogram.  floor(E B) from the float product: one
+// too much where the product rounded up to the next integer, which the sign
+// of the exact remainder tells.
+__device__ __forceinline__ int rb_bin_quick(int a, float F, float rF, float Bf, int B) {
+    const float E = quotient(float(a), F, rF);
+    float b = floorf(E * Bf);
+    b = fmaf(E, Bf, -b) < 0.0f ? b - 1.0f : b;
+    return E < 1.0f ? int(b) : B;
+}
+
+constexpr int rb_unit_threads_of(int mode) { return mode == kRbJac ? 1024 : 256; }
+
 template <int kMode, int kN>
-__global__ __launch_bounds__(kWave * kRbUnitWaves) __attribute__((amdgpu_waves_per_eu(
-    kMode == kRbFwd ? 1 : 4))) void rb_unit_kernel(
-    const RbModel* __restrict__ rbm, const RunArgs a, const uint2* __restrict__ cnt_in,
-    const float* __restrict__ F_in, const float* __restrict__ S_in,
-    const double* __restrict__ Sbar, const double* __restrict__ g,
-    const uint32_t* __restrict__ rank_offP, const uint4* __restrict__ rank_offD,
-    const float* __restrict__ poolP, unsigned long long* __restrict__ hist_acc,
-    double* __restrict__ grad,
-    uint32_t* __restrict__ work) {
+__global__ __launch_bounds__(rb_unit_threads_of(kMode)) void rb_unit_kernel(const RunArgs a,
+                                                                            const RbUnitArgs p) {
     constexpr bool kDeriv = kMode != kRbFwd;
-    extern __shared__ __align__(16) double s_unit[];
-    __shared__ RbModel sR;
-    const int tid = int(threadIdx.x), lane = tid % kWave, wave = tid / kWave;
+    constexpr int K = kN * (kN - 1), kCols = kN * kN;
+    constexpr int kThreads = rb_unit_threads_of(kMode);
+    extern __shared__ __align__(16) double s_acc[];
+    const int tid = int(threadIdx.x), lane = tid % kWave;
     const int B = a.B;
-    {
-        const uint32_t* src = reinterpret_cast<const uint32_t*>(rbm);
-        uint32_t* dst = reinterpret_cast<uint32_t*>(&sR);
-        for (uint32_t i = uint32_t(tid); i < sizeof(RbModel) / 4; i += blockDim.x) dst[i] = src[i];
-    }
-    const int head = rb_unit_head(B, kMode, kN);
-    unsigned long long* s_h = reinterpret_cast<unsigned long long*>(s_unit);
-    double* s_d = s_unit;
-    for (int i = tid; i < head; i += int(blockDim.x)) {
-        if (kMode == kRbGrad) s_d[i] = i < B ? g[i] : 0.0;
-        else if (kMode == kRbJac) s_d[i] = 0.0;
+    const int nacc = rb_unit_acc(B, kMode, kN) * p.copies;
+    float* s_pool = reinterpret_cast<float*>(s_acc + nacc);
+    uint16_t* s_order = reinterpret_cast<uint16_t*>(s_pool + (p.pool ? rb_lds_floats(kN) : 0));
+    uint32_t* s_count = reinterpret_cast<uint32_t*>(s_order + kThreads * kRbUnitPer);
+    unsigned long long* s_h = reinterpret_cast<unsigned long long*>(s_acc);
+    for (int i = tid; i < nacc; i += kThreads) {
+        if (kMode == kRbGrad) s_acc[i] = i < B ? p.g[i] : 0.0;
         else s_h[i] = 0ull;
     }
-    __syncthreads();
-    constexpr int n = kN, K = kN * (kN - 1);  // states and rate pairs of the set
-    constexpr int kRow = rb_unit_jac_row(kN);
-    double* w_x = s_unit + head + wave * rb_unit_wave_doubles(kMode, kN);
+    if (p.pool)
+        for (int i = tid; i < rb_lds_floats(kN); i += kThreads) s_pool[i] = p.poolP[i];
+    const int copy = lane & (p.copies - 1);
+    const float Bf = float(B);
+    const UnitDiv divR{a.div_m, a.div_sh};
 
     const uint32_t nq = gridDim.x < kAuxQueues ? gridDim.x : kAuxQueues;
     const uint32_t queue = blockIdx.x % nq;
     const uint32_t q_begin = uint32_t(uint64_t(a.nunits) * queue / nq);
     const uint32_t q_len = uint32_t(uint64_t(a.nunits) * (queue + 1u) / nq) - q_begin;
-    uint32_t* counter = &work[kRbUnitCounter + queue * kCounterStride];
-    double gp[kN] = {};  // adjoint: d h / d p_s over the lane's elements
-    double gk[K] = {};   // adjoint: G P (S - Sbar) over the lane's elements
+    uint32_t* counter = &p.work[kRbUnitCounter + queue * kCounterStride];
+    double gp[kN] = {};       // adjoint: d h / d p_s over the lane's units
+    double gk[K] = {};        // adjoint: h (S - Sbar) over the lane's units
+    unsigned long long acc0 = 0;  // forward: the units' outcomes 0 (bin 0)
     while (true) {
-        uint32_t off = 0;
-        if (lane == 0) off = atomicAdd(counter, a.batch);
-        off = __shfl(off, 0);
+        __syncthreads();  // the last tile's order and counters are free
+        if (tid < 64) s_count[tid] = 0u;
+        if (tid == 63) s_count[63] = atomicAdd(counter, uint32_t(p.tile));
+        __syncthreads();
+        const uint32_t off = s_count[63];
         if (off >= q_len) break;
-        const uint32_t end = q_len - off < a.batch ? q_len : off + a.batch;
-        for (uint32_t r0 = off; r0 < end; r0 += kWave) {
-            // this lane's unit of the round
-            const uint32_t o = r0 + uint32_t(lane);
-            const bool valid = o < end;
-            const uint32_t u = q_begin + (valid ? o : r0);
-            const uint2 c = valid ? cnt_in[u] : make_uint2(0u, 0u);
+        const uint32_t base = q_begin + off;
+        const uint32_t len = q_len - off < uint32_t(p.tile) ? q_len - off : uint32_t(p.tile);
+        // counting sort by total, the longest first; units with Mt >=
+        // kRbMemoCap are left out (the walk listed them for rb_big_kernel)
+        uint32_t key[kRbUnitPer], rank[kRbUnitPer];
+#pragma unroll
+        for (int j = 0; j < kRbUnitPer; ++j) {
+            const uint32_t i = uint32_t(tid + j * kThreads);
+            key[j] = kRbMemoCap;
+            if (i < len) {
+                const uint2 c = p.cnt[base + i];
+                const uint32_t mt = (c.x & 0xFFFFu) + (c.x >> 16) + (c.y & 0xFFFFu) + (c.y >> 16);
+                if (mt < uint32_t(kRbMemoCap)) key[j] = uint32_t(kRbMemoCap) - 1u - mt;
+            }
+            rank[j] = key[j] < uint32_t(kRbMemoCap) ? atomicAdd(&s_count[key[j]], 1u) : 0u;
+        }
+        __syncthreads();
+        if (tid < kWave) {
+            const uint32_t v = lane < kRbMemoCap ? s_count[lane] : 0u;
+            const uint32_t incl = uint32_t(wave_scan_sum(int(v), lane));
+            s_count[lane] = lane <= kRbMemoCap ? incl - v : 0u;  // [kRbMemoCap]: how many
+        }
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < kRbUnitPer; ++j)
+            if (key[j] < uint32_t(kRbMemoCap))
+                s_order[s_count[key[j]] + rank[j]] = uint16_t(tid + j * kThreads);
+        const uint32_t count = s_count[kRbMemoCap];
+        __syncthreads();
+
+        while (true) {
+            uint32_t first = 0;
+            if (lane == 0) first = atomicAdd(&s_count[62], uint32_t(kWave));
+            first = uint32_t(__builtin_amdgcn_readfirstlane(int(first)));
+            if (first >= count) break;
+            const bool valid = first + uint32_t(lane) < count;
+            const uint32_t u = base + s_order[valid ? first + uint32_t(lane) : first];
+            const uint2 c = p.cnt[u];
+            const float F = p.F[u];
             int mm[kRbMaxStates] = {0, 0, 0, 0};
-            int Mt = 0;
+            int total = 0;
 #pragma unroll
             for (int s = 0; s < kN; ++s) {
                 mm[s] = int(rb_count(c, s));
-                Mt += mm[s];
+                total += mm[s];
             }
-            // units with Mt >= kRbMemoCap: listed by the walk for rb_big_kernel
-            const bool memo = valid && Mt < kRbMemoCap;
-            const int len = memo ? Mt + 1 : 0;
-            uint32_t offP = 0;
-            uint4 offD = make_uint4(0u, 0u, 0u, 0u);
-            float F = 0.0f;
-            // derivative passes: the unit's score less its burst's mean, in
-            // the wave's LDS
-            double* w_sc = w_x + lane * K;
-            if (memo) {
-                const uint32_t rk = rb_rank(mm, n, kRbMemoCap - 1);
-                offP = rank_offP[rk];
-                F = F_in[u];
-                if (kDeriv) offD = rank_offD[rk];
-            }
+            const int Mt = valid ? total : -1;
+            const int longest = __builtin_amdgcn_readfirstlane(total);  // sorted
+            const uint32_t rk = rb_rank(mm, kN, kRbMemoCap - 1);
+            const uint32_t offP = p.rank_offP[rk];
+            uint32_t offD[kN];  // the pmfs without a trial of state s (uncounted: any block)
             if (kDeriv) {
-                const uint32_t bl = u / a.R;
+                const uint4 d = p.rank_offD[rk];
+                int js = 0;
+#pragma unroll
+                for (int s = 0; s < kN; ++s) {
+                    const bool counted = mm[s] > 0;
+                    const uint32_t o = js == 0 ? d.x : js == 1 ? d.y : js == 2 ? d.z : d.w;
+                    offD[s] = counted ? o : offP;
+                    js += counted ? 1 : 0;
+                }
+            }
+            double sc[kMode == kRbJac ? K : 1];  // Jacobian: S - Sbar
+            const uint32_t bl = kDeriv ? unit_div(u, divR) : 0u;
+            if (kMode == kRbJac) {
 #pragma unroll
                 for (int k = 0; k < K; ++k)
-                    w_sc[k] = memo ? double(S_in[size_t(u) * size_t(K) + size_t(k)]) -
-                                                  Sbar[size_t(bl) * size_t(K) + size_t(k)]
-                                            : 0.0;
+                    sc[k] = double(p.S[size_t(u) * size_t(K) + size_t(k)]) -
+                            p.Sbar[size_t(bl) * size_t(K) + size_t(k)];
             }
-            const int incl = wave_scan_sum(len, lane);
-            const int pos = incl - len;
-            const int total = __shfl(incl, kWave - 1);
-            if (kDeriv) wave_lds_sync();
-
-            auto fetch = [&](int wb, RbElem& e) {
-                const int j = wb + lane;
-                e.act = j < total;
-                e.own = wave_owner(pos, j, &e.pown);
-                e.ai = j - e.pown;
-                e.F = __shfl(F, e.own);
-                const uint32_t op = __shfl(offP, e.own);
-                e.P = e.act ? poolP[op + uint32_t(e.ai)] : 0.0f;
-                if (kDeriv) {
-                    e.cx = __shfl(c.x, e.own);
-                    e.cy = __shfl(c.y, e.own);
-                    const uint2 ci = make_uint2(e.cx, e.cy);
-                    const uint32_t d0 = __shfl(offD.x, e.own), d1 = __shfl(offD.y, e.own);
-                    const uint32_t d2 = __shfl(offD.z, e.own), d3 = __shfl(offD.w, e.own);
-                    int Mi = 0;
+            const bool in_range = quotient_range(F);
+            const float rF = 1.0f / F;
+            const bool quick = __all(in_range);  // F = 0, or far from 1: the plain quotient
+            double h = 0.0, G_last = 0.0, hs[kN] = {};
+            float pd_last[kN] = {};
+            // four outcomes at a time; four(offset, v): entries offset ..
+            // offset + 3.  Lanes past their unit's outcomes read on into the
+            // blocks that follow.
+            auto outcomes = [&](auto&& four) {
+                for (int q0 = 0; q0 <= longest; q0 += 4) {
+                    float P4[4], D4[kN][4];
+                    four(offP + uint32_t(q0), P4);
+                    if (kDeriv) {
 #pragma unroll
-                    for (int s = 0; s < kN; ++s) Mi += int(rb_count(ci, s));
-                    e.Mi = Mi;
-                    const bool inner = e.act && e.ai < Mi;
-                    int js = 0;
-#pragma unroll
-                    for (int s = 0; s < kN; ++s) {
-                        const bool counted = rb_count(ci, s) > 0u;
-                        const uint32_t base = js == 0 ? d0 : js == 1 ? d1 : js == 2 ? d2 : d3;
-                        e.pd[s] = inner && counted ? poolP[base + uint32_t(e.ai)] : 0.0f;
-                        js += counted ? 1 : 0;
+                        for (int s = 0; s < kN; ++s) four(offD[s] + uint32_t(q0), D4[s]);
                     }
-                }
-            };
-            auto process = [&](const RbElem& e, int wb) {
-                const int b0 = e.act ? rb_bin(e.ai, e.F, B) : -1;
-                if (kMode == kRbFwd) {
-                    if (b0 >= 0) atomicAdd(&s_h[b0], (unsigned long long)rb_fixed(e.P));
-                    return;
-                }
-                // the next outcome's bin: from the next lane, which holds it
-                // unless this lane is the window's last
-                int b1 = __shfl_down(b0, 1);
-                const bool inner = e.act && e.ai < e.Mi;
-                if (inner && lane == kWave - 1) b1 = rb_bin(e.ai + 1, e.F, B);
-                const uint2 ci = make_uint2(e.cx, e.cy);
-                if (kMode == kRbGrad) {
-                    const double G0 = b0 >= 0 ? s_d[b0] : 0.0;
-                    if (inner) {
-                        const double G1 = b1 >= 0 ? s_d[b1] : 0.0;
-                        const double dG = double(float(G1 - G0));
 #pragma unroll
-                        for (int s = 0; s < kN; ++s)
-                            gp[s] += double(rb_count(ci, s)) * double(e.pd[s]) * dG;
-                    }
-                    // h (S - Sbar) of the unit, one element at a time (h is
-                    // the sum of G(bin(a)) P(a) over the unit's outcomes)
-                    if (e.act && b0 >= 0) {
-                        const double hv = G0 * double(e.P);
-                        const double* scu = w_x + e.own * K;
+                    for (int j = 0; j < 4; ++j) {
+                        const int q = q0 + j;
+                        const bool act = q <= Mt;
+                        const float P = P4[j];
+                        int b = 0;
+                        if (quick) {
+                            b = rb_bin_quick(q, F, rF, Bf, B);
+                        } else {
+                            b = rb_bin(q, F, B);
+                            b = b < 0 ? B : b;
+                        }
+                        if constexpr (kMode == kRbFwd) {
+                            const uint64_t w = act ? rb_fixed(P) : 0u;
+                            if (q == 0) acc0 += w;  // E = 0: bin 0
+                            else if (act && b < B)
+                                atomicAdd(&s_h[b * p.copies + copy], (unsigned long long)w);
+                        } else if constexpr (kMode == kRbGrad) {
+                            // sum_c P_s(c) (G(bin(c + 1)) - G(bin(c))), c = q - 1
+                            const double G = s_acc[b];
+                            const double dG = act ? double(float(G - G_last)) : 0.0;
+                            h += G * double(act ? P : 0.0f);
+                            G_last = G;
 #pragma unroll
-                        for (int k = 0; k < K; ++k)
-                            gk[k] += hv * scu[k];
-                    }
-                } else {
-                    if (b0 >= 0) {
-                        double* row = s_d + b0 * kRow + kN;
-                        const double* scu = w_x + e.own * K;
+                            for (int s = 0; s < kN; ++s) {
+                                hs[s] += double(pd_last[s]) * dG;
+                                pd_last[s] = D4[s][j];
+                            }
+                        } else {
+                            double e[kN];
 #pragma unroll
-                        for (int k = 0; k < K; ++k)
-                            atomicAdd(&row[k], double(e.P) * scu[k]);
-                    }
-                    if (inner && b0 != b1) {
+                            for (int s = 0; s < kN; ++s) {
+                                const float pd = q < Mt ? D4[s][j] : 0.0f;
+                                e[s] = double(mm[s]) * (double(pd_last[s]) - double(pd));
+                                pd_last[s] = pd;
+                            }
+                            if (act && b < B) {
+                                double* row = s_acc + size_t(b * kCols) * size_t(p.copies) + copy;
 #pragma unroll
-                        for (int s = 0; s < kN; ++s) {
-                            const uint32_t m = rb_count(ci, s);
-                            if (m > 0u) {
-                                const double w = double(m) * double(e.pd[s]);
-                                if (b1 >= 0) atomicAdd(&s_d[b1 * kRow + s], w);
-                                if (b0 >= 0) atomicAdd(&s_d[b0 * kRow + s], -w);
+                                for (int s = 0; s < kN; ++s) atomicAdd(&row[s * p.copies], e[s]);
+#pragma unroll
+                                for (int k = 0; k < K; ++k)
+                                    atomicAdd(&row[(kN + k) * p.copies], double(P) * sc[k]);
                             }
                         }
                     }
                 }
             };
-            if (total > 0) {
-                RbElem cur, nxt;
-                fetch(0, cur);
-                for (int wb = 0; wb < total; wb += kWave) {
-                    if (wb + kWave < total) fetch(wb + kWave, nxt);
-                    process(cur, wb);
-                    cur = nxt;
-                }
+            if (p.pool && longest < rb_lds_totals(kN))
+                outcomes([&](uint32_t o, float* v) {
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) v[j] = s_pool[o + uint32_t(j)];
+                });
+            else
+                outcomes([&](uint32_t o, float* v) {
+                    const Floats4 x = *reinterpret_cast<const Floats4*>(p.poolP + o);
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) v[j] = x[j];
+                });
+            if (kMode == kRbGrad && valid) {
+#pragma unroll
+                for (int s = 0; s < kN; ++s) gp[s] += double(mm[s]) * hs[s];
+#pragma unroll
+                for (int k = 0; k < K; ++k)
+                    gk[k] += h * (double(p.S[size_t(u) * size_t(K) + size_t(k)]) -
+                                  p.Sbar[size_t(bl) * size_t(K) + size_t(k)]);
             }
-            if (kDeriv) wave_lds_sync();  // the round's LDS reads before the next round's writes
         }
     }
+    const double f = a.R > 1 ? double(a.R) / double(a.R - 1) : 0.0;
     if (kMode == kRbFwd) {
+        atomicAdd(&s_h[copy], acc0);
         __syncthreads();
-        unsigned long long* row = hist_acc + size_t(blockIdx.x & 7u) * kMaxBins;
-        for (int i = tid; i < B; i += int(blockDim.x))
-            if (s_h[i]) atomicAdd(&row[i], s_h[i]);
+        unsigned long long* row = p.hist_acc + size_t(blockIdx.x & 7u) * kMaxBins;
+        for (int i = tid; i < B; i += kThreads) {
+            unsigned long long v = 0;
+            for (int x = 0; x < p.copies; ++x) v += s_h[i * p.copies + x];
+            if (v) atomicAdd(&row[i], v);
+        }
     } else if (kMode == kRbGrad) {
-        const double f = a.R > 1 ? double(a.R) / double(a.R - 1) : 0.0;
+        // the workgroup's sums, in the cotangent's place
+        double* s_sum = reinterpret_cast<double*>(s_acc);
+        __syncthreads();
+        if (tid < kCols) s_sum[tid] = 0.0;
+        __syncthreads();
 #pragma unroll
-        for (int s = 0; s < kN; ++s) {
-            const double v = wave_sum(gp[s]);
-            if (lane == 0 && s < n) atomicAdd(&grad[s], v);
+        for (int i = 0; i < kCols; ++i) {
+            const double v = wave_sum(i < kN ? gp[i < kN ? i : 0] : f * gk[i < kN ? 0 : i - kN]);
+            if (lane == 0) atomicAdd(&s_sum[i], v);
         }
-#pragma unroll
-        for (int k = 0; k < K; ++k) {
-            const double v = wave_sum(gk[k]);
-            if (lane == 0) atomicAdd(&grad[n + k], f * v);
-        }
+        __syncthreads();
+        double* row = p.grad + size_t(blockIdx.x % kRbGradRows) * kRbGradLen;
+        if (tid < kCols) atomicAdd(&row[tid], s_sum[tid]);
     } else {
         // grad holds J[b][i], i < n + K (efficiencies, then rates in args
-        // order), B rows of kRbJacCols
+        // order), B rows of kRbGradLen, kRbJacRows times
         __syncthreads();
-        const double f = a.R > 1 ? double(a.R) / double(a.R - 1) : 0.0;
-        const int w = n + K;
-        for (int i = tid; i < B * w; i += int(blockDim.x)) {
-            const int b = i / w, col = i - b * w;
-            const double v = col < n ? s_d[b * kRow + col] : f * s_d[b * kRow + col];
-            if (v != 0.0) atomicAdd(&grad[size_t(b) * kRbJacCols + size_t(col)], v);
+        double* J = p.grad + size_t(blockIdx.x % kRbJacRows) * size_t(B) * kRbGradLen;
+        for (int i = tid; i < B * kCols; i += kThreads) {
+            const int b = i / kCols, col = i - b * kCols;
+            double v = 0.0;
+            for (int x = 0; x < p.copies; ++x) v += s_acc[size_t(i) * size_t(p.copies) + size_t(x)];
+            if (col >= kN) v *= f;
+            if (v != 0.0) atomicAdd(&J[size_t(b) * kRbGradLen + size_t(col)], v);
         }
     }
 }
@@ -862,16 +909,18 @@ __global__ __launch_bounds__(kWave) void rb_big_kernel(
             if (s_h[i]) atomicAdd(&row[i], s_h[i]);
     } else if (kMode == kRbGrad) {
         const double f = a.R > 1 ? double(a.R) / double(a.R - 1) : 0.0;
-        if (int(lane) < n) atomicAdd(&grad[lane], gp_acc);
-        if (int(lane) < K) atomicAdd(&grad[n + int(lane)], f * gk_acc);
+        double* row = grad + size_t(blockIdx.x % kRbGradRows) * kRbGradLen;
+        if (int(lane) < n) atomicAdd(&row[lane], gp_acc);
+        if (int(lane) < K) atomicAdd(&row[n + int(lane)], f * gk_acc);
     } else {
         const double f = a.R > 1 ? double(a.R) / double(a.R - 1) : 0.0;
         const int w = n + K;
+        double* J = grad + size_t(blockIdx.x % kRbJacRows) * size_t(B) * kRbGradLen;
         for (int i = int(lane); i < B * w; i += kWave) {
             const int b = i / w, col = i - b * w;
             const double v = col < n ? s_d[b * kRbJacCols + col]
                                      : f * s_d[b * kRbJacCols + kRbMaxStates + (col - n)];
-            if (v != 0.0) atomicAdd(&grad[size_t(b) * kRbJacCols + size_t(col)], v);
+            if (v != 0.0) atomicAdd(&J[size_t(b) * kRbGradLen + size_t(col)], v);
         }
     }
 }
@@ -932,6 +981,22 @@ __global__ void rb_table_kernel(const RbModel* __restrict__ rbm, const double* _
     pmf_tab[i] = float(rb_binom_pmf(m, k, lf, rbm->p[s], rbm->lp[s], rbm->lq[s]));
 }
 
+// Sums the rows of a derivative pass: n sums of `rows` values `stride` apart, a
+// group of kLanes lanes per sum.
+template <int kLanes>
+__global__ __launch_bounds__(256) void rb_rows_kernel(const double* __restrict__ rows_in, int n,
+                                                      int rows, int stride,
+                                                      double* __restrict__ out) {
+    const int t = int(blockIdx.x * blockDim.x + threadIdx.x);
+    const int i = t / kLanes, l = t % kLanes;
+    double v = 0.0;
+    if (i < n)
+        for (int r = l; r < rows; r += kLanes) v += rows_in[size_t(r) * size_t(stride) + size_t(i)];
+#pragma unroll
+    for (int o = kLanes / 2; o > 0; o >>= 1) v += __shfl_xor(v, o);
+    if (i < n && l == 0) out[i] = v;
+}
+
 // Device result of an RB run, followed by uint64 M[B] (2^-32 units).
 struct RbResultHeader {
     double chi2;
@@ -988,7 +1053,7 @@ hipError_t rb_walk_occupancy(bool scores, int n, int* per_cu) {
 
 template <int kMode>
 static hipError_t rb_unit_occupancy_m(int n, size_t l, int* per_cu) {
-    const int tu = kWave * kRbUnitWaves;
+    const int tu = rb_unit_threads_of(kMode);
     if (n == 2) return hipOccupancyMaxActiveBlocksPerMultiprocessor(per_cu, rb_unit_kernel<kMode, 2>, tu, l);
     if (n == 3) return hipOccupancyMaxActiveBlocksPerMultiprocessor(per_cu, rb_unit_kernel<kMode, 3>, tu, l);
     return hipOccupancyMaxActiveBlocksPerMultiprocessor(per_cu, rb_unit_kernel<kMode, 4>, tu, l);
@@ -1049,8 +1114,10 @@ hipError_t launch_rb_walk(bool scores, int n, uint32_t grid, uint32_t replay_gri
     return hipGetLastError();
 }
 
-int rb_unit_threads() { return kWave * kRbUnitWaves; }
-size_t rb_unit_lds_bytes(int B, int mode, int n) { return rb_unit_lds(B, mode, n); }
+int rb_unit_threads(int mode) { return rb_unit_threads_of(mode); }
+size_t rb_unit_lds_bytes(int B, int mode, int n, int copies, bool pool) {
+    return rb_unit_lds(B, mode, n, copies, rb_unit_threads_of(mode), pool);
+}
 size_t rb_big_lds_bytes(int B, int cap, int mode, bool wide) { return rb_big_lds(B, cap, mode, wide); }
 
 hipError_t launch_rb_table(const RbModel* rbm, const double* lf, float* pmf_tab, int n,
@@ -1077,30 +1144,26 @@ hipError_t launch_rb_memo(int n, const float* pmf_tab, const uint4* items, uint3
 }
 
 template <int kMode, int kN>
-static void launch_rb_unit_n(uint32_t grid, size_t lds, const RbModel* rbm, const RunArgs& a,
-                             const uint2* cnt, const float* F, const float* S, const double* Sbar,
-                             const double* g, const uint32_t* rank_offP, const uint4* rank_offD,
-                             const float* poolP, unsigned long long* hist_acc, double* grad,
-                             uint32_t* work, hipStream_t stream) {
-    hipLaunchKernelGGL((rb_unit_kernel<kMode, kN>), dim3(grid), dim3(uint32_t(kWave * kRbUnitWaves)),
-                       lds, stream, rbm, a, cnt, F, S, Sbar, g, rank_offP, rank_offD, poolP,
-                       hist_acc, grad, work);
+static void launch_rb_unit_n(uint32_t grid, const RunArgs& a, const RbUnitArgs& p,
+                             hipStream_t stream) {
+    const int threads = rb_unit_threads_of(kMode);
+    hipLaunchKernelGGL((rb_unit_kernel<kMode, kN>), dim3(grid), dim3(uint32_t(threads)),
+                       rb_unit_lds(a.B, kMode, kN, p.copies, threads, p.pool != 0), stream, a, p);
 }
 
-hipError_t launch_rb_unit(int mode, int n, uint32_t grid, const RbModel* rbm, const RunArgs& a,
-                          const uint2* cnt, const float* F, const float* S, const double* Sbar,
-                          const double* g, const uint32_t* rank_offP, const uint4* rank_offD,
-                          const float* poolP, unsigned long long* hist_acc, double* grad,
-                          uint32_t* work, hipStream_t stream) {
+hipError_t launch_rb_unit(int mode, int n, uint32_t grid, int copies, int tile, bool pool,
+                          const RunArgs& a, const uint2* cnt, const float* F, const float* S,
+                          const double* Sbar, const double* g, const uint32_t* rank_offP,
+                          const uint4* rank_offD, const float* poolP,
+                          unsigned long long* hist_acc, double* grad, uint32_t* work,
+                          hipStream_t stream) {
     if (n < 2 || n > kRbMaxStates) return hipErrorInvalidValue;
-    const size_t lds = rb_unit_lds(a.B, mode, n);
-#define PDA_RB_UNIT(M, N)                                                                      \
-    launch_rb_unit_n<M, N>(grid, lds, rbm, a, cnt, F, S, Sbar, g, rank_offP, rank_offD, poolP, \
-                           hist_acc, grad, work, stream)
-#define PDA_RB_UNIT_M(M)            \
-    if (n == 2) PDA_RB_UNIT(M, 2);  \
-    else if (n == 3) PDA_RB_UNIT(M, 3); \
-    else PDA_RB_UNIT(M, 4)
+    const RbUnitArgs p{cnt,      F,    S,    Sbar,   g,    rank_offP, rank_offD, poolP,
+                       hist_acc, grad, work, copies, tile, pool ? 1 : 0};
+#define PDA_RB_UNIT_M(M)                                       \
+    if (n == 2) launch_rb_unit_n<M, 2>(grid, a, p, stream);    \
+    else if (n == 3) launch_rb_unit_n<M, 3>(grid, a, p, stream); \
+    else launch_rb_unit_n<M, 4>(grid, a, p, stream)
     if (mode == kRbGrad) {
         PDA_RB_UNIT_M(kRbGrad);
     } else if (mode == kRbJac) {
@@ -1109,7 +1172,6 @@ hipError_t launch_rb_unit(int mode, int n, uint32_t grid, const RbModel* rbm, co
         PDA_RB_UNIT_M(kRbFwd);
     }
 #undef PDA_RB_UNIT_M
-#undef PDA_RB_UNIT
     return hipGetLastError();
 }
 
@@ -1155,6 +1217,16 @@ hipError_t launch_rb_score_mean(const RunArgs& a, int K, const float* S, double*
     const uint64_t cap = uint64_t(num_cu > 0 ? num_cu : 1) * 4u;
     const uint32_t grid = uint32_t(std::max<uint64_t>(1, std::min<uint64_t>(want, cap)));
     hipLaunchKernelGGL(rb_score_mean_kernel, dim3(grid), dim3(256), 0, stream, a, K, S, Sbar);
+    return hipGetLastError();
+}
+
+hipError_t launch_rb_rows(const double* rows, int n, int nrows, double* out, hipStream_t stream) {
+    if (nrows >= kWave)
+        hipLaunchKernelGGL(rb_rows_kernel<kWave>, dim3(uint32_t((n * kWave + 255) / 256)),
+                           dim3(256), 0, stream, rows, n, nrows, n, out);
+    else
+        hipLaunchKernelGGL(rb_rows_kernel<8>, dim3(uint32_t((n * 8 + 255) / 256)), dim3(256), 0,
+                           stream, rows, n, nrows, n, out);
     return hipGetLastError();
 }
 
