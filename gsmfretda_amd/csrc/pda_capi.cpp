@@ -154,7 +154,11 @@ int load_common(pda_ctx* ctx, const int64_t* start, const int64_t* stop, const i
     ctx->nbursts = nbursts;
     ctx->nphotons = total;
     ctx->h_P.resize(size_t(nbursts));
-    for (int64_t i = 0; i < nbursts; ++i) ctx->h_P[size_t(i)] = bursts[size_t(i)].P;
+    ctx->max_P = 0;
+    for (int64_t i = 0; i < nbursts; ++i) {
+        ctx->h_P[size_t(i)] = bursts[size_t(i)].P;
+        ctx->max_P = std::max(ctx->max_P, bursts[size_t(i)].P);
+    }
     ctx->clk_p = clk_p;
     ctx->bg_ad = bg_ad;
     ctx->bg_dd = bg_dd;
@@ -480,7 +484,7 @@ int pda_run(pda_ctx* ctx, int sid, int R, uint32_t seed, uint32_t set_id, int fl
     a.replay_cap = uint32_t(s->replay_cap);
     HIP_TRY(hipEventRecord(s->ev0, s->stream));
     const BinomGuide guide{s->d_thr, s->d_guide};
-    const FastArgs fa = fast_args(s->n, s->quick_rates, a.clk_p, s->ph.r0);
+    const FastArgs fa = fast_args(s->n, s->quick_rates, a.clk_p, s->ph.r0, ctx->max_P);
     HIP_TRY(launch_walk(pass, grid, ctx->d_bursts, ctx->d_ticks, ctx->d_links, s->d_blob, guide, a,
                         fa, s->d_hist_acc, s->d_replay, s->d_replay_count, s->d_work, outE, outAcc,
                         outF, s->stream));

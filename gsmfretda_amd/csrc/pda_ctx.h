@@ -233,6 +233,7 @@ struct pda_ctx {
     float* d_obs = nullptr;
     pda::LaunchShape shape;
     std::vector<uint32_t> h_P;      // photons per burst (host copy)
+    uint32_t max_P = 0;             // the most photons of a burst
     double* d_lf = nullptr;         // log k! for the RB form
     size_t lds_per_block = 65536;   // LDS a workgroup may allocate
     pda::RbMemoLayout rb_memo[5];   // by state count (2..4 used)

@@ -132,7 +132,9 @@ __device__ __forceinline__ void flush_hist(int32_t* h, int32_t* __restrict__ row
 // arguments cannot have, correctly rounded quotients from reciprocals kept
 // per model, and the launch's divisions done on the host (unit / R, the
 // queues' shares) took a 3-state evaluation of 100,000 bursts x 100 from 459
-// to 407 us and the 256-set generation from 16.7 to 14.7 ms.  The register
+// to 407 us and the 256-set generation from 16.7 to 14.7 ms; a search in
+// uniform steps, 32-bit draws and windows without early returns from there to
+// 387 us and 13.2 ms.  The register
 // limit keeps 8 waves on a SIMD (single set) or 7 (population, where 64 VGPRs
 // would spill): the window loop waits on dependent loads, which the other
 // waves hide.  (Starting 64 units at a time and queueing in LDS those that
@@ -269,11 +271,8 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(
                 r = fast_window<false, BroadDraw>(M, &draw, key, d.P, d.stop_rel, d.T, ticks,
                                                   links, a, fa, st);
             } else if (kPass == kPassGuided) {
-                const size_t base = kPop ? size_t(M.guide_base) : 0;
-                const BinomGuide g{io.guide.thr + base * kGuideStatePairs,
-                                   io.guide.guide + base * kBinomTable * kGuideBuckets};
-                r = fast_window<false, BinomGuide>(M, &g, key, d.P, d.stop_rel, d.T, ticks, links,
-                                                   a, fa, st);
+                r = fast_window<false, BinomGuide>(M, &io.guide, key, d.P, d.stop_rel, d.T, ticks,
+                                                   links, a, fa, st);
             } else {
                 r = fast_window<false, BinomTable>(M, &io.blobs[set].tab, key, d.P, d.stop_rel,
                                                    d.T, ticks, links, a, fa, st);

@@ -145,7 +145,8 @@ int enqueue_population(pda_ctx* ctx, Slot& s, int pass, uint32_t grid, const Run
         guide = BinomGuide{p.d_thr, p.d_guide};
     }
     HIP_TRY(launch_pop_walk(pass, grid, ctx->d_bursts, ctx->d_ticks, ctx->d_links, ctl, blobs,
-                            guide, a, fast_args(p.max_states, p.quick_rates, a.clk_p, p.r0),
+                            guide, a, fast_args(p.max_states, p.quick_rates, a.clk_p, p.r0,
+                                             ctx->max_P),
                             p.d_hist_acc, p.d_replay, p.d_replay_count, p.d_work,
                             s.stream));
     if (pass != kPassGeneral)

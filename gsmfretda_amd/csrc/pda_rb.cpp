@@ -455,7 +455,7 @@ int rb_enqueue_forward(pda_ctx* ctx, Slot& s, RbState& r, const Model& M,
     HIP_TRY(hipEventRecord(s.rb_join, s.rb_aux));
     HIP_TRY(launch_rb_walk(scores, n, grid, uint32_t(ctx->num_cu) * 4u, ctx->d_bursts, ctx->d_ticks,
                            ctx->d_links, d_blob, d_rbm, a,
-                           fast_args(n, M.quick_rates != 0, a.clk_p, M.r0), r.d_cnt, r.d_F, r.d_S, r.d_work,
+                           fast_args(n, M.quick_rates != 0, a.clk_p, M.r0, ctx->max_P), r.d_cnt, r.d_F, r.d_S, r.d_work,
                            r.d_big, r.d_huge, r.d_big_count, r.d_replay, r.d_replay_count,
                            s.stream));
     HIP_TRY(hipEventRecord(r.ev_walk, s.stream));

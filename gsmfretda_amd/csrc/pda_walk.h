@@ -152,34 +152,47 @@ inline int build_guide_row_host(const Model& M, const BinomTable& tab, int s, in
     return end + 1;
 }
 
+// ThrPair at index i of a table, as one load.
+PDA_HD ThrPair load_pair(const ThrPair* t, uint32_t i) {
+#ifdef __HIP_DEVICE_COMPILE__
+    typedef long Pair __attribute__((ext_vector_type(2)));
+    const Pair v = *reinterpret_cast<const Pair*>(reinterpret_cast<const char*>(t) + i * 16u);
+    return ThrPair{v.x, v.y};
+#else
+    return t[i];
+#endif
+}
+static_assert(sizeof(ThrPair) == 16, "a pair is one load");
+
 // binomial_table by the thresholds: the same X for every uniform, or -1
 // where binomial_table returns -1 and where u falls between lo_X and up_X
 // (2 kGuideBand + 2 grid points around each threshold, ~5e-13 of the grid:
 // the general form then runs the loop).
 // Two dependent loads instead of X + 1 loop passes whose count differs from
 // lane to lane.
+//
+// guided_count: X before the flip of p > 1/2, for 0 < n < kBinomTable; row is
+// the state's in the table.  Offsets are 32-bit from the tables' starts (a
+// table holds at most 1 GiB), and a pair is one 16-byte load.
+PDA_HD int guided_count(int n, uint32_t row, const BinomGuide& G, uint32_t hi, uint32_t lo) {
+    const int64_t u = (int64_t(hi >> 5) << 26) | int64_t(lo >> 6);
+    int X = G.guide[(row * uint32_t(kBinomTable) + uint32_t(n)) * uint32_t(kGuideBuckets) +
+                    (hi >> 26)];
+    uint32_t at = row * uint32_t(kGuideStatePairs) + uint32_t(n) * uint32_t(n + 3) / 2u + uint32_t(X);
+    ThrPair e = load_pair(G.thr, at);
+    while (u >= e.up) {
+        ++X;
+        e = load_pair(G.thr, ++at);
+    }
+    return u > e.lo ? -1 : X;
+}
+
 PDA_HD int64_t binomial_guided(int n, int s, const Model& M, const BinomGuide& G, uint32_t hi,
                                uint32_t lo) {
     if (n <= 0) return 0;
     if (n >= kBinomTable) return -1;
-    const int64_t u = (int64_t(hi >> 5) << 26) | int64_t(lo >> 6);
-    const size_t row = size_t(s) * kBinomTable + size_t(n);
-    int X = G.guide[row * kGuideBuckets + size_t(u >> kGuideShift)];
-    const ThrPair* t = G.thr + guide_row_offset(s, n);
-    ThrPair e = t[X];
-    while (u >= e.up) e = t[++X];
-    if (u > e.lo) return -1;
-    return M.flip[s] ? int64_t(n - X) : int64_t(X);
-}
-
-PDA_HD int64_t binomial_fast(int n, int s, const Model& M, const BinomTable& tab, uint32_t hi,
-                             uint32_t lo) {
-    return binomial_table(n, s, M, tab, hi, lo);
-}
-
-PDA_HD int64_t binomial_fast(int n, int s, const Model& M, const BinomGuide& g, uint32_t hi,
-                             uint32_t lo) {
-    return binomial_guided(n, s, M, g, hi, lo);
+    const int X = guided_count(n, uint32_t(s), G, hi, lo);
+    return X < 0 ? -1 : M.flip[s] ? n - X : X;
 }
 
 // binomial() for n < kBinomTable trials of any p, or -1 where the uniform lies
@@ -266,8 +279,9 @@ struct NoDeduce {
     using type = T;
 };
 
-// background_count() for means <= 64 (one inversion chunk); -1 otherwise
-// (also for caps of 2^30 photons or more, which a 32-bit counter could pass).
+// background_count() for means <= 64 (one inversion chunk) and caps below 2^30
+// photons, which a 32-bit counter cannot pass (background_single: -1 for
+// others).
 // The inversion's first two steps run for every lane without a branch: their
 // divisions by 1 and 2 are exact (the identity and a power-of-two scaling),
 // so pk * lam and (pk * lam) * 0.5 round to the loop's values; the loop then
@@ -276,8 +290,7 @@ struct NoDeduce {
 // longer runs the loop as often as its longest draw needs.  (The cumulative
 // sums do not decrease, so a uniform beyond one is beyond those before; a
 // mean of 0 or less has exp(0) = 1, which no uniform exceeds.)
-PDA_HD float background_single(float lam, float cap, float u_first, float u_cap) {
-    if (lam > 64.0f || !(cap < 0x1p30f)) return -1.0f;
+PDA_HD float background_capped(float lam, float cap, float u_first, float u_cap) {
     lam = fmaxf(lam, 0.0f);
     const float pk0 = fexp_minus(lam);
     const float pk1 = pk0 * lam;
@@ -296,6 +309,10 @@ PDA_HD float background_single(float lam, float cap, float u_first, float u_cap)
         }
     }
     return float(k) <= cap ? float(k) : floorf(cap * u_cap);
+}
+PDA_HD float background_single(float lam, float cap, float u_first, float u_cap) {
+    if (lam > 64.0f || !(cap < 0x1p30f)) return -1.0f;
+    return background_capped(lam, cap, u_first, u_cap);
 }
 
 // Walk state of one unit between windows.  The fast form keeps the window
@@ -451,15 +468,43 @@ PDA_HD int general_window(const Model& M, const UnitKey& key, uint32_t P, uint32
 // launch: jumps = the largest state count - 2, the comparisons of the
 // next-state draw; quick: the rates and the tick length are in quotient()'s
 // range; clk_r: 1 / clk_p rounded to float; r0_r: 1 / r0, or 0 when r0 is
-// out of that range.
+// out of that range; top: the largest power of two up to the photons of the
+// longest burst, the first step of the window ends' search.
 struct FastArgs {
     int32_t jumps;
     int32_t quick;
     float clk_r, r0_r;
+    uint32_t top;
 };
-PDA_HD FastArgs fast_args(int max_states, bool quick_rates, float clk_p, float r0) {
+PDA_HD FastArgs fast_args(int max_states, bool quick_rates, float clk_p, float r0,
+                          uint32_t max_photons) {
+    uint32_t top = 1;
+    while (top <= max_photons / 2u) top *= 2u;
     return FastArgs{max_states - 2, quick_rates && quotient_range(clk_p) ? 1 : 0, 1.0f / clk_p,
-                    quotient_range(r0) ? 1.0f / r0 : 0.0f};
+                    quotient_range(r0) ? 1.0f / r0 : 0.0f, top};
+}
+
+// window_close() by steps of decreasing powers of two, the same for every
+// lane: pos is the last photon found so far whose tick is below w1 (c - 1:
+// none).  A step past the burst looks at its last photon: were that below w1,
+// so were all.  Five vector instructions a step and a uniform loop, where the
+// halving of each lane's own interval took eight and the wave's exec mask.
+PDA_HD uint32_t step_close(const uint32_t* tick, const uint2* link, uint32_t c, uint32_t last,
+                           uint32_t w1, uint32_t top) {
+    uint32_t pos = c - 1u;
+    uint32_t step = top;
+#ifdef __HIP_DEVICE_COMPILE__
+    while (step > 1u && !__any(last - c >= step)) step >>= 1;
+#endif
+#pragma unroll 1
+    for (; step > 0u; step >>= 1) {
+        const uint32_t next = pos + step;
+        const uint32_t i = next < last ? next : last;
+        pos = tick[i] < w1 ? i : pos;
+    }
+    const uint32_t at = pos + 1u < last ? pos + 1u : last;
+    const uint32_t f1 = link[at].x & kIndexMask;
+    return f1 < last ? f1 : last;
 }
 
 // Tab of fast_window for models with distance broadening: the efficiency is
@@ -482,25 +527,22 @@ PDA_HD int fast_window(const Model& M, const typename NoDeduce<Tab>::type* tab, 
     // next state: the running sums do not decrease, so the first one above u
     // comes after as many as are not above it (a rate sum of 0 makes them
     // NaN, never above); the entries from n - 2 on are +inf
-    int j = 0;
-    if (fa.jumps > 0) {
-        const float u = uniform24(A.w[0]);
-        j = (M.nscum[s][0] > u ? 0 : 1) + (M.nscum[s][1] > u ? 0 : 1);
-        for (int i = 2; i < fa.jumps; ++i) j += M.nscum[s][i] > u ? 0 : 1;
-    }
+    const float us = uniform24(A.w[0]);
+    int j = (M.nscum[s][0] > us ? 0 : 1) + (M.nscum[s][1] > us ? 0 : 1);
+#pragma unroll 1
+    for (int i = 2; i < fa.jumps; ++i) j += M.nscum[s][i] > us ? 0 : 1;
     j += j >= s ? 1 : 0;
     const float lg = flog_uniform24(A.w[1]);
     const float mk = M.kdiv[s][j][0];
     const float tau = fa.quick ? quotient(lg, mk, M.kdiv[s][j][1]) : lg / mk;
     const float tsum = st.tsum + tau;
-    uint32_t w1 = stop_rel;
-    if (tsum < T) {
-        const float ticks = fa.quick ? quotient(tsum, a.clk_p, fa.clk_r) : tsum / a.clk_p;
-        const float wf = float(st.w0) + ticks;
-        if (!(wf < 0x1p31f)) return kStepReplay;
-        w1 = uint32_t(wf);
-    }
-    const uint32_t close = window_close(tick, link, st.c, last, w1);
+    const float ticks = fa.quick ? quotient(tsum, a.clk_p, fa.clk_r) : tsum / a.clk_p;
+    const float wf = float(st.w0) + ticks;
+    const bool ends = !(tsum < T);
+    // bad: the window needs the general form (its values below are not used)
+    bool bad = !ends && !(wf < 0x1p31f);
+    const uint32_t w1 = ends ? stop_rel : bad ? 0u : uint32_t(wf);
+    const uint32_t close = step_close(tick, link, st.c, last, w1, fa.top);
     // the count of the one colour the window has (0 for a photon in both
     // channels, whose run ends at itself)
     const uint2 L = link[st.c];
@@ -516,26 +558,25 @@ PDA_HD int fast_window(const Model& M, const typename NoDeduce<Tab>::type* tab, 
         // 0 whatever its uniforms are (k = 0, or past the cap with
         // floor(0 u) = 0): only the other is made, on its channel's rate and
         // words (the window leaves the fast form when either mean is above
-        // 64).  One exponential and one inversion
-        // loop per window instead of two, whose lanes had each waited for
-        // the other channel's (with two draws a 3-state evaluation of
-        // 100,000 bursts x 100 took 434 us and the 256-set generation
-        // 19.9 ms, with one 417 us and 19.1 ms; under a 30 kHz background
-        // 323 and 275 us).  (fv - bgd) - bga is fv - bg then, exactly.
+        // 64).  One exponential and one inversion loop per window instead of
+        // two, whose lanes had each waited for the other channel's (with two
+        // draws a 3-state evaluation of 100,000 bursts x 100 took 434 us and
+        // the 256-set generation 19.9 ms, with one 417 us and 19.1 ms; under
+        // a 30 kHz background 323 and 275 us).  (fv - bgd) - bga is fv - bg
+        // then, exactly.
         const Block Bk = draw_block(key, w, kSubBackground);
         const float dt = float(int32_t(w1 - st.w0)) * a.clk_p;
-        const float lam = dt * (donor ? a.bg_dd : a.bg_ad);
-        if (dt * fmaxf(a.bg_ad, a.bg_dd) > 64.0f) return kStepReplay;
-        const float bg = background_single(lam, fv, uniform24(donor ? Bk.w[1] : Bk.w[0]),
-                                           uniform24(donor ? Bk.w[3] : Bk.w[2]));
-        if (bg < 0.0f) return kStepReplay;
-        m = fv - bg;
+        bad = bad || dt * fmaxf(a.bg_ad, a.bg_dd) > 64.0f || !(fv < 0x1p30f);
+        const float lam = fminf(dt * (donor ? a.bg_dd : a.bg_ad), 64.0f);
+        m = fv - background_capped(lam, bad ? 0.0f : fv, uniform24(donor ? Bk.w[1] : Bk.w[0]),
+                                   uniform24(donor ? Bk.w[3] : Bk.w[2]));
     }
     m = floorf(m + 0.5f);
     if (kCounts) {
         *wi = WindowInfo{s, j, tau, int32_t(m)};
     } else {
-        int x;
+        const int n = int(m);
+        int x = 0;
         if constexpr (std::is_same<Tab, BroadDraw>::value) {
             // broadened efficiency (drawE, src/gen_rand.cuh:63-68)
             float de = M.ep0[s];
@@ -545,11 +586,19 @@ PDA_HD int fast_window(const Model& M, const typename NoDeduce<Tab>::type* tab, 
                 de = fa.r0_r != 0.0f ? distance_efficiency_quick(rd, M.r0, fa.r0_r)
                                      : distance_efficiency(rd, M.r0);
             }
-            x = binomial_broad(int(m), de, A.w[2], A.w[3]);
+            x = binomial_broad(n, de, A.w[2], A.w[3]);
+            bad = bad || x < 0;
+        } else if constexpr (std::is_same<Tab, BinomGuide>::value) {
+            bad = bad || n >= kBinomTable;
+            if (n > 0 && !bad) {
+                x = guided_count(n, uint32_t(M.guide_base + s), *tab, A.w[2], A.w[3]);
+                bad = x < 0;
+                x = M.flip[s] ? n - x : x;
+            }
         } else {
-            x = int(binomial_fast(int(m), s, M, *tab, A.w[2], A.w[3]));
+            x = int(binomial_table(n, s, M, *tab, A.w[2], A.w[3]));
+            bad = bad || x < 0;
         }
-        if (x < 0) return kStepReplay;
         st.acc += float(x);
     }
     st.F += fv;
@@ -558,6 +607,7 @@ PDA_HD int fast_window(const Model& M, const typename NoDeduce<Tab>::type* tab, 
     st.s = j;
     st.c = close;
     st.w = w + 1u;
+    if (bad) return kStepReplay;
     if (close == last || !(T > tsum) || st.w >= kMaxWindows) return kStepDone;
     return kStepMore;
 }
@@ -570,7 +620,7 @@ PDA_HD WalkOut walk_unit(const Model& M, const typename NoDeduce<Tab>::type* tab
     WalkState<kFast> st;
     int r = begin_unit<kFast>(M, key, P, T, st);
     if constexpr (kFast) {
-        const FastArgs fa = fast_args(M.n, M.quick_rates != 0, a.clk_p, M.r0);
+        const FastArgs fa = fast_args(M.n, M.quick_rates != 0, a.clk_p, M.r0, P);
         while (r == kStepMore)
             r = fast_window<false, Tab>(M, tab, key, P, stop_rel, T, tick, link, a, fa, st);
     } else {
