@@ -134,19 +134,20 @@ __device__ __forceinline__ void flush_hist(int32_t* h, int32_t* __restrict__ row
 // queues' shares) took a 3-state evaluation of 100,000 bursts x 100 from 459
 // to 407 us and the 256-set generation from 16.7 to 14.7 ms; a search in
 // uniform steps, 32-bit draws and windows without early returns from there to
-// 387 us and 13.2 ms.  The register
-// limit keeps 8 waves on a SIMD (single set) or 7 (population, where 64 VGPRs
-// would spill): the window loop waits on dependent loads, which the other
-// waves hide.  (Starting 64 units at a time and queueing in LDS those that
+// 387 us and 13.2 ms.  The register limit
+// keeps 8 waves on a SIMD: the window loop waits on dependent loads, which the
+// other waves hide (the 256-set generation 11.3 ms on the GPU with 7 and 10.6
+// with 8, 64 sets of fast dynamics 12.1 and 11.3).  (Starting 64 units at a time and queueing in LDS those that
 // outlast their first window was slower: 14 % more instructions, the first
 // window's close running for half of the lanes.)
 // The draw of a broadened efficiency and its binomial (kPassBroad) need up to
-// 77 registers.  They had been the general form's, at 186 registers and two
+// 74 registers (7 waves for populations: 0.94 ms against 0.98 with 6 on the
+// 64 sets below; no difference for single sets).  They had been the general form's, at 186 registers and two
 // waves per SIMD with logarithms, exponentials and divisions in double per
 // window: 50,000 bursts x 50 of a 3-state model 371 -> 197 us, 64 sets x
 // 20,000 x 16 2.74 -> 1.41 ms.
 constexpr int fast_waves_per_eu(bool pop, int pass) {
-    return pass == kPassBroad ? 6 : pop ? 7 : 8;
+    return pass != kPassBroad ? 8 : pop ? 7 : 6;
 }
 
 struct FastIO {
