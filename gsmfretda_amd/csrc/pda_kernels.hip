@@ -137,18 +137,33 @@ __device__ __forceinline__ void flush_hist(int32_t* h, int32_t* __restrict__ row
 // 387 us and 13.2 ms.  The register limit
 // keeps 8 waves on a SIMD: the window loop waits on dependent loads, which the
 // other waves hide (the 256-set generation 11.3 ms on the GPU with 7 and 10.6
-// with 8, 64 sets of fast dynamics 12.1 and 11.3).  (Starting 64 units at a time and queueing in LDS those that
-// outlast their first window was slower: 14 % more instructions, the first
+// with 8, 64 sets of fast dynamics 12.1 and 11.3).
+// Units are started 64 at a time into LDS and taken from there one lane at a
+// time as lanes fall idle, and ended ones wait in LDS until 64 can be binned:
+// a start (a Philox block and the unit's division) and a tally (a division and
+// a floor in double) would otherwise run for the one or two lanes of a pass
+// that need them.  64 sets of fast dynamics 11.27 -> 10.53 ms on the GPU,
+// 100,000 x 100 of 3 states 293 -> 288 us; 256 sets of slow dynamics the same
+// (10.62).  The population's workgroup has to stay within 5,120 bytes of LDS
+// for 32 of them on a CU (LDS is handed out in 1,280), which is why the models
+// come in parts; at 6,400 the 256 sets took 12.9 ms.  (Starting units together
+// with their first windows was slower: 14 % more instructions, the first
 // window's close running for half of the lanes.)
 // The draw of a broadened efficiency and its binomial (kPassBroad) need up to
 // 74 registers (7 waves for populations: 0.94 ms against 0.98 with 6 on the
-// 64 sets below; no difference for single sets).  They had been the general form's, at 186 registers and two
-// waves per SIMD with logarithms, exponentials and divisions in double per
-// window: 50,000 bursts x 50 of a 3-state model 371 -> 197 us, 64 sets x
+// 64 sets below; no difference for single sets).  They had been the general
+// form's, at 186 registers and two waves per SIMD with logarithms,
+// exponentials and divisions in double per window: 50,000 bursts x 50 of a 3-state model 371 -> 197 us, 64 sets x
 // 20,000 x 16 2.74 -> 1.41 ms.
 constexpr int fast_waves_per_eu(bool pop, int pass) {
     return pass != kPassBroad ? 8 : pop ? 7 : 6;
 }
+
+// A unit that has been started: its burst, its key and its first state.
+struct StartedUnit {
+    BurstDesc d;
+    uint32_t r, b;
+};
 
 struct FastIO {
     const BurstDesc* bursts;
@@ -171,17 +186,25 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(
     fast_waves_per_eu(kPop, kPass)))) void fast_walk_kernel(const FastIO io, const RunArgs a,
                                                             const FastArgs fa) {
     constexpr int kSlots = kPop ? 2 : 1;
-    __shared__ Model sM[kSlots];
-    extern __shared__ int32_t s_hist[];  // [kSlots][a.B]
+    using Mod = typename std::conditional<
+        kPass == kPassGuided, FastModel,
+        typename std::conditional<kPass == kPassBroad, BroadModel, Model>::type>::type;
+    __shared__ Mod sM[kSlots];
+    __shared__ StartedUnit s_start[kWave];    // units started and not yet taken
+    __shared__ uint8_t s_state[kWave];        // their first states
+    __shared__ float2 s_done[2 * kWave];      // (acc, F) of units not yet binned
+    extern __shared__ int32_t s_hist[];       // [kSlots][a.B]
     const uint32_t lane = threadIdx.x;
     for (uint32_t i = lane; i < uint32_t(kSlots) * uint32_t(a.B); i += kWave) s_hist[i] = 0;
-    if (!kPop) {
-        const uint32_t* src = reinterpret_cast<const uint32_t*>(&io.blobs->m);
-        uint32_t* dst = reinterpret_cast<uint32_t*>(&sM[0]);
-        for (uint32_t i = lane; i < sizeof(Model) / 4; i += kWave) dst[i] = src[i];
-    }
-    wave_lds_sync();
+    auto load_model = [&](uint32_t into, uint32_t set) {
+        const uint32_t* src = reinterpret_cast<const uint32_t*>(&io.blobs[set].m);
+        uint32_t* dst = reinterpret_cast<uint32_t*>(&sM[into]);
+        for (uint32_t i = lane; i < sizeof(Mod) / 4; i += kWave) dst[i] = src[i];
+        wave_lds_sync();
+    };
+    if (!kPop) load_model(0u, 0u);
 
+    const uint32_t seed = kPop ? io.ctl->seed : a.seed;
     const uint32_t queue = blockIdx.x % a.queues;
     // this queue's work: a contiguous share of the units, or every
     // a.queues-th batch of the generation
@@ -191,109 +214,160 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(
     const uint32_t xrow = blockIdx.x & 7u;
     const UnitDiv divR{a.div_m, a.div_sh};
     int set0 = kPop ? -1 : 0, set1 = -1;  // the set each LDS slot holds
-    uint32_t cur = 0;                     // slot that receives new units
+    uint32_t cur = 0;                     // slot whose units are being started
     uint32_t pool_set = 0, pool_next = 0, pool_end = 0;
+    uint32_t started = 0, start_next = 0;  // entries of s_start, the next to take
+    uint32_t done = 0;                     // entries of s_done
     bool drained = false;
     bool busy = false;
     uint32_t slot = 0;
     WalkState<true> st{};
-    UnitKey key{kPop ? io.ctl->seed : a.seed, a.set, 0u, 0u};
+    UnitKey key{seed, a.set, 0u, 0u};
     BurstDesc d{0u, 0u, 0u, 0.0f};
+    // bins the first `count` (at most 64) waiting units, one per lane
+    auto bin_done = [&](uint32_t first, uint32_t count) {
+        wave_lds_sync();
+        if (lane < count) {
+            const float2 r = s_done[first + lane];
+            const uint32_t sl = kPop ? fbits(r.y) >> 31 : 0u;  // F's sign: the slot
+            tally(s_hist + sl * uint32_t(a.B), a.B, r.x, kPop ? fabsf(r.y) : r.y);
+        }
+    };
     while (true) {
-        bool need = !busy;
-        while (!drained) {
-            const uint64_t want = __ballot(need);
+        while (true) {
+            const uint64_t want = __ballot(!busy);
             if (want == 0) break;
-            if (pool_next >= pool_end) {
-                uint32_t k = 0;
-                if (lane == 0) k = atomicAdd(&io.work[queue * kCounterStride], kPop ? 1u : a.batch);
-                k = __builtin_amdgcn_readfirstlane(k);
-                if (k >= q_len) {
-                    drained = true;
-                    break;
+            if (start_next == started) {  // start 64 units
+                if (pool_next >= pool_end) {
+                    if (drained) break;
+                    uint32_t k = 0;
+                    if (lane == 0)
+                        k = atomicAdd(&io.work[queue * kCounterStride], kPop ? 1u : a.batch);
+                    k = __builtin_amdgcn_readfirstlane(k);
+                    if (k >= q_len) {
+                        drained = true;
+                        break;
+                    }
+                    if (kPop) {
+                        k = k * a.queues + queue;
+                        pool_set = k / a.bps;
+                        pool_next = (k - pool_set * a.bps) * a.batch;
+                        pool_end = a.nunits - pool_next < a.batch ? a.nunits : pool_next + a.batch;
+                    } else {
+                        pool_next = q.begin + k;
+                        pool_end = q.end - pool_next < a.batch ? q.end : pool_next + a.batch;
+                    }
                 }
-                if (kPop) {
-                    k = k * a.queues + queue;
-                    pool_set = k / a.bps;
-                    pool_next = (k - pool_set * a.bps) * a.batch;
-                    pool_end = a.nunits - pool_next < a.batch ? a.nunits : pool_next + a.batch;
-                } else {
-                    pool_next = q.begin + k;
-                    pool_end = q.end - pool_next < a.batch ? q.end : pool_next + a.batch;
+                if (kPop && int(pool_set) != (cur ? set1 : set0)) {
+                    const uint32_t other = cur ^ 1u;
+                    if (__any(busy && slot == other)) break;  // the older set is still walking
+                    const int old = other ? set1 : set0;
+                    if (old >= 0) {
+                        bin_done(0u, done);
+                        done = 0;
+                        wave_lds_sync();
+                        flush_hist(s_hist + other * uint32_t(a.B),
+                                   io.hist_acc + (size_t(old) * 8u + xrow) * size_t(a.B), a.B,
+                                   lane);
+                    }
+                    load_model(other, pool_set);
+                    if (other) set1 = int(pool_set);
+                    else set0 = int(pool_set);
+                    cur = other;
                 }
-            }
-            if (kPop && int(pool_set) != (cur ? set1 : set0)) {
-                const uint32_t other = cur ^ 1u;
-                if (__any(busy && slot == other)) break;  // the older set is still walking
-                const int old = other ? set1 : set0;
-                if (old >= 0) {
-                    wave_lds_sync();
-                    flush_hist(s_hist + other * uint32_t(a.B),
-                               io.hist_acc + (size_t(old) * 8u + xrow) * size_t(a.B), a.B, lane);
+                const uint32_t u = pool_next + lane;
+                bool walks = false;
+                int state = 0;
+                StartedUnit e;
+                if (u < pool_end) {
+                    const uint32_t bl = unit_div(u, divR);
+                    e.d = io.bursts[a.begin + bl];
+                    e.r = u - bl * a.R;
+                    e.b = a.begin + bl;
+                    const UnitKey k{seed,
+                                    kPop ? io.ctl->set_base + pool_set * io.ctl->set_stride : a.set,
+                                    e.r, e.b};
+                    WalkState<true> s0;
+                    walks = begin_unit<true>(sM[kPop ? cur : 0u], k, e.d.P, e.d.T, s0) == kStepMore;
+                    state = s0.s;
+                    if (!walks) {
+                        tally(s_hist + (kPop ? cur : 0u) * uint32_t(a.B), a.B, 0.0f, 0.0f);
+                        if (kSamples) store_sample(u, 0.0f, 0.0f, io.outE, io.outAcc, io.outF);
+                    }
                 }
-                const uint32_t* src = reinterpret_cast<const uint32_t*>(&io.blobs[pool_set].m);
-                uint32_t* dst = reinterpret_cast<uint32_t*>(&sM[other]);
-                for (uint32_t i = lane; i < sizeof(Model) / 4; i += kWave) dst[i] = src[i];
+                pool_next = pool_end - pool_next < kWave ? pool_end : pool_next + kWave;
+                const uint64_t walking = __ballot(walks);
+                if (walks) {
+                    s_start[lanes_below(walking)] = e;
+                    s_state[lanes_below(walking)] = uint8_t(state);
+                }
                 wave_lds_sync();
-                if (other) set1 = int(pool_set);
-                else set0 = int(pool_set);
-                cur = other;
+                start_next = 0;
+                started = uint32_t(__popcll(walking));
+                continue;
             }
+            const uint32_t left = started - start_next;
             const uint32_t rank = lanes_below(want);
-            const uint32_t avail = pool_end - pool_next;
-            if (need && rank < avail) {
-                const uint32_t u = pool_next + rank;
-                const uint32_t bl = unit_div(u, divR);
+            if (!busy && rank < left) {
+                const StartedUnit e = s_start[start_next + rank];
+                d = e.d;
+                key.r = e.r;
+                key.b = e.b;
                 slot = cur;
-                d = io.bursts[a.begin + bl];
-                if (kPop) key.set = io.ctl->set_base + pool_set * io.ctl->set_stride;
-                key.r = u - bl * a.R;
-                key.b = a.begin + bl;
-                if (begin_unit<true>(sM[kPop ? slot : 0u], key, d.P, d.T, st) == kStepMore) {
-                    busy = true;
-                    need = false;
-                } else {
-                    tally(s_hist + slot * uint32_t(a.B), a.B, 0.0f, 0.0f);
-                    if (kSamples) store_sample(u, 0.0f, 0.0f, io.outE, io.outAcc, io.outF);
-                }
+                if (kPop) key.set = io.ctl->set_base + uint32_t(cur ? set1 : set0) * io.ctl->set_stride;
+                st = WalkState<true>{};
+                st.s = s_state[start_next + rank];
+                busy = true;
             }
             const uint32_t taken = uint32_t(__popcll(want));
-            pool_next += taken < avail ? taken : avail;
+            start_next += taken < left ? taken : left;
         }
         if (!__any(busy)) break;
+        bool ended = false;
         if (busy) {
-            const Model& M = sM[kPop ? slot : 0u];
+            const Mod& M = sM[kPop ? slot : 0u];
             const uint32_t set = kPop ? uint32_t(slot ? set1 : set0) : 0u;
             const uint32_t* ticks = io.ticks + d.off;
             const uint2* links = io.links + d.off;
             int r;
-            if (kPass == kPassBroad) {
+            if constexpr (kPass == kPassBroad) {
                 const BroadDraw draw{};
                 r = fast_window<false, BroadDraw>(M, &draw, key, d.P, d.stop_rel, d.T, ticks,
                                                   links, a, fa, st);
-            } else if (kPass == kPassGuided) {
+            } else if constexpr (kPass == kPassGuided) {
                 r = fast_window<false, BinomGuide>(M, &io.guide, key, d.P, d.stop_rel, d.T, ticks,
                                                    links, a, fa, st);
             } else {
                 r = fast_window<false, BinomTable>(M, &io.blobs[set].tab, key, d.P, d.stop_rel,
                                                    d.T, ticks, links, a, fa, st);
             }
-            if (r != kStepMore) {
-                busy = false;
+            busy = r == kStepMore;
+            ended = r == kStepDone;
+            if (r == kStepReplay) {
                 const uint32_t u = (key.b - a.begin) * a.R + key.r;
-                if (r == kStepReplay) {
-                    const uint32_t i = atomicAdd(io.replay_count, 1u);
-                    if (i < a.replay_cap) {
-                        if (kPop) static_cast<uint64_t*>(io.replay)[i] = (uint64_t(set) << 32) | u;
-                        else static_cast<uint32_t*>(io.replay)[i] = u;
-                    }
-                } else {
-                    tally(s_hist + slot * uint32_t(a.B), a.B, st.acc, st.F);
-                    if (kSamples) store_sample(u, st.acc, st.F, io.outE, io.outAcc, io.outF);
+                const uint32_t i = atomicAdd(io.replay_count, 1u);
+                if (i < a.replay_cap) {
+                    if (kPop) static_cast<uint64_t*>(io.replay)[i] = (uint64_t(set) << 32) | u;
+                    else static_cast<uint32_t*>(io.replay)[i] = u;
                 }
             }
+            if (kSamples && ended)
+                store_sample((key.b - a.begin) * a.R + key.r, st.acc, st.F, io.outE, io.outAcc,
+                             io.outF);
+        }
+        // ended units wait until 64 can be binned together
+        const uint64_t ends = __ballot(ended);
+        if (ended)
+            s_done[done + lanes_below(ends)] =
+                make_float2(st.acc, kPop ? bitsf(fbits(st.F > 0.0f ? st.F : 0.0f) | slot << 31)
+                                         : st.F);
+        done += uint32_t(__popcll(ends));
+        if (done >= kWave) {
+            done -= kWave;
+            bin_done(done, kWave);  // the last 64: those before them keep their places
         }
     }
+    bin_done(0u, done);
     wave_lds_sync();
     if (kPop) {
         if (set0 >= 0)

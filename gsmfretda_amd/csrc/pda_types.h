@@ -56,8 +56,11 @@ struct BurstDesc {
 // min(close, link[c].y) - f for f = link[c].x < close (src/mc.cu:136-181).
 
 // Model tables of one parameter set, built on the host from the args of
-// mc::set_params (src/mc.cu:790-800, src/eigenhelper.cpp:4-54).
-struct Model {
+// mc::set_params (src/mc.cu:790-800, src/eigenhelper.cpp:4-54).  In three
+// parts, each the beginning of the next, for the kernels that keep a copy in
+// LDS: what the fast form reads, what it reads besides for models with
+// distance broadening, and the rest, which the general form reads.
+struct FastModel {
     int32_t n;
     int32_t any_v;                // some v[s] != 0: broadening draws needed
     int32_t init_state;           // >= 0: the initial-state draw always gives this state
@@ -67,24 +70,26 @@ struct Model {
     // first state row of this set in its threshold table (population runs:
     // the sets' rows follow one another; 0 for a slot's single set)
     int32_t guide_base;
-    float pad0;
-    float p0cum[kMaxStates];                      // running sums of genMatP's inflow
+    int32_t quick_rates;          // every rate within quotient()'s range
+    int32_t flip[kMaxStates];     // p > 1/2: the acceptor draw is n - X
+    float p0cum[kMaxStates];      // running sums of genMatP's inflow
     // [s][jj] running sums of P_i2j column s; the last of the n - 1 entries,
     // which every draw past the others takes, and the rest are +inf
     float nscum[kMaxStates][kMaxStates];
-    float krate[kMaxStates][kMaxStates];          // [s][j] = K(j, s), rate s -> j
     // [s][j]: -K(j, s) and its reciprocal rounded to float (quotient())
     float kdiv[kMaxStates][kMaxStates][2];
-    int32_t quick_rates;          // every rate within quotient()'s range
-    int32_t pad1;
+};
+struct BroadModel : FastModel {
     float v[kMaxStates];
     float base[kMaxStates];                       // r0 (1/E - 1)^(1/6)
     float ep0[kMaxStates];                        // broadened E when v == 0
+};
+struct Model : BroadModel {
+    float krate[kMaxStates][kMaxStates];          // [s][j] = K(j, s), rate s -> j
     // Binomial(m, ep0[s]) by inversion (src/binom.cuh:135-169) on
-    // pp = min(p, 1-p): pp, q = 1 - pp, and whether p > 1/2 (draw n - X).
+    // pp = min(p, 1-p): pp and q = 1 - pp.
     double pp[kMaxStates];
     double qq[kMaxStates];
-    int32_t flip[kMaxStates];
 };
 
 // q^m and the inversion bound min(m, mp + 10 sqrt(mpq + 1)) per state and

@@ -344,7 +344,7 @@ struct WindowInfo {
 // Returns kStepDone when the unit has no window that counts anything
 // (zero or one photon, or T <= 0: E = 0).
 template <bool kFast>
-PDA_HD int begin_unit(const Model& M, const UnitKey& key, uint32_t P, float T,
+PDA_HD int begin_unit(const FastModel& M, const UnitKey& key, uint32_t P, float T,
                       WalkState<kFast>& st) {
     st.s = 0;
     st.tsum = 0.0f;
@@ -515,8 +515,8 @@ struct BroadDraw {};
 // kStepReplay where the window needs the general form.  Tab: BinomGuide
 // (thresholds) or BinomTable (inversion loop) for the acceptor draw of a
 // model without distance broadening, BroadDraw for one with.
-template <bool kCounts = false, class Tab = BinomTable>
-PDA_HD int fast_window(const Model& M, const typename NoDeduce<Tab>::type* tab, const UnitKey& key,
+template <bool kCounts = false, class Tab = BinomTable, class Mod = Model>
+PDA_HD int fast_window(const Mod& M, const typename NoDeduce<Tab>::type* tab, const UnitKey& key,
                        uint32_t P, uint32_t stop_rel, float T, const uint32_t* tick,
                        const uint2* link, const RunArgs& a, const FastArgs& fa,
                        WalkState<true>& st, WindowInfo* wi = nullptr) {

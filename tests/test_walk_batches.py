@@ -1,0 +1,47 @@
+"""GPU: the walk kernels start units 64 at a time and bin ended ones 64 at a
+time; runs of less than that, of that and a unit more, units that end where
+they start, and populations whose batches hold a few units each, so that a
+wave goes through many sets."""
+import numpy as np
+import pytest
+
+from gsmfretda_amd import pda, synth
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("bursts,R,B,nsets,v", [
+    (1, 1, 50, 3, 0.0),
+    (63, 1, 7, 5, 0.0),
+    (13, 5, 200, 300, 0.0),
+    (64, 2, 1, 9, 4.0),
+    (129, 7, 50, 40, 0.0),
+    (43, 3, 1024, 70, 4.0),
+])
+def test_walk_batches(gpu_mc, oracle, bursts, R, B, nsets, v):
+    rng = np.random.default_rng(bursts + nsets)
+    # some rates so slow that most units end in their first window
+    sets = []
+    for i in range(nsets):
+        n = int(rng.integers(2, 5))
+        a = synth.make_args(np.sort(rng.uniform(0.1, 0.9, n)),
+                            synth.loguniform_rates(rng, n * (n - 1), *((1.0, 9.0), (3e2, 8e3))[i % 2]))
+        a = np.array(a, np.float32)
+        a[n * n:] = v * (i % 3 == 0)
+        sets.append((n, a))
+    d = synth.generate(bursts, sets[1][1], sets[1][0], seed=bursts)
+    m = gpu_mc
+    m.load(d, SgDivSr=rng.uniform(0, 1, bursts).astype(np.float32), nbins=B, left_pad=0)
+    m.set_photophysics(0, *synth.PHOTOPHYSICS)
+    m.set_burst_range(0, -1, 0)
+    m.set_population([n for n, _ in sets], [a for _, a in sets])
+    m.run_population(R=R, seed=31, set_base=2, set_stride=5)
+    hist, _, _, _ = m.get_population_result()
+    od = oracle.Data.from_bursts(d)
+    for i, (n, a) in enumerate(sets):
+        p = oracle.make_params(n, a, *synth.PHOTOPHYSICS)
+        want = oracle.run(od, p, R=R, seed=31, set_id=2 + 5 * i, B=B, want_units=False)["hist"]
+        assert np.array_equal(hist[i].astype(np.int64), want), f"set {i}"
+        if i < 4:
+            h1, _, _, _ = pda.evaluate(m, n, a, R, 31, set_id=2 + 5 * i)
+            assert np.array_equal(h1.astype(np.int64), want), f"set {i} alone"
