@@ -92,6 +92,14 @@ Launch plan_launch(const pda_ctx* ctx, int pass, bool population, uint64_t units
     return L;
 }
 
+uint32_t replay_grid(const pda_ctx* ctx, uint64_t units) {
+    int per_cu = 0;
+    if (walk_occupancy(kPassReplay, ctx->B, &per_cu) != hipSuccess || per_cu < 1) per_cu = 1;
+    const uint64_t want = (units + kWave - 1) / kWave;
+    return uint32_t(
+        std::max<uint64_t>(1, std::min<uint64_t>(want, uint64_t(ctx->num_cu) * per_cu)));
+}
+
 void plan_args(RunArgs& a, uint64_t items, uint32_t align) {
     const UnitDiv q = make_unit_div(a.R);
     a.div_m = q.m;
@@ -239,10 +247,10 @@ int pda_create(int device, int nstreams, pda_ctx** out) {
             hipMemset(s.d_work, 0, sizeof(uint32_t) * kWorkWords) != hipSuccess ||
             hipEventCreateWithFlags(&s.model_copied, hipEventDisableTiming) != hipSuccess ||
             hipMalloc(&s.d_hist_acc, sizeof(int32_t) * kMaxBins * 8) != hipSuccess ||
-
-            hipMalloc(&s.d_result, sizeof(ResultHeader) + sizeof(int32_t) * kMaxBins) != hipSuccess ||
             hipHostMalloc(reinterpret_cast<void**>(&s.h_result),
-                          sizeof(ResultHeader) + sizeof(int32_t) * kMaxBins, hipHostMallocDefault) != hipSuccess ||
+                          sizeof(ResultHeader) + sizeof(int32_t) * kMaxBins,
+                          hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess ||
+            hipHostGetDevicePointer(reinterpret_cast<void**>(&s.d_result), s.h_result, 0) != hipSuccess ||
             hipEventCreate(&s.ev0) != hipSuccess || hipEventCreate(&s.ev_mid) != hipSuccess ||
             hipEventCreate(&s.ev1) != hipSuccess ||
             hipMemset(s.d_hist_acc, 0, sizeof(int32_t) * kMaxBins * 8) != hipSuccess ||
@@ -272,7 +280,6 @@ int pda_destroy(pda_ctx* ctx) {
         (void)hipFree(s.d_replay_count);
         (void)hipFree(s.d_work);
         (void)hipFree(s.d_hist_acc);
-        (void)hipFree(s.d_result);
         (void)hipHostFree(s.h_result);
         (void)hipFree(s.d_E);
         (void)hipFree(s.d_acc);
@@ -487,27 +494,16 @@ int pda_run(pda_ctx* ctx, int sid, int R, uint32_t seed, uint32_t set_id, int fl
     const FastArgs fa = fast_args(s->n, s->quick_rates, a.clk_p, s->ph.r0, ctx->max_P);
     HIP_TRY(launch_walk(pass, grid, ctx->d_bursts, ctx->d_ticks, ctx->d_links, s->d_blob, guide, a,
                         fa, s->d_hist_acc, s->d_replay, s->d_replay_count, s->d_work, outE, outAcc,
-                        outF, s->stream));
+                        outF, nullptr, nullptr, s->stream));
     HIP_TRY(hipEventRecord(s->ev_mid, s->stream));
-    if (nunits > 0) {
-        // the abandoned units, in the general form over the whole GPU; the
-        // grid is sized for the worst case and its unneeded workgroups exit
-        // at once
-        int per_cu = 0;
-        if (walk_occupancy(kPassReplay, ctx->B, &per_cu) != hipSuccess || per_cu < 1) per_cu = 1;
-        const uint64_t want = (uint64_t(nunits) + kWave - 1) / kWave;
-        const uint32_t rgrid =
-            uint32_t(std::max<uint64_t>(1, std::min<uint64_t>(want, uint64_t(ctx->num_cu) * per_cu)));
-        HIP_TRY(launch_walk(kPassReplay, rgrid, ctx->d_bursts, ctx->d_ticks, ctx->d_links,
-                            s->d_blob, guide, a, fa, s->d_hist_acc, s->d_replay, s->d_replay_count,
-                            s->d_work,
-                            outE, outAcc, outF, s->stream));
-    }
-    HIP_TRY(launch_finish(a, ctx->d_obs, s->d_hist_acc, s->d_replay_count, s->d_work, s->d_result,
-                          s->stream));
+    // the abandoned units, in the general form over the whole GPU, and the end
+    // of the run; the grid is sized for the worst case and its unneeded
+    // workgroups exit at once
+    HIP_TRY(launch_walk(kPassReplay, replay_grid(ctx, uint64_t(nunits)), ctx->d_bursts,
+                        ctx->d_ticks, ctx->d_links, s->d_blob, guide, a, fa, s->d_hist_acc,
+                        s->d_replay, s->d_replay_count, s->d_work, outE, outAcc, outF, ctx->d_obs,
+                        s->d_result, s->stream));
     HIP_TRY(hipEventRecord(s->ev1, s->stream));
-    HIP_TRY(hipMemcpyAsync(s->h_result, s->d_result, sizeof(ResultHeader) + sizeof(int32_t) * size_t(a.B),
-                           hipMemcpyDeviceToHost, s->stream));
     if (outE)
         HIP_TRY(hipMemcpyAsync(s->h_E, outE, sizeof(float) * size_t(nunits), hipMemcpyDeviceToHost,
                                s->stream));

@@ -73,8 +73,10 @@ struct Population {
     uint8_t* d_in = nullptr;
     int cap_B = 0;
     int32_t* d_hist_acc = nullptr;   // [cap_sets][8][cap_B], zero between runs
-    uint8_t* d_out = nullptr;        // PopStatus + SetResult[cap_sets] + int32 hist[cap_sets][B]
-    uint8_t* h_out = nullptr;        // pinned
+    // PopStatus + SetResult[cap_sets] + int32 hist[cap_sets][B], pinned, written
+    // by the run's last kernel
+    uint8_t* h_out = nullptr;
+    uint8_t* d_out = nullptr;        // its device address
     size_t out_bytes = 0;
     uint64_t* d_replay = nullptr;
     uint32_t* d_replay_count = nullptr;
@@ -179,8 +181,8 @@ struct Slot {
     std::vector<float> args;
     int64_t begin = 0, end = -1;
     int32_t* d_hist_acc = nullptr;
-    ResultHeader* d_result = nullptr;
-    ResultHeader* h_result = nullptr;  // pinned
+    ResultHeader* h_result = nullptr;  // pinned, written by the run's last kernel
+    ResultHeader* d_result = nullptr;  // its device address
     int last_B = 0;
     int64_t last_units = 0;
     bool ran = false;
@@ -257,6 +259,8 @@ struct Launch {
     uint32_t grid = 1, batch = kWave, queues = 1;
 };
 Launch plan_launch(const pda_ctx* ctx, int pass, bool population, uint64_t units);
+// Workgroups of the replay pass of a run of `units` units.
+uint32_t replay_grid(const pda_ctx* ctx, uint64_t units);
 // The fields of a walk's arguments that follow from the others: R's
 // multiply-shift divisor, and the `items` (units, or a population's batches)
 // each of the a.queues work counters hands out, in whole waves of units.
@@ -265,16 +269,14 @@ void plan_args(RunArgs& a, uint64_t items, uint32_t align);
 // kernels (pda_kernels.hip)
 hipError_t walk_occupancy(int pass, int B, int* blocks_per_cu);
 hipError_t pop_walk_occupancy(int pass, int B, int* blocks_per_cu);
+// kPassReplay also ends the run: histogram and chi2 against obs into result
 hipError_t launch_walk(int pass, uint32_t grid, const BurstDesc* bursts, const uint32_t* ticks,
                        const uint2* links, const ModelBlob* blob, const BinomGuide& guide,
                        const RunArgs& a, const FastArgs& fa, int32_t* hist_acc, uint32_t* replay,
                        uint32_t* replay_count, uint32_t* work, float* outE, int32_t* outAcc,
-                       float* outF, hipStream_t stream);
+                       float* outF, const float* obs, ResultHeader* result, hipStream_t stream);
 hipError_t launch_guide(const ModelBlob* blobs, int nsets, int max_states, ThrPair* thr,
                         uint8_t* guide, hipStream_t stream);
-hipError_t launch_finish(const RunArgs& a, const float* obs, int32_t* hist_acc,
-                         uint32_t* replay_count, uint32_t* work, ResultHeader* result,
-                         hipStream_t stream);
 hipError_t launch_pop_walk(int pass, uint32_t grid, const BurstDesc* bursts,
                            const uint32_t* ticks, const uint2* links, const PopControl* ctl,
                            const ModelBlob* blobs, const BinomGuide& guide, const RunArgs& a,

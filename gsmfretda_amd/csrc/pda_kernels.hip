@@ -1,7 +1,7 @@
 // pda_kernels.hip -- gfx950 kernels of the Monte-Carlo PDA hot path.
 //
-// fast_walk_kernel, walk_kernel and finish_kernel replace gSMFRETda's mc_kernel (src/mc.cu:83-197)
-// together with the host histogram and chi2 of src/streamWorker.cpp:184-206:
+// fast_walk_kernel and walk_kernel replace gSMFRETda's mc_kernel
+// (src/mc.cu:83-197) together with the host histogram and chi2 of src/streamWorker.cpp:184-206:
 //   * one-wave workgroups; every lane streams through (burst, resample)
 //     units taken from per-XCD work counters, advancing one dwell window
 //     per loop pass, so lanes and waves never wait for the longest unit;
@@ -15,8 +15,8 @@
 //   * the common case runs in a lean form (fast_walk_kernel, at most 72
 //     VGPRs); the rare units that need BTPE draws, inversion restarts or
 //     large background means are listed and replayed in full by walk_kernel
-//     over the whole grid; finish_kernel then reduces the LDS histograms of
-//     all workgroups and computes chi2 on the device.
+//     over the whole grid, whose last workgroup sums the accumulator rows,
+//     computes chi2 and writes both to the host's result buffer.
 #include <hip/hip_runtime.h>
 
 #include "pda_math.h"
@@ -380,33 +380,120 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(
     }
 }
 
+// chi2 of one histogram by one wave, as src/streamWorker.cpp:194-206: the
+// reference's float accumulation and FP64.  Reads the 8 accumulator rows
+// (`pitch` apart, left zero for the next run) and writes their sum.
+//
+// The reference's sum is a chain of dependent conversions and additions, one
+// per bin.  Lane b forms bin b's terms, 64 bins at a time; the chain then
+// runs over the lanes by readlane, a bin's terms ready before its turn.  An
+// empty bin's terms are zero, which adds nothing: no branch in the chain.
+// (It had been a loop of one thread over LDS: 24 us for 200 bins, 8.6 for
+// 50, of which the rest of the kernel is 3.)
+struct Chi2Sum {
+    float c32;
+    double c64;
+    int filled;  // bins of the sum that are not empty
+};
+__device__ __forceinline__ double lane_value(double v, int l) {
+    const uint64_t b = __double_as_longlong(v);
+    const uint32_t lo = __builtin_amdgcn_readlane(uint32_t(b), l);
+    const uint32_t hi = __builtin_amdgcn_readlane(uint32_t(b >> 32), l);
+    return __longlong_as_double((long long)(uint64_t(hi) << 32 | lo));
+}
+__device__ __forceinline__ Chi2Sum chi2_fold(const RunArgs& a, const float* __restrict__ obs,
+                                             int32_t* __restrict__ rows, size_t pitch,
+                                             int32_t* __restrict__ hist, uint32_t lane) {
+    Chi2Sum r{0.0f, 0.0, 0};
+    const uint32_t B = uint32_t(a.B);
+    const float Rf = float(a.R);
+    int32_t next[8];  // the next 64 bins' rows, on their way during the chain
+    float next_obs = 0.0f;
+    auto fetch = [&](uint32_t b) {
+        if (b < B) {
+#pragma unroll
+            for (uint32_t x = 0; x < 8u; ++x)
+                next[x] = __hip_atomic_load(&rows[x * pitch + b], __ATOMIC_RELAXED,
+                                            __HIP_MEMORY_SCOPE_AGENT);
+            next_obs = obs[b];
+        }
+    };
+    fetch(lane);
+    for (uint32_t base = 0; base < B; base += kWave) {
+        const uint32_t b = base + lane;
+        int32_t Mb = 0;
+        const float ob = next_obs;
+        if (b < B) {
+#pragma unroll
+            for (uint32_t x = 0; x < 8u; ++x) {
+                if (next[x]) rows[x * pitch + b] = 0;
+                Mb += next[x];
+            }
+            hist[b] = Mb;
+        }
+        fetch(b + kWave);
+        // per-bin terms: FP64, and the reference's double term of a float
+        // difference (pow(float, 2) / float, src/streamWorker.cpp:200-201)
+        double t64 = 0.0, t32 = 0.0;
+        const bool filled = Mb > 0 && int(b) >= a.left_pad;
+        if (filled) {
+            const float Mf = float(Mb);
+            const float dlt = ob - Mf / Rf;
+            t32 = (double(dlt) * double(dlt)) / double(Mf / Rf);
+            const double md = double(Mb) / double(a.R);
+            const double dd = double(ob) - md;
+            t64 = dd * dd / md;
+        }
+        r.filled += __popcll(__ballot(filled));
+#pragma unroll 8
+        for (int l = 0; l < kWave; ++l) {
+            r.c32 = float(double(r.c32) + lane_value(t32, l));
+            r.c64 += lane_value(t64, l);
+        }
+    }
+    return r;
+}
+
+// Ends a single set's run (one wave): histogram, chi2, and the run's counters
+// (walk and replay queues, replay count) back to zero.
+__device__ __forceinline__ void finish_run(const RunArgs& a, const float* __restrict__ obs,
+                                           int32_t* __restrict__ hist_acc,
+                                           uint32_t* __restrict__ replay_count, uint32_t replays,
+                                           uint32_t* __restrict__ work,
+                                           ResultHeader* __restrict__ result, uint32_t lane) {
+    const Chi2Sum c = chi2_fold(a, obs, hist_acc, kMaxBins,
+                                reinterpret_cast<int32_t*>(result + 1), lane);
+    if (lane == 0) {
+        const int dof = c.filled - a.nstates * (a.nstates + 1);
+        ResultHeader r{};
+        r.chi2_ref = c.c32 / float(dof);
+        r.chi2_64 = c.c64 / double(dof);
+        r.effN = c.filled;
+        r.units = int64_t(a.nunits);
+        r.B = a.B;
+        r.replays = int32_t(replays);
+        *result = r;
+        *replay_count = 0u;
+    }
+    for (uint32_t q = lane; q < kMaxQueues + kAuxQueues + 1u; q += kWave)
+        work[q * kCounterStride] = 0u;
+}
+
 // ---- walk in the general form ---------------------------------------------------
 //
-// The units the fast form abandoned, launched right after it on the same
-// stream, so the replay list and its count are final.  Each one-wave
-// workgroup keeps an LDS histogram and adds it to its XCD's accumulator row
-// at the end (workgroups are dispatched to the 8 XCDs round-robin, so the
-// atomics of a launch spread over 8 x B addresses).  No completion ticket and
-// no fence: the finish kernel, launched behind on the same stream, reads the
-// rows.
-__global__ __launch_bounds__(kWave) void walk_kernel(
+// Walks this workgroup's share of a replay list in the general form and adds
+// its histogram to its XCD's accumulator row (workgroups are dispatched to the
+// 8 XCDs round-robin, so the atomics of a launch spread over 8 x B addresses).
+__device__ __forceinline__ void replay_units(
     const BurstDesc* __restrict__ bursts, const uint32_t* __restrict__ ticks,
-    const uint2* __restrict__ links, const ModelBlob* __restrict__ blob, const RunArgs a,
-    int32_t* __restrict__ hist_acc, const uint32_t* __restrict__ replay,
-    const uint32_t* __restrict__ replay_count, uint32_t* __restrict__ work,
-    float* __restrict__ outE, int32_t* __restrict__ outAcc, float* __restrict__ outF) {
-    const uint32_t c = *replay_count;
-    const uint32_t nunits = c < a.replay_cap ? c : a.replay_cap;
-    // as many workgroups as the list needs a wave for, each queue served by
-    // at least one of them
-    const uint32_t waves = (nunits + kWave - 1u) / kWave;
-    const uint32_t alive = waves < gridDim.x ? waves : gridDim.x;
-    if (blockIdx.x >= alive) return;  // uniform over the workgroup
-    const uint32_t queues = alive < kReplayQueues ? alive : kReplayQueues;
-    const uint32_t queue = blockIdx.x % queues;
+    const uint2* __restrict__ links, const ModelBlob* __restrict__ blob, const RunArgs& a,
+    int32_t* __restrict__ hist_acc, const uint32_t* __restrict__ replay, uint32_t nunits,
+    uint32_t alive, uint32_t* __restrict__ work, float* __restrict__ outE,
+    int32_t* __restrict__ outAcc, float* __restrict__ outF, uint32_t lane) {
     __shared__ Model sM;
     extern __shared__ int32_t s_hist[];  // [a.B]
-    const uint32_t lane = threadIdx.x;
+    const uint32_t queues = alive < kReplayQueues ? alive : kReplayQueues;
+    const uint32_t queue = blockIdx.x % queues;
     {
         const uint32_t* src = reinterpret_cast<const uint32_t*>(&blob->m);
         uint32_t* dst = reinterpret_cast<uint32_t*>(&sM);
@@ -477,6 +564,42 @@ __global__ __launch_bounds__(kWave) void walk_kernel(
     flush_hist(s_hist, hist_acc + size_t(blockIdx.x & 7u) * kMaxBins, a.B, lane);
 }
 
+// The units the fast form abandoned, launched right after it on the same
+// stream, so the replay list and its count are final; and the end of the run.
+// The workgroup that adds its histogram last ends the run; where nothing was
+// abandoned -- most runs -- that is workgroup 0 at once, without a counter.
+// With the end as a launch of its own, on one thread's chain, and a copy of the
+// result behind it, 5,000 bursts x 20 of 2 states at 50 bins took 80 us and
+// 20,000 x 4 of 3 broadened states at 200 bins 115; now 69 and 89.
+__global__ __launch_bounds__(kWave) void walk_kernel(
+    const BurstDesc* __restrict__ bursts, const uint32_t* __restrict__ ticks,
+    const uint2* __restrict__ links, const ModelBlob* __restrict__ blob, const RunArgs a,
+    int32_t* __restrict__ hist_acc, const uint32_t* __restrict__ replay,
+    uint32_t* __restrict__ replay_count, uint32_t* __restrict__ work, float* __restrict__ outE,
+    int32_t* __restrict__ outAcc, float* __restrict__ outF, const float* __restrict__ obs,
+    ResultHeader* __restrict__ result) {
+    const uint32_t c = *replay_count;
+    const uint32_t nunits = c < a.replay_cap ? c : a.replay_cap;
+    // as many workgroups as the list needs a wave for, each queue served by
+    // at least one of them
+    const uint32_t waves = (nunits + kWave - 1u) / kWave;
+    const uint32_t alive = waves < gridDim.x ? waves : gridDim.x;
+    const uint32_t lane = threadIdx.x;
+    if (blockIdx.x >= (alive ? alive : 1u)) return;  // uniform over the workgroup
+    if (alive) {
+        replay_units(bursts, ticks, links, blob, a, hist_acc, replay, nunits, alive, work, outE,
+                     outAcc, outF, lane);
+        __threadfence();
+        uint32_t ended = 0;
+        if (lane == 0) ended = atomicAdd(&work[(kMaxQueues + kAuxQueues) * kCounterStride], 1u);
+        if (__builtin_amdgcn_readfirstlane(ended) + 1u != alive) return;
+        __threadfence();
+    }
+    // (a workgroup that has not yet read the replay count, and now reads
+    // zero, is not workgroup 0, which has been counted: it returns)
+    finish_run(a, obs, hist_acc, replay_count, c, work, result, lane);
+}
+
 // Threshold rows of the fast walk's binomial draws, one wave per (state,
 // photon count) row of a parameter set (the operations and their order are
 // those of build_guide_row_host): blockIdx.x = state * kBinomTable + count,
@@ -543,65 +666,6 @@ __global__ __launch_bounds__(kWave) void guide_kernel(const ModelBlob* __restric
         else hi_i = mid;
     }
     guide[(size_t(srow) * kBinomTable + size_t(m)) * kGuideBuckets + size_t(lane)] = uint8_t(lo_i);
-}
-
-constexpr uint32_t kFinishWaves = 16;
-
-// Finishes a run in one workgroup of 16 waves: reduces the 8 accumulator
-// rows (leaving them zero for the next run), computes the reduced chi2 of
-// src/streamWorker.cpp:194-206 in the reference's float accumulation and in
-// FP64, and resets the run's counters (walk and replay queues, replay count).
-__global__ __launch_bounds__(kWave * kFinishWaves) void finish_kernel(
-    const RunArgs a, const float* __restrict__ obs, int32_t* __restrict__ hist_acc,
-    uint32_t* __restrict__ replay_count, uint32_t* __restrict__ work,
-    ResultHeader* __restrict__ result) {
-    __shared__ int32_t s_hist[kMaxBins];
-    __shared__ double s_t64[kMaxBins];
-    __shared__ double s_t32[kMaxBins];
-    const uint32_t tid = threadIdx.x;
-    int32_t* rhist = reinterpret_cast<int32_t*>(result + 1);
-    const float Rf = float(a.R);
-    for (uint32_t b = tid; b < uint32_t(a.B); b += blockDim.x) {
-        int32_t Mb = 0;
-        for (uint32_t x = 0; x < 8u; ++x) Mb += atomicExch(&hist_acc[size_t(x) * kMaxBins + b], 0);
-        s_hist[b] = Mb;
-        rhist[b] = Mb;
-        // per-bin terms: FP64, and the reference's double term of a float
-        // difference (pow(float, 2) / float, src/streamWorker.cpp:200-201)
-        double t64 = 0.0, t32 = 0.0;
-        if (Mb > 0) {
-            const float Mf = float(Mb);
-            const float dlt = obs[b] - Mf / Rf;
-            t32 = (double(dlt) * double(dlt)) / double(Mf / Rf);
-            const double md = double(Mb) / double(a.R);
-            const double dd = double(obs[b]) - md;
-            t64 = dd * dd / md;
-        }
-        s_t64[b] = t64;
-        s_t32[b] = t32;
-    }
-    __syncthreads();
-    if (tid == 0) {
-        int effN = a.B - a.left_pad;
-        float c32 = 0.0f;
-        double c64 = 0.0;
-        for (int b = a.left_pad; b < a.B; ++b) {
-            if (s_hist[b] > 0) {
-                c32 = float(double(c32) + s_t32[b]);
-                c64 += s_t64[b];
-            } else {
-                --effN;
-            }
-        }
-        const int dof = effN - a.nstates * (a.nstates + 1);
-        result->chi2_ref = c32 / float(dof);
-        result->chi2_64 = c64 / double(dof);
-        result->effN = effN;
-        result->units = int64_t(a.nunits);
-        result->B = a.B;
-        result->replays = int32_t(atomicExch(replay_count, 0u));
-    }
-    if (tid < kMaxQueues + kReplayQueues) atomicExch(&work[tid * kCounterStride], 0u);
 }
 
 // ---- population runs ---------------------------------------------------------
@@ -736,7 +800,7 @@ __global__ __launch_bounds__(kWave) void pop_replay_kernel(
 }
 
 // One workgroup per set: reduces the set's 8 accumulator rows (leaving them
-// zero), computes its chi2 as finish_kernel does, with the set's own degrees
+// zero), computes its chi2 as finish_run does, with the set's own degrees
 // of freedom; workgroup 0 reports and resets the replay count and the work
 // counters.
 __global__ __launch_bounds__(kWave) void pop_finish_kernel(
@@ -744,63 +808,32 @@ __global__ __launch_bounds__(kWave) void pop_finish_kernel(
     int32_t* __restrict__ hist_acc, uint32_t* __restrict__ replay_count,
     uint32_t* __restrict__ work, PopStatus* __restrict__ status, SetResult* __restrict__ results,
     int32_t* __restrict__ hists) {
-    __shared__ int32_t s_M[kMaxBins];
-    __shared__ double s_t64[kMaxBins];
-    __shared__ double s_t32[kMaxBins];
     const uint32_t set = blockIdx.x, lane = threadIdx.x;
-    const uint32_t B = uint32_t(a.B);
-    int32_t* rows = hist_acc + size_t(set) * 8u * B;
-    const float Rf = float(a.R);
-    for (uint32_t b = lane; b < B; b += kWave) {
-        int32_t Mb = 0;
-        for (uint32_t x = 0; x < 8u; ++x) Mb += atomicExch(&rows[x * B + b], 0);
-        s_M[b] = Mb;
-        hists[size_t(set) * B + b] = Mb;
-        double t64 = 0.0, t32 = 0.0;
-        if (Mb > 0) {
-            const float Mf = float(Mb);
-            const float dlt = obs[b] - Mf / Rf;
-            t32 = (double(dlt) * double(dlt)) / double(Mf / Rf);
-            const double md = double(Mb) / double(a.R);
-            const double dd = double(obs[b]) - md;
-            t64 = dd * dd / md;
-        }
-        s_t64[b] = t64;
-        s_t32[b] = t32;
-    }
-    __syncthreads();
+    const size_t B = size_t(a.B);
+    const Chi2Sum c = chi2_fold(a, obs, hist_acc + size_t(set) * 8u * B, B,
+                                hists + size_t(set) * B, lane);
     if (lane == 0) {
-        int effN = a.B - a.left_pad;
-        float c32 = 0.0f;
-        double c64 = 0.0;
-        for (int b = a.left_pad; b < a.B; ++b) {
-            if (s_M[b] > 0) {
-                c32 = float(double(c32) + s_t32[b]);
-                c64 += s_t64[b];
-            } else {
-                --effN;
-            }
-        }
         const int n = blobs[set].m.n;
-        const int dof = effN - n * (n + 1);
+        const int dof = c.filled - n * (n + 1);
         SetResult r;
-        r.chi2_ref = c32 / float(dof);
-        r.chi2_64 = c64 / double(dof);
-        r.effN = effN;
+        r.chi2_ref = c.c32 / float(dof);
+        r.chi2_64 = c.c64 / double(dof);
+        r.effN = c.filled;
         r.n = n;
         r.pad = 0;
         results[set] = r;
     }
     if (set == 0) {
         if (lane == 0) {
-            const uint32_t c = atomicExch(replay_count, 0u);
+            const uint32_t n = *replay_count;
+            *replay_count = 0u;
             PopStatus st;
-            st.replays = c;
-            st.overflow = c > a.replay_cap ? 1u : 0u;
+            st.replays = n;
+            st.overflow = n > a.replay_cap ? 1u : 0u;
             st.pad[0] = st.pad[1] = 0;
             *status = st;
         }
-        for (uint32_t q = lane; q < kMaxQueues; q += kWave) atomicExch(&work[q * kCounterStride], 0u);
+        for (uint32_t q = lane; q < kMaxQueues; q += kWave) work[q * kCounterStride] = 0u;
     }
 }
 
@@ -1059,13 +1092,14 @@ hipError_t launch_walk(int pass, uint32_t grid, const BurstDesc* bursts, const u
                        const uint2* links, const ModelBlob* blob, const BinomGuide& guide,
                        const RunArgs& a, const FastArgs& fa, int32_t* hist_acc, uint32_t* replay,
                        uint32_t* replay_count, uint32_t* work, float* outE, int32_t* outAcc,
-                       float* outF, hipStream_t stream) {
+                       float* outF, const float* obs, ResultHeader* result, hipStream_t stream) {
     const size_t lds = sizeof(int32_t) * size_t(a.B);
     const FastIO io{bursts, ticks, links, blob, nullptr, guide, hist_acc, replay,
                     replay_count, work, outE, outAcc, outF};
     if (pass == kPassReplay)
         hipLaunchKernelGGL(walk_kernel, dim3(grid), dim3(kWave), lds, stream, bursts, ticks, links,
-                           blob, a, hist_acc, replay, replay_count, work, outE, outAcc, outF);
+                           blob, a, hist_acc, replay, replay_count, work, outE, outAcc, outF, obs,
+                           result);
     else if (pass == kPassBroad && outE)
         launch_fast<false, kPassBroad, true>(grid, lds, io, a, fa, stream);
     else if (pass == kPassBroad)
@@ -1081,14 +1115,6 @@ hipError_t launch_guide(const ModelBlob* blobs, int nsets, int max_states, ThrPa
                         uint8_t* guide, hipStream_t stream) {
     hipLaunchKernelGGL(guide_kernel, dim3(uint32_t(max_states) * kBinomTable, uint32_t(nsets)),
                        dim3(kWave), 0, stream, blobs, thr, guide);
-    return hipGetLastError();
-}
-
-hipError_t launch_finish(const RunArgs& a, const float* obs, int32_t* hist_acc,
-                         uint32_t* replay_count, uint32_t* work, ResultHeader* result,
-                         hipStream_t stream) {
-    hipLaunchKernelGGL(finish_kernel, dim3(1), dim3(kWave * kFinishWaves), 0, stream, a, obs,
-                       hist_acc, replay_count, work, result);
     return hipGetLastError();
 }
 

@@ -60,7 +60,7 @@ __global__ __launch_bounds__(1024) void clear_scratch_kernel(uint32_t* __restric
                                                              uint32_t* __restrict__ count,
                                                              int32_t* __restrict__ hist_acc) {
     const uint32_t t = threadIdx.x;
-    if (t < kMaxQueues + kAuxQueues) work[size_t(t) * kCounterStride] = 0u;
+    if (t < kMaxQueues + kAuxQueues + 1u) work[size_t(t) * kCounterStride] = 0u;
     if (t == 0) *count = 0u;
     for (uint32_t i = t; i < uint32_t(kMaxBins) * 8u; i += blockDim.x) hist_acc[i] = 0;
 }
@@ -143,18 +143,11 @@ extern "C" int pda_run_noalloc(pda_ctx* ctx, int sid, int R, uint32_t seed, uint
     const BinomGuide guide{s->d_thr, s->d_guide};
     const FastArgs fa = fast_args(s->n, s->quick_rates, a.clk_p, s->ph.r0, ctx->max_P);
     HIP_TRY(launch_walk(pass, L.grid, ctx->d_bursts, ctx->d_ticks, ctx->d_links, s->d_blob, guide,
-                        a, fa, hist_acc, replay, count, work, nullptr, nullptr, nullptr, s->stream));
-    if (nunits > 0) {
-        int per_cu = 0;
-        if (walk_occupancy(kPassReplay, ctx->B, &per_cu) != hipSuccess || per_cu < 1) per_cu = 1;
-        const uint64_t want = (uint64_t(nunits) + kWave - 1) / kWave;
-        const uint32_t rgrid = uint32_t(
-            std::max<uint64_t>(1, std::min<uint64_t>(want, uint64_t(ctx->num_cu) * per_cu)));
-        HIP_TRY(launch_walk(kPassReplay, rgrid, ctx->d_bursts, ctx->d_ticks, ctx->d_links,
-                            s->d_blob, guide, a, fa, hist_acc, replay, count, work, nullptr, nullptr,
-                            nullptr, s->stream));
-    }
-    HIP_TRY(launch_finish(a, ctx->d_obs, hist_acc, count, work,
-                          static_cast<ResultHeader*>(d_result), s->stream));
+                        a, fa, hist_acc, replay, count, work, nullptr, nullptr, nullptr, nullptr,
+                        nullptr, s->stream));
+    HIP_TRY(launch_walk(kPassReplay, replay_grid(ctx, uint64_t(nunits)), ctx->d_bursts,
+                        ctx->d_ticks, ctx->d_links, s->d_blob, guide, a, fa, hist_acc, replay,
+                        count, work, nullptr, nullptr, nullptr, ctx->d_obs,
+                        static_cast<ResultHeader*>(d_result), s->stream));
     return PDA_OK;
 }

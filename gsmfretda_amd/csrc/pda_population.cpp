@@ -54,7 +54,6 @@ void free_population(Population& p) {
     p.d_guide = nullptr;
     p.cap_guide_states = 0;
     (void)hipFree(p.d_hist_acc);
-    (void)hipFree(p.d_out);
     (void)hipHostFree(p.h_out);
     (void)hipFree(p.d_replay);
     (void)hipFree(p.d_replay_count);
@@ -116,12 +115,12 @@ int ensure_pop_buffers(pda_ctx* ctx, Slot& s, int B) {
     const size_t ob = out_bytes(p.cap_sets, p.cap_B);
     if (ob > p.out_bytes) {
         drop_graph(p);
-        (void)hipFree(p.d_out);
         (void)hipHostFree(p.h_out);
         p.d_out = p.h_out = nullptr;
         p.out_bytes = 0;
-        HIP_TRY(hipMalloc(&p.d_out, ob));
-        HIP_TRY(hipHostMalloc(reinterpret_cast<void**>(&p.h_out), ob, hipHostMallocDefault));
+        HIP_TRY(hipHostMalloc(reinterpret_cast<void**>(&p.h_out), ob,
+                              hipHostMallocMapped | hipHostMallocCoherent));
+        HIP_TRY(hipHostGetDevicePointer(reinterpret_cast<void**>(&p.d_out), p.h_out, 0));
         p.out_bytes = ob;
     }
     (void)ctx;
@@ -155,8 +154,6 @@ int enqueue_population(pda_ctx* ctx, Slot& s, int pass, uint32_t grid, const Run
                                   uint32_t(ctx->num_cu) * 4u, s.stream));
     HIP_TRY(launch_pop_finish(blobs, a, ctx->d_obs, p.d_hist_acc, p.d_replay_count, p.d_work,
                               status, results, hists, s.stream));
-    HIP_TRY(hipMemcpyAsync(p.h_out, p.d_out, out_bytes(size_t(p.nsets), a.B),
-                           hipMemcpyDeviceToHost, s.stream));
     return PDA_OK;
 }
 

@@ -15,10 +15,10 @@ constexpr uint32_t kDefaultQueues = 32;  // four per XCD unless tuned
 // Each work counter sits on its own 256-byte line: device-scope atomics on
 // one line serialise, and counters sharing a line would serialise together.
 constexpr uint32_t kCounterStride = 64;  // uint32 words between counters
-// Counter words of a run: kMaxQueues queue counters and kAuxQueues more
+// Counter words of a run: kMaxQueues queue counters and kAuxQueues + 1 more
 // (the RB pmf pass's burst counters), each on its own line.
 constexpr uint32_t kAuxQueues = 8;
-constexpr size_t kWorkWords = size_t(kMaxQueues + kAuxQueues) * kCounterStride;
+constexpr size_t kWorkWords = size_t(kMaxQueues + kAuxQueues + 1u) * kCounterStride;
 
 // How a walk launch runs: the fast form with the acceptor draws of models
 // without distance broadening from threshold rows (kPassGuided) or by the
@@ -166,7 +166,7 @@ struct PopControl {
     uint32_t pad[60];  // the models that follow start 256-byte aligned
 };
 
-// Population runs: what the finish kernel reports besides the sets' results.
+// Population runs: what pop_finish_kernel reports besides the sets' results.
 struct PopStatus {
     uint32_t replays;   // units the fast pass abandoned
     uint32_t overflow;  // 1: more than the replay list holds (results invalid)

@@ -45,3 +45,40 @@ def test_walk_batches(gpu_mc, oracle, bursts, R, B, nsets, v):
         if i < 4:
             h1, _, _, _ = pda.evaluate(m, n, a, R, 31, set_id=2 + 5 * i)
             assert np.array_equal(h1.astype(np.int64), want), f"set {i} alone"
+
+
+@pytest.mark.parametrize("B,left_pad", [(1, 0), (63, 2), (64, 64), (65, 0), (129, 63), (1024, 5)])
+@pytest.mark.parametrize("bg", [0.0, 6e4])
+def test_run_end(gpu_mc, oracle, B, left_pad, bg):
+    """The end of a run by one wave, 64 bins at a time, with units replayed
+    (a background whose mean leaves the fast form) and without, twice: the
+    last workgroup leaves the rows and the counters zero."""
+    n, R, seed = 3, 6, 77
+    rng = np.random.default_rng(B)
+    args = synth.make_args([0.2, 0.5, 0.8], synth.loguniform_rates(rng, 6, 3e2, 8e3))
+    d = synth.generate(300, args, n, seed=B + 1)
+    if bg:
+        d.bg_dd, d.bg_ad = bg, bg
+    obs = rng.uniform(0, 1, 300).astype(np.float32)
+    m = gpu_mc
+    m.load(d, SgDivSr=obs, nbins=B, left_pad=left_pad)
+    m.set_photophysics(0, *synth.PHOTOPHYSICS)
+    m.set_burst_range(0, -1, 0)
+    od = oracle.Data.from_bursts(d)
+    p = oracle.make_params(n, args, *synth.PHOTOPHYSICS)
+    want = oracle.run(od, p, R=R, seed=seed, set_id=3, B=B, want_units=False)["hist"]
+    c32, c64, eff = oracle.chi2(oracle.hist(obs, B).astype(np.float32), want, R, n,
+                                left_pad=left_pad)
+    m.set_population([n, n], [args, args])
+    for _ in range(2):
+        h, g64, g32, geff = pda.evaluate(m, n, args, R, seed, set_id=3)
+        assert np.array_equal(h.astype(np.int64), want)
+        # the oracle's sums, operation for operation
+        assert geff == eff and np.array_equal([g32, g64], [c32, c64], equal_nan=True)
+        assert (m.run_stats(0)[1] > 0) == (bg > 0)
+        m.run_population(R=R, seed=seed, set_base=3, set_stride=0)
+        h, g64, g32, geff = m.get_population_result()
+        for i in range(2):
+            assert np.array_equal(h[i].astype(np.int64), want)
+            assert geff[i] == eff
+            assert np.array_equal([g32[i], g64[i]], [c32, c64], equal_nan=True)
