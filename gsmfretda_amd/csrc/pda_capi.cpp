@@ -191,18 +191,9 @@ int upload_model(Slot& s) {
         set_error(err);
         return rc;
     }
-    if (s.model_pending) {
-        HIP_TRY(hipEventSynchronize(s.model_copied));
-        s.model_pending = false;
-    }
-    s.h_blob->m = M;
-    build_binom_table(M, s.h_blob->tab);
     s.any_v = M.any_v != 0;
     s.quick_rates = M.quick_rates != 0;
-    HIP_TRY(hipMemcpyAsync(s.d_blob, s.h_blob, sizeof(ModelBlob), hipMemcpyHostToDevice, s.stream));
-    HIP_TRY(hipEventRecord(s.model_copied, s.stream));
-    if (!s.any_v) HIP_TRY(launch_guide(s.d_blob, 1, M.n, s.d_thr, s.d_guide, s.stream));
-    s.model_pending = true;
+    HIP_TRY(launch_model(M, s.d_model, s.d_thr, s.d_guide, s.stream));
     return PDA_OK;
 }
 
@@ -237,15 +228,13 @@ int pda_create(int device, int nstreams, pda_ctx** out) {
     ctx->slots.resize(size_t(nstreams));
     for (auto& s : ctx->slots) {
         if (hipStreamCreateWithFlags(&s.stream, hipStreamNonBlocking) != hipSuccess ||
-            hipHostMalloc(reinterpret_cast<void**>(&s.h_blob), sizeof(ModelBlob), hipHostMallocDefault) != hipSuccess ||
-            hipMalloc(&s.d_blob, sizeof(ModelBlob)) != hipSuccess ||
+            hipMalloc(&s.d_model, sizeof(Model)) != hipSuccess ||
             hipMalloc(&s.d_thr, sizeof(ThrPair) * kGuideThrPairs) != hipSuccess ||
             hipMalloc(&s.d_guide, kGuideBytes) != hipSuccess ||
             hipMalloc(&s.d_replay_count, sizeof(uint32_t)) != hipSuccess ||
             hipMemset(s.d_replay_count, 0, sizeof(uint32_t)) != hipSuccess ||
             hipMalloc(&s.d_work, sizeof(uint32_t) * kWorkWords) != hipSuccess ||
             hipMemset(s.d_work, 0, sizeof(uint32_t) * kWorkWords) != hipSuccess ||
-            hipEventCreateWithFlags(&s.model_copied, hipEventDisableTiming) != hipSuccess ||
             hipMalloc(&s.d_hist_acc, sizeof(int32_t) * kMaxBins * 8) != hipSuccess ||
             hipHostMalloc(reinterpret_cast<void**>(&s.h_result),
                           sizeof(ResultHeader) + sizeof(int32_t) * kMaxBins,
@@ -272,10 +261,9 @@ int pda_destroy(pda_ctx* ctx) {
     (void)hipSetDevice(ctx->device);
     for (auto& s : ctx->slots) {
         if (s.stream) (void)hipStreamSynchronize(s.stream);
-        (void)hipFree(s.d_blob);
+        (void)hipFree(s.d_model);
         (void)hipFree(s.d_thr);
         (void)hipFree(s.d_guide);
-        (void)hipHostFree(s.h_blob);
         (void)hipFree(s.d_replay);
         (void)hipFree(s.d_replay_count);
         (void)hipFree(s.d_work);
@@ -285,7 +273,6 @@ int pda_destroy(pda_ctx* ctx) {
         (void)hipFree(s.d_acc);
         (void)hipFree(s.d_F);
         (void)hipHostFree(s.h_E);
-        if (s.model_copied) (void)hipEventDestroy(s.model_copied);
         if (s.ev0) (void)hipEventDestroy(s.ev0);
         if (s.ev_mid) (void)hipEventDestroy(s.ev_mid);
         if (s.ev1) (void)hipEventDestroy(s.ev1);
@@ -492,7 +479,7 @@ int pda_run(pda_ctx* ctx, int sid, int R, uint32_t seed, uint32_t set_id, int fl
     HIP_TRY(hipEventRecord(s->ev0, s->stream));
     const BinomGuide guide{s->d_thr, s->d_guide};
     const FastArgs fa = fast_args(s->n, s->quick_rates, a.clk_p, s->ph.r0, ctx->max_P);
-    HIP_TRY(launch_walk(pass, grid, ctx->d_bursts, ctx->d_ticks, ctx->d_links, s->d_blob, guide, a,
+    HIP_TRY(launch_walk(pass, grid, ctx->d_bursts, ctx->d_ticks, ctx->d_links, s->d_model, guide, a,
                         fa, s->d_hist_acc, s->d_replay, s->d_replay_count, s->d_work, outE, outAcc,
                         outF, nullptr, nullptr, s->stream));
     HIP_TRY(hipEventRecord(s->ev_mid, s->stream));
@@ -500,7 +487,7 @@ int pda_run(pda_ctx* ctx, int sid, int R, uint32_t seed, uint32_t set_id, int fl
     // of the run; the grid is sized for the worst case and its unneeded
     // workgroups exit at once
     HIP_TRY(launch_walk(kPassReplay, replay_grid(ctx, uint64_t(nunits)), ctx->d_bursts,
-                        ctx->d_ticks, ctx->d_links, s->d_blob, guide, a, fa, s->d_hist_acc,
+                        ctx->d_ticks, ctx->d_links, s->d_model, guide, a, fa, s->d_hist_acc,
                         s->d_replay, s->d_replay_count, s->d_work, outE, outAcc, outF, ctx->d_obs,
                         s->d_result, s->stream));
     HIP_TRY(hipEventRecord(s->ev1, s->stream));

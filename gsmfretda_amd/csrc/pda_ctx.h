@@ -69,7 +69,7 @@ struct Population {
     bool quick_rates = false;        // of every set
     float r0 = 0.f;                  // photophysics the sets were built with
     size_t cap_sets = 0;             // allocated sets
-    uint8_t* h_in = nullptr;         // pinned: PopControl + ModelBlob[cap_sets]
+    uint8_t* h_in = nullptr;         // pinned: PopControl + Model[cap_sets]
     uint8_t* d_in = nullptr;
     int cap_B = 0;
     int32_t* d_hist_acc = nullptr;   // [cap_sets][8][cap_B], zero between runs
@@ -88,6 +88,8 @@ struct Population {
     uint8_t* d_guide = nullptr;
     size_t cap_guide_states = 0;
     bool guided = false;
+    BinomTable* d_tabs = nullptr;    // else, where the sets draw by the table: theirs
+    size_t cap_tabs = 0;
     int max_states = 0;
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
@@ -110,9 +112,9 @@ struct RbState {
     void* d_rbm = nullptr;             // RbModel
     void* h_rbm = nullptr;             // pinned
     // the walk's model when the state is one set of an RB population (the
-    // single-set forward walks the slot's own d_blob)
-    ModelBlob* d_blob = nullptr;
-    ModelBlob* h_blob = nullptr;       // pinned
+    // single-set forward walks the slot's own d_model)
+    Model* d_model = nullptr;
+    Model* h_model = nullptr;          // pinned
     uint2* d_cnt = nullptr;            // per unit: photon counts per state
     float* d_F = nullptr;              // per unit: F
     float* d_S = nullptr;              // per unit: scores of the rates
@@ -162,8 +164,7 @@ struct RbState {
 struct Slot {
     bool quick_rates = false;     // every rate of the set is in quotient()'s range
     hipStream_t stream = nullptr;
-    ModelBlob* h_blob = nullptr;  // pinned staging of the model tables
-    ModelBlob* d_blob = nullptr;
+    Model* d_model = nullptr;
     // threshold rows of the fast walk's binomial draws for the uploaded set
     // (guide_kernel, enqueued with every model upload)
     ThrPair* d_thr = nullptr;     // kGuideThrPairs
@@ -173,8 +174,6 @@ struct Slot {
     uint32_t* d_replay_count = nullptr;
     uint32_t* d_work = nullptr;    // kWorkWords: work counters of the run, one per line
     size_t replay_cap = 0;
-    hipEvent_t model_copied = nullptr;
-    bool model_pending = false;
     int n = 0;
     bool have_params = false;
     Photophysics ph;
@@ -271,22 +270,26 @@ hipError_t walk_occupancy(int pass, int B, int* blocks_per_cu);
 hipError_t pop_walk_occupancy(int pass, int B, int* blocks_per_cu);
 // kPassReplay also ends the run: histogram and chi2 against obs into result
 hipError_t launch_walk(int pass, uint32_t grid, const BurstDesc* bursts, const uint32_t* ticks,
-                       const uint2* links, const ModelBlob* blob, const BinomGuide& guide,
+                       const uint2* links, const Model* model, const BinomGuide& guide,
                        const RunArgs& a, const FastArgs& fa, int32_t* hist_acc, uint32_t* replay,
                        uint32_t* replay_count, uint32_t* work, float* outE, int32_t* outAcc,
                        float* outF, const float* obs, ResultHeader* result, hipStream_t stream);
-hipError_t launch_guide(const ModelBlob* blobs, int nsets, int max_states, ThrPair* thr,
+// stores the model of a parameter set and builds its threshold rows
+hipError_t launch_model(const Model& M, Model* model, ThrPair* thr, uint8_t* guide,
+                        hipStream_t stream);
+hipError_t launch_guide(const Model* models, int nsets, int max_states, ThrPair* thr,
                         uint8_t* guide, hipStream_t stream);
 hipError_t launch_pop_walk(int pass, uint32_t grid, const BurstDesc* bursts,
                            const uint32_t* ticks, const uint2* links, const PopControl* ctl,
-                           const ModelBlob* blobs, const BinomGuide& guide, const RunArgs& a,
+                           const Model* models, const BinomTable* tabs,
+                           const BinomGuide& guide, const RunArgs& a,
                            const FastArgs& fa, int32_t* hist_acc, uint64_t* replay,
                            uint32_t* replay_count, uint32_t* work, hipStream_t stream);
 hipError_t launch_pop_replay(const BurstDesc* bursts, const uint32_t* ticks, const uint2* links,
-                             const PopControl* ctl, const ModelBlob* blobs, const RunArgs& a,
+                             const PopControl* ctl, const Model* models, const RunArgs& a,
                              int32_t* hist_acc, const uint64_t* replay,
                              const uint32_t* replay_count, uint32_t grid, hipStream_t stream);
-hipError_t launch_pop_finish(const ModelBlob* blobs, const RunArgs& a, const float* obs,
+hipError_t launch_pop_finish(const Model* models, const RunArgs& a, const float* obs,
                              int32_t* hist_acc, uint32_t* replay_count, uint32_t* work,
                              PopStatus* status, SetResult* results, int32_t* hists,
                              hipStream_t stream);
@@ -308,7 +311,7 @@ hipError_t rb_walk_occupancy(bool scores, int n, int* per_cu);
 // abandoned (replay_grid workgroups; those beyond the list's need exit)
 hipError_t launch_rb_walk(bool scores, int n, uint32_t grid, uint32_t replay_grid,
                           const BurstDesc* bursts, const uint32_t* ticks, const uint2* links,
-                          const ModelBlob* blob, const RbModel* rbm, const RunArgs& a,
+                          const Model* model, const RbModel* rbm, const RunArgs& a,
                           const FastArgs& fa, uint2* cnt, float* F, float* S, uint32_t* work,
                           uint32_t* big, uint32_t* huge,
                           uint32_t* big_count, uint32_t* replay, uint32_t* replay_count,

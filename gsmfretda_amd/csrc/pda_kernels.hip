@@ -169,7 +169,8 @@ struct FastIO {
     const BurstDesc* bursts;
     const uint32_t* ticks;
     const uint2* links;
-    const ModelBlob* blobs;    // [1], or the population's sets
+    const Model* models;       // [1], or the population's sets
+    const BinomTable* tabs;    // kPassTable: [sets]
     const PopControl* ctl;     // population: the sets' stream keys
     BinomGuide guide;
     int32_t* hist_acc;
@@ -197,7 +198,7 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(
     const uint32_t lane = threadIdx.x;
     for (uint32_t i = lane; i < uint32_t(kSlots) * uint32_t(a.B); i += kWave) s_hist[i] = 0;
     auto load_model = [&](uint32_t into, uint32_t set) {
-        const uint32_t* src = reinterpret_cast<const uint32_t*>(&io.blobs[set].m);
+        const uint32_t* src = reinterpret_cast<const uint32_t*>(&io.models[set]);
         uint32_t* dst = reinterpret_cast<uint32_t*>(&sM[into]);
         for (uint32_t i = lane; i < sizeof(Mod) / 4; i += kWave) dst[i] = src[i];
         wave_lds_sync();
@@ -338,7 +339,7 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(
                 r = fast_window<false, BinomGuide>(M, &io.guide, key, d.P, d.stop_rel, d.T, ticks,
                                                    links, a, fa, st);
             } else {
-                r = fast_window<false, BinomTable>(M, &io.blobs[set].tab, key, d.P, d.stop_rel,
+                r = fast_window<false, BinomTable>(M, &io.tabs[set], key, d.P, d.stop_rel,
                                                    d.T, ticks, links, a, fa, st);
             }
             busy = r == kStepMore;
@@ -486,7 +487,7 @@ __device__ __forceinline__ void finish_run(const RunArgs& a, const float* __rest
 // 8 XCDs round-robin, so the atomics of a launch spread over 8 x B addresses).
 __device__ __forceinline__ void replay_units(
     const BurstDesc* __restrict__ bursts, const uint32_t* __restrict__ ticks,
-    const uint2* __restrict__ links, const ModelBlob* __restrict__ blob, const RunArgs& a,
+    const uint2* __restrict__ links, const Model* __restrict__ model, const RunArgs& a,
     int32_t* __restrict__ hist_acc, const uint32_t* __restrict__ replay, uint32_t nunits,
     uint32_t alive, uint32_t* __restrict__ work, float* __restrict__ outE,
     int32_t* __restrict__ outAcc, float* __restrict__ outF, uint32_t lane) {
@@ -495,7 +496,7 @@ __device__ __forceinline__ void replay_units(
     const uint32_t queues = alive < kReplayQueues ? alive : kReplayQueues;
     const uint32_t queue = blockIdx.x % queues;
     {
-        const uint32_t* src = reinterpret_cast<const uint32_t*>(&blob->m);
+        const uint32_t* src = reinterpret_cast<const uint32_t*>(model);
         uint32_t* dst = reinterpret_cast<uint32_t*>(&sM);
         for (uint32_t i = lane; i < sizeof(Model) / 4; i += kWave) dst[i] = src[i];
         for (uint32_t i = lane; i < uint32_t(a.B); i += kWave) s_hist[i] = 0;
@@ -573,7 +574,7 @@ __device__ __forceinline__ void replay_units(
 // 20,000 x 4 of 3 broadened states at 200 bins 115; now 69 and 89.
 __global__ __launch_bounds__(kWave) void walk_kernel(
     const BurstDesc* __restrict__ bursts, const uint32_t* __restrict__ ticks,
-    const uint2* __restrict__ links, const ModelBlob* __restrict__ blob, const RunArgs a,
+    const uint2* __restrict__ links, const Model* __restrict__ model, const RunArgs a,
     int32_t* __restrict__ hist_acc, const uint32_t* __restrict__ replay,
     uint32_t* __restrict__ replay_count, uint32_t* __restrict__ work, float* __restrict__ outE,
     int32_t* __restrict__ outAcc, float* __restrict__ outF, const float* __restrict__ obs,
@@ -587,7 +588,7 @@ __global__ __launch_bounds__(kWave) void walk_kernel(
     const uint32_t lane = threadIdx.x;
     if (blockIdx.x >= (alive ? alive : 1u)) return;  // uniform over the workgroup
     if (alive) {
-        replay_units(bursts, ticks, links, blob, a, hist_acc, replay, nunits, alive, work, outE,
+        replay_units(bursts, ticks, links, model, a, hist_acc, replay, nunits, alive, work, outE,
                      outAcc, outF, lane);
         __threadfence();
         uint32_t ended = 0;
@@ -600,26 +601,19 @@ __global__ __launch_bounds__(kWave) void walk_kernel(
     finish_run(a, obs, hist_acc, replay_count, c, work, result, lane);
 }
 
-// Threshold rows of the fast walk's binomial draws, one wave per (state,
-// photon count) row of a parameter set (the operations and their order are
-// those of build_guide_row_host): blockIdx.x = state * kBinomTable + count,
-// blockIdx.y = set; set i's state s takes table row blobs[i].m.guide_base + s.
-// Runs on the stream after the model upload, so the walks that follow read
-// finished rows.
-__global__ __launch_bounds__(kWave) void guide_kernel(const ModelBlob* __restrict__ blobs,
-                                                      ThrPair* __restrict__ thr,
-                                                      uint8_t* __restrict__ guide) {
+// One threshold row of the fast walk's binomial draws, by one wave: state s
+// with m photons (the operations and their order are those of
+// build_guide_row_host), in table row M.guide_base + s.
+__device__ __forceinline__ void guide_row(const Model& M, int s, int m, ThrPair* __restrict__ thr,
+                                          uint8_t* __restrict__ guide) {
     __shared__ int64_t s_up[kBinomTable + 1];
-    const ModelBlob* blob = blobs + blockIdx.y;
-    const int s = int(blockIdx.x) / kBinomTable;
-    const int m = int(blockIdx.x) % kBinomTable;
-    if (s >= blob->m.n) return;  // uniform over the workgroup
-    const int srow = blob->m.guide_base + s;
+    const int srow = M.guide_base + s;
     const int lane = int(threadIdx.x);
-    const double pp = blob->m.pp[s];
-    const double q = blob->m.qq[s];
-    const int bound = blob->tab.bound[s][m];
-    const double qn = blob->tab.qn[s][m];
+    const double pp = M.pp[s];
+    const double q = M.qq[s];
+    double qn;
+    int32_t bound;
+    inversion_constants(m, pp, q, M.lq[s], &qn, &bound);
     ThrPair* t = thr + guide_row_offset(srow, m);
     double carryP = 1.0, carryC = 0.0;
     int end = -1;
@@ -668,6 +662,36 @@ __global__ __launch_bounds__(kWave) void guide_kernel(const ModelBlob* __restric
     guide[(size_t(srow) * kBinomTable + size_t(m)) * kGuideBuckets + size_t(lane)] = uint8_t(lo_i);
 }
 
+// A slot's parameter set: its model tables into the slot's device copy, and
+// its threshold rows (one workgroup each: state * kBinomTable + count) for the
+// walks behind on the stream.  The model is an argument of the launch, which
+// is taken when it is made: no staging buffer, no copy in front of it.  With
+// the copy, and the rows' constants formed on the host (131,072 exponentials
+// for a generation of 256 sets of 4 states), 5,000 bursts x 20 of 2 states took
+// 69 us and that generation 12.5 ms; now 52 us and 10.9 ms.
+__global__ __launch_bounds__(kWave) void model_kernel(const Model M, Model* __restrict__ model,
+                                                      ThrPair* __restrict__ thr,
+                                                      uint8_t* __restrict__ guide) {
+    if (blockIdx.x == 0) {
+        const uint32_t* src = reinterpret_cast<const uint32_t*>(&M);
+        uint32_t* dst = reinterpret_cast<uint32_t*>(model);
+        for (uint32_t i = threadIdx.x; i < sizeof(Model) / 4; i += kWave) dst[i] = src[i];
+    }
+    if (M.any_v) return;  // draws by the loop, no rows
+    guide_row(M, int(blockIdx.x) / kBinomTable, int(blockIdx.x) % kBinomTable, thr, guide);
+}
+
+// The threshold rows of a population's sets: blockIdx.x as above, blockIdx.y
+// the set.
+__global__ __launch_bounds__(kWave) void guide_kernel(const Model* __restrict__ models,
+                                                      ThrPair* __restrict__ thr,
+                                                      uint8_t* __restrict__ guide) {
+    const Model& M = models[blockIdx.y];
+    const int s = int(blockIdx.x) / kBinomTable;
+    if (s >= M.n) return;  // uniform over the workgroup
+    guide_row(M, s, int(blockIdx.x) % kBinomTable, thr, guide);
+}
+
 // ---- population runs ---------------------------------------------------------
 //
 // A population of parameter sets (an optimiser generation) over the same
@@ -683,7 +707,7 @@ __global__ __launch_bounds__(kWave) void guide_kernel(const ModelBlob* __restric
 __global__ __launch_bounds__(kWave) void pop_walk_kernel(
     const BurstDesc* __restrict__ bursts, const uint32_t* __restrict__ ticks,
     const uint2* __restrict__ links, const PopControl* __restrict__ ctl,
-    const ModelBlob* __restrict__ blobs, const RunArgs a, int32_t* __restrict__ hist_acc,
+    const Model* __restrict__ models, const RunArgs a, int32_t* __restrict__ hist_acc,
     uint32_t* __restrict__ work) {
     __shared__ Model sM[2];
     extern __shared__ int32_t s_hist[];  // [2][a.B]
@@ -730,7 +754,7 @@ __global__ __launch_bounds__(kWave) void pop_walk_kernel(
                 if (old >= 0)
                     flush_hist(s_hist + other * uint32_t(a.B),
                                hist_acc + (size_t(old) * 8u + xrow) * size_t(a.B), a.B, lane);
-                const uint32_t* src = reinterpret_cast<const uint32_t*>(&blobs[pool_set].m);
+                const uint32_t* src = reinterpret_cast<const uint32_t*>(&models[pool_set]);
                 uint32_t* dst = reinterpret_cast<uint32_t*>(&sM[other]);
                 for (uint32_t i = lane; i < sizeof(Model) / 4; i += kWave) dst[i] = src[i];
                 __syncthreads();
@@ -782,7 +806,7 @@ __global__ __launch_bounds__(kWave) void pop_walk_kernel(
 __global__ __launch_bounds__(kWave) void pop_replay_kernel(
     const BurstDesc* __restrict__ bursts, const uint32_t* __restrict__ ticks,
     const uint2* __restrict__ links, const PopControl* __restrict__ ctl,
-    const ModelBlob* __restrict__ blobs, const RunArgs a, int32_t* __restrict__ hist_acc,
+    const Model* __restrict__ models, const RunArgs a, int32_t* __restrict__ hist_acc,
     const uint64_t* __restrict__ replay, const uint32_t* __restrict__ replay_count) {
     const uint32_t count = *replay_count < a.replay_cap ? *replay_count : a.replay_cap;
     const uint32_t stride = gridDim.x * blockDim.x;
@@ -793,7 +817,7 @@ __global__ __launch_bounds__(kWave) void pop_replay_kernel(
         const uint32_t b = a.begin + bl;
         const BurstDesc d = bursts[b];
         const UnitKey key{ctl->seed, ctl->set_base + set * ctl->set_stride, u - bl * a.R, b};
-        const WalkOut o = walk_unit<false>(blobs[set].m, nullptr, key, d.P, d.stop_rel, d.T,
+        const WalkOut o = walk_unit<false>(models[set], nullptr, key, d.P, d.stop_rel, d.T,
                                            ticks + d.off, links + d.off, a);
         tally(hist_acc + size_t(set) * 8u * size_t(a.B), a.B, o.acc, o.F);
     }
@@ -804,7 +828,7 @@ __global__ __launch_bounds__(kWave) void pop_replay_kernel(
 // of freedom; workgroup 0 reports and resets the replay count and the work
 // counters.
 __global__ __launch_bounds__(kWave) void pop_finish_kernel(
-    const ModelBlob* __restrict__ blobs, const RunArgs a, const float* __restrict__ obs,
+    const Model* __restrict__ models, const RunArgs a, const float* __restrict__ obs,
     int32_t* __restrict__ hist_acc, uint32_t* __restrict__ replay_count,
     uint32_t* __restrict__ work, PopStatus* __restrict__ status, SetResult* __restrict__ results,
     int32_t* __restrict__ hists) {
@@ -813,7 +837,7 @@ __global__ __launch_bounds__(kWave) void pop_finish_kernel(
     const Chi2Sum c = chi2_fold(a, obs, hist_acc + size_t(set) * 8u * B, B,
                                 hists + size_t(set) * B, lane);
     if (lane == 0) {
-        const int n = blobs[set].m.n;
+        const int n = models[set].n;
         const int dof = c.filled - n * (n + 1);
         SetResult r;
         r.chi2_ref = c.c32 / float(dof);
@@ -1089,16 +1113,16 @@ static void launch_fast(uint32_t grid, size_t lds, const FastIO& io, const RunAr
 }
 
 hipError_t launch_walk(int pass, uint32_t grid, const BurstDesc* bursts, const uint32_t* ticks,
-                       const uint2* links, const ModelBlob* blob, const BinomGuide& guide,
+                       const uint2* links, const Model* model, const BinomGuide& guide,
                        const RunArgs& a, const FastArgs& fa, int32_t* hist_acc, uint32_t* replay,
                        uint32_t* replay_count, uint32_t* work, float* outE, int32_t* outAcc,
                        float* outF, const float* obs, ResultHeader* result, hipStream_t stream) {
     const size_t lds = sizeof(int32_t) * size_t(a.B);
-    const FastIO io{bursts, ticks, links, blob, nullptr, guide, hist_acc, replay,
+    const FastIO io{bursts, ticks, links, model, nullptr, nullptr, guide, hist_acc, replay,
                     replay_count, work, outE, outAcc, outF};
     if (pass == kPassReplay)
         hipLaunchKernelGGL(walk_kernel, dim3(grid), dim3(kWave), lds, stream, bursts, ticks, links,
-                           blob, a, hist_acc, replay, replay_count, work, outE, outAcc, outF, obs,
+                           model, a, hist_acc, replay, replay_count, work, outE, outAcc, outF, obs,
                            result);
     else if (pass == kPassBroad && outE)
         launch_fast<false, kPassBroad, true>(grid, lds, io, a, fa, stream);
@@ -1111,10 +1135,17 @@ hipError_t launch_walk(int pass, uint32_t grid, const BurstDesc* bursts, const u
     return hipGetLastError();
 }
 
-hipError_t launch_guide(const ModelBlob* blobs, int nsets, int max_states, ThrPair* thr,
+hipError_t launch_model(const Model& M, Model* model, ThrPair* thr, uint8_t* guide,
+                        hipStream_t stream) {
+    hipLaunchKernelGGL(model_kernel, dim3(M.any_v ? 1u : uint32_t(M.n) * kBinomTable), dim3(kWave),
+                       0, stream, M, model, thr, guide);
+    return hipGetLastError();
+}
+
+hipError_t launch_guide(const Model* models, int nsets, int max_states, ThrPair* thr,
                         uint8_t* guide, hipStream_t stream) {
     hipLaunchKernelGGL(guide_kernel, dim3(uint32_t(max_states) * kBinomTable, uint32_t(nsets)),
-                       dim3(kWave), 0, stream, blobs, thr, guide);
+                       dim3(kWave), 0, stream, models, thr, guide);
     return hipGetLastError();
 }
 
@@ -1132,15 +1163,16 @@ hipError_t pop_walk_occupancy(int pass, int B, int* blocks_per_cu) {
 
 hipError_t launch_pop_walk(int pass, uint32_t grid, const BurstDesc* bursts,
                            const uint32_t* ticks, const uint2* links, const PopControl* ctl,
-                           const ModelBlob* blobs, const BinomGuide& guide, const RunArgs& a,
+                           const Model* models, const BinomTable* tabs,
+                           const BinomGuide& guide, const RunArgs& a,
                            const FastArgs& fa, int32_t* hist_acc, uint64_t* replay,
                            uint32_t* replay_count, uint32_t* work, hipStream_t stream) {
     const size_t lds = sizeof(int32_t) * 2u * size_t(a.B);
-    const FastIO io{bursts, ticks, links, blobs, ctl, guide, hist_acc, replay,
+    const FastIO io{bursts, ticks, links, models, tabs, ctl, guide, hist_acc, replay,
                     replay_count, work, nullptr, nullptr, nullptr};
     if (pass == kPassGeneral)
         hipLaunchKernelGGL(pop_walk_kernel, dim3(grid), dim3(kWave), lds, stream, bursts, ticks,
-                           links, ctl, blobs, a, hist_acc, work);
+                           links, ctl, models, a, hist_acc, work);
     else if (pass == kPassBroad)
         launch_fast<true, kPassBroad, false>(grid, lds, io, a, fa, stream);
     else if (pass == kPassTable)
@@ -1151,19 +1183,19 @@ hipError_t launch_pop_walk(int pass, uint32_t grid, const BurstDesc* bursts,
 }
 
 hipError_t launch_pop_replay(const BurstDesc* bursts, const uint32_t* ticks, const uint2* links,
-                             const PopControl* ctl, const ModelBlob* blobs, const RunArgs& a,
+                             const PopControl* ctl, const Model* models, const RunArgs& a,
                              int32_t* hist_acc, const uint64_t* replay,
                              const uint32_t* replay_count, uint32_t grid, hipStream_t stream) {
     hipLaunchKernelGGL(pop_replay_kernel, dim3(grid), dim3(kWave), 0, stream, bursts, ticks,
-                       links, ctl, blobs, a, hist_acc, replay, replay_count);
+                       links, ctl, models, a, hist_acc, replay, replay_count);
     return hipGetLastError();
 }
 
-hipError_t launch_pop_finish(const ModelBlob* blobs, const RunArgs& a, const float* obs,
+hipError_t launch_pop_finish(const Model* models, const RunArgs& a, const float* obs,
                              int32_t* hist_acc, uint32_t* replay_count, uint32_t* work,
                              PopStatus* status, SetResult* results, int32_t* hists,
                              hipStream_t stream) {
-    hipLaunchKernelGGL(pop_finish_kernel, dim3(a.nsets), dim3(kWave), 0, stream, blobs, a, obs,
+    hipLaunchKernelGGL(pop_finish_kernel, dim3(a.nsets), dim3(kWave), 0, stream, models, a, obs,
                        hist_acc, replay_count, work, status, results, hists);
     return hipGetLastError();
 }

@@ -202,6 +202,7 @@ int build_model(const Photophysics& s, int n, const float* args, int nargs, Mode
         M.flip[i] = p > 0.5 ? 1 : 0;
         M.pp[i] = M.flip[i] ? 1.0 - p : p;
         M.qq[i] = 1.0 - M.pp[i];
+        M.lq[i] = dlog(M.qq[i]);
     }
     return PDA_OK;
 }
@@ -210,15 +211,8 @@ int build_model(const Photophysics& s, int n, const float* args, int nargs, Mode
 void build_binom_table(const Model& M, BinomTable& T) {
     std::memset(&T, 0, sizeof T);
     for (int s = 0; s < M.n; ++s) {
-        const double pp = M.pp[s], q = M.qq[s];
-        const double lq = dlog(q);
-        for (int n = 0; n < kBinomTable; ++n) {
-            T.qn[s][n] = dexp(double(n) * lq);
-            const double np = double(n) * pp;
-            double lim = np + 10.0 * std::sqrt(np * q + 1.0);
-            if (double(n) < lim) lim = double(n);
-            T.bound[s][n] = int32_t(lim);
-        }
+        for (int n = 0; n < kBinomTable; ++n)
+            inversion_constants(n, M.pp[s], M.qq[s], M.lq[s], &T.qn[s][n], &T.bound[s][n]);
     }
 }
 

@@ -381,6 +381,16 @@ PDA_HD float distance_efficiency_quick(float rd, float r0, float r0_r) {
 // typical burst produces.
 constexpr int kInversionMaxN = 128;
 
+// q^n and the inversion bound min(n, np + 10 sqrt(npq + 1)) (src/binom.cuh:
+// 135-169) of Binomial(n, p), p <= 1/2; lq = log(q).
+PDA_HD void inversion_constants(int n, double p, double q, double lq, double* qn, int32_t* bound) {
+    *qn = dexp(double(n) * lq);
+    const double np = double(n) * p;
+    double lim = np + 10.0 * sqrt(np * q + 1.0);
+    if (double(n) < lim) lim = double(n);
+    *bound = int32_t(lim);
+}
+
 PDA_HD int64_t binomial_inversion(int n, double p, double U, const UnitKey& key, uint32_t w) {
     const double q = 1.0 - p;
     const double qn = dexp(double(n) * dlog(q));

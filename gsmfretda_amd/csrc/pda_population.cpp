@@ -50,9 +50,12 @@ void free_population(Population& p) {
     (void)hipFree(p.d_in);
     (void)hipFree(p.d_thr);
     (void)hipFree(p.d_guide);
+    (void)hipFree(p.d_tabs);
     p.d_thr = nullptr;
     p.d_guide = nullptr;
     p.cap_guide_states = 0;
+    p.d_tabs = nullptr;
+    p.cap_tabs = 0;
     (void)hipFree(p.d_hist_acc);
     (void)hipHostFree(p.h_out);
     (void)hipFree(p.d_replay);
@@ -76,10 +79,10 @@ constexpr int kMaxSets = 1 << 16;
 // larger population draws by the inversion loop.
 constexpr size_t kPopGuideBudget = size_t(1) << 30;
 
-size_t in_bytes(size_t nsets) { return sizeof(PopControl) + sizeof(ModelBlob) * nsets; }
+size_t in_bytes(size_t nsets) { return sizeof(PopControl) + sizeof(Model) * nsets; }
 
-const ModelBlob* blobs_of(const uint8_t* base) {
-    return reinterpret_cast<const ModelBlob*>(base + sizeof(PopControl));
+const Model* models_of(const uint8_t* base) {
+    return reinterpret_cast<const Model*>(base + sizeof(PopControl));
 }
 
 size_t out_bytes(size_t nsets, int B) {
@@ -131,7 +134,7 @@ int ensure_pop_buffers(pda_ctx* ctx, Slot& s, int B) {
 int enqueue_population(pda_ctx* ctx, Slot& s, int pass, uint32_t grid, const RunArgs& a) {
     Population& p = s.pop;
     const PopControl* ctl = reinterpret_cast<const PopControl*>(p.d_in);
-    const ModelBlob* blobs = blobs_of(p.d_in);
+    const Model* models = models_of(p.d_in);
     PopStatus* status = reinterpret_cast<PopStatus*>(p.d_out);
     SetResult* results = reinterpret_cast<SetResult*>(p.d_out + sizeof(PopStatus));
     int32_t* hists = reinterpret_cast<int32_t*>(p.d_out + sizeof(PopStatus) +
@@ -140,19 +143,19 @@ int enqueue_population(pda_ctx* ctx, Slot& s, int pass, uint32_t grid, const Run
                            s.stream));
     BinomGuide guide{nullptr, nullptr};
     if (pass == kPassGuided) {
-        HIP_TRY(launch_guide(blobs, p.nsets, p.max_states, p.d_thr, p.d_guide, s.stream));
+        HIP_TRY(launch_guide(models, p.nsets, p.max_states, p.d_thr, p.d_guide, s.stream));
         guide = BinomGuide{p.d_thr, p.d_guide};
     }
-    HIP_TRY(launch_pop_walk(pass, grid, ctx->d_bursts, ctx->d_ticks, ctx->d_links, ctl, blobs,
-                            guide, a, fast_args(p.max_states, p.quick_rates, a.clk_p, p.r0,
+    HIP_TRY(launch_pop_walk(pass, grid, ctx->d_bursts, ctx->d_ticks, ctx->d_links, ctl, models,
+                            p.d_tabs, guide, a, fast_args(p.max_states, p.quick_rates, a.clk_p, p.r0,
                                              ctx->max_P),
                             p.d_hist_acc, p.d_replay, p.d_replay_count, p.d_work,
                             s.stream));
     if (pass != kPassGeneral)
-        HIP_TRY(launch_pop_replay(ctx->d_bursts, ctx->d_ticks, ctx->d_links, ctl, blobs, a,
+        HIP_TRY(launch_pop_replay(ctx->d_bursts, ctx->d_ticks, ctx->d_links, ctl, models, a,
                                   p.d_hist_acc, p.d_replay, p.d_replay_count,
                                   uint32_t(ctx->num_cu) * 4u, s.stream));
-    HIP_TRY(launch_pop_finish(blobs, a, ctx->d_obs, p.d_hist_acc, p.d_replay_count, p.d_work,
+    HIP_TRY(launch_pop_finish(models, a, ctx->d_obs, p.d_hist_acc, p.d_replay_count, p.d_work,
                               status, results, hists, s.stream));
     return PDA_OK;
 }
@@ -368,13 +371,24 @@ int pda_set_population(pda_ctx* ctx, int sid, int nsets, const int32_t* nstates,
         HIP_TRY(hipMalloc(&p.d_guide, states * size_t(kBinomTable) * kGuideBuckets));
         p.cap_guide_states = states;
     }
+    if (!guided && !any_v) {
+        if (size_t(nsets) > p.cap_tabs) {
+            drop_graph(p);
+            (void)hipFree(p.d_tabs);
+            p.d_tabs = nullptr;
+            p.cap_tabs = 0;
+            HIP_TRY(hipMalloc(&p.d_tabs, sizeof(BinomTable) * size_t(nsets)));
+            p.cap_tabs = size_t(nsets);
+        }
+        std::vector<BinomTable> tabs(static_cast<size_t>(nsets));
+        for (int i = 0; i < nsets; ++i) build_binom_table(models[size_t(i)], tabs[size_t(i)]);
+        HIP_TRY(hipMemcpyAsync(p.d_tabs, tabs.data(), sizeof(BinomTable) * size_t(nsets),
+                               hipMemcpyHostToDevice, s->stream));
+        HIP_TRY(hipStreamSynchronize(s->stream));
+    }
     p.guided = guided;
     p.max_states = max_states;
-    ModelBlob* hb = reinterpret_cast<ModelBlob*>(p.h_in + sizeof(PopControl));
-    for (int i = 0; i < nsets; ++i) {
-        hb[i].m = models[size_t(i)];
-        build_binom_table(models[size_t(i)], hb[i].tab);
-    }
+    std::memcpy(p.h_in + sizeof(PopControl), models.data(), sizeof(Model) * size_t(nsets));
     p.nsets = nsets;
     p.n.assign(nstates, nstates + nsets);
     p.args.assign(args, args + nargs_total);

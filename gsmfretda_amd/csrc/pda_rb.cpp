@@ -29,8 +29,8 @@ namespace pda {
 void free_rb(RbState& r) {
     (void)hipFree(r.d_rbm);
     (void)hipHostFree(r.h_rbm);
-    (void)hipFree(r.d_blob);
-    (void)hipHostFree(r.h_blob);
+    (void)hipFree(r.d_model);
+    (void)hipHostFree(r.h_model);
     (void)hipFree(r.d_cnt);
     (void)hipFree(r.d_F);
     (void)hipFree(r.d_S);
@@ -316,11 +316,11 @@ int pass_shape(pda_ctx* ctx, int mode, int n, bool wide, int B, int cap, uint32_
 }
 
 // Enqueues one RB forward of model M -- the walk reading M from the device
-// blob d_blob -- over the slot's burst range into state r, on the slot's
+// model d_model -- over the slot's burst range into state r, on the slot's
 // stream.  sync_model: first wait for the stream, whose last run may still be
 // copying r's pinned model (a population forward waits once for all sets).
 int rb_enqueue_forward(pda_ctx* ctx, Slot& s, RbState& r, const Model& M,
-                       const ModelBlob* d_blob, int R, uint32_t seed, uint32_t set_id, int flags,
+                       const Model* d_model, int R, uint32_t seed, uint32_t set_id, int flags,
                        bool sync_model) {
     int rc = ensure_rb(ctx, r);
     if (rc) return rc;
@@ -454,7 +454,7 @@ int rb_enqueue_forward(pda_ctx* ctx, Slot& s, RbState& r, const Model& M,
                            s.rb_aux));
     HIP_TRY(hipEventRecord(s.rb_join, s.rb_aux));
     HIP_TRY(launch_rb_walk(scores, n, grid, uint32_t(ctx->num_cu) * 4u, ctx->d_bursts, ctx->d_ticks,
-                           ctx->d_links, d_blob, d_rbm, a,
+                           ctx->d_links, d_model, d_rbm, a,
                            fast_args(n, M.quick_rates != 0, a.clk_p, M.r0, ctx->max_P), r.d_cnt, r.d_F, r.d_S, r.d_work,
                            r.d_big, r.d_huge, r.d_big_count, r.d_replay, r.d_replay_count,
                            s.stream));
@@ -516,7 +516,7 @@ int pda_rb_forward(pda_ctx* ctx, int sid, int R, uint32_t seed, uint32_t set_id,
         int rc = build_model(s->ph, s->n, s->args.data(), int(s->args.size()), M, err);
         if (rc) return fail(rc, "%s", err.c_str());
     }
-    return rb_enqueue_forward(ctx, *s, s->rb, M, s->d_blob, R, seed, set_id, flags, true);
+    return rb_enqueue_forward(ctx, *s, s->rb, M, s->d_model, R, seed, set_id, flags, true);
 }
 
 int pda_rb_get_result(pda_ctx* ctx, int sid, uint64_t* M_fixed, double* M, int nbins,
@@ -711,14 +711,14 @@ int pda_rb_forward_population(pda_ctx* ctx, int sid, int R, uint32_t seed, uint3
     if (s->rbpop.size() < size_t(p.nsets)) s->rbpop.resize(size_t(p.nsets));
     for (int k = 0; k < p.nsets; ++k) {
         RbState& r = s->rbpop[size_t(k)];
-        if (!r.d_blob) HIP_TRY(hipMalloc(reinterpret_cast<void**>(&r.d_blob), sizeof(ModelBlob)));
-        if (!r.h_blob)
-            HIP_TRY(hipHostMalloc(reinterpret_cast<void**>(&r.h_blob), sizeof(ModelBlob),
+        if (!r.d_model) HIP_TRY(hipMalloc(reinterpret_cast<void**>(&r.d_model), sizeof(Model)));
+        if (!r.h_model)
+            HIP_TRY(hipHostMalloc(reinterpret_cast<void**>(&r.h_model), sizeof(Model),
                                   hipHostMallocDefault));
-        r.h_blob->m = models[size_t(k)];
-        HIP_TRY(hipMemcpyAsync(r.d_blob, r.h_blob, sizeof(Model), hipMemcpyHostToDevice,
+        *r.h_model = models[size_t(k)];
+        HIP_TRY(hipMemcpyAsync(r.d_model, r.h_model, sizeof(Model), hipMemcpyHostToDevice,
                                s->stream));
-        int rc = rb_enqueue_forward(ctx, *s, r, models[size_t(k)], r.d_blob, R, seed,
+        int rc = rb_enqueue_forward(ctx, *s, r, models[size_t(k)], r.d_model, R, seed,
                                     set_base + uint32_t(k) * set_stride, flags, false);
         if (rc) {
             s->rbpop_sets = 0;

@@ -150,7 +150,7 @@ struct RbAcc {
 template <bool kScores, int kN>
 __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(7))) void rb_walk_kernel(
     const BurstDesc* __restrict__ bursts, const uint32_t* __restrict__ ticks,
-    const uint2* __restrict__ links, const ModelBlob* __restrict__ blob,
+    const uint2* __restrict__ links, const Model* __restrict__ model,
     const RbModel* __restrict__ rbm, const RunArgs a, const FastArgs fa,
     uint2* __restrict__ cnt_out,
     float* __restrict__ F_out, float* __restrict__ S_out, uint32_t* __restrict__ work,
@@ -160,7 +160,7 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(7))) void
     __shared__ RbModel sR;
     const uint32_t lane = threadIdx.x;
     {
-        const uint32_t* src = reinterpret_cast<const uint32_t*>(&blob->m);
+        const uint32_t* src = reinterpret_cast<const uint32_t*>(model);
         uint32_t* dst = reinterpret_cast<uint32_t*>(&sM);
         for (uint32_t i = lane; i < sizeof(Model) / 4; i += kWave) dst[i] = src[i];
         const uint32_t* src2 = reinterpret_cast<const uint32_t*>(rbm);
@@ -244,7 +244,7 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(7))) void
 template <bool kScores, int kN>
 __global__ __launch_bounds__(kWave) void rb_replay_kernel(
     const BurstDesc* __restrict__ bursts, const uint32_t* __restrict__ ticks,
-    const uint2* __restrict__ links, const ModelBlob* __restrict__ blob,
+    const uint2* __restrict__ links, const Model* __restrict__ model,
     const RbModel* __restrict__ rbm, const RunArgs a, uint2* __restrict__ cnt_out,
     float* __restrict__ F_out, float* __restrict__ S_out, uint32_t* __restrict__ big,
     uint32_t* __restrict__ huge, uint32_t* __restrict__ big_count,
@@ -255,7 +255,7 @@ __global__ __launch_bounds__(kWave) void rb_replay_kernel(
     __shared__ RbModel sR;
     const uint32_t lane = threadIdx.x;
     {
-        const uint32_t* src = reinterpret_cast<const uint32_t*>(&blob->m);
+        const uint32_t* src = reinterpret_cast<const uint32_t*>(model);
         uint32_t* dst = reinterpret_cast<uint32_t*>(&sM);
         for (uint32_t i = lane; i < sizeof(Model) / 4; i += kWave) dst[i] = src[i];
         const uint32_t* src2 = reinterpret_cast<const uint32_t*>(rbm);
@@ -1079,26 +1079,26 @@ hipError_t rb_big_occupancy(int mode, bool wide, int dyn_lds, int* per_cu) {
 
 template <bool kScores, int kN>
 static void launch_rb_walk_n(uint32_t grid, uint32_t replay_grid, const BurstDesc* bursts,
-                             const uint32_t* ticks, const uint2* links, const ModelBlob* blob,
+                             const uint32_t* ticks, const uint2* links, const Model* model,
                              const RbModel* rbm, const RunArgs& a, const FastArgs& fa, uint2* cnt,
                              float* F, float* S, uint32_t* work, uint32_t* big, uint32_t* huge, uint32_t* big_count,
                              uint32_t* replay, uint32_t* replay_count, hipStream_t stream) {
     hipLaunchKernelGGL((rb_walk_kernel<kScores, kN>), dim3(grid), dim3(kWave), 0, stream, bursts,
-                       ticks, links, blob, rbm, a, fa, cnt, F, S, work, big, huge, big_count,
+                       ticks, links, model, rbm, a, fa, cnt, F, S, work, big, huge, big_count,
                        replay, replay_count);
     hipLaunchKernelGGL((rb_replay_kernel<kScores, kN>), dim3(replay_grid), dim3(kWave), 0, stream,
-                       bursts, ticks, links, blob, rbm, a, cnt, F, S, big, huge, big_count, replay,
+                       bursts, ticks, links, model, rbm, a, cnt, F, S, big, huge, big_count, replay,
                        replay_count);
 }
 
 hipError_t launch_rb_walk(bool scores, int n, uint32_t grid, uint32_t replay_grid,
                           const BurstDesc* bursts, const uint32_t* ticks, const uint2* links,
-                          const ModelBlob* blob, const RbModel* rbm, const RunArgs& a,
+                          const Model* model, const RbModel* rbm, const RunArgs& a,
                           const FastArgs& fa, uint2* cnt, float* F, float* S, uint32_t* work,
                           uint32_t* big, uint32_t* huge, uint32_t* big_count,
                           uint32_t* replay, uint32_t* replay_count, hipStream_t stream) {
 #define PDA_RB_WALK(SC, N)                                                                    \
-    launch_rb_walk_n<SC, N>(grid, replay_grid, bursts, ticks, links, blob, rbm, a, fa, cnt, F, \
+    launch_rb_walk_n<SC, N>(grid, replay_grid, bursts, ticks, links, model, rbm, a, fa, cnt, F, \
                             S, work, big, huge, big_count, replay, replay_count, stream)
     if (n < 2 || n > kRbMaxStates) return hipErrorInvalidValue;
     if (scores) {

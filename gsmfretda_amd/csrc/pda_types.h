@@ -90,6 +90,7 @@ struct Model : BroadModel {
     // pp = min(p, 1-p): pp and q = 1 - pp.
     double pp[kMaxStates];
     double qq[kMaxStates];
+    double lq[kMaxStates];                        // log q
 };
 
 // q^m and the inversion bound min(m, mp + 10 sqrt(mpq + 1)) per state and
@@ -123,12 +124,6 @@ struct BinomGuide {
     const uint8_t* guide;  // [kMaxStates][kBinomTable][kGuideBuckets]
 };
 constexpr size_t kGuideBytes = size_t(kMaxStates) * kBinomTable * kGuideBuckets;
-
-// What a stream slot uploads per parameter set.
-struct ModelBlob {
-    Model m;
-    BinomTable tab;
-};
 
 // Arguments of one launch of the walk kernel (passed by value).
 struct RunArgs {
