@@ -159,12 +159,6 @@ constexpr int fast_waves_per_eu(bool pop, int pass) {
     return pass != kPassBroad ? 8 : pop ? 7 : 6;
 }
 
-// A unit that has been started: its burst, its key and its first state.
-struct StartedUnit {
-    BurstDesc d;
-    uint32_t r, b;
-};
-
 struct FastIO {
     const BurstDesc* bursts;
     const uint32_t* ticks;

@@ -55,71 +55,111 @@ constexpr int kRbJacCols = kRbMaxStates + kRbMaxPairs;
 
 constexpr int kRbFwd = 0, kRbGrad = 1, kRbJac = 2;
 
-// What an RB walk accumulates over a unit's windows, in registers (kN
-// states, known at compile time, so every index below is a constant): the
-// photon counts per state and the score of the walk's draws per rate pair,
+// Orders the LDS accesses of the wave's lanes: every lane's earlier LDS
+// writes are visible to every lane's later LDS reads.  The lanes of a wave
+// share data through LDS here without a workgroup barrier; the compiler
+// treats each lane as a thread of its own and, without this fence, may keep
+// a value a lane stored in a register instead of reading what another lane
+// wrote over it, or move accesses across the exchange.
+__device__ __forceinline__ void wave_lds_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+}
+
+// Lanes of the mask below this one.
+__device__ __forceinline__ uint32_t lanes_below(uint64_t mask) {
+    return __builtin_amdgcn_mbcnt_hi(uint32_t(mask >> 32),
+                                     __builtin_amdgcn_mbcnt_lo(uint32_t(mask), 0u));
+}
+
+// What an RB walk accumulates over a unit's windows (kN states, known at
+// compile time): the photon counts per state, in registers, and the score of
+// the walk's draws per rate pair, in the lane's column of an LDS array,
 //   d/dK(j', s) log[P(j | s) K(j, s) exp(-K(j, s) tau)]
 //     = [j' = j] (2 / K(j, s) - tau) - 1 / sum_{j''} K(j'', s)
 // summed over the windows in float, in the order of the oracle's
 // restatement: per window, the taken pair's 2 / K - tau first, then
 // 1 / sum K off every pair leaving the window's state.
-template <int kN, bool kScores>
+template <int kN, bool kScores, int kStride>
 struct RbAcc {
     static constexpr int kK = kN * (kN - 1);
+    static constexpr bool kHasScores = kScores;
     uint32_t cnt[kN];
-    float S[kScores ? kK : 1];
+    float* S;  // the lane's scores, kStride apart
 
     __device__ __forceinline__ void clear() {
 #pragma unroll
         for (int s = 0; s < kN; ++s) cnt[s] = 0u;
+        if (kScores) {
 #pragma unroll
-        for (int i = 0; i < (kScores ? kK : 1); ++i) S[i] = 0.0f;
+            for (int i = 0; i < kK; ++i) S[i * kStride] = 0.0f;
+        }
     }
 
-    __device__ __forceinline__ void absorb(const RbModel& R, const WindowInfo& wi) {
+    template <class R_t>
+    __device__ __forceinline__ void absorb(const R_t& R, const WindowInfo& wi) {
         const uint32_t m = wi.m > 0 ? uint32_t(wi.m) : 0u;
 #pragma unroll
         for (int s = 0; s < kN; ++s) cnt[s] += s == wi.s ? m : 0u;
         if (kScores) {
-            const int p = rate_pair(kN, wi.s, wi.j);
             const float v = R.two_over_k[wi.s][wi.j] - wi.tau;
             const float inv = R.inv_sum[wi.s];
+            // the pairs leaving wi.s: rate_pair(kN, wi.s, to)
+            float t[kN - 1];
 #pragma unroll
-            for (int i = 0; i < kK; ++i) {
-                // pair i = rate_pair(kN, from, to): to = i / (kN - 1)
-                const int to = i / (kN - 1), r = i % (kN - 1);
-                const int from = r < to ? r : r + 1;
-                const float t = i == p ? S[i] + v : S[i];
-                S[i] = from == wi.s ? t - inv : S[i];
+            for (int k = 0; k < kN - 1; ++k) t[k] = S[out_pair(wi.s, k) * kStride];
+#pragma unroll
+            for (int k = 0; k < kN - 1; ++k) {
+                const int to = k < wi.s ? k : k + 1;
+                t[k] = to == wi.j ? t[k] + v : t[k];
+                S[out_pair(wi.s, k) * kStride] = t[k] - inv;
             }
         }
     }
 
+    // rate_pair(kN, s, to) of the k-th state `to` other than s
+    __device__ __forceinline__ static int out_pair(int s, int k) {
+        return k < s ? k * (kN - 1) + s - 1 : (k + 1) * (kN - 1) + s;
+    }
+
+    // rb_pack of the counts (states >= n hold 0)
+    __device__ __forceinline__ uint2 packed() const {
+        uint32_t c[kRbMaxStates] = {0u, 0u, 0u, 0u};
+#pragma unroll
+        for (int s = 0; s < kN; ++s) c[s] = cnt[s];
+        return make_uint2((c[0] & 0xFFFFu) | (c[1] << 16), (c[2] & 0xFFFFu) | (c[3] << 16));
+    }
+
     // Stores the unit: its packed counts, F and scores; a unit too long for
-    // the memo joins the big list (total < kRbBigSplit, count big_count[0])
-    // or the huge one (count big_count[1]): one atomic per wave, list and
-    // call site, the lanes storing now ranked among themselves.
+    // the memo joins the big list (total < kRbBigSplit, count big_count[0]) or the huge one (count
+    // big_count[1]): one atomic per wave, list and call site, the lanes
+    // storing now ranked among themselves.
     __device__ __forceinline__ void store(uint32_t unit, float F, uint32_t lane,
                                           uint2* __restrict__ cnt_out, float* __restrict__ F_out,
                                           float* __restrict__ S_out, uint32_t* __restrict__ big,
                                           uint32_t* __restrict__ huge,
                                           uint32_t* __restrict__ big_count) const {
-        uint32_t c[kRbMaxStates] = {0u, 0u, 0u, 0u};
-#pragma unroll
-        for (int s = 0; s < kN; ++s) c[s] = cnt[s];
-        uint2 packed;  // rb_pack of the four counts (states >= n hold 0)
-        packed.x = (c[0] & 0xFFFFu) | (c[1] << 16);
-        packed.y = (c[2] & 0xFFFFu) | (c[3] << 16);
-        cnt_out[unit] = packed;
+        const uint2 c = packed();
+        cnt_out[unit] = c;
         F_out[unit] = F;
         if (kScores) {
-            // kK (2, 6 or 12) floats per unit: 8-byte aligned rows, two floats
-            // a store
-            float2* row = reinterpret_cast<float2*>(S_out + size_t(unit) * size_t(kK));
+            // kK (2, 6 or 12) floats per unit, 8-byte aligned rows: as few
+            // stores as there can be, each lane's going to a line of its own
+            struct __attribute__((packed, aligned(8))) Quad {
+                float v[4];
+            };
+            float* row = S_out + size_t(unit) * size_t(kK);
 #pragma unroll
-            for (int i = 0; i < kK / 2; ++i) row[i] = make_float2(S[2 * i], S[2 * i + 1]);
+            for (int i = 0; i + 4 <= kK; i += 4)
+                *reinterpret_cast<Quad*>(row + i) = Quad{{S[i * kStride], S[(i + 1) * kStride],
+                                                          S[(i + 2) * kStride],
+                                                          S[(i + 3) * kStride]}};
+            if (kK % 4)
+                *reinterpret_cast<float2*>(row + kK / 4 * 4) =
+                    make_float2(S[(kK - 2) * kStride], S[(kK - 1) * kStride]);
         }
-        const uint32_t mt = c[0] + c[1] + c[2] + c[3];
+        const uint32_t mt = (c.x & 0xFFFFu) + (c.x >> 16) + (c.y & 0xFFFFu) + (c.y >> 16);
         append(mt >= uint32_t(kRbMemoCap) && mt < uint32_t(kRbBigSplit), unit, lane, big,
                &big_count[0]);
         append(mt >= uint32_t(kRbBigSplit), unit, lane, huge, &big_count[1]);
@@ -141,14 +181,46 @@ struct RbAcc {
     }
 };
 
+// Units that rb_walk_kernel starts at a time: its LDS then stays within 5,120
+// bytes, and 32 workgroups share a CU.
+template <int kN>
+constexpr uint32_t kRbWalkStart = kN > 3 ? 32u : 64u;
+
+// A unit without a window: no counts, no scores.
+template <class Acc>
+__device__ __forceinline__ void zero_unit(uint32_t unit, uint2* __restrict__ cnt_out,
+                                          float* __restrict__ F_out, float* __restrict__ S_out) {
+    cnt_out[unit] = make_uint2(0u, 0u);
+    F_out[unit] = 0.0f;
+    if (Acc::kHasScores)
+        for (int i = 0; i < Acc::kK; ++i) S_out[size_t(unit) * Acc::kK + i] = 0.0f;
+}
+
+// What absorb() reads of an RbModel.
+struct RbScoreModel {
+    float two_over_k[kRbMaxStates][kRbMaxStates];
+    float inv_sum[kRbMaxStates];
+};
+
 // The walk of every unit in the fast form (32-bit window ends, background
 // means <= 64: the plain walk's common case) with the work stealing of
-// walk_kernel; a unit that leaves the common case is listed for
+// fast_walk_kernel; a unit that leaves the common case is listed for
 // rb_replay_kernel, which walks it again from its start in the general form
 // with the same keyed draws, so every unit's stored summary is the general
-// form's.
+// form's.  As there, units are started into LDS many at a time.
+//
+// Bound by the memory its results go to (100,000 bursts x 64 of 3 states: 231
+// MB of counts, F and scores, of which 400 MB arrive, lines being written back
+// before the last of their five units ends; with the scores stored to one
+// small region instead the walk takes 65 us less), VALU at 60 %.  Scores summed
+// in LDS instead of registers: a window touches the n - 1 rates out of its
+// state where the register form had to select among all n (n - 1), 594 VALU
+// instructions against 835 and 59 registers against 71, so 8 waves on a SIMD.
+// That run 324 -> 300 us, 4 states of fast dynamics 160 -> 157 us per set and
+// derivative step.  (Ended units kept in LDS and stored 64 at a time: 315 us
+// with 3 states, spills with 4.)
 template <bool kScores, int kN>
-__global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(7))) void rb_walk_kernel(
+__global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(8))) void rb_walk_kernel(
     const BurstDesc* __restrict__ bursts, const uint32_t* __restrict__ ticks,
     const uint2* __restrict__ links, const Model* __restrict__ model,
     const RbModel* __restrict__ rbm, const RunArgs a, const FastArgs fa,
@@ -156,74 +228,109 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(7))) void
     float* __restrict__ F_out, float* __restrict__ S_out, uint32_t* __restrict__ work,
     uint32_t* __restrict__ big, uint32_t* __restrict__ huge, uint32_t* __restrict__ big_count,
     uint32_t* __restrict__ replay, uint32_t* __restrict__ replay_count) {
-    __shared__ Model sM;
-    __shared__ RbModel sR;
+    using Acc = RbAcc<kN, kScores, kWave>;
+    constexpr uint32_t kStart = kRbWalkStart<kN>;
+    constexpr int kS = kScores ? Acc::kK : 1;
+    __shared__ FastModel sM;
+    __shared__ RbScoreModel sR;
+    __shared__ StartedUnit s_start[kStart];   // units started and not yet taken
+    __shared__ uint8_t s_state[kStart];       // their first states
+    __shared__ float s_S[kS][kWave];          // the lanes' scores
     const uint32_t lane = threadIdx.x;
     {
         const uint32_t* src = reinterpret_cast<const uint32_t*>(model);
         uint32_t* dst = reinterpret_cast<uint32_t*>(&sM);
-        for (uint32_t i = lane; i < sizeof(Model) / 4; i += kWave) dst[i] = src[i];
-        const uint32_t* src2 = reinterpret_cast<const uint32_t*>(rbm);
-        uint32_t* dst2 = reinterpret_cast<uint32_t*>(&sR);
-        for (uint32_t i = lane; i < sizeof(RbModel) / 4; i += kWave) dst2[i] = src2[i];
+        for (uint32_t i = lane; i < sizeof(FastModel) / 4; i += kWave) dst[i] = src[i];
+        const float* src2 = &rbm->two_over_k[0][0];
+        float* dst2 = reinterpret_cast<float*>(&sR);
+        static_assert(offsetof(RbModel, inv_sum) ==
+                          offsetof(RbModel, two_over_k) + offsetof(RbScoreModel, inv_sum),
+                      "the two lie together in both");
+        for (uint32_t i = lane; i < sizeof(RbScoreModel) / 4; i += kWave) dst2[i] = src2[i];
     }
     __syncthreads();
-    RbAcc<kN, kScores> acc;
+    Acc acc;
+    acc.S = &s_S[0][lane];
 
     const uint32_t queue = blockIdx.x % a.queues;
     const uint64_t q_first = uint64_t(queue) * a.q_share;
     const uint32_t q_begin = q_first < a.nunits ? uint32_t(q_first) : a.nunits;
     const uint32_t q_end = a.nunits - q_begin < a.q_share ? a.nunits : q_begin + a.q_share;
     uint32_t pool_next = 0, pool_end = 0;
+    uint32_t started = 0, start_next = 0;  // entries of s_start, the next to take
     bool busy = false;
-    uint32_t u = 0;
     WalkState<true> st{};
     UnitKey key{a.seed, a.set, 0u, 0u};
     BurstDesc d{0u, 0u, 0u, 0.0f};
     const UnitDiv divR{a.div_m, a.div_sh};
     bool drained = false;
     while (true) {
-        bool need = !busy;
-        while (!drained) {
-            const uint64_t want = __ballot(need);
+        while (true) {
+            const uint64_t want = __ballot(!busy);
             if (want == 0) break;
-            if (pool_next >= pool_end) {
-                uint32_t off = 0;
-                if (lane == 0) off = atomicAdd(&work[queue * kCounterStride], a.batch);
-                off = __shfl(off, 0);
-                if (off >= q_end - q_begin) {
-                    drained = true;
-                    break;
+            if (start_next == started) {  // start the next units
+                if (pool_next >= pool_end) {
+                    if (drained) break;
+                    uint32_t off = 0;
+                    if (lane == 0) off = atomicAdd(&work[queue * kCounterStride], a.batch);
+                    off = __builtin_amdgcn_readfirstlane(off);
+                    if (off >= q_end - q_begin) {
+                        drained = true;
+                        break;
+                    }
+                    pool_next = q_begin + off;
+                    pool_end = pool_next + a.batch < q_end ? pool_next + a.batch : q_end;
                 }
-                pool_next = q_begin + off;
-                pool_end = pool_next + a.batch < q_end ? pool_next + a.batch : q_end;
+                const uint32_t v = pool_next + lane;
+                bool walks = false;
+                int state = 0;
+                StartedUnit e;
+                if (lane < kStart && v < pool_end) {
+                    const uint32_t bl = unit_div(v, divR);
+                    e.d = bursts[a.begin + bl];
+                    e.r = v - bl * a.R;
+                    e.b = a.begin + bl;
+                    const UnitKey k{a.seed, a.set, e.r, e.b};
+                    WalkState<true> s0;
+                    walks = begin_unit<true>(sM, k, e.d.P, e.d.T, s0) == kStepMore;
+                    state = s0.s;
+                    if (!walks) {
+                        zero_unit<Acc>(v, cnt_out, F_out, S_out);
+                    }
+                }
+                pool_next = pool_end - pool_next < kStart ? pool_end : pool_next + kStart;
+                const uint64_t walking = __ballot(walks);
+                if (walks) {
+                    s_start[lanes_below(walking)] = e;
+                    s_state[lanes_below(walking)] = uint8_t(state);
+                }
+                wave_lds_sync();
+                start_next = 0;
+                started = uint32_t(__popcll(walking));
+                continue;
             }
-            const uint32_t rank = __builtin_amdgcn_mbcnt_hi(
-                uint32_t(want >> 32), __builtin_amdgcn_mbcnt_lo(uint32_t(want), 0u));
-            const uint32_t avail = pool_end - pool_next;
-            if (need && rank < avail) {
-                u = pool_next + rank;
-                const uint32_t bl = unit_div(u, divR);
-                const uint32_t b = a.begin + bl;
-                d = bursts[b];
-                key.r = u - bl * a.R;
-                key.b = b;
+            const uint32_t left = started - start_next;
+            const uint32_t rank = lanes_below(want);
+            if (!busy && rank < left) {
+                const StartedUnit e = s_start[start_next + rank];
+                d = e.d;
+                key.r = e.r;
+                key.b = e.b;
+                st = WalkState<true>{};
+                st.s = s_state[start_next + rank];
                 acc.clear();
-                if (begin_unit<true>(sM, key, d.P, d.T, st) == kStepMore) {
-                    busy = true;
-                    need = false;
-                } else {
-                    acc.store(u, st.F, lane, cnt_out, F_out, S_out, big, huge, big_count);
-                }
+                busy = true;
             }
             const uint32_t taken = uint32_t(__popcll(want));
-            pool_next += taken < avail ? taken : avail;
+            start_next += taken < left ? taken : left;
         }
         if (!__any(busy)) break;
         if (busy) {
             WindowInfo wi;
-            const int r = fast_window<true>(sM, nullptr, key, d.P, d.stop_rel, d.T, ticks + d.off,
-                                            links + d.off, a, fa, st, &wi);
+            const uint32_t u = (key.b - a.begin) * a.R + key.r;
+            const int r = fast_window<true, BinomGuide>(sM, nullptr, key, d.P, d.stop_rel, d.T,
+                                                        ticks + d.off, links + d.off, a, fa, st,
+                                                        &wi);
             if (r == kStepReplay) {
                 replay[atomicAdd(replay_count, 1u)] = u;
                 busy = false;
@@ -253,6 +360,7 @@ __global__ __launch_bounds__(kWave) void rb_replay_kernel(
     if (blockIdx.x * kWave >= count) return;  // uniform over the workgroup
     __shared__ Model sM;
     __shared__ RbModel sR;
+    __shared__ float s_S[kScores ? kN * (kN - 1) : 1][kWave];
     const uint32_t lane = threadIdx.x;
     {
         const uint32_t* src = reinterpret_cast<const uint32_t*>(model);
@@ -274,7 +382,8 @@ __global__ __launch_bounds__(kWave) void rb_replay_kernel(
             const BurstDesc d = bursts[b];
             const UnitKey key{a.seed, a.set, u - bl * a.R, b};
             WalkState<false> st{};
-            RbAcc<kN, kScores> acc;
+            RbAcc<kN, kScores, kWave> acc;
+            acc.S = &s_S[0][lane];
             acc.clear();
             int r = begin_unit<false>(sM, key, d.P, d.T, st);
             while (r == kStepMore) {
@@ -303,18 +412,6 @@ __device__ __forceinline__ int wave_scan_sum(int v, int lane) {
         if (lane >= d) v += t;
     }
     return v;
-}
-
-// Orders the LDS accesses of the wave's lanes: every lane's earlier LDS
-// writes are visible to every lane's later LDS reads.  The lanes of a wave
-// share data through LDS here without a workgroup barrier; the compiler
-// treats each lane as a thread of its own and, without this fence, may keep
-// a value a lane stored in a register instead of reading what another lane
-// wrote over it, or move accesses across the exchange.
-__device__ __forceinline__ void wave_lds_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
 }
 
 // What the passes compute per unit, with P(a), a = 0..Mt, the unit's pmf

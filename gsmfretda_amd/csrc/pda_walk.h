@@ -340,6 +340,12 @@ struct WindowInfo {
     int32_t m;
 };
 
+// A unit that has been started: its burst and its key.
+struct StartedUnit {
+    BurstDesc d;
+    uint32_t r, b;
+};
+
 // Start of a unit (src/mc.cu:92-116): initial state from genMatP's inflow.
 // Returns kStepDone when the unit has no window that counts anything
 // (zero or one photon, or T <= 0: E = 0).
