@@ -261,6 +261,9 @@ int pda_destroy(pda_ctx* ctx) {
     (void)hipSetDevice(ctx->device);
     for (auto& s : ctx->slots) {
         if (s.stream) (void)hipStreamSynchronize(s.stream);
+        if (s.rb_aux) (void)hipStreamSynchronize(s.rb_aux);
+        for (hipStream_t st : s.rb_par)
+            if (st) (void)hipStreamSynchronize(st);
         (void)hipFree(s.d_model);
         (void)hipFree(s.d_thr);
         (void)hipFree(s.d_guide);
@@ -279,10 +282,11 @@ int pda_destroy(pda_ctx* ctx) {
         free_population(s.pop);
         free_rb(s.rb);
         for (auto& r : s.rbpop) free_rb(r);
-        if (s.rb_aux) {
-            (void)hipStreamSynchronize(s.rb_aux);
-            (void)hipStreamDestroy(s.rb_aux);
-        }
+        if (s.rb_aux) (void)hipStreamDestroy(s.rb_aux);
+        for (hipStream_t st : s.rb_par)
+            if (st) (void)hipStreamDestroy(st);
+        for (hipEvent_t e : s.rb_par_done)
+            if (e) (void)hipEventDestroy(e);
         if (s.rb_fork) (void)hipEventDestroy(s.rb_fork);
         if (s.rb_join) (void)hipEventDestroy(s.rb_join);
         if (s.stream) (void)hipStreamDestroy(s.stream);

@@ -106,31 +106,40 @@ struct Population {
     bool ready = false;  // counters and events allocated
 };
 
+// Sets of an RB population that run beside each other, less one: with 1, 2, 3
+// and 5 a Jacobian step of four sets of 4 states (50,000 bursts x 8, fast
+// dynamics) takes 1.21, 1.12, 1.26 and 1.26 ms (1.38 without), the runtime's
+// four hardware queues also serving the process's other streams.
+constexpr int kRbParallel = 2;
+
+struct RbModel;
+
 // Rao-Blackwellised runs of a slot: per-unit walk summaries of the last
 // forward run (reused by the adjoint), histogram rows, result, gradient.
 struct RbState {
-    void* d_rbm = nullptr;             // RbModel
-    void* h_rbm = nullptr;             // pinned
+    RbModel* d_rbm = nullptr;
     // the walk's model when the state is one set of an RB population (the
     // single-set forward walks the slot's own d_model)
     Model* d_model = nullptr;
-    Model* h_model = nullptr;          // pinned
     uint2* d_cnt = nullptr;            // per unit: photon counts per state
     float* d_F = nullptr;              // per unit: F
     float* d_S = nullptr;              // per unit: scores of the rates
     size_t cap_units = 0, cap_scores = 0;
     unsigned long long* d_hist = nullptr;  // [8][kMaxBins]
     uint32_t* d_work = nullptr;        // kWorkWords: walk queues + pmf pass queues
-    uint8_t* d_res = nullptr;          // header + uint64 M[kMaxBins]
-    uint8_t* h_res = nullptr;          // pinned
+    // header + uint64 M[kMaxBins], pinned, written by the run's last kernel
+    uint8_t* h_res = nullptr;
+    uint8_t* d_res = nullptr;          // its device address
     double* d_g = nullptr;             // cotangent per bin
-    double* h_g = nullptr;             // pinned
-    double* d_grad = nullptr;          // kRbGradRows rows of n + K, then their sum
+    double* h_g = nullptr;             // pinned, and its device address
+    double* d_hg = nullptr;
+    double* d_grad = nullptr;          // kRbGradRows rows of n + K
     float* d_pmf_tab = nullptr;        // binomial pmfs of the states, counts < 256
-    // kRbJacRows times [B][n + K] rows of 16, then their sum (capacity in bins)
+    // kRbJacRows times [B][n + K] rows of 16 (capacity in bins)
     double* d_jac = nullptr;
     int cap_jac = 0;
-    double* h_jac = nullptr;           // pinned
+    double* h_jac = nullptr;           // the rows' sum, pinned, and its device address
+    double* d_hjac = nullptr;
     // units whose acceptor total is too large for the memo, listed by the
     // walk: totals below kRbBigSplit (d_big) and the rest (d_huge), each of
     // capacity cap_units, with their counts d_big_count[0] and [1]
@@ -149,7 +158,8 @@ struct RbState {
     float* d_poolP = nullptr;
     size_t cap_poolP = 0;
     bool sbar_valid = false;           // d_Sbar holds the last forward's means
-    double* h_grad = nullptr;          // pinned
+    double* h_grad = nullptr;          // the rows' sum, pinned, and its device address
+    double* d_hgrad = nullptr;
     hipEvent_t ev0 = nullptr, ev_walk = nullptr, ev1 = nullptr, ev_a0 = nullptr, ev_a1 = nullptr;
     bool ready = false;                // every fixed-size buffer above allocated
     bool ran = false, scores = false, adj_ran = false;
@@ -198,6 +208,9 @@ struct Slot {
     // runs on stream (fork after the model copy, join before the pmf pass)
     hipStream_t rb_aux = nullptr;
     hipEvent_t rb_fork = nullptr, rb_join = nullptr;
+    // RB population: set k runs on the slot's stream or one of these
+    hipStream_t rb_par[kRbParallel] = {};
+    hipEvent_t rb_par_done[kRbParallel] = {};
     std::vector<RbState> rbpop;  // RB population: one state per set
     int rbpop_sets = 0;          // sets of the last RB population forward
 };
@@ -299,7 +312,6 @@ hipError_t launch_primitive(int op, const void* in, void* out, int64_t n, hipStr
 hipError_t microbench_shape(int op, uint32_t* grid, uint32_t* threads);
 hipError_t launch_microbench(int op, uint32_t grid, int iters, float param, const double* qn,
                              const int32_t* bound, uint64_t* out, hipStream_t stream);
-struct RbModel;
 // rb_big_kernel, mode 0 forward, 1 adjoint, 2 Jacobian; wide: derivative
 // passes in double
 hipError_t rb_big_occupancy(int mode, bool wide, int dyn_lds, int* per_cu);
@@ -320,8 +332,12 @@ hipError_t launch_rb_walk(bool scores, int n, uint32_t grid, uint32_t replay_gri
 int rb_unit_threads(int mode);
 size_t rb_unit_lds_bytes(int B, int mode, int n, int copies, bool pool);
 size_t rb_big_lds_bytes(int B, int cap, int mode, bool wide);
-hipError_t launch_rb_table(const RbModel* rbm, const double* lf, float* pmf_tab, int n,
-                           hipStream_t stream);
+hipError_t launch_rb_table(const RbModel& R, const Model& M, RbModel* rbm, Model* model,
+                           const double* lf, float* pmf_tab, uint32_t* work, uint32_t* big_count,
+                           uint32_t* replay_count, hipStream_t stream);
+// g_host (or null): the adjoint's cotangent, B entries
+hipError_t launch_rb_begin(double* rows, uint32_t n, uint32_t* work, const double* g_host,
+                           double* g, int B, hipStream_t stream);
 hipError_t launch_rb_memo(int n, const float* pmf_tab, const uint4* items, uint32_t nitems,
                           const uint32_t* rank_offP, float* poolP, hipStream_t stream);
 // copies: of the LDS accumulators; tile: units a workgroup takes at a time;
@@ -343,6 +359,6 @@ hipError_t launch_rb_score_mean(const RunArgs& a, int K, const float* S, double*
 // out[i] = sum of the nrows rows of n doubles
 hipError_t launch_rb_rows(const double* rows, int n, int nrows, double* out, hipStream_t stream);
 hipError_t launch_rb_finish(const RunArgs& a, const float* obs, unsigned long long* hist_acc,
-                            uint32_t* work, void* res, hipStream_t stream);
+                            void* res, hipStream_t stream);
 
 }  // namespace pda

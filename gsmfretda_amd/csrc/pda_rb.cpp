@@ -28,15 +28,12 @@ namespace pda {
 
 void free_rb(RbState& r) {
     (void)hipFree(r.d_rbm);
-    (void)hipHostFree(r.h_rbm);
     (void)hipFree(r.d_model);
-    (void)hipHostFree(r.h_model);
     (void)hipFree(r.d_cnt);
     (void)hipFree(r.d_F);
     (void)hipFree(r.d_S);
     (void)hipFree(r.d_hist);
     (void)hipFree(r.d_work);
-    (void)hipFree(r.d_res);
     (void)hipHostFree(r.h_res);
     (void)hipFree(r.d_g);
     (void)hipHostFree(r.h_g);
@@ -81,36 +78,44 @@ constexpr size_t kRbResBytes = sizeof(RbResultHeaderH) + sizeof(uint64_t) * kMax
 constexpr int kGradLen = kRbGradLen;
 constexpr size_t kRbCounters = kWorkWords;  // queue counters + the pmf pass's
 
+// Pinned host memory that kernels read or write, and its device address, once.
+template <class T>
+hipError_t mapped(T** host, T** device, size_t bytes) {
+    if (*host) return hipSuccess;
+    void* h = nullptr;
+    hipError_t e = hipHostMalloc(&h, bytes, hipHostMallocMapped | hipHostMallocCoherent);
+    if (e != hipSuccess) return e;
+    void* d = nullptr;
+    e = hipHostGetDevicePointer(&d, h, 0);
+    if (e != hipSuccess) {
+        (void)hipHostFree(h);
+        return e;
+    }
+    *host = static_cast<T*>(h);
+    *device = static_cast<T*>(d);
+    return hipSuccess;
+}
+
 int ensure_rb(pda_ctx* ctx, RbState& r) {
     if (!r.ready) {
         // each buffer once: a call that fails part way (out of memory) leaves
         // what it got for the next call, which allocates the rest
         if (!r.d_rbm) HIP_TRY(hipMalloc(&r.d_rbm, sizeof(RbModel)));
-        if (!r.h_rbm) HIP_TRY(hipHostMalloc(&r.h_rbm, sizeof(RbModel), hipHostMallocDefault));
         if (!r.d_hist) HIP_TRY(hipMalloc(&r.d_hist, sizeof(unsigned long long) * 8u * kMaxBins));
         HIP_TRY(hipMemset(r.d_hist, 0, sizeof(unsigned long long) * 8u * kMaxBins));
         if (!r.d_work) HIP_TRY(hipMalloc(&r.d_work, sizeof(uint32_t) * kRbCounters));
         if (!r.d_big_count) HIP_TRY(hipMalloc(&r.d_big_count, 2 * sizeof(uint32_t)));
         if (!r.d_replay_count) HIP_TRY(hipMalloc(&r.d_replay_count, sizeof(uint32_t)));
         HIP_TRY(hipMemset(r.d_work, 0, sizeof(uint32_t) * kRbCounters));
-        if (!r.d_res) HIP_TRY(hipMalloc(&r.d_res, kRbResBytes));
-        if (!r.h_res)
-            HIP_TRY(hipHostMalloc(reinterpret_cast<void**>(&r.h_res), kRbResBytes,
-                                  hipHostMallocDefault));
+        HIP_TRY(mapped(&r.h_res, &r.d_res, kRbResBytes));
         if (!r.d_g) HIP_TRY(hipMalloc(&r.d_g, sizeof(double) * kMaxBins));
-        if (!r.h_g)
-            HIP_TRY(hipHostMalloc(reinterpret_cast<void**>(&r.h_g), sizeof(double) * kMaxBins,
-                                  hipHostMallocDefault));
+        HIP_TRY(mapped(&r.h_g, &r.d_hg, sizeof(double) * kMaxBins));
         if (!r.d_grad)
-            HIP_TRY(hipMalloc(&r.d_grad, sizeof(double) * kGradLen * (kRbGradRows + 1)));
+            HIP_TRY(hipMalloc(&r.d_grad, sizeof(double) * kGradLen * kRbGradRows));
         if (!r.d_pmf_tab)
             HIP_TRY(hipMalloc(&r.d_pmf_tab, sizeof(float) * size_t(kRbMaxStates) * kRbPmfStride));
-        if (!r.h_jac)
-            HIP_TRY(hipHostMalloc(reinterpret_cast<void**>(&r.h_jac),
-                                  sizeof(double) * kGradLen * kMaxBins, hipHostMallocDefault));
-        if (!r.h_grad)
-            HIP_TRY(hipHostMalloc(reinterpret_cast<void**>(&r.h_grad), sizeof(double) * kGradLen,
-                                  hipHostMallocDefault));
+        HIP_TRY(mapped(&r.h_jac, &r.d_hjac, sizeof(double) * kGradLen * kMaxBins));
+        HIP_TRY(mapped(&r.h_grad, &r.d_hgrad, sizeof(double) * kGradLen));
         for (hipEvent_t* e : {&r.ev0, &r.ev_walk, &r.ev1, &r.ev_a0, &r.ev_a1})
             if (!*e) HIP_TRY(hipEventCreate(e));
         HIP_TRY(hipDeviceSynchronize());
@@ -316,12 +321,13 @@ int pass_shape(pda_ctx* ctx, int mode, int n, bool wide, int B, int cap, uint32_
 }
 
 // Enqueues one RB forward of model M -- the walk reading M from the device
-// model d_model -- over the slot's burst range into state r, on the slot's
-// stream.  sync_model: first wait for the stream, whose last run may still be
-// copying r's pinned model (a population forward waits once for all sets).
+// copy d_model, which the first launch writes if store_model is set -- over the
+// slot's burst range into state r, on `stream`, the memo on `aux` where there
+// is one; timed: with the events of pda_rb_stats.
 int rb_enqueue_forward(pda_ctx* ctx, Slot& s, RbState& r, const Model& M,
-                       const Model* d_model, int R, uint32_t seed, uint32_t set_id, int flags,
-                       bool sync_model) {
+                       const Model* d_model, Model* store_model, int R, uint32_t seed,
+                       uint32_t set_id, int flags, bool timed, hipStream_t stream,
+                       hipStream_t aux) {
     int rc = ensure_rb(ctx, r);
     if (rc) return rc;
     const int n = M.n;
@@ -334,7 +340,9 @@ int rb_enqueue_forward(pda_ctx* ctx, Slot& s, RbState& r, const Model& M,
     // with c = max(gamma - crosstalk, 1 - dexdir); at most the burst's photons
     // when c <= 1
     uint32_t maxP = 0;
-    for (int64_t b = b0; b < b1; ++b) maxP = std::max(maxP, ctx->h_P[size_t(b)]);
+    if (b0 == 0 && b1 == int64_t(ctx->h_P.size())) maxP = ctx->max_P;
+    else
+        for (int64_t b = b0; b < b1; ++b) maxP = std::max(maxP, ctx->h_P[size_t(b)]);
     const float coef = std::max({M.gmx, M.omdd, 0.0f});
     const int bound = rb_total_bound(maxP, coef);
     if (bound > kRbMaxCount)
@@ -386,12 +394,11 @@ int rb_enqueue_forward(pda_ctx* ctx, Slot& s, RbState& r, const Model& M,
         HIP_TRY(hipMalloc(&r.d_Sbar, sizeof(double) * nsb));
         r.cap_sbar = nsb;
     }
-    if (sync_model) HIP_TRY(hipStreamSynchronize(s.stream));  // the pinned model may be in use
-    RbModel* hm = static_cast<RbModel*>(r.h_rbm);
+    RbModel rbm;
     bool rates_positive = false, p_interior = false;
-    build_rb_model(M, *hm, &rates_positive, &p_interior);
+    build_rb_model(M, rbm, &rates_positive, &p_interior);
     bool wide = false;  // a state whose leave-one-out recurrence barely damps errors
-    for (int st = 0; st < n; ++st) wide = wide || (hm->p[st] > 0.4f && hm->p[st] < 0.6f);
+    for (int st = 0; st < n; ++st) wide = wide || (rbm.p[st] > 0.4f && rbm.p[st] < 0.6f);
 
     RunArgs a{};
     a.begin = uint32_t(b0);
@@ -436,44 +443,38 @@ int rb_enqueue_forward(pda_ctx* ctx, Slot& s, RbState& r, const Model& M,
         r.cap_poolP = ML.poolP;
     }
 
-    if (!s.rb_aux) HIP_TRY(hipStreamCreateWithFlags(&s.rb_aux, hipStreamNonBlocking));
-    if (!s.rb_fork) HIP_TRY(hipEventCreateWithFlags(&s.rb_fork, hipEventDisableTiming));
-    if (!s.rb_join) HIP_TRY(hipEventCreateWithFlags(&s.rb_join, hipEventDisableTiming));
-    HIP_TRY(hipMemsetAsync(r.d_work, 0, sizeof(uint32_t) * kRbCounters, s.stream));
-    HIP_TRY(hipMemsetAsync(r.d_big_count, 0, 2 * sizeof(uint32_t), s.stream));
-    HIP_TRY(hipMemsetAsync(r.d_replay_count, 0, sizeof(uint32_t), s.stream));
-    HIP_TRY(hipMemcpyAsync(r.d_rbm, r.h_rbm, sizeof(RbModel), hipMemcpyHostToDevice, s.stream));
-    const RbModel* d_rbm = static_cast<const RbModel*>(r.d_rbm);
-    HIP_TRY(hipEventRecord(r.ev0, s.stream));
-    // the pmf table and memo depend on the model only: built on the side
-    // stream while the walk runs (the memo's few, long waves hide under it)
-    HIP_TRY(hipEventRecord(s.rb_fork, s.stream));
-    HIP_TRY(hipStreamWaitEvent(s.rb_aux, s.rb_fork, 0));
-    HIP_TRY(launch_rb_table(d_rbm, ctx->d_lf, r.d_pmf_tab, n, s.rb_aux));
+    const RbModel* d_rbm = r.d_rbm;
+    if (timed) HIP_TRY(hipEventRecord(r.ev0, stream));
+    HIP_TRY(launch_rb_table(rbm, M, r.d_rbm, store_model, ctx->d_lf, r.d_pmf_tab, r.d_work,
+                            r.d_big_count, r.d_replay_count, stream));
+    // the memo depends on the model only: built on the side stream, where
+    // there is one, while the walk runs (its few, long waves hide under it)
+    if (aux) {
+        HIP_TRY(hipEventRecord(s.rb_fork, stream));
+        HIP_TRY(hipStreamWaitEvent(aux, s.rb_fork, 0));
+    }
     HIP_TRY(launch_rb_memo(n, r.d_pmf_tab, ML.d_items, ML.nitems, ML.d_rank_offP, r.d_poolP,
-                           s.rb_aux));
-    HIP_TRY(hipEventRecord(s.rb_join, s.rb_aux));
+                           aux ? aux : stream));
+    if (aux) HIP_TRY(hipEventRecord(s.rb_join, aux));
     HIP_TRY(launch_rb_walk(scores, n, grid, uint32_t(ctx->num_cu) * 4u, ctx->d_bursts, ctx->d_ticks,
                            ctx->d_links, d_model, d_rbm, a,
                            fast_args(n, M.quick_rates != 0, a.clk_p, M.r0, ctx->max_P), r.d_cnt, r.d_F, r.d_S, r.d_work,
                            r.d_big, r.d_huge, r.d_big_count, r.d_replay, r.d_replay_count,
-                           s.stream));
-    HIP_TRY(hipEventRecord(r.ev_walk, s.stream));
-    HIP_TRY(hipStreamWaitEvent(s.stream, s.rb_join, 0));
+                           stream));
+    if (timed) HIP_TRY(hipEventRecord(r.ev_walk, stream));
+    if (aux) HIP_TRY(hipStreamWaitEvent(stream, s.rb_join, 0));
     HIP_TRY(launch_rb_unit(0, n, ps.unit_grid, ps.copies, ps.tile, ps.pool, a, r.d_cnt, r.d_F,
                            nullptr, nullptr, nullptr, ML.d_rank_offP, ML.d_rank_offD, r.d_poolP,
-                           r.d_hist, nullptr, r.d_work, s.stream));
+                           r.d_hist, nullptr, r.d_work, stream));
     HIP_TRY(launch_rb_big(0, false, ps.big_grid, ps.big_cap, d_rbm, ctx->d_lf, r.d_pmf_tab, a, r.d_cnt,
                           r.d_F, nullptr, nullptr, nullptr, r.d_big, r.d_big_count, r.d_hist,
-                          nullptr, s.stream));
+                          nullptr, stream));
     if (cap > kRbBigSplit)
         HIP_TRY(launch_rb_big(0, false, ps.huge_grid, cap, d_rbm, ctx->d_lf, r.d_pmf_tab, a, r.d_cnt,
                               r.d_F, nullptr, nullptr, nullptr, r.d_huge, r.d_big_count + 1,
-                              r.d_hist, nullptr, s.stream));
-    HIP_TRY(launch_rb_finish(a, ctx->d_obs, r.d_hist, r.d_work, r.d_res, s.stream));
-    HIP_TRY(hipEventRecord(r.ev1, s.stream));
-    HIP_TRY(hipMemcpyAsync(r.h_res, r.d_res, sizeof(RbResultHeaderH) + sizeof(uint64_t) * size_t(a.B),
-                           hipMemcpyDeviceToHost, s.stream));
+                              r.d_hist, nullptr, stream));
+    HIP_TRY(launch_rb_finish(a, ctx->d_obs, r.d_hist, r.d_res, stream));
+    if (timed) HIP_TRY(hipEventRecord(r.ev1, stream));
     r.ran = true;
     r.adj_ran = false;
     r.scores = scores;
@@ -516,7 +517,11 @@ int pda_rb_forward(pda_ctx* ctx, int sid, int R, uint32_t seed, uint32_t set_id,
         int rc = build_model(s->ph, s->n, s->args.data(), int(s->args.size()), M, err);
         if (rc) return fail(rc, "%s", err.c_str());
     }
-    return rb_enqueue_forward(ctx, *s, s->rb, M, s->d_model, R, seed, set_id, flags, true);
+    if (!s->rb_aux) HIP_TRY(hipStreamCreateWithFlags(&s->rb_aux, hipStreamNonBlocking));
+    if (!s->rb_fork) HIP_TRY(hipEventCreateWithFlags(&s->rb_fork, hipEventDisableTiming));
+    if (!s->rb_join) HIP_TRY(hipEventCreateWithFlags(&s->rb_join, hipEventDisableTiming));
+    return rb_enqueue_forward(ctx, *s, s->rb, M, s->d_model, nullptr, R, seed, set_id, flags, true,
+                              s->stream, s->rb_aux);
 }
 
 int pda_rb_get_result(pda_ctx* ctx, int sid, uint64_t* M_fixed, double* M, int nbins,
@@ -560,7 +565,8 @@ int check_derivative_run(const RbState& r, int sid, int nbins, int nargs) {
 // Enqueues the lane and long-unit kernels of a derivative pass (mode 1
 // adjoint with cotangent r.d_g, 2 Jacobian) of state r's last forward,
 // accumulating into out (zeroed by the caller).
-int enqueue_derivative(pda_ctx* ctx, Slot& s, RbState& r, int mode, double* out) {
+int enqueue_derivative(pda_ctx* ctx, RbState& r, int mode, double* out, uint32_t rows,
+                       bool timed, hipStream_t stream) {
     RunArgs a{};
     a.begin = uint32_t(r.b0);
     a.nunits = uint32_t((r.b1 - r.b0) * int64_t(r.R));
@@ -572,43 +578,40 @@ int enqueue_derivative(pda_ctx* ctx, Slot& s, RbState& r, int mode, double* out)
     if (int rc = pass_shape(ctx, mode, r.n, r.wide, r.B, r.cap, a.nunits, ps)) return rc;
     a.queues = 1;
     plan_args(a, a.nunits, kWave);
-    const RbModel* d_rbm = static_cast<const RbModel*>(r.d_rbm);
+    const RbModel* d_rbm = r.d_rbm;
     const RbMemoLayout& ML = ctx->rb_memo[r.n];
     const double* g = mode == 1 ? r.d_g : nullptr;
-    HIP_TRY(hipMemsetAsync(r.d_work, 0, sizeof(uint32_t) * kRbCounters, s.stream));
-    HIP_TRY(hipEventRecord(r.ev_a0, s.stream));
+    HIP_TRY(launch_rb_begin(out, rows, r.d_work, mode == 1 ? r.d_hg : nullptr, r.d_g, r.B,
+                            stream));
+    if (timed) HIP_TRY(hipEventRecord(r.ev_a0, stream));
     if (!r.sbar_valid) {
-        HIP_TRY(launch_rb_score_mean(a, r.K, r.d_S, r.d_Sbar, ctx->num_cu, s.stream));
+        HIP_TRY(launch_rb_score_mean(a, r.K, r.d_S, r.d_Sbar, ctx->num_cu, stream));
         r.sbar_valid = true;
     }
     HIP_TRY(launch_rb_unit(mode, r.n, ps.unit_grid, ps.copies, ps.tile, ps.pool, a, r.d_cnt,
                            r.d_F, r.d_S, r.d_Sbar, g, ML.d_rank_offP, ML.d_rank_offD, r.d_poolP,
-                           nullptr, out, r.d_work, s.stream));
+                           nullptr, out, r.d_work, stream));
     HIP_TRY(launch_rb_big(mode, ps.wide, ps.big_grid, ps.big_cap, d_rbm, ctx->d_lf, r.d_pmf_tab, a,
                           r.d_cnt, r.d_F, r.d_S, r.d_Sbar, g, r.d_big, r.d_big_count, nullptr, out,
-                          s.stream));
+                          stream));
     if (r.cap > kRbBigSplit)
         HIP_TRY(launch_rb_big(mode, ps.wide, ps.huge_grid, r.cap, d_rbm, ctx->d_lf, r.d_pmf_tab, a,
                               r.d_cnt, r.d_F, r.d_S, r.d_Sbar, g, r.d_huge, r.d_big_count + 1,
-                              nullptr, out, s.stream));
-    HIP_TRY(hipEventRecord(r.ev_a1, s.stream));
+                              nullptr, out, stream));
+    if (timed) HIP_TRY(hipEventRecord(r.ev_a1, stream));
     return PDA_OK;
 }
 
 // Enqueues the adjoint pass of state r's last forward for the cotangent g
 // (nbins entries; r's pinned buffers must be free: the caller waited for the
-// stream), its gradient copied to r.h_grad.
-int rb_enqueue_adjoint(pda_ctx* ctx, Slot& s, RbState& r, const double* g) {
+// stream), its gradient written to r.h_grad.
+int rb_enqueue_adjoint(pda_ctx* ctx, RbState& r, const double* g, bool timed,
+                       hipStream_t stream) {
     std::memcpy(r.h_g, g, sizeof(double) * size_t(r.B));
-    HIP_TRY(hipMemsetAsync(r.d_grad, 0, sizeof(double) * kGradLen * kRbGradRows, s.stream));
-    HIP_TRY(hipMemcpyAsync(r.d_g, r.h_g, sizeof(double) * size_t(r.B), hipMemcpyHostToDevice,
-                           s.stream));
-    if (int rc = enqueue_derivative(ctx, s, r, 1, r.d_grad)) return rc;
-    double* sum = r.d_grad + kGradLen * kRbGradRows;
-    HIP_TRY(launch_rb_rows(r.d_grad, kGradLen, kRbGradRows, sum, s.stream));
-    HIP_TRY(hipMemcpyAsync(r.h_grad, sum, sizeof(double) * kGradLen, hipMemcpyDeviceToHost,
-                           s.stream));
-    HIP_TRY(hipMemsetAsync(r.d_work, 0, sizeof(uint32_t) * kRbCounters, s.stream));
+    if (int rc = enqueue_derivative(ctx, r, 1, r.d_grad, uint32_t(kGradLen * kRbGradRows), timed,
+                                    stream))
+        return rc;
+    HIP_TRY(launch_rb_rows(r.d_grad, kGradLen, kRbGradRows, r.d_hgrad, stream));
     r.adj_ran = true;
     return PDA_OK;
 }
@@ -621,22 +624,19 @@ void rb_collect_adjoint(const RbState& r, double* grad, int nargs) {
     for (int i = n + K; i < nargs; ++i) grad[i] = 0.0;            // v (held at 0)
 }
 
-// Enqueues the Jacobian pass of state r's last forward, copied to r.h_jac.
-int rb_enqueue_jacobian(pda_ctx* ctx, Slot& s, RbState& r) {
-    const size_t bytes = sizeof(double) * kGradLen * size_t(r.B);
+// Enqueues the Jacobian pass of state r's last forward, written to r.h_jac.
+int rb_enqueue_jacobian(pda_ctx* ctx, RbState& r, bool timed, hipStream_t stream) {
     if (r.B > r.cap_jac) {  // the caller waited for the stream
         (void)hipFree(r.d_jac);
         r.d_jac = nullptr;
         r.cap_jac = 0;
-        HIP_TRY(hipMalloc(&r.d_jac, bytes * (kRbJacRows + 1)));
+        HIP_TRY(hipMalloc(&r.d_jac, sizeof(double) * kGradLen * size_t(r.B) * kRbJacRows));
         r.cap_jac = r.B;
     }
-    HIP_TRY(hipMemsetAsync(r.d_jac, 0, bytes * kRbJacRows, s.stream));
-    if (int rc = enqueue_derivative(ctx, s, r, 2, r.d_jac)) return rc;
-    double* sum = r.d_jac + size_t(kGradLen) * size_t(r.B) * kRbJacRows;
-    HIP_TRY(launch_rb_rows(r.d_jac, kGradLen * r.B, kRbJacRows, sum, s.stream));
-    HIP_TRY(hipMemcpyAsync(r.h_jac, sum, bytes, hipMemcpyDeviceToHost, s.stream));
-    HIP_TRY(hipMemsetAsync(r.d_work, 0, sizeof(uint32_t) * kRbCounters, s.stream));
+    const int n = kGradLen * r.B;
+    if (int rc = enqueue_derivative(ctx, r, 2, r.d_jac, uint32_t(n) * kRbJacRows, timed, stream))
+        return rc;
+    HIP_TRY(launch_rb_rows(r.d_jac, n, kRbJacRows, r.d_hjac, stream));
     r.adj_ran = true;
     return PDA_OK;
 }
@@ -648,6 +648,36 @@ void rb_collect_jacobian(const RbState& r, double* J, int nbins, int nargs) {
         for (int i = 0; i < w; ++i) J[size_t(b) * size_t(nargs) + size_t(i)] = r.h_jac[size_t(b) * kGradLen + size_t(i)];
         for (int i = w; i < nargs; ++i) J[size_t(b) * size_t(nargs) + size_t(i)] = 0.0;  // v
     }
+}
+
+// The sets of a population run beside each other on up to 1 + kRbParallel
+// streams: one set's walk is as long as its longest unit's, with most of its
+// lanes idle towards the end, and its passes are a chain of short launches.
+// The parallel streams start behind the slot's stream and end in front of it.
+hipStream_t rb_set_stream(const Slot& s, int k) {
+    const int lane = k % (kRbParallel + 1);
+    return lane ? s.rb_par[lane - 1] : s.stream;
+}
+
+int rb_sets_fork(Slot& s, int nsets) {
+    if (!s.rb_fork) HIP_TRY(hipEventCreateWithFlags(&s.rb_fork, hipEventDisableTiming));
+    for (int i = 0; i < kRbParallel && i + 1 < nsets; ++i) {
+        if (!s.rb_par[i]) HIP_TRY(hipStreamCreateWithFlags(&s.rb_par[i], hipStreamNonBlocking));
+        if (!s.rb_par_done[i])
+            HIP_TRY(hipEventCreateWithFlags(&s.rb_par_done[i], hipEventDisableTiming));
+    }
+    if (nsets > 1) HIP_TRY(hipEventRecord(s.rb_fork, s.stream));
+    for (int i = 0; i < kRbParallel && i + 1 < nsets; ++i)
+        HIP_TRY(hipStreamWaitEvent(s.rb_par[i], s.rb_fork, 0));
+    return PDA_OK;
+}
+
+int rb_sets_join(Slot& s, int nsets) {
+    for (int i = 0; i < kRbParallel && i + 1 < nsets; ++i) {
+        HIP_TRY(hipEventRecord(s.rb_par_done[i], s.rb_par[i]));
+        HIP_TRY(hipStreamWaitEvent(s.stream, s.rb_par_done[i], 0));
+    }
+    return PDA_OK;
 }
 
 }  // namespace
@@ -663,7 +693,7 @@ int pda_rb_adjoint(pda_ctx* ctx, int sid, const double* g, int nbins, double* gr
         if (!std::isfinite(g[b])) return fail(PDA_E_ARG, "g[%d] not finite", b);
     HIP_TRY(hipSetDevice(ctx->device));
     HIP_TRY(hipStreamSynchronize(s->stream));
-    if (int rc = rb_enqueue_adjoint(ctx, *s, s->rb, g)) return rc;
+    if (int rc = rb_enqueue_adjoint(ctx, s->rb, g, true, s->stream)) return rc;
     HIP_TRY(hipStreamSynchronize(s->stream));
     rb_collect_adjoint(s->rb, grad, nargs);
     return PDA_OK;
@@ -676,7 +706,7 @@ int pda_rb_jacobian(pda_ctx* ctx, int sid, double* J, int nbins, int nargs) {
     if (int rc = check_derivative_run(s->rb, sid, nbins, nargs)) return rc;
     HIP_TRY(hipSetDevice(ctx->device));
     HIP_TRY(hipStreamSynchronize(s->stream));
-    if (int rc = rb_enqueue_jacobian(ctx, *s, s->rb)) return rc;
+    if (int rc = rb_enqueue_jacobian(ctx, s->rb, true, s->stream)) return rc;
     HIP_TRY(hipStreamSynchronize(s->stream));
     rb_collect_jacobian(s->rb, J, nbins, nargs);
     return PDA_OK;
@@ -706,25 +736,25 @@ int pda_rb_forward_population(pda_ctx* ctx, int sid, int R, uint32_t seed, uint3
         if (models[size_t(k)].any_v)
             return fail(PDA_E_ARG, "set %d: the RB form needs v = 0 in every state", k);
     }
-    // every set's pinned model may still be in use by the previous run
+    // the sets' buffers may be in use by the previous run, or grow
     HIP_TRY(hipStreamSynchronize(s->stream));
     if (s->rbpop.size() < size_t(p.nsets)) s->rbpop.resize(size_t(p.nsets));
-    for (int k = 0; k < p.nsets; ++k) {
+    for (int k = 0; k < p.nsets; ++k)
+        if (!s->rbpop[size_t(k)].d_model)
+            HIP_TRY(hipMalloc(reinterpret_cast<void**>(&s->rbpop[size_t(k)].d_model),
+                              sizeof(Model)));
+    s->rbpop_sets = 0;
+    if (int rc = rb_sets_fork(*s, p.nsets)) return rc;
+    int rc = PDA_OK;
+    for (int k = 0; k < p.nsets && !rc; ++k) {
         RbState& r = s->rbpop[size_t(k)];
-        if (!r.d_model) HIP_TRY(hipMalloc(reinterpret_cast<void**>(&r.d_model), sizeof(Model)));
-        if (!r.h_model)
-            HIP_TRY(hipHostMalloc(reinterpret_cast<void**>(&r.h_model), sizeof(Model),
-                                  hipHostMallocDefault));
-        *r.h_model = models[size_t(k)];
-        HIP_TRY(hipMemcpyAsync(r.d_model, r.h_model, sizeof(Model), hipMemcpyHostToDevice,
-                               s->stream));
-        int rc = rb_enqueue_forward(ctx, *s, r, models[size_t(k)], r.d_model, R, seed,
-                                    set_base + uint32_t(k) * set_stride, flags, false);
-        if (rc) {
-            s->rbpop_sets = 0;
-            return fail(rc, "set %d: %s", k, last_error().c_str());
-        }
+        rc = rb_enqueue_forward(ctx, *s, r, models[size_t(k)], r.d_model, r.d_model, R, seed,
+                                set_base + uint32_t(k) * set_stride, flags, false,
+                                rb_set_stream(*s, k), nullptr);
+        if (rc) rc = fail(rc, "set %d: %s", k, last_error().c_str());
     }
+    if (int rj = rb_sets_join(*s, p.nsets)) return rj;
+    if (rc) return rc;
     s->rbpop_sets = p.nsets;
     return PDA_OK;
 }
@@ -767,9 +797,13 @@ int pda_rb_adjoint_population(pda_ctx* ctx, int sid, const double* g, int nbins,
     }
     HIP_TRY(hipSetDevice(ctx->device));
     HIP_TRY(hipStreamSynchronize(s->stream));
-    for (int k = 0; k < K; ++k)
-        if (int rc = rb_enqueue_adjoint(ctx, *s, s->rbpop[size_t(k)], g + size_t(k) * size_t(nbins)))
-            return rc;
+    if (int rc = rb_sets_fork(*s, K)) return rc;
+    int rc = PDA_OK;
+    for (int k = 0; k < K && !rc; ++k)
+        rc = rb_enqueue_adjoint(ctx, s->rbpop[size_t(k)], g + size_t(k) * size_t(nbins), false,
+                                rb_set_stream(*s, k));
+    if (int rj = rb_sets_join(*s, K)) return rj;
+    if (rc) return rc;
     HIP_TRY(hipStreamSynchronize(s->stream));
     for (int k = 0; k < K; ++k)
         rb_collect_adjoint(s->rbpop[size_t(k)], grad + size_t(k) * size_t(nargs), nargs);
@@ -789,9 +823,13 @@ int pda_rb_jacobian_population(pda_ctx* ctx, int sid, const int32_t* which, doub
                 return fail(rc, "set %d: %s", k, last_error().c_str());
     HIP_TRY(hipSetDevice(ctx->device));
     HIP_TRY(hipStreamSynchronize(s->stream));
-    for (int k = 0; k < K; ++k)
+    if (int rc = rb_sets_fork(*s, K)) return rc;
+    int rc = PDA_OK;
+    for (int k = 0; k < K && !rc; ++k)
         if (!which || which[k])
-            if (int rc = rb_enqueue_jacobian(ctx, *s, s->rbpop[size_t(k)])) return rc;
+            rc = rb_enqueue_jacobian(ctx, s->rbpop[size_t(k)], false, rb_set_stream(*s, k));
+    if (int rj = rb_sets_join(*s, K)) return rj;
+    if (rc) return rc;
     HIP_TRY(hipStreamSynchronize(s->stream));
     const size_t per = size_t(nbins) * size_t(nargs);
     for (int k = 0; k < K; ++k) {

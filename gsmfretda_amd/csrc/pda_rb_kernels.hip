@@ -67,6 +67,22 @@ __device__ __forceinline__ void wave_lds_sync() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
 }
 
+// Lane l's value, in every lane.
+__device__ __forceinline__ double lane_value(double v, int l) {
+    const uint64_t b = __double_as_longlong(v);
+    const uint32_t lo = __builtin_amdgcn_readlane(uint32_t(b), l);
+    const uint32_t hi = __builtin_amdgcn_readlane(uint32_t(b >> 32), l);
+    return __longlong_as_double((long long)(uint64_t(hi) << 32 | lo));
+}
+
+// *dst = src by `threads` threads, this one being t.
+template <class T>
+__device__ __forceinline__ void store_words(T* dst, const T& src, uint32_t t, uint32_t threads) {
+    const uint32_t* from = reinterpret_cast<const uint32_t*>(&src);
+    uint32_t* to = reinterpret_cast<uint32_t*>(dst);
+    for (uint32_t i = t; i < sizeof(T) / 4; i += threads) to[i] = from[i];
+}
+
 // Lanes of the mask below this one.
 __device__ __forceinline__ uint32_t lanes_below(uint64_t mask) {
     return __builtin_amdgcn_mbcnt_hi(uint32_t(mask >> 32),
@@ -1026,12 +1042,14 @@ __global__ __launch_bounds__(kWave) void rb_big_kernel(
 // summed r ascending in double.  A workgroup stages the scores of a run of
 // whole bursts in LDS with coalesced loads, then one thread per (burst,
 // rate) sums them; bursts whose R K scores exceed the stage are summed
-// straight from global memory.
-constexpr uint32_t kRbSbarStage = 8192;  // floats
+// straight from global memory.  Bound by the scores' 154 MB (100,000 bursts x 64
+// of 3 states): 33 us, 82 with single-float loads and half as many workgroups
+// of twice the stage.
+constexpr uint32_t kRbSbarStage = 4096;  // floats
 __global__ __launch_bounds__(256) void rb_score_mean_kernel(const RunArgs a, int K,
                                                             const float* __restrict__ S,
                                                             double* __restrict__ Sbar) {
-    __shared__ float st[kRbSbarStage];
+    __shared__ __align__(8) float st[kRbSbarStage];
     const uint64_t nb = a.nunits / a.R;
     const uint32_t per = a.R * uint32_t(K);  // scores per burst
     const uint32_t bpb = per <= kRbSbarStage ? kRbSbarStage / per : 0u;
@@ -1050,32 +1068,65 @@ __global__ __launch_bounds__(256) void rb_score_mean_kernel(const RunArgs a, int
         const uint32_t nbh = uint32_t(nb - b0 < bpb ? nb - b0 : bpb);
         const float* src = S + b0 * per;
         __syncthreads();
-        for (uint32_t i = threadIdx.x; i < nbh * per; i += blockDim.x) st[i] = src[i];
+        // K is even: whole pairs, 8-byte aligned
+        const float2* src2 = reinterpret_cast<const float2*>(src);
+        float2* st2 = reinterpret_cast<float2*>(st);
+#pragma unroll 8
+        for (uint32_t i = threadIdx.x; i < nbh * per / 2u; i += 256u) st2[i] = src2[i];
         __syncthreads();
         for (uint32_t t = threadIdx.x; t < nbh * uint32_t(K); t += blockDim.x) {
             const uint32_t bl = t / uint32_t(K), k = t - bl * uint32_t(K);
             const float* x = st + bl * per + k;
             double sum = 0.0;
+#pragma unroll 8
             for (uint32_t r = 0; r < a.R; ++r) sum += double(x[r * uint32_t(K)]);
             Sbar[(b0 + bl) * uint64_t(K) + k] = sum / double(a.R);
         }
     }
 }
 
-// The binomial pmfs of every state for counts m < kRbPmfTable (one thread
-// per entry), read by the pmf passes instead of recomputing them per unit.
-__global__ void rb_table_kernel(const RbModel* __restrict__ rbm, const double* __restrict__ lf,
-                                float* __restrict__ pmf_tab) {
-    const int i = int(blockIdx.x * blockDim.x + threadIdx.x);
-    const int n = rbm->n;
-    if (i >= n * kRbPmfStride) return;
-    const int s = i / kRbPmfStride, r = i - s * kRbPmfStride;
+// Start of a forward: the binomial pmfs of every state (blockIdx.y) for
+// counts m < kRbPmfTable, one thread per entry, read by the pmf passes instead
+// of recomputing them per unit; and from the first workgroup the run's device
+// copies of its models and zeroed counters.  The models are arguments of the
+// launch: no staging buffer whose reuse the host has to wait for, no copies
+// and fills in front of the walk.  (With those, six small launches here and as
+// many at the derivative passes' ends, 3 states of 100,000 bursts x 64 with
+// their adjoint took 775 us; now 653.)
+__global__ __launch_bounds__(256) void rb_table_kernel(
+    const RbModel R, const Model M, RbModel* __restrict__ rbm, Model* __restrict__ model,
+    const double* __restrict__ lf, float* __restrict__ pmf_tab, uint32_t* __restrict__ work,
+    uint32_t* __restrict__ big_count, uint32_t* __restrict__ replay_count) {
+    if (blockIdx.x == 0 && blockIdx.y == 0) {
+        const uint32_t t = threadIdx.x;
+        store_words(rbm, R, t, 256u);
+        if (model) store_words(model, M, t, 256u);
+        for (uint32_t i = t; i < kMaxQueues + kAuxQueues + 1u; i += 256u)
+            work[i * kCounterStride] = 0u;
+        if (t < 2u) big_count[t] = 0u;
+        if (t == 0u) *replay_count = 0u;
+    }
+    const int r = int(blockIdx.x * blockDim.x + threadIdx.x);
+    if (r >= kRbPmfStride) return;
+    const int s = int(blockIdx.y);
     // r = m (m + 1) / 2 + k with 0 <= k <= m
     int m = int((sqrt(8.0 * double(r) + 1.0) - 1.0) * 0.5);
     while (m * (m + 1) / 2 > r) --m;
     while ((m + 1) * (m + 2) / 2 <= r) ++m;
     const int k = r - m * (m + 1) / 2;
-    pmf_tab[i] = float(rb_binom_pmf(m, k, lf, rbm->p[s], rbm->lp[s], rbm->lq[s]));
+    pmf_tab[s * kRbPmfStride + r] = float(rb_binom_pmf(m, k, lf, R.p[s], R.lp[s], R.lq[s]));
+}
+
+// Start of a derivative pass: its accumulator rows and counters zero, and for
+// the adjoint the cotangent from the host's buffer.
+__global__ __launch_bounds__(256) void rb_begin_kernel(double* __restrict__ rows, uint32_t n,
+                                                       uint32_t* __restrict__ work,
+                                                       const double* __restrict__ g_host,
+                                                       double* __restrict__ g, int B) {
+    const uint32_t i = blockIdx.x * 256u + threadIdx.x;
+    if (i < n) rows[i] = 0.0;
+    if (i < kMaxQueues + kAuxQueues + 1u) work[i * kCounterStride] = 0u;
+    if (g_host && i < uint32_t(B)) g[i] = g_host[i];
 }
 
 // Sums the rows of a derivative pass: n sums of `rows` values `stride` apart, a
@@ -1101,43 +1152,50 @@ struct RbResultHeader {
     int32_t B;
 };
 
-// One workgroup: sums the 8 rows (leaving them zero), chi2 of the expected
+// One wave: sums the 8 rows (leaving them zero), chi2 of the expected
 // counts M_b / R against the observed histogram with the reference's rules
-// (src/streamWorker.cpp:197-206), counter reset.
+// (src/streamWorker.cpp:197-206), into the host's result buffer.  Lane b forms
+// bin b's term, 64 bins at a time, and the sum runs over the lanes; an empty
+// bin's term is zero.
 __global__ __launch_bounds__(kWave) void rb_finish_kernel(
     const RunArgs a, const float* __restrict__ obs, unsigned long long* __restrict__ hist_acc,
-    uint32_t* __restrict__ work, RbResultHeader* __restrict__ res) {
-    __shared__ double s_t[kMaxBins];
-    __shared__ unsigned long long s_M[kMaxBins];
+    RbResultHeader* __restrict__ res) {
     const uint32_t lane = threadIdx.x;
     unsigned long long* M = reinterpret_cast<unsigned long long*>(res + 1);
-    for (uint32_t b = lane; b < uint32_t(a.B); b += kWave) {
-        unsigned long long v = 0;
-        for (uint32_t x = 0; x < 8u; ++x) v += atomicExch(&hist_acc[size_t(x) * kMaxBins + b], 0ull);
-        s_M[b] = v;
-        M[b] = v;
+    double c = 0.0;
+    int effN = 0;
+    for (uint32_t base = 0; base < uint32_t(a.B); base += kWave) {
+        const uint32_t b = base + lane;
         double t = 0.0;
-        if (v > 0) {
-            const double m = double(v) * 0x1p-32 / double(a.R);
-            const double dd = double(obs[b]) - m;
-            t = dd * dd / m;
+        bool filled = false;
+        if (b < uint32_t(a.B)) {
+            unsigned long long x[8], v = 0;
+#pragma unroll
+            for (uint32_t k = 0; k < 8u; ++k)
+                x[k] = __hip_atomic_load(&hist_acc[size_t(k) * kMaxBins + b], __ATOMIC_RELAXED,
+                                         __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+            for (uint32_t k = 0; k < 8u; ++k) {
+                if (x[k]) hist_acc[size_t(k) * kMaxBins + b] = 0ull;
+                v += x[k];
+            }
+            M[b] = v;
+            filled = v > 0 && int(b) >= a.left_pad;
+            if (filled) {
+                const double m = double(v) * 0x1p-32 / double(a.R);
+                const double dd = double(obs[b]) - m;
+                t = dd * dd / m;
+            }
         }
-        s_t[b] = t;
+        effN += __popcll(__ballot(filled));
+#pragma unroll 8
+        for (int l = 0; l < kWave; ++l) c += lane_value(t, l);
     }
-    __syncthreads();
     if (lane == 0) {
-        int effN = a.B - a.left_pad;
-        double c = 0.0;
-        for (int b = a.left_pad; b < a.B; ++b) {
-            if (s_M[b] > 0) c += s_t[b];
-            else --effN;
-        }
         res->chi2 = c / double(effN - a.nstates * (a.nstates + 1));
         res->effN = effN;
         res->B = a.B;
     }
-    for (uint32_t q = lane; q < kMaxQueues + kAuxQueues; q += kWave)
-        atomicExch(&work[q * kCounterStride], 0u);
 }
 
 hipError_t rb_walk_occupancy(bool scores, int n, int* per_cu) {
@@ -1217,11 +1275,21 @@ size_t rb_unit_lds_bytes(int B, int mode, int n, int copies, bool pool) {
 }
 size_t rb_big_lds_bytes(int B, int cap, int mode, bool wide) { return rb_big_lds(B, cap, mode, wide); }
 
-hipError_t launch_rb_table(const RbModel* rbm, const double* lf, float* pmf_tab, int n,
-                           hipStream_t stream) {
-    const int total = n * kRbPmfStride;
-    hipLaunchKernelGGL(rb_table_kernel, dim3(uint32_t((total + 255) / 256)), dim3(256), 0, stream,
-                       rbm, lf, pmf_tab);
+hipError_t launch_rb_table(const RbModel& R, const Model& M, RbModel* rbm, Model* model,
+                           const double* lf, float* pmf_tab, uint32_t* work, uint32_t* big_count,
+                           uint32_t* replay_count, hipStream_t stream) {
+    hipLaunchKernelGGL(rb_table_kernel, dim3(uint32_t((kRbPmfStride + 255) / 256), uint32_t(R.n)),
+                       dim3(256), 0, stream, R, M, rbm, model, lf, pmf_tab, work, big_count,
+                       replay_count);
+    return hipGetLastError();
+}
+
+hipError_t launch_rb_begin(double* rows, uint32_t n, uint32_t* work, const double* g_host,
+                           double* g, int B, hipStream_t stream) {
+    const uint32_t most = std::max<uint32_t>(std::max<uint32_t>(n, uint32_t(B)),
+                                             kMaxQueues + kAuxQueues + 1u);
+    hipLaunchKernelGGL(rb_begin_kernel, dim3((most + 255u) / 256u), dim3(256), 0, stream, rows, n,
+                       work, g_host, g, B);
     return hipGetLastError();
 }
 
@@ -1311,7 +1379,7 @@ hipError_t launch_rb_score_mean(const RunArgs& a, int K, const float* S, double*
     const uint64_t bpb = per <= kRbSbarStage ? kRbSbarStage / per : 0;
     const uint64_t want = bpb ? (nb + bpb - 1) / bpb : (nb * uint64_t(K) + 255) / 256;
     // a few workgroups per CU, each looping over its share
-    const uint64_t cap = uint64_t(num_cu > 0 ? num_cu : 1) * 4u;
+    const uint64_t cap = uint64_t(num_cu > 0 ? num_cu : 1) * 8u;
     const uint32_t grid = uint32_t(std::max<uint64_t>(1, std::min<uint64_t>(want, cap)));
     hipLaunchKernelGGL(rb_score_mean_kernel, dim3(grid), dim3(256), 0, stream, a, K, S, Sbar);
     return hipGetLastError();
@@ -1328,8 +1396,8 @@ hipError_t launch_rb_rows(const double* rows, int n, int nrows, double* out, hip
 }
 
 hipError_t launch_rb_finish(const RunArgs& a, const float* obs, unsigned long long* hist_acc,
-                            uint32_t* work, void* res, hipStream_t stream) {
-    hipLaunchKernelGGL(rb_finish_kernel, dim3(1), dim3(kWave), 0, stream, a, obs, hist_acc, work,
+                            void* res, hipStream_t stream) {
+    hipLaunchKernelGGL(rb_finish_kernel, dim3(1), dim3(kWave), 0, stream, a, obs, hist_acc,
                        static_cast<RbResultHeader*>(res));
     return hipGetLastError();
 }

@@ -44,3 +44,35 @@ def test_rb_tiles(gpu_mc, oracle, n, bursts, R, B, ph):
     scale = np.abs(g) @ np.abs(J) + np.abs(J).max() * R
     assert np.all(np.abs(g @ J - adj) <= 1e-9 * scale), (g @ J, adj)
     gpu_mc.set_photophysics(0, *DEFAULT)
+
+
+@pytest.mark.parametrize("nsets,bursts,R", [(1, 40, 5), (2, 7, 700), (3, 300, 3), (8, 33, 7)])
+def test_rb_sets_beside_each_other(gpu_mc, nsets, bursts, R):
+    """Sets of an RB population, on as many streams as there are sets or
+    fewer, forward and Jacobian twice: each equal to its run alone (with an
+    odd number of resamples, and with one whose scores of a burst exceed the
+    mean kernel's stage)."""
+    rng = np.random.default_rng(nsets)
+    sets = [(n, synth.make_args(np.sort(rng.uniform(0.1, 0.9, n)),
+                                synth.loguniform_rates(rng, n * (n - 1), 3e2, 8e3)))
+            for n in rng.integers(2, 5, 1).repeat(nsets)]
+    n = sets[0][0]
+    d = synth.generate(bursts, sets[0][1], n, seed=bursts)
+    m = gpu_mc
+    m.load(d, SgDivSr=rng.uniform(0, 1, bursts).astype(np.float32), nbins=20, left_pad=1)
+    m.set_photophysics(0, *DEFAULT)
+    m.set_burst_range(0, -1, 0)
+    m.set_population([k for k, _ in sets], [a for _, a in sets])
+    for seed in (5, 6):
+        m.rb_forward_population(R=R, seed=seed, set_base=1, set_stride=2)
+        _, fixed, chi2, eff = m.rb_population_result()
+        J = m.rb_jacobian_population(n, 20)
+        for k, (_, a) in enumerate(sets):
+            assert m.set_params(n, 0, a)
+            m.rb_forward(R=R, seed=seed, set_id=1 + 2 * k)
+            _, f1, c1, e1 = m.rb_result()
+            assert np.array_equal(fixed[k], f1) and eff[k] == e1
+            assert np.array_equal([chi2[k]], [c1], equal_nan=True)
+            # the same terms in double, fewer than 2^20, in another order
+            J1 = m.rb_jacobian(n, 20)
+            assert np.all(np.abs(J[k] - J1) <= 1e-9 * (np.abs(J1).max() + R))
