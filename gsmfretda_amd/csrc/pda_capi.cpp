@@ -83,13 +83,19 @@ Launch plan_launch(const pda_ctx* ctx, int pass, bool population, uint64_t units
         batch = (units / (max_grid * grabs) + kWave - 1) / kWave * kWave;
         batch = std::min<uint64_t>(std::max<uint64_t>(batch, kWave), 4096);
     }
-    const uint64_t batches = (units + batch - 1) / batch;
     Launch L;
-    L.grid = uint32_t(std::max<uint64_t>(1, std::min(max_grid, batches)));
     L.batch = uint32_t(batch);
     const uint32_t q = ctx->shape.queues ? ctx->shape.queues : kDefaultQueues;
-    L.queues = std::min<uint32_t>(q, L.grid);
+    size_grid(L, max_grid, units, q);
     return L;
+}
+
+void size_grid(Launch& L, uint64_t max_grid, uint64_t units, uint32_t queues) {
+    const uint64_t batches = (units + L.batch - 1) / L.batch;
+    L.queues = uint32_t(std::max<uint64_t>(
+        1, std::min<uint64_t>(queues, std::min(max_grid, batches))));
+    const uint64_t share = (batches + L.queues - 1) / L.queues;
+    L.grid = uint32_t(std::min(max_grid, std::max<uint64_t>(share, 1) * L.queues));
 }
 
 uint32_t replay_grid(const pda_ctx* ctx, uint64_t units) {
@@ -100,12 +106,17 @@ uint32_t replay_grid(const pda_ctx* ctx, uint64_t units) {
         std::max<uint64_t>(1, std::min<uint64_t>(want, uint64_t(ctx->num_cu) * per_cu)));
 }
 
-void plan_args(RunArgs& a, uint64_t items, uint32_t align) {
+void plan_args(RunArgs& a) {
     const UnitDiv q = make_unit_div(a.R);
     a.div_m = q.m;
     a.div_sh = q.sh;
-    const uint64_t share = (items + a.queues - 1u) / a.queues;
-    a.q_share = uint32_t(std::max<uint64_t>(1, (share + align - 1u) / align * align));
+    a.bps = a.batch ? uint32_t((uint64_t(a.nunits) + a.batch - 1) / a.batch) : 0u;
+    const uint64_t share = (uint64_t(a.nunits) + a.queues - 1u) / a.queues;
+    a.q_share = uint32_t(std::max<uint64_t>(1, (share + kWave - 1u) / kWave * kWave));
+}
+
+const WalkBurst* run_order(const pda_ctx* ctx, int64_t b0, int64_t b1) {
+    return b0 == 0 && b1 == ctx->nbursts ? ctx->d_order : ctx->d_plain;
 }
 
 }  // namespace pda
@@ -116,9 +127,13 @@ namespace {
 
 void free_data(pda_ctx* ctx) {
     (void)hipFree(ctx->d_bursts);
+    (void)hipFree(ctx->d_plain);
+    (void)hipFree(ctx->d_order);
     (void)hipFree(ctx->d_ticks);
     (void)hipFree(ctx->d_links);
     ctx->d_bursts = nullptr;
+    ctx->d_plain = nullptr;
+    ctx->d_order = nullptr;
     ctx->d_ticks = nullptr;
     ctx->d_links = nullptr;
     ctx->nbursts = ctx->nphotons = 0;
@@ -150,6 +165,13 @@ int load_common(pda_ctx* ctx, const int64_t* start, const int64_t* stop, const i
         HIP_TRY(hipMalloc(&ctx->d_bursts, sizeof(BurstDesc) * size_t(nbursts)));
         HIP_TRY(hipMemcpy(ctx->d_bursts, bursts.data(), sizeof(BurstDesc) * size_t(nbursts),
                           hipMemcpyHostToDevice));
+        std::vector<WalkBurst> plain, order;
+        burst_order(bursts, plain, order);
+        const size_t bytes = sizeof(WalkBurst) * size_t(nbursts);
+        HIP_TRY(hipMalloc(&ctx->d_plain, bytes));
+        HIP_TRY(hipMemcpy(ctx->d_plain, plain.data(), bytes, hipMemcpyHostToDevice));
+        HIP_TRY(hipMalloc(&ctx->d_order, bytes));
+        HIP_TRY(hipMemcpy(ctx->d_order, order.data(), bytes, hipMemcpyHostToDevice));
     }
     if (total > 0) {
         HIP_TRY(hipMalloc(&ctx->d_ticks, sizeof(uint32_t) * size_t(total)));
@@ -441,8 +463,7 @@ int pda_run(pda_ctx* ctx, int sid, int R, uint32_t seed, uint32_t set_id, int fl
     a.batch = L.batch;
     a.queues = L.queues;
     a.nsets = 1;
-    a.bps = 0;
-    plan_args(a, uint64_t(nunits), kWave);
+    plan_args(a);
 
     float* outE = nullptr;
     int32_t* outAcc = nullptr;
@@ -483,7 +504,7 @@ int pda_run(pda_ctx* ctx, int sid, int R, uint32_t seed, uint32_t set_id, int fl
     HIP_TRY(hipEventRecord(s->ev0, s->stream));
     const BinomGuide guide{s->d_thr, s->d_guide};
     const FastArgs fa = fast_args(s->n, s->quick_rates, a.clk_p, s->ph.r0, ctx->max_P);
-    HIP_TRY(launch_walk(pass, grid, ctx->d_bursts, ctx->d_ticks, ctx->d_links, s->d_model, guide, a,
+    HIP_TRY(launch_walk(pass, grid, ctx->d_bursts, run_order(ctx, b0, b1), ctx->d_ticks, ctx->d_links, s->d_model, guide, a,
                         fa, s->d_hist_acc, s->d_replay, s->d_replay_count, s->d_work, outE, outAcc,
                         outF, nullptr, nullptr, s->stream));
     HIP_TRY(hipEventRecord(s->ev_mid, s->stream));
@@ -491,7 +512,7 @@ int pda_run(pda_ctx* ctx, int sid, int R, uint32_t seed, uint32_t set_id, int fl
     // of the run; the grid is sized for the worst case and its unneeded
     // workgroups exit at once
     HIP_TRY(launch_walk(kPassReplay, replay_grid(ctx, uint64_t(nunits)), ctx->d_bursts,
-                        ctx->d_ticks, ctx->d_links, s->d_model, guide, a, fa, s->d_hist_acc,
+                        nullptr, ctx->d_ticks, ctx->d_links, s->d_model, guide, a, fa, s->d_hist_acc,
                         s->d_replay, s->d_replay_count, s->d_work, outE, outAcc, outF, ctx->d_obs,
                         s->d_result, s->stream));
     HIP_TRY(hipEventRecord(s->ev1, s->stream));

@@ -240,6 +240,9 @@ struct pda_ctx {
     int64_t nbursts = 0, nphotons = 0;
     uint64_t data_gen = 0;          // bumped by every burst load
     pda::BurstDesc* d_bursts = nullptr;
+    // the bursts as the walk starts them: as they come, and by falling duration
+    pda::WalkBurst* d_plain = nullptr;
+    pda::WalkBurst* d_order = nullptr;
     uint32_t* d_ticks = nullptr;
     uint2* d_links = nullptr;
     float clk_p = 0.f, bg_ad = 0.f, bg_dd = 0.f;
@@ -271,18 +274,27 @@ struct Launch {
     uint32_t grid = 1, batch = kWave, queues = 1;
 };
 Launch plan_launch(const pda_ctx* ctx, int pass, bool population, uint64_t units);
+// Queues and workgroups of a launch over `units` units, L.batch at a time: a
+// workgroup per batch of every queue as long as they fit the GPU.  One per
+// batch of the run left some queues a workgroup short, and their last batch
+// to a second turn: a run of 20,000 bursts x 4 of 3 broadened states walked
+// for 41 us, 33 now.
+void size_grid(Launch& L, uint64_t max_grid, uint64_t units, uint32_t queues);
 // Workgroups of the replay pass of a run of `units` units.
 uint32_t replay_grid(const pda_ctx* ctx, uint64_t units);
 // The fields of a walk's arguments that follow from the others: R's
-// multiply-shift divisor, and the `items` (units, or a population's batches)
-// each of the a.queues work counters hands out, in whole waves of units.
-void plan_args(RunArgs& a, uint64_t items, uint32_t align);
+// multiply-shift divisor and the batches per set.
+void plan_args(RunArgs& a);
+// The bursts in the order in which a run over [b0, b1) starts them, entry b0
+// first: by falling duration for all of them, as they come for a part.
+const WalkBurst* run_order(const pda_ctx* ctx, int64_t b0, int64_t b1);
 
 // kernels (pda_kernels.hip)
 hipError_t walk_occupancy(int pass, int B, int* blocks_per_cu);
 hipError_t pop_walk_occupancy(int pass, int B, int* blocks_per_cu);
 // kPassReplay also ends the run: histogram and chi2 against obs into result
-hipError_t launch_walk(int pass, uint32_t grid, const BurstDesc* bursts, const uint32_t* ticks,
+hipError_t launch_walk(int pass, uint32_t grid, const BurstDesc* bursts, const WalkBurst* order,
+                       const uint32_t* ticks,
                        const uint2* links, const Model* model, const BinomGuide& guide,
                        const RunArgs& a, const FastArgs& fa, int32_t* hist_acc, uint32_t* replay,
                        uint32_t* replay_count, uint32_t* work, float* outE, int32_t* outAcc,
@@ -293,7 +305,7 @@ hipError_t launch_model(const Model& M, Model* model, ThrPair* thr, uint8_t* gui
 hipError_t launch_guide(const Model* models, int nsets, int max_states, ThrPair* thr,
                         uint8_t* guide, hipStream_t stream);
 hipError_t launch_pop_walk(int pass, uint32_t grid, const BurstDesc* bursts,
-                           const uint32_t* ticks, const uint2* links, const PopControl* ctl,
+                           const WalkBurst* order, const uint32_t* ticks, const uint2* links, const PopControl* ctl,
                            const Model* models, const BinomTable* tabs,
                            const BinomGuide& guide, const RunArgs& a,
                            const FastArgs& fa, int32_t* hist_acc, uint64_t* replay,
@@ -322,8 +334,8 @@ hipError_t rb_walk_occupancy(bool scores, int n, int* per_cu);
 // the fast-form walk and, behind it, the general-form replay of the units it
 // abandoned (replay_grid workgroups; those beyond the list's need exit)
 hipError_t launch_rb_walk(bool scores, int n, uint32_t grid, uint32_t replay_grid,
-                          const BurstDesc* bursts, const uint32_t* ticks, const uint2* links,
-                          const Model* model, const RbModel* rbm, const RunArgs& a,
+                          const BurstDesc* bursts, const WalkBurst* order, const uint32_t* ticks,
+                          const uint2* links, const Model* model, const RbModel* rbm, const RunArgs& a,
                           const FastArgs& fa, uint2* cnt, float* F, float* S, uint32_t* work,
                           uint32_t* big, uint32_t* huge,
                           uint32_t* big_count, uint32_t* replay, uint32_t* replay_count,

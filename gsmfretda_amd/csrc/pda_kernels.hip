@@ -31,28 +31,6 @@ namespace pda {
 constexpr uint32_t kReplayQueues = 8;
 static_assert(kReplayQueues <= kAuxQueues, "replay counters live on the auxiliary lines");
 
-// Contiguous share of a run's work items (units or batches) that one work
-// counter hands out.
-struct QueueRange {
-    uint32_t begin, end;
-};
-__device__ __forceinline__ QueueRange queue_range(uint32_t queue, uint32_t share, uint32_t n) {
-    const uint64_t b = uint64_t(queue) * share;
-    const uint32_t begin = b < n ? uint32_t(b) : n;
-    return QueueRange{begin, n - begin < share ? n : begin + share};
-}
-
-// Batches of a population that a work counter hands out: every queues-th of
-// the flat list (set 0's batches, set 1's, ...), the first being `queue`.  A
-// set's units take a multiple of another's under faster dynamics; dealt out
-// like this every queue has its share of every set, where contiguous shares
-// gave whole sets to a queue, whose waves (only they take from it) ended
-// long after the others'.
-__device__ __forceinline__ uint32_t pop_queue_length(uint32_t batches, uint32_t queue,
-                                                     uint32_t queues) {
-    return batches > queue ? (batches - queue + queues - 1u) / queues : 0u;
-}
-
 // Lanes of the mask below this one.
 __device__ __forceinline__ uint32_t lanes_below(uint64_t mask) {
     return __builtin_amdgcn_mbcnt_hi(uint32_t(mask >> 32),
@@ -117,7 +95,10 @@ __device__ __forceinline__ void flush_hist(int32_t* h, int32_t* __restrict__ row
 //
 // A population's work is a flat list of batches: set s owns batches
 // [s * bps, (s + 1) * bps), each covering up to a.batch consecutive units of
-// that set; the list is dealt out to the counters in turn (pop_queue_length).
+// that set; the list is dealt out to the counters in turn: a set's units take a
+// multiple of another's under faster dynamics, and with contiguous shares a
+// queue had whole sets, its waves (only they take from it) ending long after
+// the others'.
 // A wave's lanes may be walking units of two sets at once: the workgroup keeps
 // two LDS model slots with an LDS histogram each, and a wave moves to a third
 // set only after the older slot's lanes have finished, so it never drains to
@@ -138,6 +119,14 @@ __device__ __forceinline__ void flush_hist(int32_t* h, int32_t* __restrict__ row
 // keeps 8 waves on a SIMD: the window loop waits on dependent loads, which the
 // other waves hide (the 256-set generation 11.3 ms on the GPU with 7 and 10.6
 // with 8, 64 sets of fast dynamics 12.1 and 11.3).
+// A single set's bursts are started by falling duration within each queue's
+// share (burst_order in pda_layout.cpp), so that a run ends with units of few
+// windows and not with some lane's thirtieth: 50,000 bursts x 16 of 3 states
+// under a 30 kHz background 277 -> 231 us, 100,000 x 100 of 3 states 317 -> 310.
+// Sorted over all bursts, which takes the queues' photons apart, the latter
+// took 318 and a population 6 % more; populations, whose other sets fill the
+// end of each, and the RB walk, which writes per burst, start them as they
+// come.
 // Units are started 64 at a time into LDS and taken from there one lane at a
 // time as lanes fall idle, and ended ones wait in LDS until 64 can be binned:
 // a start (a Philox block and the unit's division) and a tally (a division and
@@ -160,7 +149,7 @@ constexpr int fast_waves_per_eu(bool pop, int pass) {
 }
 
 struct FastIO {
-    const BurstDesc* bursts;
+    const WalkBurst* bursts;
     const uint32_t* ticks;
     const uint2* links;
     const Model* models;       // [1], or the population's sets
@@ -201,11 +190,8 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(
 
     const uint32_t seed = kPop ? io.ctl->seed : a.seed;
     const uint32_t queue = blockIdx.x % a.queues;
-    // this queue's work: a contiguous share of the units, or every
-    // a.queues-th batch of the generation
     const QueueRange q = queue_range(queue, a.q_share, kPop ? 0u : a.nunits);
-    const uint32_t q_len = kPop ? pop_queue_length(a.nsets * a.bps, queue, a.queues)
-                                : q.end - q.begin;
+    const uint32_t batches = a.nsets * a.bps;
     const uint32_t xrow = blockIdx.x & 7u;
     const UnitDiv divR{a.div_m, a.div_sh};
     int set0 = kPop ? -1 : 0, set1 = -1;  // the set each LDS slot holds
@@ -239,19 +225,15 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(
                     if (lane == 0)
                         k = atomicAdd(&io.work[queue * kCounterStride], kPop ? 1u : a.batch);
                     k = __builtin_amdgcn_readfirstlane(k);
-                    if (k >= q_len) {
+                    if (kPop) k = k * a.queues + queue;
+                    if (k >= (kPop ? batches : q.end - q.begin)) {
                         drained = true;
                         break;
                     }
-                    if (kPop) {
-                        k = k * a.queues + queue;
-                        pool_set = k / a.bps;
-                        pool_next = (k - pool_set * a.bps) * a.batch;
-                        pool_end = a.nunits - pool_next < a.batch ? a.nunits : pool_next + a.batch;
-                    } else {
-                        pool_next = q.begin + k;
-                        pool_end = q.end - pool_next < a.batch ? q.end : pool_next + a.batch;
-                    }
+                    if (kPop) pool_set = k / a.bps;
+                    pool_next = kPop ? (k - pool_set * a.bps) * a.batch : q.begin + k;
+                    const uint32_t end = kPop ? a.nunits : q.end;
+                    pool_end = end - pool_next < a.batch ? end : pool_next + a.batch;
                 }
                 if (kPop && int(pool_set) != (cur ? set1 : set0)) {
                     const uint32_t other = cur ^ 1u;
@@ -275,10 +257,10 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(
                 int state = 0;
                 StartedUnit e;
                 if (u < pool_end) {
-                    const uint32_t bl = unit_div(u, divR);
-                    e.d = io.bursts[a.begin + bl];
-                    e.r = u - bl * a.R;
-                    e.b = a.begin + bl;
+                    const uint32_t i = unit_div(u, divR);
+                    e.d = io.bursts[a.begin + i].d;
+                    e.b = io.bursts[a.begin + i].b;
+                    e.r = u - i * a.R;
                     const UnitKey k{seed,
                                     kPop ? io.ctl->set_base + pool_set * io.ctl->set_stride : a.set,
                                     e.r, e.b};
@@ -287,7 +269,9 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(
                     state = s0.s;
                     if (!walks) {
                         tally(s_hist + (kPop ? cur : 0u) * uint32_t(a.B), a.B, 0.0f, 0.0f);
-                        if (kSamples) store_sample(u, 0.0f, 0.0f, io.outE, io.outAcc, io.outF);
+                        if (kSamples)
+                            store_sample((e.b - a.begin) * a.R + e.r, 0.0f, 0.0f, io.outE,
+                                         io.outAcc, io.outF);
                     }
                 }
                 pool_next = pool_end - pool_next < kWave ? pool_end : pool_next + kWave;
@@ -498,7 +482,9 @@ __device__ __forceinline__ void replay_units(
     __syncthreads();
 
     // handed out as in fast_walk_kernel, a wave's worth at a time
-    const QueueRange q = queue_range(queue, (nunits + queues - 1u) / queues, nunits);
+    const uint32_t share = (nunits + queues - 1u) / queues;
+    const uint32_t q_begin = queue * share < nunits ? queue * share : nunits;
+    const uint32_t q_end = nunits - q_begin < share ? nunits : q_begin + share;
     uint32_t* counter = &work[(kMaxQueues + queue) * kCounterStride];
     uint32_t pool_next = 0, pool_end = 0;  // the wave's current batch
     bool busy = false;
@@ -517,12 +503,12 @@ __device__ __forceinline__ void replay_units(
                 uint32_t off = 0;
                 if (lane == 0) off = atomicAdd(counter, uint32_t(kWave));
                 off = __shfl(off, 0);
-                if (off >= q.end - q.begin) {
+                if (off >= q_end - q_begin) {
                     drained = true;
                     break;
                 }
-                pool_next = q.begin + off;
-                pool_end = q.end - pool_next < kWave ? q.end : pool_next + kWave;
+                pool_next = q_begin + off;
+                pool_end = q_end - pool_next < kWave ? q_end : pool_next + kWave;
             }
             const uint32_t rank = lanes_below(want);
             const uint32_t avail = pool_end - pool_next;
@@ -711,7 +697,7 @@ __global__ __launch_bounds__(kWave) void pop_walk_kernel(
 
     const uint32_t seed = ctl->seed, set_base = ctl->set_base, set_stride = ctl->set_stride;
     const uint32_t queue = blockIdx.x % a.queues;
-    const uint32_t q_len = pop_queue_length(a.nsets * a.bps, queue, a.queues);
+    const uint32_t batches = a.nsets * a.bps;
     const uint32_t xrow = blockIdx.x & 7u;
     int set0 = -1, set1 = -1;    // wave-uniform: the set each LDS slot holds
     uint32_t cur = 0;            // slot that receives new units
@@ -732,11 +718,11 @@ __global__ __launch_bounds__(kWave) void pop_walk_kernel(
                 uint32_t k = 0;
                 if (lane == 0) k = atomicAdd(&work[queue * kCounterStride], 1u);
                 k = __shfl(k, 0);
-                if (k >= q_len) {
+                k = k * a.queues + queue;
+                if (k >= batches) {
                     drained = true;
                     break;
                 }
-                k = k * a.queues + queue;
                 pool_set = k / a.bps;
                 pool_next = (k - pool_set * a.bps) * a.batch;
                 pool_end = pool_next + a.batch < a.nunits ? pool_next + a.batch : a.nunits;
@@ -1106,13 +1092,14 @@ static void launch_fast(uint32_t grid, size_t lds, const FastIO& io, const RunAr
                        stream, io, a, fa);
 }
 
-hipError_t launch_walk(int pass, uint32_t grid, const BurstDesc* bursts, const uint32_t* ticks,
+hipError_t launch_walk(int pass, uint32_t grid, const BurstDesc* bursts, const WalkBurst* order,
+                       const uint32_t* ticks,
                        const uint2* links, const Model* model, const BinomGuide& guide,
                        const RunArgs& a, const FastArgs& fa, int32_t* hist_acc, uint32_t* replay,
                        uint32_t* replay_count, uint32_t* work, float* outE, int32_t* outAcc,
                        float* outF, const float* obs, ResultHeader* result, hipStream_t stream) {
     const size_t lds = sizeof(int32_t) * size_t(a.B);
-    const FastIO io{bursts, ticks, links, model, nullptr, nullptr, guide, hist_acc, replay,
+    const FastIO io{order, ticks, links, model, nullptr, nullptr, guide, hist_acc, replay,
                     replay_count, work, outE, outAcc, outF};
     if (pass == kPassReplay)
         hipLaunchKernelGGL(walk_kernel, dim3(grid), dim3(kWave), lds, stream, bursts, ticks, links,
@@ -1156,13 +1143,13 @@ hipError_t pop_walk_occupancy(int pass, int B, int* blocks_per_cu) {
 }
 
 hipError_t launch_pop_walk(int pass, uint32_t grid, const BurstDesc* bursts,
-                           const uint32_t* ticks, const uint2* links, const PopControl* ctl,
+                           const WalkBurst* order, const uint32_t* ticks, const uint2* links, const PopControl* ctl,
                            const Model* models, const BinomTable* tabs,
                            const BinomGuide& guide, const RunArgs& a,
                            const FastArgs& fa, int32_t* hist_acc, uint64_t* replay,
                            uint32_t* replay_count, uint32_t* work, hipStream_t stream) {
     const size_t lds = sizeof(int32_t) * 2u * size_t(a.B);
-    const FastIO io{bursts, ticks, links, models, tabs, ctl, guide, hist_acc, replay,
+    const FastIO io{order, ticks, links, models, tabs, ctl, guide, hist_acc, replay,
                     replay_count, work, nullptr, nullptr, nullptr};
     if (pass == kPassGeneral)
         hipLaunchKernelGGL(pop_walk_kernel, dim3(grid), dim3(kWave), lds, stream, bursts, ticks,

@@ -1,6 +1,7 @@
 // pda_layout.cpp -- see pda_layout.h.
 #include "pda_layout.h"
 
+#include <algorithm>
 #include <cmath>
 #include <cstdarg>
 #include <cstdio>
@@ -205,6 +206,38 @@ int build_model(const Photophysics& s, int n, const float* args, int nargs, Mode
         M.lq[i] = dlog(M.qq[i]);
     }
     return PDA_OK;
+}
+
+// A counting sort of each of kDefaultQueues parts.  A unit's windows grow with
+// its burst's duration: the walk starts the long ones first, and a run ends with
+// short ones.
+void burst_order(const std::vector<BurstDesc>& bursts, std::vector<WalkBurst>& plain,
+                 std::vector<WalkBurst>& order) {
+    constexpr uint32_t kOrderBuckets = 256;
+    constexpr size_t kOrderParts = kDefaultQueues;
+    float longest = 0.0f;
+    for (const BurstDesc& d : bursts)
+        if (d.T < INFINITY && d.T > longest) longest = d.T;
+    const float scale = longest > 0.0f ? float(kOrderBuckets - 1) / longest : 0.0f;
+    auto bucket = [&](const BurstDesc& d) {  // 0: the longest
+        const float x = d.T * scale;
+        return x >= 1.0f ? kOrderBuckets - 1u - std::min(uint32_t(std::min(x, float(kOrderBuckets))),
+                                                         kOrderBuckets - 1u)
+                         : kOrderBuckets - 1u;
+    };
+    const size_t n = bursts.size();
+    plain.resize(n);
+    order.resize(n);
+    for (size_t i = 0; i < n; ++i) plain[i] = WalkBurst{bursts[i], uint32_t(i), {0u, 0u, 0u}};
+    // each queue's share by itself: a share stays one region of the photon arrays
+    const size_t part = std::max<size_t>((n + kOrderParts - 1) / kOrderParts, 1);
+    for (size_t b0 = 0; b0 < n; b0 += part) {
+        const size_t b1 = std::min(n, b0 + part);
+        uint32_t next[kOrderBuckets + 1] = {};
+        for (size_t i = b0; i < b1; ++i) ++next[bucket(bursts[i]) + 1];
+        for (uint32_t i = 0; i < kOrderBuckets; ++i) next[i + 1] += next[i];
+        for (size_t i = b0; i < b1; ++i) order[b0 + next[bucket(bursts[i])]++] = plain[i];
+    }
 }
 
 // Inversion constants of binomial_inversion() (pda_math.h) per state and count.

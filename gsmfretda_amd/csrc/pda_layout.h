@@ -48,6 +48,11 @@ int encode_bursts(const int64_t* start, const int64_t* stop, const int64_t* ista
 int build_model(const Photophysics& ph, int n, const float* args, int nargs, Model& M,
                 std::string& err);
 
+// The bursts as a walk starts them: as they come, and by falling duration (in
+// 256 steps of the longest, a step's bursts in their order) within each of
+// kDefaultQueues equal parts.
+void burst_order(const std::vector<BurstDesc>& bursts, std::vector<WalkBurst>& plain,
+                 std::vector<WalkBurst>& order);
 // Tabulated inversion constants for the fast walk (needs M from build_model).
 void build_binom_table(const Model& M, BinomTable& T);
 

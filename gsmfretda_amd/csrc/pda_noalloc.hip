@@ -130,23 +130,22 @@ extern "C" int pda_run_noalloc(pda_ctx* ctx, int sid, int R, uint32_t seed, uint
     a.nstates = s->n;
     a.replay_cap = uint32_t(kReplayCapacity);
     a.nsets = 1;
-    a.bps = 0;
     const int pass = s->any_v ? kPassBroad : kPassGuided;
     const Launch L = plan_launch(ctx, pass, false, uint64_t(nunits));
     a.batch = L.batch;
     a.queues = L.queues;
-    plan_args(a, uint64_t(nunits), kWave);
+    plan_args(a);
 
     hipLaunchKernelGGL(clear_scratch_kernel, dim3(1), dim3(1024), 0, s->stream, work, count,
                        hist_acc);
     HIP_TRY(hipGetLastError());
     const BinomGuide guide{s->d_thr, s->d_guide};
     const FastArgs fa = fast_args(s->n, s->quick_rates, a.clk_p, s->ph.r0, ctx->max_P);
-    HIP_TRY(launch_walk(pass, L.grid, ctx->d_bursts, ctx->d_ticks, ctx->d_links, s->d_model, guide,
+    HIP_TRY(launch_walk(pass, L.grid, ctx->d_bursts, run_order(ctx, b0, b1), ctx->d_ticks, ctx->d_links, s->d_model, guide,
                         a, fa, hist_acc, replay, count, work, nullptr, nullptr, nullptr, nullptr,
                         nullptr, s->stream));
     HIP_TRY(launch_walk(kPassReplay, replay_grid(ctx, uint64_t(nunits)), ctx->d_bursts,
-                        ctx->d_ticks, ctx->d_links, s->d_model, guide, a, fa, hist_acc, replay,
+                        nullptr, ctx->d_ticks, ctx->d_links, s->d_model, guide, a, fa, hist_acc, replay,
                         count, work, nullptr, nullptr, nullptr, ctx->d_obs,
                         static_cast<ResultHeader*>(d_result), s->stream));
     return PDA_OK;

@@ -146,7 +146,8 @@ int enqueue_population(pda_ctx* ctx, Slot& s, int pass, uint32_t grid, const Run
         HIP_TRY(launch_guide(models, p.nsets, p.max_states, p.d_thr, p.d_guide, s.stream));
         guide = BinomGuide{p.d_thr, p.d_guide};
     }
-    HIP_TRY(launch_pop_walk(pass, grid, ctx->d_bursts, ctx->d_ticks, ctx->d_links, ctl, models,
+    HIP_TRY(launch_pop_walk(pass, grid, ctx->d_bursts,
+                            ctx->d_plain, ctx->d_ticks, ctx->d_links, ctl, models,
                             p.d_tabs, guide, a, fast_args(p.max_states, p.quick_rates, a.clk_p, p.r0,
                                              ctx->max_P),
                             p.d_hist_acc, p.d_replay, p.d_replay_count, p.d_work,
@@ -219,8 +220,7 @@ int run_population(pda_ctx* ctx, Slot& s, int R, uint32_t seed, uint32_t set_bas
     a.nstates = 0;
     a.replay_cap = uint32_t(std::min<size_t>(p.replay_cap, 0xFFFFFFFFu));
     a.nsets = uint32_t(p.nsets);
-    a.bps = uint32_t(bps);
-    plan_args(a, bps * uint64_t(p.nsets), 1u);
+    plan_args(a);
     const uint32_t grid = units > 0 ? L.grid : 1u;
 
     // the generation's stream keys travel with its models

@@ -425,10 +425,12 @@ int rb_enqueue_forward(pda_ctx* ctx, Slot& s, RbState& r, const Model& M,
         batch = (uint64_t(units) / (max_grid * 6u) + kWave - 1) / kWave * kWave;
         batch = std::min<uint64_t>(std::max<uint64_t>(batch, kWave), 4096);
     }
-    const uint32_t grid = uint32_t(std::max<uint64_t>(1, std::min(max_grid, (uint64_t(units) + batch - 1) / batch)));
-    a.batch = uint32_t(batch);
-    a.queues = std::min<uint32_t>(ctx->shape.queues ? ctx->shape.queues : kDefaultQueues, grid);
-    plan_args(a, uint64_t(units), kWave);
+    Launch L;
+    L.batch = uint32_t(batch);
+    size_grid(L, max_grid, uint64_t(units), ctx->shape.queues ? ctx->shape.queues : kDefaultQueues);
+    a.batch = L.batch;
+    a.queues = L.queues;
+    plan_args(a);
     PassShape ps;
     if (int rc = pass_shape(ctx, 0, n, false, a.B, cap, a.nunits, ps)) return rc;
     // the memo of this set: every count vector's pmf
@@ -456,8 +458,8 @@ int rb_enqueue_forward(pda_ctx* ctx, Slot& s, RbState& r, const Model& M,
     HIP_TRY(launch_rb_memo(n, r.d_pmf_tab, ML.d_items, ML.nitems, ML.d_rank_offP, r.d_poolP,
                            aux ? aux : stream));
     if (aux) HIP_TRY(hipEventRecord(s.rb_join, aux));
-    HIP_TRY(launch_rb_walk(scores, n, grid, uint32_t(ctx->num_cu) * 4u, ctx->d_bursts, ctx->d_ticks,
-                           ctx->d_links, d_model, d_rbm, a,
+    HIP_TRY(launch_rb_walk(scores, n, L.grid, uint32_t(ctx->num_cu) * 4u, ctx->d_bursts,
+                           ctx->d_plain, ctx->d_ticks, ctx->d_links, d_model, d_rbm, a,
                            fast_args(n, M.quick_rates != 0, a.clk_p, M.r0, ctx->max_P), r.d_cnt, r.d_F, r.d_S, r.d_work,
                            r.d_big, r.d_huge, r.d_big_count, r.d_replay, r.d_replay_count,
                            stream));
@@ -577,7 +579,7 @@ int enqueue_derivative(pda_ctx* ctx, RbState& r, int mode, double* out, uint32_t
     PassShape ps;
     if (int rc = pass_shape(ctx, mode, r.n, r.wide, r.B, r.cap, a.nunits, ps)) return rc;
     a.queues = 1;
-    plan_args(a, a.nunits, kWave);
+    plan_args(a);
     const RbModel* d_rbm = r.d_rbm;
     const RbMemoLayout& ML = ctx->rb_memo[r.n];
     const double* g = mode == 1 ? r.d_g : nullptr;

@@ -237,7 +237,7 @@ struct RbScoreModel {
 // with 3 states, spills with 4.)
 template <bool kScores, int kN>
 __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(8))) void rb_walk_kernel(
-    const BurstDesc* __restrict__ bursts, const uint32_t* __restrict__ ticks,
+    const WalkBurst* __restrict__ bursts, const uint32_t* __restrict__ ticks,
     const uint2* __restrict__ links, const Model* __restrict__ model,
     const RbModel* __restrict__ rbm, const RunArgs a, const FastArgs fa,
     uint2* __restrict__ cnt_out,
@@ -269,9 +269,7 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(8))) void
     acc.S = &s_S[0][lane];
 
     const uint32_t queue = blockIdx.x % a.queues;
-    const uint64_t q_first = uint64_t(queue) * a.q_share;
-    const uint32_t q_begin = q_first < a.nunits ? uint32_t(q_first) : a.nunits;
-    const uint32_t q_end = a.nunits - q_begin < a.q_share ? a.nunits : q_begin + a.q_share;
+    const QueueRange q = queue_range(queue, a.q_share, a.nunits);
     uint32_t pool_next = 0, pool_end = 0;
     uint32_t started = 0, start_next = 0;  // entries of s_start, the next to take
     bool busy = false;
@@ -287,31 +285,31 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(8))) void
             if (start_next == started) {  // start the next units
                 if (pool_next >= pool_end) {
                     if (drained) break;
-                    uint32_t off = 0;
-                    if (lane == 0) off = atomicAdd(&work[queue * kCounterStride], a.batch);
-                    off = __builtin_amdgcn_readfirstlane(off);
-                    if (off >= q_end - q_begin) {
+                    uint32_t k = 0;
+                    if (lane == 0) k = atomicAdd(&work[queue * kCounterStride], a.batch);
+                    k = __builtin_amdgcn_readfirstlane(k);
+                    if (k >= q.end - q.begin) {
                         drained = true;
                         break;
                     }
-                    pool_next = q_begin + off;
-                    pool_end = pool_next + a.batch < q_end ? pool_next + a.batch : q_end;
+                    pool_next = q.begin + k;
+                    pool_end = q.end - pool_next < a.batch ? q.end : pool_next + a.batch;
                 }
                 const uint32_t v = pool_next + lane;
                 bool walks = false;
                 int state = 0;
                 StartedUnit e;
                 if (lane < kStart && v < pool_end) {
-                    const uint32_t bl = unit_div(v, divR);
-                    e.d = bursts[a.begin + bl];
-                    e.r = v - bl * a.R;
-                    e.b = a.begin + bl;
+                    const uint32_t i = unit_div(v, divR);
+                    e.d = bursts[a.begin + i].d;
+                    e.b = bursts[a.begin + i].b;
+                    e.r = v - i * a.R;
                     const UnitKey k{a.seed, a.set, e.r, e.b};
                     WalkState<true> s0;
                     walks = begin_unit<true>(sM, k, e.d.P, e.d.T, s0) == kStepMore;
                     state = s0.s;
                     if (!walks) {
-                        zero_unit<Acc>(v, cnt_out, F_out, S_out);
+                        zero_unit<Acc>((e.b - a.begin) * a.R + e.r, cnt_out, F_out, S_out);
                     }
                 }
                 pool_next = pool_end - pool_next < kStart ? pool_end : pool_next + kStart;
@@ -1234,11 +1232,11 @@ hipError_t rb_big_occupancy(int mode, bool wide, int dyn_lds, int* per_cu) {
 
 template <bool kScores, int kN>
 static void launch_rb_walk_n(uint32_t grid, uint32_t replay_grid, const BurstDesc* bursts,
-                             const uint32_t* ticks, const uint2* links, const Model* model,
+                             const WalkBurst* order, const uint32_t* ticks, const uint2* links, const Model* model,
                              const RbModel* rbm, const RunArgs& a, const FastArgs& fa, uint2* cnt,
                              float* F, float* S, uint32_t* work, uint32_t* big, uint32_t* huge, uint32_t* big_count,
                              uint32_t* replay, uint32_t* replay_count, hipStream_t stream) {
-    hipLaunchKernelGGL((rb_walk_kernel<kScores, kN>), dim3(grid), dim3(kWave), 0, stream, bursts,
+    hipLaunchKernelGGL((rb_walk_kernel<kScores, kN>), dim3(grid), dim3(kWave), 0, stream, order,
                        ticks, links, model, rbm, a, fa, cnt, F, S, work, big, huge, big_count,
                        replay, replay_count);
     hipLaunchKernelGGL((rb_replay_kernel<kScores, kN>), dim3(replay_grid), dim3(kWave), 0, stream,
@@ -1247,14 +1245,14 @@ static void launch_rb_walk_n(uint32_t grid, uint32_t replay_grid, const BurstDes
 }
 
 hipError_t launch_rb_walk(bool scores, int n, uint32_t grid, uint32_t replay_grid,
-                          const BurstDesc* bursts, const uint32_t* ticks, const uint2* links,
-                          const Model* model, const RbModel* rbm, const RunArgs& a,
-                          const FastArgs& fa, uint2* cnt, float* F, float* S, uint32_t* work,
+                          const BurstDesc* bursts, const WalkBurst* order, const uint32_t* ticks,
+                          const uint2* links, const Model* model, const RbModel* rbm,
+                          const RunArgs& a, const FastArgs& fa, uint2* cnt, float* F, float* S, uint32_t* work,
                           uint32_t* big, uint32_t* huge, uint32_t* big_count,
                           uint32_t* replay, uint32_t* replay_count, hipStream_t stream) {
 #define PDA_RB_WALK(SC, N)                                                                    \
-    launch_rb_walk_n<SC, N>(grid, replay_grid, bursts, ticks, links, model, rbm, a, fa, cnt, F, \
-                            S, work, big, huge, big_count, replay, replay_count, stream)
+    launch_rb_walk_n<SC, N>(grid, replay_grid, bursts, order, ticks, links, model, rbm, a, fa, \
+                            cnt, F, S, work, big, huge, big_count, replay, replay_count, stream)
     if (n < 2 || n > kRbMaxStates) return hipErrorInvalidValue;
     if (scores) {
         if (n == 2) PDA_RB_WALK(true, 2);

@@ -43,6 +43,13 @@ struct BurstDesc {
     float T;            // T_burst_duration, seconds
 };
 
+// A burst in the order in which a walk starts them: its index and itself.
+struct WalkBurst {
+    BurstDesc d;
+    uint32_t b;
+    uint32_t pad[3];
+};
+
 // Per photon i of a burst (local indices):
 //   tick[i]   burst-relative tick; photons in neither channel carry the tick
 //             of the next channel photon (kTickSentinel if none), so the
@@ -137,11 +144,12 @@ struct RunArgs {
     float clk_p, bg_ad, bg_dd;
     int32_t nstates;     // for the chi2 degrees of freedom
     uint32_t replay_cap; // capacity of the replay list
-    uint32_t nsets;      // population runs: parameter sets
-    uint32_t bps;        // population runs: work batches per set
-    // derived by plan_args: floor(u / R) as (u div_m) >> div_sh (UnitDiv of
-    // R), and the work items (units; population runs: batches) of a queue
-    uint32_t div_m, div_sh, q_share;
+    uint32_t nsets;      // parameter sets (1, or the population's)
+    // derived by plan_args: work batches per set, and floor(u / R) as
+    // (u div_m) >> div_sh (UnitDiv of R)
+    uint32_t bps;
+    uint32_t div_m, div_sh;
+    uint32_t q_share;    // units of a queue of a single set's run
 };
 
 // Device result of one run, followed by int32 hist[B].

@@ -340,6 +340,17 @@ struct WindowInfo {
     int32_t m;
 };
 
+// What a work counter hands out: of a single set's units a contiguous share,
+// of a population's batches (set 0's, set 1's, ...) every queues-th.
+struct QueueRange {
+    uint32_t begin, end;
+};
+PDA_HD QueueRange queue_range(uint32_t queue, uint32_t share, uint32_t n) {
+    const uint64_t b = uint64_t(queue) * share;
+    const uint32_t begin = b < n ? uint32_t(b) : n;
+    return QueueRange{begin, n - begin < share ? n : begin + share};
+}
+
 // A unit that has been started: its burst and its key.
 struct StartedUnit {
     BurstDesc d;

@@ -82,3 +82,48 @@ def test_run_end(gpu_mc, oracle, B, left_pad, bg):
             assert np.array_equal(h[i].astype(np.int64), want)
             assert geff[i] == eff
             assert np.array_equal([g32[i], g64[i]], [c32, c64], equal_nan=True)
+
+
+@pytest.mark.parametrize("bursts,R", [(1, 3), (31, 70), (33, 2), (1000, 5)])
+@pytest.mark.parametrize("spread", ["usual", "equal", "zeros", "one long"])
+def test_bursts_started_by_duration(gpu_mc, oracle, bursts, R, spread):
+    """A run over all bursts starts them by duration, one over a part of them
+    as they come: the same units, at the same places, whatever the durations
+    (all the same, none for some, one far longer than the rest)."""
+    n, seed = 3, 5
+    rng = np.random.default_rng(bursts)
+    args = synth.make_args([0.2, 0.5, 0.8], synth.loguniform_rates(rng, 6, 3e2, 8e3))
+    d = synth.generate(bursts, args, n, seed=bursts + 7)
+    d.T = np.array(d.T, np.float32)
+    if spread == "equal":
+        d.T[:] = d.T[0]
+    elif spread == "zeros":
+        d.T[::3] = 0.0
+        d.T[1::7] = -1.0
+    elif spread == "one long":
+        d.T[bursts // 2] = 3e4
+    m = gpu_mc
+    m.load(d, SgDivSr=rng.uniform(0, 1, bursts).astype(np.float32), nbins=50, left_pad=0)
+    m.set_photophysics(0, *synth.PHOTOPHYSICS)
+    assert m.set_params(n, 0, args)
+    m.reSampleTimes = R
+
+    def units(b0, b1):
+        k = m.set_burst_range(b0, b1, 0)
+        m.run_kernel(sid=0, seed=seed, set_id=4, samples=True)
+        m.synchronize(0)
+        h = m.get_hist_chi2(0)[0]
+        return (h, *m.get_samples(0, k * R))
+    whole = units(0, -1)
+    o = oracle.run(oracle.Data.from_bursts(d), oracle.make_params(n, args, *synth.PHOTOPHYSICS),
+                   R=R, seed=seed, set_id=4, B=50)
+    assert np.array_equal(whole[0].astype(np.int64), o["hist"])
+    assert np.array_equal(whole[2], o["acc"])
+    if bursts > 1:
+        k = bursts // 2
+        a, b = units(0, k), units(k, bursts)
+        assert np.array_equal(whole[0], a[0] + b[0])
+        for x, y, z in zip(whole[1:], a[1:], b[1:]):
+            assert np.array_equal(np.asarray(x).view(np.uint32),
+                                  np.concatenate([y, z]).view(np.uint32))
+    m.set_burst_range(0, -1, 0)
