@@ -119,6 +119,10 @@ const WalkBurst* run_order(const pda_ctx* ctx, int64_t b0, int64_t b1) {
     return b0 == 0 && b1 == ctx->nbursts ? ctx->d_order : ctx->d_plain;
 }
 
+float clock_ms(const pda_ctx* ctx, uint64_t from, uint64_t to) {
+    return float(double(to - from) / double(ctx->clock_khz));
+}
+
 }  // namespace pda
 
 using namespace pda;
@@ -247,6 +251,9 @@ int pda_create(int device, int nstreams, pda_ctx** out) {
         ctx->num_cu = prop.multiProcessorCount;
         if (prop.sharedMemPerBlock > 0) ctx->lds_per_block = prop.sharedMemPerBlock;
     }
+    int khz = 0;
+    if (hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, device) == hipSuccess && khz > 0)
+        ctx->clock_khz = khz;
     ctx->slots.resize(size_t(nstreams));
     for (auto& s : ctx->slots) {
         if (hipStreamCreateWithFlags(&s.stream, hipStreamNonBlocking) != hipSuccess ||
@@ -262,8 +269,9 @@ int pda_create(int device, int nstreams, pda_ctx** out) {
                           sizeof(ResultHeader) + sizeof(int32_t) * kMaxBins,
                           hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess ||
             hipHostGetDevicePointer(reinterpret_cast<void**>(&s.d_result), s.h_result, 0) != hipSuccess ||
-            hipEventCreate(&s.ev0) != hipSuccess || hipEventCreate(&s.ev_mid) != hipSuccess ||
-            hipEventCreate(&s.ev1) != hipSuccess ||
+            hipHostMalloc(reinterpret_cast<void**>(&s.h_times), sizeof(RunTimes),
+                          hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess ||
+            hipHostGetDevicePointer(reinterpret_cast<void**>(&s.d_times), s.h_times, 0) != hipSuccess ||
             hipMemset(s.d_hist_acc, 0, sizeof(int32_t) * kMaxBins * 8) != hipSuccess ||
             hipDeviceSynchronize() != hipSuccess) {
             pda_destroy(ctx);
@@ -298,9 +306,7 @@ int pda_destroy(pda_ctx* ctx) {
         (void)hipFree(s.d_acc);
         (void)hipFree(s.d_F);
         (void)hipHostFree(s.h_E);
-        if (s.ev0) (void)hipEventDestroy(s.ev0);
-        if (s.ev_mid) (void)hipEventDestroy(s.ev_mid);
-        if (s.ev1) (void)hipEventDestroy(s.ev1);
+        (void)hipHostFree(s.h_times);
         free_population(s.pop);
         free_rb(s.rb);
         for (auto& r : s.rbpop) free_rb(r);
@@ -501,21 +507,18 @@ int pda_run(pda_ctx* ctx, int sid, int R, uint32_t seed, uint32_t set_id, int fl
         s->replay_cap = size_t(nunits);
     }
     a.replay_cap = uint32_t(s->replay_cap);
-    HIP_TRY(hipEventRecord(s->ev0, s->stream));
     const BinomGuide guide{s->d_thr, s->d_guide};
     const FastArgs fa = fast_args(s->n, s->quick_rates, a.clk_p, s->ph.r0, ctx->max_P);
     HIP_TRY(launch_walk(pass, grid, ctx->d_bursts, run_order(ctx, b0, b1), ctx->d_ticks, ctx->d_links, s->d_model, guide, a,
                         fa, s->d_hist_acc, s->d_replay, s->d_replay_count, s->d_work, outE, outAcc,
-                        outF, nullptr, nullptr, s->stream));
-    HIP_TRY(hipEventRecord(s->ev_mid, s->stream));
+                        outF, nullptr, nullptr, s->d_times, s->stream));
     // the abandoned units, in the general form over the whole GPU, and the end
     // of the run; the grid is sized for the worst case and its unneeded
     // workgroups exit at once
     HIP_TRY(launch_walk(kPassReplay, replay_grid(ctx, uint64_t(nunits)), ctx->d_bursts,
                         nullptr, ctx->d_ticks, ctx->d_links, s->d_model, guide, a, fa, s->d_hist_acc,
                         s->d_replay, s->d_replay_count, s->d_work, outE, outAcc, outF, ctx->d_obs,
-                        s->d_result, s->stream));
-    HIP_TRY(hipEventRecord(s->ev1, s->stream));
+                        s->d_result, s->d_times, s->stream));
     if (outE)
         HIP_TRY(hipMemcpyAsync(s->h_E, outE, sizeof(float) * size_t(nunits), hipMemcpyDeviceToHost,
                                s->stream));
@@ -597,8 +600,8 @@ int pda_last_run_ms(pda_ctx* ctx, int sid, float* ms) {
     Slot* s = slot_of(ctx, sid);
     if (!s || !ms) return fail(PDA_E_ARG, "bad argument");
     if (!s->ran) return fail(PDA_E_STATE, "stream %d has not run", sid);
-    HIP_TRY(hipEventSynchronize(s->ev1));
-    HIP_TRY(hipEventElapsedTime(ms, s->ev0, s->ev1));
+    HIP_TRY(hipStreamSynchronize(s->stream));
+    *ms = clock_ms(ctx, s->h_times->start, s->h_times->end);
     return PDA_OK;
 }
 
@@ -606,12 +609,10 @@ int pda_last_pass_ms(pda_ctx* ctx, int sid, float* walk_ms, float* finish_ms) {
     Slot* s = slot_of(ctx, sid);
     if (!s) return fail(PDA_E_ARG, "bad stream id %d", sid);
     if (!s->ran) return fail(PDA_E_STATE, "stream %d has not run", sid);
-    HIP_TRY(hipEventSynchronize(s->ev1));
-    float a = 0.f, b = 0.f;
-    HIP_TRY(hipEventElapsedTime(&a, s->ev0, s->ev_mid));
-    HIP_TRY(hipEventElapsedTime(&b, s->ev_mid, s->ev1));
-    if (walk_ms) *walk_ms = a;
-    if (finish_ms) *finish_ms = b;
+    HIP_TRY(hipStreamSynchronize(s->stream));
+    const RunTimes& t = *s->h_times;
+    if (walk_ms) *walk_ms = clock_ms(ctx, t.start, t.walked);
+    if (finish_ms) *finish_ms = clock_ms(ctx, t.walked, t.end);
     return PDA_OK;
 }
 

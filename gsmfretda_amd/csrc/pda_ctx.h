@@ -160,7 +160,10 @@ struct RbState {
     bool sbar_valid = false;           // d_Sbar holds the last forward's means
     double* h_grad = nullptr;          // the rows' sum, pinned, and its device address
     double* d_hgrad = nullptr;
-    hipEvent_t ev0 = nullptr, ev_walk = nullptr, ev1 = nullptr, ev_a0 = nullptr, ev_a1 = nullptr;
+    // clock readings of the last forward and, [1], the last derivative pass
+    // (start and end), pinned, and their device address
+    RunTimes* h_times = nullptr;
+    RunTimes* d_times = nullptr;
     bool ready = false;                // every fixed-size buffer above allocated
     bool ran = false, scores = false, adj_ran = false;
     int R = 0, B = 0, n = 0, K = 0, cap = 0, left_pad = 0;
@@ -201,7 +204,8 @@ struct Slot {
     float* h_E = nullptr;  // pinned (the reference's hmcE[sid])
     size_t sample_cap = 0;
     bool samples_valid = false;
-    hipEvent_t ev0 = nullptr, ev_mid = nullptr, ev1 = nullptr;
+    RunTimes* h_times = nullptr;       // pinned, of the last run
+    RunTimes* d_times = nullptr;       // its device address
     Population pop;
     RbState rb;
     // RB forward: the pmf table and memo are built on rb_aux while the walk
@@ -236,6 +240,7 @@ struct RbMemoLayout {
 struct pda_ctx {
     int device = 0;
     int num_cu = 256;
+    int clock_khz = 100000;         // of the kernels' clock readings
     std::vector<pda::Slot> slots;
     int64_t nbursts = 0, nphotons = 0;
     uint64_t data_gen = 0;          // bumped by every burst load
@@ -285,6 +290,8 @@ uint32_t replay_grid(const pda_ctx* ctx, uint64_t units);
 // The fields of a walk's arguments that follow from the others: R's
 // multiply-shift divisor and the batches per set.
 void plan_args(RunArgs& a);
+// The time between two clock readings.
+float clock_ms(const pda_ctx* ctx, uint64_t from, uint64_t to);
 // The bursts in the order in which a run over [b0, b1) starts them, entry b0
 // first: by falling duration for all of them, as they come for a part.
 const WalkBurst* run_order(const pda_ctx* ctx, int64_t b0, int64_t b1);
@@ -292,13 +299,15 @@ const WalkBurst* run_order(const pda_ctx* ctx, int64_t b0, int64_t b1);
 // kernels (pda_kernels.hip)
 hipError_t walk_occupancy(int pass, int B, int* blocks_per_cu);
 hipError_t pop_walk_occupancy(int pass, int B, int* blocks_per_cu);
-// kPassReplay also ends the run: histogram and chi2 against obs into result
+// kPassReplay also ends the run: histogram and chi2 against obs into result;
+// times (or null): where the clock readings go
 hipError_t launch_walk(int pass, uint32_t grid, const BurstDesc* bursts, const WalkBurst* order,
                        const uint32_t* ticks,
                        const uint2* links, const Model* model, const BinomGuide& guide,
                        const RunArgs& a, const FastArgs& fa, int32_t* hist_acc, uint32_t* replay,
                        uint32_t* replay_count, uint32_t* work, float* outE, int32_t* outAcc,
-                       float* outF, const float* obs, ResultHeader* result, hipStream_t stream);
+                       float* outF, const float* obs, ResultHeader* result, RunTimes* times,
+                       hipStream_t stream);
 // stores the model of a parameter set and builds its threshold rows
 hipError_t launch_model(const Model& M, Model* model, ThrPair* thr, uint8_t* guide,
                         hipStream_t stream);
@@ -344,12 +353,13 @@ hipError_t launch_rb_walk(bool scores, int n, uint32_t grid, uint32_t replay_gri
 int rb_unit_threads(int mode);
 size_t rb_unit_lds_bytes(int B, int mode, int n, int copies, bool pool);
 size_t rb_big_lds_bytes(int B, int cap, int mode, bool wide);
+// times (or null): where the launches of a run put their clock readings
 hipError_t launch_rb_table(const RbModel& R, const Model& M, RbModel* rbm, Model* model,
                            const double* lf, float* pmf_tab, uint32_t* work, uint32_t* big_count,
-                           uint32_t* replay_count, hipStream_t stream);
+                           uint32_t* replay_count, RunTimes* times, hipStream_t stream);
 // g_host (or null): the adjoint's cotangent, B entries
 hipError_t launch_rb_begin(double* rows, uint32_t n, uint32_t* work, const double* g_host,
-                           double* g, int B, hipStream_t stream);
+                           double* g, int B, RunTimes* times, hipStream_t stream);
 hipError_t launch_rb_memo(int n, const float* pmf_tab, const uint4* items, uint32_t nitems,
                           const uint32_t* rank_offP, float* poolP, hipStream_t stream);
 // copies: of the LDS accumulators; tile: units a workgroup takes at a time;
@@ -359,7 +369,7 @@ hipError_t launch_rb_unit(int mode, int n, uint32_t grid, int copies, int tile, 
                           const double* Sbar, const double* g, const uint32_t* rank_offP,
                           const uint4* rank_offD, const float* poolP,
                           unsigned long long* hist_acc, double* grad, uint32_t* work,
-                          hipStream_t stream);
+                          RunTimes* times, hipStream_t stream);
 hipError_t launch_rb_big(int mode, bool wide, uint32_t grid, int cap, const RbModel* rbm,
                          const double* lf,
                          const float* pmf_tab, const RunArgs& a, const uint2* cnt, const float* F,
@@ -369,8 +379,9 @@ hipError_t launch_rb_big(int mode, bool wide, uint32_t grid, int cap, const RbMo
 hipError_t launch_rb_score_mean(const RunArgs& a, int K, const float* S, double* Sbar,
                                 int num_cu, hipStream_t stream);
 // out[i] = sum of the nrows rows of n doubles
-hipError_t launch_rb_rows(const double* rows, int n, int nrows, double* out, hipStream_t stream);
+hipError_t launch_rb_rows(const double* rows, int n, int nrows, double* out, RunTimes* times,
+                          hipStream_t stream);
 hipError_t launch_rb_finish(const RunArgs& a, const float* obs, unsigned long long* hist_acc,
-                            void* res, hipStream_t stream);
+                            void* res, RunTimes* times, hipStream_t stream);
 
 }  // namespace pda

@@ -163,6 +163,7 @@ struct FastIO {
     float* outE;
     int32_t* outAcc;
     float* outF;
+    RunTimes* times;           // or null
 };
 
 template <bool kPop, int kPass, bool kSamples>
@@ -187,6 +188,8 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(
         wave_lds_sync();
     };
     if (!kPop) load_model(0u, 0u);
+
+    if (!kPop && io.times && blockIdx.x == 0 && lane == 0) stamp(&io.times->start);
 
     const uint32_t seed = kPop ? io.ctl->seed : a.seed;
     const uint32_t queue = blockIdx.x % a.queues;
@@ -558,7 +561,8 @@ __global__ __launch_bounds__(kWave) void walk_kernel(
     int32_t* __restrict__ hist_acc, const uint32_t* __restrict__ replay,
     uint32_t* __restrict__ replay_count, uint32_t* __restrict__ work, float* __restrict__ outE,
     int32_t* __restrict__ outAcc, float* __restrict__ outF, const float* __restrict__ obs,
-    ResultHeader* __restrict__ result) {
+    ResultHeader* __restrict__ result, RunTimes* __restrict__ times) {
+    if (times && blockIdx.x == 0 && threadIdx.x == 0) stamp(&times->walked);
     const uint32_t c = *replay_count;
     const uint32_t nunits = c < a.replay_cap ? c : a.replay_cap;
     // as many workgroups as the list needs a wave for, each queue served by
@@ -579,6 +583,7 @@ __global__ __launch_bounds__(kWave) void walk_kernel(
     // (a workgroup that has not yet read the replay count, and now reads
     // zero, is not workgroup 0, which has been counted: it returns)
     finish_run(a, obs, hist_acc, replay_count, c, work, result, lane);
+    if (times && lane == 0) stamp(&times->end);
 }
 
 // One threshold row of the fast walk's binomial draws, by one wave: state s
@@ -1097,14 +1102,15 @@ hipError_t launch_walk(int pass, uint32_t grid, const BurstDesc* bursts, const W
                        const uint2* links, const Model* model, const BinomGuide& guide,
                        const RunArgs& a, const FastArgs& fa, int32_t* hist_acc, uint32_t* replay,
                        uint32_t* replay_count, uint32_t* work, float* outE, int32_t* outAcc,
-                       float* outF, const float* obs, ResultHeader* result, hipStream_t stream) {
+                       float* outF, const float* obs, ResultHeader* result, RunTimes* times,
+                       hipStream_t stream) {
     const size_t lds = sizeof(int32_t) * size_t(a.B);
     const FastIO io{order, ticks, links, model, nullptr, nullptr, guide, hist_acc, replay,
-                    replay_count, work, outE, outAcc, outF};
+                    replay_count, work, outE, outAcc, outF, times};
     if (pass == kPassReplay)
         hipLaunchKernelGGL(walk_kernel, dim3(grid), dim3(kWave), lds, stream, bursts, ticks, links,
                            model, a, hist_acc, replay, replay_count, work, outE, outAcc, outF, obs,
-                           result);
+                           result, times);
     else if (pass == kPassBroad && outE)
         launch_fast<false, kPassBroad, true>(grid, lds, io, a, fa, stream);
     else if (pass == kPassBroad)
@@ -1150,7 +1156,7 @@ hipError_t launch_pop_walk(int pass, uint32_t grid, const BurstDesc* bursts,
                            uint32_t* replay_count, uint32_t* work, hipStream_t stream) {
     const size_t lds = sizeof(int32_t) * 2u * size_t(a.B);
     const FastIO io{order, ticks, links, models, tabs, ctl, guide, hist_acc, replay,
-                    replay_count, work, nullptr, nullptr, nullptr};
+                    replay_count, work, nullptr, nullptr, nullptr, nullptr};
     if (pass == kPassGeneral)
         hipLaunchKernelGGL(pop_walk_kernel, dim3(grid), dim3(kWave), lds, stream, bursts, ticks,
                            links, ctl, models, a, hist_acc, work);

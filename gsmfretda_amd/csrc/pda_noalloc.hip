@@ -143,10 +143,10 @@ extern "C" int pda_run_noalloc(pda_ctx* ctx, int sid, int R, uint32_t seed, uint
     const FastArgs fa = fast_args(s->n, s->quick_rates, a.clk_p, s->ph.r0, ctx->max_P);
     HIP_TRY(launch_walk(pass, L.grid, ctx->d_bursts, run_order(ctx, b0, b1), ctx->d_ticks, ctx->d_links, s->d_model, guide,
                         a, fa, hist_acc, replay, count, work, nullptr, nullptr, nullptr, nullptr,
-                        nullptr, s->stream));
+                        nullptr, nullptr, s->stream));
     HIP_TRY(launch_walk(kPassReplay, replay_grid(ctx, uint64_t(nunits)), ctx->d_bursts,
                         nullptr, ctx->d_ticks, ctx->d_links, s->d_model, guide, a, fa, hist_acc, replay,
                         count, work, nullptr, nullptr, nullptr, ctx->d_obs,
-                        static_cast<ResultHeader*>(d_result), s->stream));
+                        static_cast<ResultHeader*>(d_result), nullptr, s->stream));
     return PDA_OK;
 }

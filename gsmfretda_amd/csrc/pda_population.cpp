@@ -518,7 +518,7 @@ int pda_autotune(pda_ctx* ctx, int sid, int population, int R, int reps, int* ba
                 int r2 = pda_run(ctx, sid, R, 0u, 0u, 0);
                 if (r2) return r2;
                 HIP_TRY(hipStreamSynchronize(s->stream));
-                HIP_TRY(hipEventElapsedTime(&ms, s->ev0, s->ev1));
+                ms = clock_ms(ctx, s->h_times->start, s->h_times->end);
             }
             if (i > 0) t.push_back(ms);
         }

@@ -49,8 +49,7 @@ void free_rb(RbState& r) {
     (void)hipFree(r.d_Sbar);
     (void)hipFree(r.d_poolP);
     (void)hipHostFree(r.h_grad);
-    for (hipEvent_t e : {r.ev0, r.ev_walk, r.ev1, r.ev_a0, r.ev_a1})
-        if (e) (void)hipEventDestroy(e);
+    (void)hipHostFree(r.h_times);
     r = RbState();
 }
 
@@ -116,8 +115,7 @@ int ensure_rb(pda_ctx* ctx, RbState& r) {
             HIP_TRY(hipMalloc(&r.d_pmf_tab, sizeof(float) * size_t(kRbMaxStates) * kRbPmfStride));
         HIP_TRY(mapped(&r.h_jac, &r.d_hjac, sizeof(double) * kGradLen * kMaxBins));
         HIP_TRY(mapped(&r.h_grad, &r.d_hgrad, sizeof(double) * kGradLen));
-        for (hipEvent_t* e : {&r.ev0, &r.ev_walk, &r.ev1, &r.ev_a0, &r.ev_a1})
-            if (!*e) HIP_TRY(hipEventCreate(e));
+        HIP_TRY(mapped(&r.h_times, &r.d_times, 2 * sizeof(RunTimes)));
         HIP_TRY(hipDeviceSynchronize());
         r.ready = true;
     }
@@ -323,10 +321,10 @@ int pass_shape(pda_ctx* ctx, int mode, int n, bool wide, int B, int cap, uint32_
 // Enqueues one RB forward of model M -- the walk reading M from the device
 // copy d_model, which the first launch writes if store_model is set -- over the
 // slot's burst range into state r, on `stream`, the memo on `aux` where there
-// is one; timed: with the events of pda_rb_stats.
+// is one.
 int rb_enqueue_forward(pda_ctx* ctx, Slot& s, RbState& r, const Model& M,
                        const Model* d_model, Model* store_model, int R, uint32_t seed,
-                       uint32_t set_id, int flags, bool timed, hipStream_t stream,
+                       uint32_t set_id, int flags, hipStream_t stream,
                        hipStream_t aux) {
     int rc = ensure_rb(ctx, r);
     if (rc) return rc;
@@ -446,9 +444,8 @@ int rb_enqueue_forward(pda_ctx* ctx, Slot& s, RbState& r, const Model& M,
     }
 
     const RbModel* d_rbm = r.d_rbm;
-    if (timed) HIP_TRY(hipEventRecord(r.ev0, stream));
     HIP_TRY(launch_rb_table(rbm, M, r.d_rbm, store_model, ctx->d_lf, r.d_pmf_tab, r.d_work,
-                            r.d_big_count, r.d_replay_count, stream));
+                            r.d_big_count, r.d_replay_count, r.d_times, stream));
     // the memo depends on the model only: built on the side stream, where
     // there is one, while the walk runs (its few, long waves hide under it)
     if (aux) {
@@ -463,11 +460,10 @@ int rb_enqueue_forward(pda_ctx* ctx, Slot& s, RbState& r, const Model& M,
                            fast_args(n, M.quick_rates != 0, a.clk_p, M.r0, ctx->max_P), r.d_cnt, r.d_F, r.d_S, r.d_work,
                            r.d_big, r.d_huge, r.d_big_count, r.d_replay, r.d_replay_count,
                            stream));
-    if (timed) HIP_TRY(hipEventRecord(r.ev_walk, stream));
     if (aux) HIP_TRY(hipStreamWaitEvent(stream, s.rb_join, 0));
     HIP_TRY(launch_rb_unit(0, n, ps.unit_grid, ps.copies, ps.tile, ps.pool, a, r.d_cnt, r.d_F,
                            nullptr, nullptr, nullptr, ML.d_rank_offP, ML.d_rank_offD, r.d_poolP,
-                           r.d_hist, nullptr, r.d_work, stream));
+                           r.d_hist, nullptr, r.d_work, r.d_times, stream));
     HIP_TRY(launch_rb_big(0, false, ps.big_grid, ps.big_cap, d_rbm, ctx->d_lf, r.d_pmf_tab, a, r.d_cnt,
                           r.d_F, nullptr, nullptr, nullptr, r.d_big, r.d_big_count, r.d_hist,
                           nullptr, stream));
@@ -475,8 +471,7 @@ int rb_enqueue_forward(pda_ctx* ctx, Slot& s, RbState& r, const Model& M,
         HIP_TRY(launch_rb_big(0, false, ps.huge_grid, cap, d_rbm, ctx->d_lf, r.d_pmf_tab, a, r.d_cnt,
                               r.d_F, nullptr, nullptr, nullptr, r.d_huge, r.d_big_count + 1,
                               r.d_hist, nullptr, stream));
-    HIP_TRY(launch_rb_finish(a, ctx->d_obs, r.d_hist, r.d_res, stream));
-    if (timed) HIP_TRY(hipEventRecord(r.ev1, stream));
+    HIP_TRY(launch_rb_finish(a, ctx->d_obs, r.d_hist, r.d_res, r.d_times, stream));
     r.ran = true;
     r.adj_ran = false;
     r.scores = scores;
@@ -522,8 +517,8 @@ int pda_rb_forward(pda_ctx* ctx, int sid, int R, uint32_t seed, uint32_t set_id,
     if (!s->rb_aux) HIP_TRY(hipStreamCreateWithFlags(&s->rb_aux, hipStreamNonBlocking));
     if (!s->rb_fork) HIP_TRY(hipEventCreateWithFlags(&s->rb_fork, hipEventDisableTiming));
     if (!s->rb_join) HIP_TRY(hipEventCreateWithFlags(&s->rb_join, hipEventDisableTiming));
-    return rb_enqueue_forward(ctx, *s, s->rb, M, s->d_model, nullptr, R, seed, set_id, flags, true,
-                              s->stream, s->rb_aux);
+    return rb_enqueue_forward(ctx, *s, s->rb, M, s->d_model, nullptr, R, seed, set_id, flags, s->stream,
+                              s->rb_aux);
 }
 
 int pda_rb_get_result(pda_ctx* ctx, int sid, uint64_t* M_fixed, double* M, int nbins,
@@ -568,7 +563,7 @@ int check_derivative_run(const RbState& r, int sid, int nbins, int nargs) {
 // adjoint with cotangent r.d_g, 2 Jacobian) of state r's last forward,
 // accumulating into out (zeroed by the caller).
 int enqueue_derivative(pda_ctx* ctx, RbState& r, int mode, double* out, uint32_t rows,
-                       bool timed, hipStream_t stream) {
+                       hipStream_t stream) {
     RunArgs a{};
     a.begin = uint32_t(r.b0);
     a.nunits = uint32_t((r.b1 - r.b0) * int64_t(r.R));
@@ -584,15 +579,14 @@ int enqueue_derivative(pda_ctx* ctx, RbState& r, int mode, double* out, uint32_t
     const RbMemoLayout& ML = ctx->rb_memo[r.n];
     const double* g = mode == 1 ? r.d_g : nullptr;
     HIP_TRY(launch_rb_begin(out, rows, r.d_work, mode == 1 ? r.d_hg : nullptr, r.d_g, r.B,
-                            stream));
-    if (timed) HIP_TRY(hipEventRecord(r.ev_a0, stream));
+                            r.d_times + 1, stream));
     if (!r.sbar_valid) {
         HIP_TRY(launch_rb_score_mean(a, r.K, r.d_S, r.d_Sbar, ctx->num_cu, stream));
         r.sbar_valid = true;
     }
     HIP_TRY(launch_rb_unit(mode, r.n, ps.unit_grid, ps.copies, ps.tile, ps.pool, a, r.d_cnt,
                            r.d_F, r.d_S, r.d_Sbar, g, ML.d_rank_offP, ML.d_rank_offD, r.d_poolP,
-                           nullptr, out, r.d_work, stream));
+                           nullptr, out, r.d_work, nullptr, stream));
     HIP_TRY(launch_rb_big(mode, ps.wide, ps.big_grid, ps.big_cap, d_rbm, ctx->d_lf, r.d_pmf_tab, a,
                           r.d_cnt, r.d_F, r.d_S, r.d_Sbar, g, r.d_big, r.d_big_count, nullptr, out,
                           stream));
@@ -600,20 +594,18 @@ int enqueue_derivative(pda_ctx* ctx, RbState& r, int mode, double* out, uint32_t
         HIP_TRY(launch_rb_big(mode, ps.wide, ps.huge_grid, r.cap, d_rbm, ctx->d_lf, r.d_pmf_tab, a,
                               r.d_cnt, r.d_F, r.d_S, r.d_Sbar, g, r.d_huge, r.d_big_count + 1,
                               nullptr, out, stream));
-    if (timed) HIP_TRY(hipEventRecord(r.ev_a1, stream));
     return PDA_OK;
 }
 
 // Enqueues the adjoint pass of state r's last forward for the cotangent g
 // (nbins entries; r's pinned buffers must be free: the caller waited for the
 // stream), its gradient written to r.h_grad.
-int rb_enqueue_adjoint(pda_ctx* ctx, RbState& r, const double* g, bool timed,
+int rb_enqueue_adjoint(pda_ctx* ctx, RbState& r, const double* g,
                        hipStream_t stream) {
     std::memcpy(r.h_g, g, sizeof(double) * size_t(r.B));
-    if (int rc = enqueue_derivative(ctx, r, 1, r.d_grad, uint32_t(kGradLen * kRbGradRows), timed,
-                                    stream))
+    if (int rc = enqueue_derivative(ctx, r, 1, r.d_grad, uint32_t(kGradLen * kRbGradRows), stream))
         return rc;
-    HIP_TRY(launch_rb_rows(r.d_grad, kGradLen, kRbGradRows, r.d_hgrad, stream));
+    HIP_TRY(launch_rb_rows(r.d_grad, kGradLen, kRbGradRows, r.d_hgrad, r.d_times + 1, stream));
     r.adj_ran = true;
     return PDA_OK;
 }
@@ -627,7 +619,7 @@ void rb_collect_adjoint(const RbState& r, double* grad, int nargs) {
 }
 
 // Enqueues the Jacobian pass of state r's last forward, written to r.h_jac.
-int rb_enqueue_jacobian(pda_ctx* ctx, RbState& r, bool timed, hipStream_t stream) {
+int rb_enqueue_jacobian(pda_ctx* ctx, RbState& r, hipStream_t stream) {
     if (r.B > r.cap_jac) {  // the caller waited for the stream
         (void)hipFree(r.d_jac);
         r.d_jac = nullptr;
@@ -636,9 +628,9 @@ int rb_enqueue_jacobian(pda_ctx* ctx, RbState& r, bool timed, hipStream_t stream
         r.cap_jac = r.B;
     }
     const int n = kGradLen * r.B;
-    if (int rc = enqueue_derivative(ctx, r, 2, r.d_jac, uint32_t(n) * kRbJacRows, timed, stream))
+    if (int rc = enqueue_derivative(ctx, r, 2, r.d_jac, uint32_t(n) * kRbJacRows, stream))
         return rc;
-    HIP_TRY(launch_rb_rows(r.d_jac, n, kRbJacRows, r.d_hjac, stream));
+    HIP_TRY(launch_rb_rows(r.d_jac, n, kRbJacRows, r.d_hjac, r.d_times + 1, stream));
     r.adj_ran = true;
     return PDA_OK;
 }
@@ -695,7 +687,7 @@ int pda_rb_adjoint(pda_ctx* ctx, int sid, const double* g, int nbins, double* gr
         if (!std::isfinite(g[b])) return fail(PDA_E_ARG, "g[%d] not finite", b);
     HIP_TRY(hipSetDevice(ctx->device));
     HIP_TRY(hipStreamSynchronize(s->stream));
-    if (int rc = rb_enqueue_adjoint(ctx, s->rb, g, true, s->stream)) return rc;
+    if (int rc = rb_enqueue_adjoint(ctx, s->rb, g, s->stream)) return rc;
     HIP_TRY(hipStreamSynchronize(s->stream));
     rb_collect_adjoint(s->rb, grad, nargs);
     return PDA_OK;
@@ -708,7 +700,7 @@ int pda_rb_jacobian(pda_ctx* ctx, int sid, double* J, int nbins, int nargs) {
     if (int rc = check_derivative_run(s->rb, sid, nbins, nargs)) return rc;
     HIP_TRY(hipSetDevice(ctx->device));
     HIP_TRY(hipStreamSynchronize(s->stream));
-    if (int rc = rb_enqueue_jacobian(ctx, s->rb, true, s->stream)) return rc;
+    if (int rc = rb_enqueue_jacobian(ctx, s->rb, s->stream)) return rc;
     HIP_TRY(hipStreamSynchronize(s->stream));
     rb_collect_jacobian(s->rb, J, nbins, nargs);
     return PDA_OK;
@@ -751,7 +743,7 @@ int pda_rb_forward_population(pda_ctx* ctx, int sid, int R, uint32_t seed, uint3
     for (int k = 0; k < p.nsets && !rc; ++k) {
         RbState& r = s->rbpop[size_t(k)];
         rc = rb_enqueue_forward(ctx, *s, r, models[size_t(k)], r.d_model, r.d_model, R, seed,
-                                set_base + uint32_t(k) * set_stride, flags, false,
+                                set_base + uint32_t(k) * set_stride, flags,
                                 rb_set_stream(*s, k), nullptr);
         if (rc) rc = fail(rc, "set %d: %s", k, last_error().c_str());
     }
@@ -802,7 +794,7 @@ int pda_rb_adjoint_population(pda_ctx* ctx, int sid, const double* g, int nbins,
     if (int rc = rb_sets_fork(*s, K)) return rc;
     int rc = PDA_OK;
     for (int k = 0; k < K && !rc; ++k)
-        rc = rb_enqueue_adjoint(ctx, s->rbpop[size_t(k)], g + size_t(k) * size_t(nbins), false,
+        rc = rb_enqueue_adjoint(ctx, s->rbpop[size_t(k)], g + size_t(k) * size_t(nbins),
                                 rb_set_stream(*s, k));
     if (int rj = rb_sets_join(*s, K)) return rj;
     if (rc) return rc;
@@ -829,7 +821,7 @@ int pda_rb_jacobian_population(pda_ctx* ctx, int sid, const int32_t* which, doub
     int rc = PDA_OK;
     for (int k = 0; k < K && !rc; ++k)
         if (!which || which[k])
-            rc = rb_enqueue_jacobian(ctx, s->rbpop[size_t(k)], false, rb_set_stream(*s, k));
+            rc = rb_enqueue_jacobian(ctx, s->rbpop[size_t(k)], rb_set_stream(*s, k));
     if (int rj = rb_sets_join(*s, K)) return rj;
     if (rc) return rc;
     HIP_TRY(hipStreamSynchronize(s->stream));
@@ -848,12 +840,11 @@ int pda_rb_stats(pda_ctx* ctx, int sid, float* walk_ms, float* forward_ms, float
     if (!r.ran) return fail(PDA_E_STATE, "stream %d has no RB run", sid);
     HIP_TRY(hipSetDevice(ctx->device));
     HIP_TRY(hipStreamSynchronize(s->stream));
-    if (walk_ms) HIP_TRY(hipEventElapsedTime(walk_ms, r.ev0, r.ev_walk));
-    if (forward_ms) HIP_TRY(hipEventElapsedTime(forward_ms, r.ev0, r.ev1));
-    if (adjoint_ms) {
-        *adjoint_ms = 0.f;
-        if (r.adj_ran) HIP_TRY(hipEventElapsedTime(adjoint_ms, r.ev_a0, r.ev_a1));
-    }
+    const RunTimes& f = r.h_times[0];
+    const RunTimes& d = r.h_times[1];
+    if (walk_ms) *walk_ms = clock_ms(ctx, f.start, f.walked);
+    if (forward_ms) *forward_ms = clock_ms(ctx, f.start, f.end);
+    if (adjoint_ms) *adjoint_ms = r.adj_ran ? clock_ms(ctx, d.start, d.end) : 0.f;
     return PDA_OK;
 }
 

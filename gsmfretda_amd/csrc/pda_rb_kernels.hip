@@ -587,6 +587,7 @@ struct RbUnitArgs {
     int32_t copies;  // accumulator copies, a power of two
     int32_t tile;    // units a workgroup takes at a time
     int32_t pool;    // the pool's first floats are kept in LDS
+    RunTimes* times;  // forward: where the walk's end goes, or null
 };
 
 // rb_bin() for F in quotient_range and its reciprocal rF rounded to float; B
@@ -610,6 +611,7 @@ __global__ __launch_bounds__(rb_unit_threads_of(kMode)) void rb_unit_kernel(cons
     constexpr int kThreads = rb_unit_threads_of(kMode);
     extern __shared__ __align__(16) double s_acc[];
     const int tid = int(threadIdx.x), lane = tid % kWave;
+    if (kMode == kRbFwd && p.times && blockIdx.x == 0 && tid == 0) stamp(&p.times->walked);
     const int B = a.B;
     const int nacc = rb_unit_acc(B, kMode, kN) * p.copies;
     float* s_pool = reinterpret_cast<float*>(s_acc + nacc);
@@ -1094,9 +1096,11 @@ __global__ __launch_bounds__(256) void rb_score_mean_kernel(const RunArgs a, int
 __global__ __launch_bounds__(256) void rb_table_kernel(
     const RbModel R, const Model M, RbModel* __restrict__ rbm, Model* __restrict__ model,
     const double* __restrict__ lf, float* __restrict__ pmf_tab, uint32_t* __restrict__ work,
-    uint32_t* __restrict__ big_count, uint32_t* __restrict__ replay_count) {
+    uint32_t* __restrict__ big_count, uint32_t* __restrict__ replay_count,
+    RunTimes* __restrict__ times) {
     if (blockIdx.x == 0 && blockIdx.y == 0) {
         const uint32_t t = threadIdx.x;
+        if (times && t == 0u) stamp(&times->start);
         store_words(rbm, R, t, 256u);
         if (model) store_words(model, M, t, 256u);
         for (uint32_t i = t; i < kMaxQueues + kAuxQueues + 1u; i += 256u)
@@ -1120,8 +1124,10 @@ __global__ __launch_bounds__(256) void rb_table_kernel(
 __global__ __launch_bounds__(256) void rb_begin_kernel(double* __restrict__ rows, uint32_t n,
                                                        uint32_t* __restrict__ work,
                                                        const double* __restrict__ g_host,
-                                                       double* __restrict__ g, int B) {
+                                                       double* __restrict__ g, int B,
+                                                       RunTimes* __restrict__ times) {
     const uint32_t i = blockIdx.x * 256u + threadIdx.x;
+    if (times && i == 0u) stamp(&times->start);
     if (i < n) rows[i] = 0.0;
     if (i < kMaxQueues + kAuxQueues + 1u) work[i * kCounterStride] = 0u;
     if (g_host && i < uint32_t(B)) g[i] = g_host[i];
@@ -1132,8 +1138,10 @@ __global__ __launch_bounds__(256) void rb_begin_kernel(double* __restrict__ rows
 template <int kLanes>
 __global__ __launch_bounds__(256) void rb_rows_kernel(const double* __restrict__ rows_in, int n,
                                                       int rows, int stride,
-                                                      double* __restrict__ out) {
+                                                      double* __restrict__ out,
+                                                      RunTimes* __restrict__ times) {
     const int t = int(blockIdx.x * blockDim.x + threadIdx.x);
+    if (times && t == 0) stamp(&times->end);
     const int i = t / kLanes, l = t % kLanes;
     double v = 0.0;
     if (i < n)
@@ -1157,7 +1165,7 @@ struct RbResultHeader {
 // bin's term is zero.
 __global__ __launch_bounds__(kWave) void rb_finish_kernel(
     const RunArgs a, const float* __restrict__ obs, unsigned long long* __restrict__ hist_acc,
-    RbResultHeader* __restrict__ res) {
+    RbResultHeader* __restrict__ res, RunTimes* __restrict__ times) {
     const uint32_t lane = threadIdx.x;
     unsigned long long* M = reinterpret_cast<unsigned long long*>(res + 1);
     double c = 0.0;
@@ -1193,6 +1201,7 @@ __global__ __launch_bounds__(kWave) void rb_finish_kernel(
         res->chi2 = c / double(effN - a.nstates * (a.nstates + 1));
         res->effN = effN;
         res->B = a.B;
+        if (times) stamp(&times->end);
     }
 }
 
@@ -1275,19 +1284,19 @@ size_t rb_big_lds_bytes(int B, int cap, int mode, bool wide) { return rb_big_lds
 
 hipError_t launch_rb_table(const RbModel& R, const Model& M, RbModel* rbm, Model* model,
                            const double* lf, float* pmf_tab, uint32_t* work, uint32_t* big_count,
-                           uint32_t* replay_count, hipStream_t stream) {
+                           uint32_t* replay_count, RunTimes* times, hipStream_t stream) {
     hipLaunchKernelGGL(rb_table_kernel, dim3(uint32_t((kRbPmfStride + 255) / 256), uint32_t(R.n)),
                        dim3(256), 0, stream, R, M, rbm, model, lf, pmf_tab, work, big_count,
-                       replay_count);
+                       replay_count, times);
     return hipGetLastError();
 }
 
 hipError_t launch_rb_begin(double* rows, uint32_t n, uint32_t* work, const double* g_host,
-                           double* g, int B, hipStream_t stream) {
+                           double* g, int B, RunTimes* times, hipStream_t stream) {
     const uint32_t most = std::max<uint32_t>(std::max<uint32_t>(n, uint32_t(B)),
                                              kMaxQueues + kAuxQueues + 1u);
     hipLaunchKernelGGL(rb_begin_kernel, dim3((most + 255u) / 256u), dim3(256), 0, stream, rows, n,
-                       work, g_host, g, B);
+                       work, g_host, g, B, times);
     return hipGetLastError();
 }
 
@@ -1319,10 +1328,10 @@ hipError_t launch_rb_unit(int mode, int n, uint32_t grid, int copies, int tile, 
                           const double* Sbar, const double* g, const uint32_t* rank_offP,
                           const uint4* rank_offD, const float* poolP,
                           unsigned long long* hist_acc, double* grad, uint32_t* work,
-                          hipStream_t stream) {
+                          RunTimes* times, hipStream_t stream) {
     if (n < 2 || n > kRbMaxStates) return hipErrorInvalidValue;
     const RbUnitArgs p{cnt,      F,    S,    Sbar,   g,    rank_offP, rank_offD, poolP,
-                       hist_acc, grad, work, copies, tile, pool ? 1 : 0};
+                       hist_acc, grad, work, copies, tile, pool ? 1 : 0, times};
 #define PDA_RB_UNIT_M(M)                                       \
     if (n == 2) launch_rb_unit_n<M, 2>(grid, a, p, stream);    \
     else if (n == 3) launch_rb_unit_n<M, 3>(grid, a, p, stream); \
@@ -1383,20 +1392,21 @@ hipError_t launch_rb_score_mean(const RunArgs& a, int K, const float* S, double*
     return hipGetLastError();
 }
 
-hipError_t launch_rb_rows(const double* rows, int n, int nrows, double* out, hipStream_t stream) {
+hipError_t launch_rb_rows(const double* rows, int n, int nrows, double* out, RunTimes* times,
+                          hipStream_t stream) {
     if (nrows >= kWave)
         hipLaunchKernelGGL(rb_rows_kernel<kWave>, dim3(uint32_t((n * kWave + 255) / 256)),
-                           dim3(256), 0, stream, rows, n, nrows, n, out);
+                           dim3(256), 0, stream, rows, n, nrows, n, out, times);
     else
         hipLaunchKernelGGL(rb_rows_kernel<8>, dim3(uint32_t((n * 8 + 255) / 256)), dim3(256), 0,
-                           stream, rows, n, nrows, n, out);
+                           stream, rows, n, nrows, n, out, times);
     return hipGetLastError();
 }
 
 hipError_t launch_rb_finish(const RunArgs& a, const float* obs, unsigned long long* hist_acc,
-                            void* res, hipStream_t stream) {
+                            void* res, RunTimes* times, hipStream_t stream) {
     hipLaunchKernelGGL(rb_finish_kernel, dim3(1), dim3(kWave), 0, stream, a, obs, hist_acc,
-                       static_cast<RbResultHeader*>(res));
+                       static_cast<RbResultHeader*>(res), times);
     return hipGetLastError();
 }
 

@@ -162,6 +162,14 @@ struct ResultHeader {
     int32_t replays;     // units the fast pass abandoned to the replay pass
 };
 
+// GPU clock readings of a run, written to the host by the run's own kernels.
+// (Events recorded between the launches are packets of their own: 5,000 bursts
+// x 20 of 2 states took 52 us with three of them, 47 without.  Launches that
+// record the events themselves took 75.)
+struct RunTimes {
+    uint64_t start, walked, end;
+};
+
 // Population runs: random-stream keys of the sets, uploaded with the models
 // (set s draws with key {seed, set_base + s * set_stride}).
 struct PopControl {

@@ -340,6 +340,14 @@ struct WindowInfo {
     int32_t m;
 };
 
+#ifdef __HIPCC__
+// Writes the GPU's clock (hipDeviceAttributeWallClockRate) to *t, which may be
+// host memory, unless t is null; for one thread of a launch.
+__device__ __forceinline__ void stamp(uint64_t* t) {
+    if (t) *t = wall_clock64();
+}
+#endif
+
 // What a work counter hands out: of a single set's units a contiguous share,
 // of a population's batches (set 0's, set 1's, ...) every queues-th.
 struct QueueRange {

@@ -127,3 +127,35 @@ def test_bursts_started_by_duration(gpu_mc, oracle, bursts, R, spread):
             assert np.array_equal(np.asarray(x).view(np.uint32),
                                   np.concatenate([y, z]).view(np.uint32))
     m.set_burst_range(0, -1, 0)
+
+
+def test_run_times(gpu_mc):
+    """The runs' times from the kernels' clock readings: parts of the time the
+    calls took, that of another run for another run."""
+    import time
+    n = 3
+    rng = np.random.default_rng(3)
+    args = synth.make_args([0.2, 0.5, 0.8], synth.loguniform_rates(rng, 6, 3e2, 8e3))
+    d = synth.generate(2000, args, n, seed=8)
+    m = gpu_mc
+    m.load(d, SgDivSr=rng.uniform(0, 1, 2000).astype(np.float32), nbins=50, left_pad=2)
+    m.set_photophysics(0, *synth.PHOTOPHYSICS)
+    m.set_burst_range(0, -1, 0)
+    ms = {}
+    for R in (2, 2000):
+        t0 = time.perf_counter()
+        pda.evaluate(m, n, args, R, 9)
+        wall = (time.perf_counter() - t0) * 1e3
+        w, f = m.last_pass_ms(0)
+        assert 0 < w < wall and 0 < f < wall
+        assert abs(m.last_run_ms(0) - (w + f)) <= 1e-5 * wall
+        ms[R] = w
+    assert ms[2000] > ms[2]
+    t0 = time.perf_counter()
+    m.rb_forward(R=20, seed=1, set_id=0)
+    m.rb_result()
+    wall = (time.perf_counter() - t0) * 1e3
+    w, f, a = m.rb_stats()
+    assert 0 < w < f < wall and a == 0
+    m.rb_adjoint(np.ones(50), n)
+    assert m.rb_stats()[2] > 0
