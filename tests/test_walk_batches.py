@@ -101,7 +101,7 @@ def test_bursts_started_by_duration(gpu_mc, oracle, bursts, R, spread):
         d.T[::3] = 0.0
         d.T[1::7] = -1.0
     elif spread == "one long":
-        d.T[bursts // 2] = 3e4
+        d.T[bursts // 2] = 1.0
     m = gpu_mc
     m.load(d, SgDivSr=rng.uniform(0, 1, bursts).astype(np.float32), nbins=50, left_pad=0)
     m.set_photophysics(0, *synth.PHOTOPHYSICS)
