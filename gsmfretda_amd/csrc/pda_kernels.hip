@@ -119,14 +119,14 @@ __device__ __forceinline__ void flush_hist(int32_t* h, int32_t* __restrict__ row
 // keeps 8 waves on a SIMD: the window loop waits on dependent loads, which the
 // other waves hide (the 256-set generation 11.3 ms on the GPU with 7 and 10.6
 // with 8, 64 sets of fast dynamics 12.1 and 11.3).
-// A single set's bursts are started by falling duration within each queue's
-// share (burst_order in pda_layout.cpp), so that a run ends with units of few
-// windows and not with some lane's thirtieth: 50,000 bursts x 16 of 3 states
-// under a 30 kHz background 277 -> 231 us, 100,000 x 100 of 3 states 317 -> 310.
-// Sorted over all bursts, which takes the queues' photons apart, the latter
-// took 318 and a population 6 % more; populations, whose other sets fill the
-// end of each, and the RB walk, which writes per burst, start them as they
-// come.
+// A single set's bursts are started by falling duration within each quarter of
+// a queue's share (burst_order in pda_layout.cpp), so that a run ends with units
+// of few windows and not with some lane's thirtieth: 50,000 bursts x 50 of 3
+// states under a 30 kHz background 272 -> 223 us, 100,000 x 100 of 3 states
+// 315 -> 304.  With whole shares sorted those take 244 and 313, with all bursts
+// sorted and dealt out to the queues 248 and 318, and a population 6 % more;
+// populations, whose other sets fill the end of each, and the RB walk, which
+// writes per burst, start them as they come.
 // Units are started 64 at a time into LDS and taken from there one lane at a
 // time as lanes fall idle, and ended ones wait in LDS until 64 can be binned:
 // a start (a Philox block and the unit's division) and a tally (a division and

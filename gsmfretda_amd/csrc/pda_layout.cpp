@@ -208,13 +208,12 @@ int build_model(const Photophysics& s, int n, const float* args, int nargs, Mode
     return PDA_OK;
 }
 
-// A counting sort of each of kDefaultQueues parts.  A unit's windows grow with
-// its burst's duration: the walk starts the long ones first, and a run ends with
-// short ones.
+// A counting sort of each part.  A unit's windows grow with its burst's duration:
+// the walk starts a part's long ones first, and a run ends with short ones.
 void burst_order(const std::vector<BurstDesc>& bursts, std::vector<WalkBurst>& plain,
                  std::vector<WalkBurst>& order) {
     constexpr uint32_t kOrderBuckets = 256;
-    constexpr size_t kOrderParts = kDefaultQueues;
+    constexpr size_t kOrderParts = 4u * kDefaultQueues;
     float longest = 0.0f;
     for (const BurstDesc& d : bursts)
         if (d.T < INFINITY && d.T > longest) longest = d.T;
@@ -229,7 +228,8 @@ void burst_order(const std::vector<BurstDesc>& bursts, std::vector<WalkBurst>& p
     plain.resize(n);
     order.resize(n);
     for (size_t i = 0; i < n; ++i) plain[i] = WalkBurst{bursts[i], uint32_t(i), {0u, 0u, 0u}};
-    // each queue's share by itself: a share stays one region of the photon arrays
+    // a queue's share stays one region of the photon arrays, and has long and
+    // short bursts under way together
     const size_t part = std::max<size_t>((n + kOrderParts - 1) / kOrderParts, 1);
     for (size_t b0 = 0; b0 < n; b0 += part) {
         const size_t b1 = std::min(n, b0 + part);

@@ -49,8 +49,8 @@ int build_model(const Photophysics& ph, int n, const float* args, int nargs, Mod
                 std::string& err);
 
 // The bursts as a walk starts them: as they come, and by falling duration (in
-// 256 steps of the longest, a step's bursts in their order) within each of
-// kDefaultQueues equal parts.
+// 256 steps of the longest, a step's bursts in their order) within each of equal
+// parts, four to a default queue's share.
 void burst_order(const std::vector<BurstDesc>& bursts, std::vector<WalkBurst>& plain,
                  std::vector<WalkBurst>& order);
 // Tabulated inversion constants for the fast walk (needs M from build_model).
