@@ -113,12 +113,12 @@ def roofline(units, walk_ms):
     cm = cost_model.load()
     t = walk_ms * 1e-3
     traffic = cm["hbm_traffic_bytes_per_launch"]
-    valu = valu_roofline("plain_3state", units, walk_ms, "walk_kernel<0>", traffic)
+    valu = valu_roofline("plain_3state", units, walk_ms, "fast_walk_kernel", traffic)
     ops = cm["valu_lane_ops_per_unit"] * units
     achieved = ops / t / 1e12
     peak = cm["valu_peak_lane_ops_per_s"] / 1e12
     counter = {"bound": "valu", "achieved": achieved, "peak": peak, "unit": "TOP/s",
-               "frac": achieved / peak, "traffic": traffic, "kernel": "walk_kernel<0>",
+               "frac": achieved / peak, "traffic": traffic, "kernel": "fast_walk_kernel",
                "kernel_ms_avg": walk_ms, "ops_per_unit": cm["valu_lane_ops_per_unit"],
                "basis": "SQ_THREAD_CYCLES_VALU per unit of an earlier build, frozen"}
     hb = cm["hbm_algorithmic_bytes_per_unit"] * units / t / 1e9
@@ -207,7 +207,7 @@ def population_leg(pda, synth, steps, warmup):
                         "per generation",
             "value": units * steps / dt, "unit": "burst-resamples/s",
             "roofline": valu_roofline("population_256", units, g_ms,
-                                      "pop_walk_kernel<0> (whole generation)"),
+                                      "fast_walk_kernel of a population (whole generation)"),
             "roofline_counter": {"bound": "valu", "achieved": achieved, "peak": peak,
                                  "unit": "TOP/s", "frac": achieved / peak,
                                  "ops_per_unit": cm["population_valu_lane_ops_per_unit"],
@@ -331,7 +331,7 @@ def fast_population_leg(pda, cfg, steps):
             "units_per_generation": units, "ms_per_generation": dt / steps * 1e3,
             "gpu_ms_per_generation": g_ms, "replayed_units": st[1],
             "roofline": valu_roofline("fast_dynamics_population_64", units, g_ms,
-                                      "pop_walk_kernel<0> (whole generation)")}
+                                      "fast_walk_kernel of a population (whole generation)")}
 
 
 def fit_leg(pda, cfg, limits):
@@ -443,7 +443,7 @@ def main():
 
     m.reSampleTimes = R
     seed = cfg["seeds"]["mc"]
-    # kernel durations (HIP events): one evaluation at a time on stream 0
+    # kernel durations (their own clock readings): one evaluation at a time on stream 0
     for _ in range(args.warmup):
         m.run_kernel(sid=0, seed=seed, set_id=0)
     m.synchronize(0)

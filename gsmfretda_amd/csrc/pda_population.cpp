@@ -9,8 +9,8 @@
 //   H2D copy of the generation's model tables and stream keys
 //   -> fast_walk_kernel (persistent grid)
 //   -> pop_replay_kernel (abandoned units, general form)
-//   -> pop_finish_kernel (one workgroup per set: histogram and chi2)
-//   -> D2H copy of every set's histogram and chi2.
+//   -> pop_finish_kernel (one workgroup per set: histogram and chi2, into the
+//      host's result buffer).
 // No node of the graph is a memset: the kernels leave their accumulators and
 // counters zero for the next replay.
 #include <hip/hip_runtime.h>

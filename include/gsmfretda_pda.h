@@ -142,7 +142,8 @@ int pda_get_samples(pda_ctx *ctx, int sid, float *E, int32_t *acc, float *F, int
  * completed, NULL before. */
 float *pda_samples_host(pda_ctx *ctx, int sid);
 
-/* Milliseconds spent by the slot's last run on the GPU (HIP events). */
+/* Milliseconds spent by the slot's last run on the GPU (from the kernels' clock
+ * readings). */
 int pda_last_run_ms(pda_ctx *ctx, int sid, float *ms);
 /* The same split into the walk pass over every unit and the finishing pass
  * (replayed units, histogram reduction, chi2). */
