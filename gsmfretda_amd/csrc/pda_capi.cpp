@@ -218,7 +218,6 @@ int upload_model(Slot& s) {
         return rc;
     }
     s.any_v = M.any_v != 0;
-    s.quick_rates = M.quick_rates != 0;
     HIP_TRY(launch_model(M, s.d_model, s.d_thr, s.d_guide, s.stream));
     return PDA_OK;
 }
@@ -508,7 +507,7 @@ int pda_run(pda_ctx* ctx, int sid, int R, uint32_t seed, uint32_t set_id, int fl
     }
     a.replay_cap = uint32_t(s->replay_cap);
     const BinomGuide guide{s->d_thr, s->d_guide};
-    const FastArgs fa = fast_args(s->n, s->quick_rates, a.clk_p, s->ph.r0, ctx->max_P);
+    const FastArgs fa = fast_args(a.clk_p, ctx->max_P);
     HIP_TRY(launch_walk(pass, grid, ctx->d_bursts, run_order(ctx, b0, b1), ctx->d_ticks, ctx->d_links, s->d_model, guide, a,
                         fa, s->d_hist_acc, s->d_replay, s->d_replay_count, s->d_work, outE, outAcc,
                         outF, nullptr, nullptr, s->d_times, s->stream));

@@ -54,7 +54,7 @@ struct PopGraphKey {
     // the guide kernel's state count (also the walk's), the table's buffer,
     // and what else the walk takes from the sets
     int max_states = 0;
-    float r0 = 0.f;
+    float r0_r = 0.f;
     bool quick_rates = false;
     const void* thr = nullptr;
     bool operator==(const PopGraphKey& o) const;
@@ -67,7 +67,7 @@ struct Population {
     std::vector<int64_t> off;        // start of set s in args
     bool any_v = false;
     bool quick_rates = false;        // of every set
-    float r0 = 0.f;                  // photophysics the sets were built with
+    float r0_r = 0.f;                // of the photophysics the sets were built with
     size_t cap_sets = 0;             // allocated sets
     uint8_t* h_in = nullptr;         // pinned: PopControl + Model[cap_sets]
     uint8_t* d_in = nullptr;
@@ -175,7 +175,6 @@ struct RbState {
 };
 
 struct Slot {
-    bool quick_rates = false;     // every rate of the set is in quotient()'s range
     hipStream_t stream = nullptr;
     Model* d_model = nullptr;
     // threshold rows of the fast walk's binomial draws for the uploaded set

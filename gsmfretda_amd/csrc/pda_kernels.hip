@@ -169,7 +169,7 @@ struct FastIO {
 template <bool kPop, int kPass, bool kSamples>
 __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(
     fast_waves_per_eu(kPop, kPass)))) void fast_walk_kernel(const FastIO io, const RunArgs a,
-                                                            const FastArgs fa) {
+                                                            const FastArgs launch) {
     constexpr int kSlots = kPop ? 2 : 1;
     using Mod = typename std::conditional<
         kPass == kPassGuided, FastModel,
@@ -187,7 +187,15 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(
         for (uint32_t i = lane; i < sizeof(Mod) / 4; i += kWave) dst[i] = src[i];
         wave_lds_sync();
     };
-    if (!kPop) load_model(0u, 0u);
+    FastArgs fa = launch;
+    if constexpr (!kPop) {
+        load_model(0u, 0u);
+        float r0_r = 0.0f;
+        if constexpr (kPass == kPassBroad)
+            r0_r = bitsf(__builtin_amdgcn_readfirstlane(fbits(sM[0].r0_r)));
+        fa = fast_args_of(launch, __builtin_amdgcn_readfirstlane(sM[0].n),
+                          __builtin_amdgcn_readfirstlane(sM[0].quick_rates), r0_r);
+    }
 
     if (!kPop && io.times && blockIdx.x == 0 && lane == 0) stamp(&io.times->start);
 

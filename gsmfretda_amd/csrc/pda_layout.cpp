@@ -161,6 +161,7 @@ int build_model(const Photophysics& s, int n, const float* args, int nargs, Mode
     M.gmx = s.gamma - s.crosstalk;
     M.omdd = 1.0f - s.dexdir;
     M.r0 = s.r0;
+    M.r0_r = quotient_range(s.r0) ? 1.0f / s.r0 : 0.0f;
     M.quick_rates = 1;
     // P_i2j column s, without the diagonal, as running sums (drawJ_Si2Sj)
     for (int st = 0; st < n; ++st) {

@@ -140,7 +140,7 @@ extern "C" int pda_run_noalloc(pda_ctx* ctx, int sid, int R, uint32_t seed, uint
                        hist_acc);
     HIP_TRY(hipGetLastError());
     const BinomGuide guide{s->d_thr, s->d_guide};
-    const FastArgs fa = fast_args(s->n, s->quick_rates, a.clk_p, s->ph.r0, ctx->max_P);
+    const FastArgs fa = fast_args(a.clk_p, ctx->max_P);
     HIP_TRY(launch_walk(pass, L.grid, ctx->d_bursts, run_order(ctx, b0, b1), ctx->d_ticks, ctx->d_links, s->d_model, guide,
                         a, fa, hist_acc, replay, count, work, nullptr, nullptr, nullptr, nullptr,
                         nullptr, nullptr, s->stream));

@@ -33,7 +33,7 @@ bool PopGraphKey::operator==(const PopGraphKey& o) const {
            bg_on == o.bg_on && b0 == o.b0 && b1 == o.b1 && grid == o.grid && batch == o.batch &&
            queues == o.queues && replay_cap == o.replay_cap && clk_p == o.clk_p &&
            bg_ad == o.bg_ad && bg_dd == o.bg_dd && bursts == o.bursts && ticks == o.ticks &&
-           links == o.links && data_gen == o.data_gen && obs == o.obs && r0 == o.r0 &&
+           links == o.links && data_gen == o.data_gen && obs == o.obs && r0_r == o.r0_r &&
            max_states == o.max_states && quick_rates == o.quick_rates && thr == o.thr;
 }
 
@@ -148,8 +148,9 @@ int enqueue_population(pda_ctx* ctx, Slot& s, int pass, uint32_t grid, const Run
     }
     HIP_TRY(launch_pop_walk(pass, grid, ctx->d_bursts,
                             ctx->d_plain, ctx->d_ticks, ctx->d_links, ctl, models,
-                            p.d_tabs, guide, a, fast_args(p.max_states, p.quick_rates, a.clk_p, p.r0,
-                                             ctx->max_P),
+                            p.d_tabs, guide, a,
+                            fast_args_of(fast_args(a.clk_p, ctx->max_P), p.max_states,
+                                         p.quick_rates, p.r0_r),
                             p.d_hist_acc, p.d_replay, p.d_replay_count, p.d_work,
                             s.stream));
     if (pass != kPassGeneral)
@@ -256,7 +257,7 @@ int run_population(pda_ctx* ctx, Slot& s, int R, uint32_t seed, uint32_t set_bas
         k.obs = ctx->d_obs;
         k.max_states = p.max_states;
         k.quick_rates = p.quick_rates;
-        k.r0 = p.r0;
+        k.r0_r = p.r0_r;
         k.thr = p.d_thr;
         if (!p.exec || !(k == p.key)) {
             drop_graph(p);
@@ -395,7 +396,7 @@ int pda_set_population(pda_ctx* ctx, int sid, int nsets, const int32_t* nstates,
     p.off = off;
     p.any_v = any_v;
     p.quick_rates = quick_rates;
-    p.r0 = s->ph.r0;
+    p.r0_r = models[0].r0_r;
     return PDA_OK;
 }
 

@@ -457,7 +457,8 @@ int rb_enqueue_forward(pda_ctx* ctx, Slot& s, RbState& r, const Model& M,
     if (aux) HIP_TRY(hipEventRecord(s.rb_join, aux));
     HIP_TRY(launch_rb_walk(scores, n, L.grid, uint32_t(ctx->num_cu) * 4u, ctx->d_bursts,
                            ctx->d_plain, ctx->d_ticks, ctx->d_links, d_model, d_rbm, a,
-                           fast_args(n, M.quick_rates != 0, a.clk_p, M.r0, ctx->max_P), r.d_cnt, r.d_F, r.d_S, r.d_work,
+                           fast_args_of(fast_args(a.clk_p, ctx->max_P), n, M.quick_rates, M.r0_r),
+                           r.d_cnt, r.d_F, r.d_S, r.d_work,
                            r.d_big, r.d_huge, r.d_big_count, r.d_replay, r.d_replay_count,
                            stream));
     if (aux) HIP_TRY(hipStreamWaitEvent(stream, s.rb_join, 0));

@@ -90,6 +90,7 @@ struct BroadModel : FastModel {
     float v[kMaxStates];
     float base[kMaxStates];                       // r0 (1/E - 1)^(1/6)
     float ep0[kMaxStates];                        // broadened E when v == 0
+    float r0_r;   // 1 / r0 rounded to float, 0 when r0 is out of quotient()'s range
 };
 struct Model : BroadModel {
     float krate[kMaxStates][kMaxStates];          // [s][j] = K(j, s), rate s -> j

@@ -495,18 +495,27 @@ PDA_HD int general_window(const Model& M, const UnitKey& key, uint32_t P, uint32
 // range; clk_r: 1 / clk_p rounded to float; r0_r: 1 / r0, or 0 when r0 is
 // out of that range; top: the largest power of two up to the photons of the
 // longest burst, the first step of the window ends' search.
+//
+// fast_args gives what follows from the resident bursts; the rest follows from
+// the sets' models (fast_args_of).  A single set's launch takes it from the
+// device's model when it runs: recorded into a graph it may be replayed after
+// the slot's parameters or photophysics changed.
 struct FastArgs {
     int32_t jumps;
     int32_t quick;
     float clk_r, r0_r;
     uint32_t top;
 };
-PDA_HD FastArgs fast_args(int max_states, bool quick_rates, float clk_p, float r0,
-                          uint32_t max_photons) {
+PDA_HD FastArgs fast_args(float clk_p, uint32_t max_photons) {
     uint32_t top = 1;
     while (top <= max_photons / 2u) top *= 2u;
-    return FastArgs{max_states - 2, quick_rates && quotient_range(clk_p) ? 1 : 0, 1.0f / clk_p,
-                    quotient_range(r0) ? 1.0f / r0 : 0.0f, top};
+    return FastArgs{kMaxStates - 2, quotient_range(clk_p) ? 1 : 0, 1.0f / clk_p, 0.0f, top};
+}
+PDA_HD FastArgs fast_args_of(FastArgs fa, int max_states, int quick_rates, float r0_r) {
+    fa.jumps = max_states - 2;
+    fa.quick = quick_rates ? fa.quick : 0;
+    fa.r0_r = r0_r;
+    return fa;
 }
 
 // window_close() by steps of decreasing powers of two, the same for every
@@ -645,7 +654,7 @@ PDA_HD WalkOut walk_unit(const Model& M, const typename NoDeduce<Tab>::type* tab
     WalkState<kFast> st;
     int r = begin_unit<kFast>(M, key, P, T, st);
     if constexpr (kFast) {
-        const FastArgs fa = fast_args(M.n, M.quick_rates != 0, a.clk_p, M.r0, P);
+        const FastArgs fa = fast_args_of(fast_args(a.clk_p, P), M.n, M.quick_rates, M.r0_r);
         while (r == kStepMore)
             r = fast_window<false, Tab>(M, tab, key, P, stop_rel, T, tick, link, a, fa, st);
     } else {
