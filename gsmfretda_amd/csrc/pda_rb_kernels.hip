@@ -749,7 +749,9 @@ __global__ __launch_bounds__(rb_unit_threads_of(kMode)) void rb_unit_kernel(cons
                         } else if constexpr (kMode == kRbGrad) {
                             // sum_c P_s(c) (G(bin(c + 1)) - G(bin(c))), c = q - 1
                             const double G = s_acc[b];
-                            const double dG = act ? double(float(G - G_last)) : 0.0;
+                            // (no difference before the first outcome: G alone
+                            // may be beyond float)
+                            const double dG = act && q > 0 ? double(float(G - G_last)) : 0.0;
                             h += G * double(act ? P : 0.0f);
                             G_last = G;
 #pragma unroll
