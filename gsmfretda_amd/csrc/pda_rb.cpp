@@ -509,6 +509,12 @@ int pda_rb_forward(pda_ctx* ctx, int sid, int R, uint32_t seed, uint32_t set_id,
     if (s->any_v)
         return fail(PDA_E_ARG, "the RB form needs v = 0 (no distance broadening) in every state");
     HIP_TRY(hipSetDevice(ctx->device));
+    // Recorded into a graph, the run's own tables would be the recorded set's
+    // and the walk's model whatever the slot holds at a replay.
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    HIP_TRY(hipStreamIsCapturing(s->stream, &capture));
+    if (capture != hipStreamCaptureStatusNone)
+        return fail(PDA_E_STATE, "the RB form cannot be recorded into a graph");
     Model M;
     {
         std::string err;

@@ -1,9 +1,12 @@
 """GPU: the RB adjoint where no unit has an acceptor outcome past 0, with a
-cotangent beyond float's range."""
+cotangent beyond float's range, and the RB forward on a stream that is being
+recorded."""
+import ctypes
+
 import numpy as np
 import pytest
 
-from gsmfretda_amd import synth
+from gsmfretda_amd import pda, synth
 
 pytestmark = pytest.mark.gpu
 
@@ -33,3 +36,25 @@ def test_adjoint_of_a_cotangent_beyond_float(gpu_mc):
     m.set_photophysics(0, *synth.PHOTOPHYSICS)
     assert np.array_equal(one[:2], [0.0, 0.0]) and np.array_equal(grad[:2], [0.0, 0.0])
     assert np.isfinite(grad).all()
+
+
+def test_forward_on_a_recording_stream(gpu_mc):
+    """Refused, as the other RB calls are: a replay would pair the recorded
+    set's tables with whatever model the slot holds by then."""
+    m = gpu_mc
+    _load(m, synth.PHOTOPHYSICS, 5)
+    m.rb_forward(R=6, seed=2, set_id=1)
+    want = m.rb_result()
+    hip = ctypes.CDLL("libamdhip64.so.7")
+    stream, graph = ctypes.c_void_p(m.getStreams()[0]), ctypes.c_void_p()
+    assert hip.hipStreamBeginCapture(stream, 1) == 0
+    try:
+        with pytest.raises(pda.PdaError):
+            m.rb_forward(R=6, seed=2, set_id=1)
+    finally:
+        hip.hipStreamEndCapture(stream, ctypes.byref(graph))
+        if graph:
+            hip.hipGraphDestroy(graph)
+    m.rb_forward(R=6, seed=2, set_id=1)
+    got = m.rb_result()
+    assert np.array_equal(got[1], want[1]) and got[2] == want[2]
