@@ -90,7 +90,6 @@ struct BroadModel : FastModel {
     float v[kMaxStates];
     float base[kMaxStates];                       // r0 (1/E - 1)^(1/6)
     float ep0[kMaxStates];                        // broadened E when v == 0
-    float r0_r;   // 1 / r0 rounded to float, 0 when r0 is out of quotient()'s range
 };
 struct Model : BroadModel {
     float krate[kMaxStates][kMaxStates];          // [s][j] = K(j, s), rate s -> j
@@ -99,6 +98,8 @@ struct Model : BroadModel {
     double pp[kMaxStates];
     double qq[kMaxStates];
     double lq[kMaxStates];                        // log q
+    float r0_r;  // 1 / r0 rounded to float, 0 when r0 is out of quotient()'s range
+    float pad;
 };
 
 // q^m and the inversion bound min(m, mp + 10 sqrt(mpq + 1)) per state and
