@@ -98,6 +98,13 @@ void size_grid(Launch& L, uint64_t max_grid, uint64_t units, uint32_t queues) {
     L.grid = uint32_t(std::min(max_grid, std::max<uint64_t>(share, 1) * L.queues));
 }
 
+int broad_pass(const pda_ctx* ctx, const Photophysics& ph, int64_t b0, int64_t b1, bool population) {
+    return draws_in_place(ctx->runs, ctx->nbursts, ctx->nphotons, b1 - b0, ph,
+                          !(ctx->bg_dd < 1e-4f), population)
+               ? kPassBroadAll
+               : kPassBroad;
+}
+
 uint32_t replay_grid(const pda_ctx* ctx, uint64_t units) {
     int per_cu = 0;
     if (walk_occupancy(kPassReplay, ctx->B, &per_cu) != hipSuccess || per_cu < 1) per_cu = 1;
@@ -151,9 +158,10 @@ int load_common(pda_ctx* ctx, const int64_t* start, const int64_t* stop, const i
     std::vector<BurstDesc> bursts;
     std::vector<uint32_t> ticks;
     std::vector<uint2> links;
+    LongRuns runs;
     std::string err;
     int code = encode_bursts(start, stop, istart, phcount, nbursts, src, nphotons, T, clk_p, bg_ad,
-                             bg_dd, bursts, ticks, links, err);
+                             bg_dd, bursts, ticks, links, err, &runs);
     if (code) {
         set_error(err);
         return code;
@@ -193,6 +201,7 @@ int load_common(pda_ctx* ctx, const int64_t* start, const int64_t* stop, const i
         ctx->h_P[size_t(i)] = bursts[size_t(i)].P;
         ctx->max_P = std::max(ctx->max_P, bursts[size_t(i)].P);
     }
+    ctx->runs = std::move(runs);
     ctx->clk_p = clk_p;
     ctx->bg_ad = bg_ad;
     ctx->bg_dd = bg_dd;
@@ -462,7 +471,7 @@ int pda_run(pda_ctx* ctx, int sid, int R, uint32_t seed, uint32_t set_id, int fl
     a.bg_dd = ctx->bg_dd;
     a.nstates = s->n;
     // the fast form, then the general form over the units it abandoned
-    const int pass = s->any_v ? kPassBroad : kPassGuided;
+    const int pass = s->any_v ? broad_pass(ctx, s->ph, b0, b1, false) : kPassGuided;
     const Launch L = plan_launch(ctx, pass, false, uint64_t(nunits));
     const uint32_t grid = L.grid;
     a.batch = L.batch;

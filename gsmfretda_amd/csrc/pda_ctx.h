@@ -67,7 +67,8 @@ struct Population {
     std::vector<int64_t> off;        // start of set s in args
     bool any_v = false;
     bool quick_rates = false;        // of every set
-    float r0_r = 0.f;                // of the photophysics the sets were built with
+    Photophysics ph;                 // that the sets were built with
+    float r0_r = 0.f;                // of it
     size_t cap_sets = 0;             // allocated sets
     uint8_t* h_in = nullptr;         // pinned: PopControl + Model[cap_sets]
     uint8_t* d_in = nullptr;
@@ -255,6 +256,7 @@ struct pda_ctx {
     pda::LaunchShape shape;
     std::vector<uint32_t> h_P;      // photons per burst (host copy)
     uint32_t max_P = 0;             // the most photons of a burst
+    pda::LongRuns runs;             // what broad_pass goes by
     double* d_lf = nullptr;         // log k! for the RB form
     size_t lds_per_block = 65536;   // LDS a workgroup may allocate
     pda::RbMemoLayout rb_memo[5];   // by state count (2..4 used)
@@ -284,6 +286,8 @@ Launch plan_launch(const pda_ctx* ctx, int pass, bool population, uint64_t units
 // to a second turn: a run of 20,000 bursts x 4 of 3 broadened states walked
 // for 41 us, 33 now.
 void size_grid(Launch& L, uint64_t max_grid, uint64_t units, uint32_t queues);
+// The walk of models with broadening over [b0, b1): kPassBroad or kPassBroadAll.
+int broad_pass(const pda_ctx* ctx, const Photophysics& ph, int64_t b0, int64_t b1, bool population);
 // Workgroups of the replay pass of a run of `units` units.
 uint32_t replay_grid(const pda_ctx* ctx, uint64_t units);
 // The fields of a walk's arguments that follow from the others: R's

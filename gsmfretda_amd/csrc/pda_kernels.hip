@@ -105,7 +105,7 @@ __device__ __forceinline__ void flush_hist(int32_t* h, int32_t* __restrict__ row
 // change sets.
 //
 // kPop: population (two LDS model slots with a histogram each); kPass: the
-// acceptor draw (kPassGuided, kPassTable, kPassBroad); kSamples: per-unit
+// acceptor draw (kPassGuided, kPassTable, kPassBroad, kPassBroadAll); kSamples: per-unit
 // outputs.
 //
 // Bound by VALU issue (at or above 95 % of the cycles), so what counts is the
@@ -144,8 +144,20 @@ __device__ __forceinline__ void flush_hist(int32_t* h, int32_t* __restrict__ row
 // form's, at 186 registers and two waves per SIMD with logarithms,
 // exponentials and divisions in double per window: 50,000 bursts x 50 of a 3-state model 371 -> 197 us, 64 sets x
 // 20,000 x 16 2.74 -> 1.41 ms.
+//
+// kPassBroadAll: counts beyond the table and background means above 64 are
+// drawn in the window.  A broadened unit had not been abandoned for them before
+// it had a fast form; with each of them listed by one atomic and walked again
+// (populations: the whole run again once the list was full), 64 sets of 8,000
+// bursts x 64 at efficiencies near 0.99, 17 % of their units abandoned, took
+// 8.5 ms where the general form had taken 3.5, and under a 60 kHz background
+// 17.0 against 8.3; with the draws in place 1.9 and 2.1.  The draws spill up to
+// 300 bytes where they are made; with 6 waves the 64 sets below take 1.06 ms,
+// with 5 1.09, 4 1.23 and 3 1.44, against kPassBroad's 0.95: which of the two
+// a run takes is decided by its bursts (draws_in_place in pda_layout.cpp).
+constexpr bool is_broad(int pass) { return pass == kPassBroad || pass == kPassBroadAll; }
 constexpr int fast_waves_per_eu(bool pop, int pass) {
-    return pass != kPassBroad ? 8 : pop ? 7 : 6;
+    return !is_broad(pass) ? 8 : pop && pass == kPassBroad ? 7 : 6;
 }
 
 struct FastIO {
@@ -173,7 +185,7 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(
     constexpr int kSlots = kPop ? 2 : 1;
     using Mod = typename std::conditional<
         kPass == kPassGuided, FastModel,
-        typename std::conditional<kPass == kPassBroad, BroadModel, Model>::type>::type;
+        typename std::conditional<is_broad(kPass), BroadModel, Model>::type>::type;
     __shared__ Mod sM[kSlots];
     __shared__ StartedUnit s_start[kWave];    // units started and not yet taken
     __shared__ uint8_t s_state[kWave];        // their first states
@@ -321,10 +333,11 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(
             const uint32_t* ticks = io.ticks + d.off;
             const uint2* links = io.links + d.off;
             int r;
-            if constexpr (kPass == kPassBroad) {
-                const BroadDraw draw{};
-                r = fast_window<false, BroadDraw>(M, &draw, key, d.P, d.stop_rel, d.T, ticks,
-                                                  links, a, fa, st);
+            if constexpr (is_broad(kPass)) {
+                using Draw = typename std::conditional<kPass == kPassBroad, BroadDraw, BroadAll>::type;
+                const Draw draw{};
+                r = fast_window<false, Draw>(M, &draw, key, d.P, d.stop_rel, d.T, ticks, links, a,
+                                             fa, st);
             } else if constexpr (kPass == kPassGuided) {
                 r = fast_window<false, BinomGuide>(M, &io.guide, key, d.P, d.stop_rel, d.T, ticks,
                                                    links, a, fa, st);
@@ -1095,6 +1108,9 @@ hipError_t walk_occupancy(int pass, int B, int* blocks_per_cu) {
     if (pass == kPassBroad)
         return hipOccupancyMaxActiveBlocksPerMultiprocessor(
             blocks_per_cu, fast_walk_kernel<false, kPassBroad, false>, kWave, lds);
+    if (pass == kPassBroadAll)
+        return hipOccupancyMaxActiveBlocksPerMultiprocessor(
+            blocks_per_cu, fast_walk_kernel<false, kPassBroadAll, false>, kWave, lds);
     return hipOccupancyMaxActiveBlocksPerMultiprocessor(
         blocks_per_cu, fast_walk_kernel<false, kPassGuided, false>, kWave, lds);
 }
@@ -1120,6 +1136,10 @@ hipError_t launch_walk(int pass, uint32_t grid, const BurstDesc* bursts, const W
         hipLaunchKernelGGL(walk_kernel, dim3(grid), dim3(kWave), lds, stream, bursts, ticks, links,
                            model, a, hist_acc, replay, replay_count, work, outE, outAcc, outF, obs,
                            result, times);
+    else if (pass == kPassBroadAll && outE)
+        launch_fast<false, kPassBroadAll, true>(grid, lds, io, a, fa, stream);
+    else if (pass == kPassBroadAll)
+        launch_fast<false, kPassBroadAll, false>(grid, lds, io, a, fa, stream);
     else if (pass == kPassBroad && outE)
         launch_fast<false, kPassBroad, true>(grid, lds, io, a, fa, stream);
     else if (pass == kPassBroad)
@@ -1153,6 +1173,9 @@ hipError_t pop_walk_occupancy(int pass, int B, int* blocks_per_cu) {
     if (pass == kPassBroad)
         return hipOccupancyMaxActiveBlocksPerMultiprocessor(
             blocks_per_cu, fast_walk_kernel<true, kPassBroad, false>, kWave, lds);
+    if (pass == kPassBroadAll)
+        return hipOccupancyMaxActiveBlocksPerMultiprocessor(
+            blocks_per_cu, fast_walk_kernel<true, kPassBroadAll, false>, kWave, lds);
     return hipOccupancyMaxActiveBlocksPerMultiprocessor(
         blocks_per_cu, fast_walk_kernel<true, kPassGuided, false>, kWave, lds);
 }
@@ -1171,6 +1194,8 @@ hipError_t launch_pop_walk(int pass, uint32_t grid, const BurstDesc* bursts,
                            links, ctl, models, a, hist_acc, work);
     else if (pass == kPassBroad)
         launch_fast<true, kPassBroad, false>(grid, lds, io, a, fa, stream);
+    else if (pass == kPassBroadAll)
+        launch_fast<true, kPassBroadAll, false>(grid, lds, io, a, fa, stream);
     else if (pass == kPassTable)
         launch_fast<true, kPassTable, false>(grid, lds, io, a, fa, stream);
     else

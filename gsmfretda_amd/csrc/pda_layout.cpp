@@ -26,13 +26,26 @@ int fail_to(std::string& err, int code, const char* fmt, ...) {
 
 #define fail(code, ...) fail_to(err, code, __VA_ARGS__)
 
+// The runs a burst's photons start, its links at lk.
+static void add_runs(const BurstDesc& d, const uint2* lk, LongRuns& out) {
+    for (uint32_t i = 0; i < d.P; i += LongRuns::kEvery) {
+        ++out.starts;
+        const uint32_t f = lk[i].x & kIndexMask, colour = lk[i].x >> 30;
+        if (f >= d.P || colour == 3u) continue;  // (one in both channels counts nothing)
+        std::vector<uint64_t>& h = out.at_least[colour - 1u];
+        const uint32_t run = std::min(lk[i].y - f, LongRuns::kMaxRun);
+        if (h.size() <= run) h.resize(size_t(run) + 1u, 0u);
+        ++h[run];
+    }
+}
+
 // Re-encodes the reference's burst arrays (src/loadHdf5.cpp:101-128) into the
 // resident layout of pda_types.h.
 int encode_bursts(const int64_t* start, const int64_t* stop, const int64_t* istart,
                   const int32_t* phcount, int64_t nbursts, const PhotonSrc& src, int64_t nphotons,
                   const float* T, float clk_p, float bg_ad, float bg_dd,
                   std::vector<BurstDesc>& bursts, std::vector<uint32_t>& ticks,
-                  std::vector<uint2>& links, std::string& err) {
+                  std::vector<uint2>& links, std::string& err, LongRuns* runs) {
     if (nbursts < 0 || nbursts > int64_t(0x7FFFFFFF))
         return fail(PDA_E_ARG, "nbursts %lld out of range", (long long)nbursts);
     if (nphotons < 0) return fail(PDA_E_ARG, "nphotons < 0");
@@ -127,6 +140,14 @@ int encode_bursts(const int64_t* start, const int64_t* stop, const int64_t* ista
                 lk[ii].y = P;
             }
         }
+        if (runs) add_runs(d, lk, *runs);
+    }
+    if (runs) {
+        const float bg = std::max(bg_ad, bg_dd);
+        for (const BurstDesc& d : bursts)
+            runs->long_bursts += std::max(d.T, float(d.stop_rel) * clk_p) * bg > 64.0f;
+        for (std::vector<uint64_t>& h : runs->at_least)
+            for (size_t k = h.size(); k-- > 1;) h[k - 1] += h[k];
     }
     return PDA_OK;
 }
@@ -207,6 +228,38 @@ int build_model(const Photophysics& s, int n, const float* args, int nargs, Mode
         M.lq[i] = dlog(M.qq[i]);
     }
     return PDA_OK;
+}
+
+// What share of the units kPassBroad would abandon, at most: for a count, a
+// unit's windows that start in a long run, of which a burst of P photons has
+// P / kBinomTable at most with that many; for the background mean, the units of
+// long bursts.  Taken over all bursts and held against the range's part of
+// them, so that a part that holds them all is seen too.
+//
+// kPassBroad is the faster one while hardly any unit is abandoned (64 sets of
+// 8,000 bursts x 64 without any: 0.91 ms, kPassBroadAll 1.05), and each one costs
+// it: with 0.6 % of the units abandoned 1.09 against 1.19, 1.2 % 1.23 and 1.32,
+// 1.9 % 3.9 and 3.1; a single set, whose replay no other work hides, 0.138 and
+// 0.127 at 0.6 %; under backgrounds 0.2 % (1.1 % of the bursts long) 1.74 and
+// 1.79, 2 % (6.5 %) 2.5 and 1.9.  From a sixteenth on a population's list is
+// full.
+bool draws_in_place(const LongRuns& r, int64_t nbursts, int64_t nphotons, int64_t range,
+                    const Photophysics& ph, bool bg_on, bool population) {
+    if (bg_on && r.long_bursts * 64 > range) return true;
+    const float coef[2] = {ph.gamma - ph.crosstalk, 1.0f - ph.dexdir};
+    uint64_t starts = 0;
+    for (int c = 0; c < 2; ++c) {
+        // the fewest photons whose corrected count rounds to kBinomTable
+        const double k = std::ceil((kBinomTable - 0.5) / double(coef[c]));
+        const std::vector<uint64_t>& h = r.at_least[c];
+        const double most = double(LongRuns::kMaxRun);
+        const size_t at = size_t(k < most ? k : most);  // (coef 0: k is infinite)
+        if (coef[c] > 0.0f && at < h.size()) starts += h[at];
+    }
+    if (starts == 0) return false;
+    const double windows = std::max(1.0, double(nphotons) / (double(nbursts) * kBinomTable));
+    return double(starts) / double(r.starts) * windows * double(nbursts) >
+           double(range) / (population ? 32.0 : 64.0);
 }
 
 // A counting sort of each part.  A unit's windows grow with its burst's duration:

@@ -130,7 +130,7 @@ extern "C" int pda_run_noalloc(pda_ctx* ctx, int sid, int R, uint32_t seed, uint
     a.nstates = s->n;
     a.replay_cap = uint32_t(kReplayCapacity);
     a.nsets = 1;
-    const int pass = s->any_v ? kPassBroad : kPassGuided;
+    const int pass = s->any_v ? broad_pass(ctx, s->ph, b0, b1, false) : kPassGuided;
     const Launch L = plan_launch(ctx, pass, false, uint64_t(nunits));
     a.batch = L.batch;
     a.queues = L.queues;

@@ -180,7 +180,7 @@ int run_population(pda_ctx* ctx, Slot& s, int R, uint32_t seed, uint32_t set_bas
     int rc = ensure_pop_buffers(ctx, s, ctx->B);
     if (rc) return rc;
     const int pass = force_general ? kPassGeneral
-                     : p.any_v     ? kPassBroad
+                     : p.any_v     ? broad_pass(ctx, p.ph, b0, b1, true)
                      : p.guided    ? kPassGuided
                                    : kPassTable;
     Launch L = plan_launch(ctx, pass, true, uint64_t(total));
@@ -397,6 +397,7 @@ int pda_set_population(pda_ctx* ctx, int sid, int nsets, const int32_t* nstates,
     p.any_v = any_v;
     p.quick_rates = quick_rates;
     p.r0_r = models[0].r0_r;
+    p.ph = s->ph;
     return PDA_OK;
 }
 
@@ -500,7 +501,12 @@ int pda_autotune(pda_ctx* ctx, int sid, int population, int R, int reps, int* ba
     int rc = sync_all(ctx);
     if (rc) return rc;
     int per_cu = 0;
-    const int pass = (population ? s->pop.any_v : s->any_v) ? kPassBroad : kPassGuided;
+    int64_t b0, b1;
+    range_of(ctx, *s, &b0, &b1);
+    const int pass = !(population ? s->pop.any_v : s->any_v)
+                         ? kPassGuided
+                         : broad_pass(ctx, population ? s->pop.ph : s->ph, b0, b1,
+                                      population != 0);
     HIP_TRY(population ? pop_walk_occupancy(pass, ctx->B, &per_cu) : walk_occupancy(pass, ctx->B, &per_cu));
     if (per_cu < 1) per_cu = 1;
     const LaunchShape saved = ctx->shape;

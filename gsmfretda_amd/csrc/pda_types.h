@@ -23,8 +23,9 @@ constexpr size_t kWorkWords = size_t(kMaxQueues + kAuxQueues + 1u) * kCounterStr
 // How a walk launch runs: the fast form with the acceptor draws of models
 // without distance broadening from threshold rows (kPassGuided) or by the
 // inversion loop (kPassTable: populations whose rows would take too much
-// memory), or of models with broadening (kPassBroad); the general form over
-// the units that a fast form abandoned (kPassReplay), or over every unit of a
+// memory), or of models with broadening (kPassBroad; kPassBroadAll where the
+// bursts would have it abandon units in numbers); the general form over the
+// units that a fast form abandoned (kPassReplay), or over every unit of a
 // population (kPassGeneral: its replay list overflowed).
 enum WalkPass : int {
     kPassGuided = 0,
@@ -32,6 +33,7 @@ enum WalkPass : int {
     kPassBroad = 2,
     kPassReplay = 3,
     kPassGeneral = 4,
+    kPassBroadAll = 5,
 };
 
 // One burst, original order (the range [begin, end) of mc::setBurstBd

@@ -542,18 +542,23 @@ PDA_HD uint32_t step_close(const uint32_t* tick, const uint2* link, uint32_t c, 
 }
 
 // Tab of fast_window for models with distance broadening: the efficiency is
-// drawn per window, so there is no table of its binomials.
+// drawn per window, so there is no table of its binomials.  BroadAll: counts
+// beyond the table and background means above 64 are drawn in place instead of
+// abandoning the unit.
 struct BroadDraw {};
+struct BroadAll {};
 
 // The same window in the fast form, the same values from fewer operations;
 // kStepReplay where the window needs the general form.  Tab: BinomGuide
 // (thresholds) or BinomTable (inversion loop) for the acceptor draw of a
-// model without distance broadening, BroadDraw for one with.
+// model without distance broadening, BroadDraw or BroadAll for one with.
 template <bool kCounts = false, class Tab = BinomTable, class Mod = Model>
 PDA_HD int fast_window(const Mod& M, const typename NoDeduce<Tab>::type* tab, const UnitKey& key,
                        uint32_t P, uint32_t stop_rel, float T, const uint32_t* tick,
                        const uint2* link, const RunArgs& a, const FastArgs& fa,
                        WalkState<true>& st, WindowInfo* wi = nullptr) {
+    constexpr bool kAll = std::is_same<Tab, BroadAll>::value;
+    constexpr bool kBroad = kAll || std::is_same<Tab, BroadDraw>::value;
     const int s = st.s;
     const uint32_t w = st.w;
     const uint32_t last = P - 1u;
@@ -592,7 +597,7 @@ PDA_HD int fast_window(const Mod& M, const typename NoDeduce<Tab>::type* tab, co
         // 0 whatever its uniforms are (k = 0, or past the cap with
         // floor(0 u) = 0): only the other is made, on its channel's rate and
         // words (the window leaves the fast form when either mean is above
-        // 64).  One exponential and one inversion loop per window instead of
+        // 64, unless kAll).  One exponential and one inversion loop per window instead of
         // two, whose lanes had each waited for the other channel's (with two
         // draws a 3-state evaluation of 100,000 bursts x 100 took 434 us and
         // the 256-set generation 19.9 ms, with one 417 us and 19.1 ms; under
@@ -600,10 +605,17 @@ PDA_HD int fast_window(const Mod& M, const typename NoDeduce<Tab>::type* tab, co
         // then, exactly.
         const Block Bk = draw_block(key, w, kSubBackground);
         const float dt = float(int32_t(w1 - st.w0)) * a.clk_p;
-        bad = bad || dt * fmaxf(a.bg_ad, a.bg_dd) > 64.0f || !(fv < 0x1p30f);
-        const float lam = fminf(dt * (donor ? a.bg_dd : a.bg_ad), 64.0f);
-        m = fv - background_capped(lam, bad ? 0.0f : fv, uniform24(donor ? Bk.w[1] : Bk.w[0]),
-                                   uniform24(donor ? Bk.w[3] : Bk.w[2]));
+        const bool many = dt * fmaxf(a.bg_ad, a.bg_dd) > 64.0f || !(fv < 0x1p30f);
+        const float lam = dt * (donor ? a.bg_dd : a.bg_ad);
+        const float u_first = uniform24(donor ? Bk.w[1] : Bk.w[0]);
+        const float u_cap = uniform24(donor ? Bk.w[3] : Bk.w[2]);
+        if (kAll && many && !bad) {
+            m = fv - background_count(lam, fv, u_first, u_cap, key, w,
+                                      donor ? kSubPoissonD : kSubPoissonA);
+        } else {
+            bad = bad || many;
+            m = fv - background_capped(fminf(lam, 64.0f), bad ? 0.0f : fv, u_first, u_cap);
+        }
     }
     m = floorf(m + 0.5f);
     if (kCounts) {
@@ -611,7 +623,7 @@ PDA_HD int fast_window(const Mod& M, const typename NoDeduce<Tab>::type* tab, co
     } else {
         const int n = int(m);
         int x = 0;
-        if constexpr (std::is_same<Tab, BroadDraw>::value) {
+        if constexpr (kBroad) {
             // broadened efficiency (drawE, src/gen_rand.cuh:63-68)
             float de = M.ep0[s];
             if (M.v[s] != 0.0f) {
@@ -620,7 +632,10 @@ PDA_HD int fast_window(const Mod& M, const typename NoDeduce<Tab>::type* tab, co
                 de = fa.r0_r != 0.0f ? distance_efficiency_quick(rd, M.r0, fa.r0_r)
                                      : distance_efficiency(rd, M.r0);
             }
-            x = binomial_broad(n, de, A.w[2], A.w[3]);
+            if (kAll && n >= kBinomTable && !bad)
+                x = int(binomial(n, double(de), A.w[2], A.w[3], key, w));
+            else
+                x = binomial_broad(n, de, A.w[2], A.w[3]);
             bad = bad || x < 0;
         } else if constexpr (std::is_same<Tab, BinomGuide>::value) {
             bad = bad || n >= kBinomTable;
