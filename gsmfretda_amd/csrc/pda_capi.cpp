@@ -700,9 +700,9 @@ int pda_debug_guide(pda_ctx* ctx, int sid, void* thr, int64_t thr_bytes, void* g
 
 int pda_debug_primitive(pda_ctx* ctx, int op, const void* in, void* out, int64_t n) {
     // input / output bytes per item for each op
-    static const size_t in_sz[10] = {24, 4, 4, 8, 8, 4, 8, 48, 40, 4};
-    static const size_t out_sz[10] = {16, 4, 4, 8, 8, 4, 4, 8, 4, 4};
-    if (!ctx || !in || !out || op < 0 || op > 9 || n < 0 || n > (int64_t(1) << 28))
+    static const size_t in_sz[17] = {24, 4, 4, 8, 8, 4, 8, 48, 40, 4, 4, 4, 8, 8, 8, 48, 8};
+    static const size_t out_sz[17] = {16, 4, 4, 8, 8, 4, 4, 8, 4, 4, 4, 4, 4, 4, 4, 8, 8};
+    if (!ctx || !in || !out || op < 0 || op > 16 || n < 0 || n > (int64_t(1) << 28))
         return fail(PDA_E_ARG, "bad argument");
     if (n == 0) return PDA_OK;
     HIP_TRY(hipSetDevice(ctx->device));

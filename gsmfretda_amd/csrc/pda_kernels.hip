@@ -916,6 +916,29 @@ __global__ void primitive_kernel(int op, const void* __restrict__ in, void* __re
             break;
         }
         case 9: static_cast<uint32_t*>(out)[i] = static_cast<const uint32_t*>(in)[i]; break;
+        case 10: static_cast<float*>(out)[i] = flog_uniform24(static_cast<const uint32_t*>(in)[i]); break;
+        case 11: static_cast<float*>(out)[i] = fexp_minus(static_cast<const float*>(in)[i]); break;
+        case 12: {
+            const float* q = static_cast<const float*>(in) + 2 * i;
+            static_cast<float*>(out)[i] = quotient(q[0], q[1], 1.0f / q[1]);
+            break;
+        }
+        case 13: {
+            const uint32_t* q = static_cast<const uint32_t*>(in) + 2 * i;
+            static_cast<float*>(out)[i] = gauss_uniform24(q[0], q[1]);
+            break;
+        }
+        case 14: {
+            const float* q = static_cast<const float*>(in) + 2 * i;
+            static_cast<float*>(out)[i] = distance_efficiency_quick(q[0], q[1], 1.0f / q[1]);
+            break;
+        }
+        case 15: {
+            const BinomItem it = static_cast<const BinomItem*>(in)[i];
+            static_cast<int64_t*>(out)[i] = binomial_broad(it.n, float(it.p), it.hi, it.lo);
+            break;
+        }
+        case 16: static_cast<double*>(out)[i] = reciprocal_close(static_cast<const double*>(in)[i]); break;
         default: break;
     }
 }

@@ -371,6 +371,17 @@ PDA_HD float distance_efficiency_quick(float rd, float r0, float r0_r) {
 #endif
 }
 
+// 1 / x within 2^-50 relative, for x in [1/2, 2^20].
+PDA_HD double reciprocal_close(double x) {
+#ifdef __HIP_DEVICE_COMPILE__
+    double r = __builtin_amdgcn_rcp(x);
+    r = fma(fma(-x, r, 1.0), r, r);
+    return fma(fma(-x, r, 1.0), r, r);
+#else
+    return 1.0 / x;
+#endif
+}
+
 // ---- binomial -------------------------------------------------------------
 // Inversion (src/binom.cuh:135-169) when n < kInversionMaxN or
 // min(p,1-p) n <= 30, BTPE (Kachitvichyanukul & Schmeiser 1988,

@@ -221,28 +221,14 @@ PDA_HD int binomial_broad(int n, float p, uint32_t hi, uint32_t lo) {
         if (e & 1) C *= sq;
         sq *= sq;
     }
-#ifdef __HIP_DEVICE_COMPILE__
-    double rq = __builtin_amdgcn_rcp(q);
-    rq = fma(fma(-q, rq, 1.0), rq, rq);
-    rq = fma(fma(-q, rq, 1.0), rq, rq);
-#else
-    const double rq = 1.0 / q;
-#endif
-    const double ratio = pp * rq;
+    const double ratio = pp * reciprocal_close(q);
     const double U = uniform53(hi, lo);
     double px = C;
     double left = double(n);  // n - X
     int X = 0;
     while (U > C && X < n) {
         ++X;
-#ifdef __HIP_DEVICE_COMPILE__
-        double inv = __builtin_amdgcn_rcp(double(X));
-        inv = fma(fma(-double(X), inv, 1.0), inv, inv);
-        inv = fma(fma(-double(X), inv, 1.0), inv, inv);
-#else
-        const double inv = 1.0 / double(X);
-#endif
-        px = (px * ratio) * (left * inv);
+        px = (px * ratio) * (left * reciprocal_close(double(X)));
         left -= 1.0;
         if (U < C + kBroadBand) return -1;  // too near the threshold passed
         C += px;
@@ -529,6 +515,8 @@ PDA_HD uint32_t step_close(const uint32_t* tick, const uint2* link, uint32_t c, 
     uint32_t step = top;
 #ifdef __HIP_DEVICE_COMPILE__
     while (step > 1u && !__any(last - c >= step)) step >>= 1;
+#else
+    while (step > 1u && !(last - c >= step)) step >>= 1;  // a wave of one lane
 #endif
 #pragma unroll 1
     for (; step > 0u; step >>= 1) {

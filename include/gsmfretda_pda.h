@@ -313,7 +313,10 @@ int pda_run_noalloc(pda_ctx *ctx, int sid, int R, uint32_t seed, uint32_t set_id
  * 7 binomial (in: n i32, p f64, key 4 u32, w u32, words 2 u32 -> i64),
  * 8 background_count (in: lam, cap, u1, u2 f32, key 4 u32, w, sub -> f32),
  * 9 plain copy of u32 words (a kernel of known traffic, for counter
- * calibration).
+ * calibration); of the fast form: 10 flog_uniform24 (u32 -> f32),
+ * 11 fexp_minus, 12 quotient (a, b f32 -> f32), 13 gauss_uniform24 (2 u32 ->
+ * f32), 14 distance_efficiency_quick (rd, r0 f32 -> f32), 15 binomial_broad
+ * (as 7), 16 reciprocal_close (f64 -> f64).
  * in/out are host arrays; the layout per op is documented in pda_capi.cpp. */
 int pda_debug_primitive(pda_ctx *ctx, int op, const void *in, void *out, int64_t n);
 
