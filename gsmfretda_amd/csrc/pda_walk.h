@@ -228,7 +228,8 @@ PDA_HD int binomial_broad(int n, float p, uint32_t hi, uint32_t lo) {
     int X = 0;
     while (U > C && X < n) {
         ++X;
-        px = (px * ratio) * (left * reciprocal_close(double(X)));
+        const double inv = reciprocal_close(double(X));
+        px = (px * ratio) * (left * inv);
         left -= 1.0;
         if (U < C + kBroadBand) return -1;  // too near the threshold passed
         C += px;
