@@ -127,7 +127,7 @@ const WalkBurst* run_order(const pda_ctx* ctx, int64_t b0, int64_t b1) {
 }
 
 float clock_ms(const pda_ctx* ctx, uint64_t from, uint64_t to) {
-    return float(double(to - from) / double(ctx->clock_khz));
+    return float(double(int64_t(to - from)) / double(ctx->clock_khz));
 }
 
 }  // namespace pda

@@ -491,7 +491,7 @@ int pda_get_launch_shape(const pda_ctx* ctx, int* batch_tiles, int* waves_per_cu
 // Coordinate search over the launch shape on the slot's current work (its
 // single set, or its population): batch size, then resident waves per CU,
 // then the number of work counters; each candidate is run `reps` times after
-// one untimed run and scored by its median HIP-event time.  Results do not
+// one untimed run and scored by its median GPU time.  Results do not
 // depend on the shape (every unit's draws are keyed), only the time does.
 int pda_autotune(pda_ctx* ctx, int sid, int population, int R, int reps, int* batch_tiles,
                  int* waves_per_cu, int* queues, float* best_ms) {

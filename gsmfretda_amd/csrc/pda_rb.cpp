@@ -604,6 +604,11 @@ int enqueue_derivative(pda_ctx* ctx, RbState& r, int mode, double* out, uint32_t
     return PDA_OK;
 }
 
+// The counter of the pass's last launch: the line after the unit pass's.
+uint32_t* rb_ended(const RbState& r) {
+    return r.d_work + size_t(kMaxQueues + kAuxQueues) * kCounterStride;
+}
+
 // Enqueues the adjoint pass of state r's last forward for the cotangent g
 // (nbins entries; r's pinned buffers must be free: the caller waited for the
 // stream), its gradient written to r.h_grad.
@@ -612,7 +617,8 @@ int rb_enqueue_adjoint(pda_ctx* ctx, RbState& r, const double* g,
     std::memcpy(r.h_g, g, sizeof(double) * size_t(r.B));
     if (int rc = enqueue_derivative(ctx, r, 1, r.d_grad, uint32_t(kGradLen * kRbGradRows), stream))
         return rc;
-    HIP_TRY(launch_rb_rows(r.d_grad, kGradLen, kRbGradRows, r.d_hgrad, r.d_times + 1, stream));
+    HIP_TRY(launch_rb_rows(r.d_grad, kGradLen, kRbGradRows, r.d_hgrad, rb_ended(r), r.d_times + 1,
+                           stream));
     r.adj_ran = true;
     return PDA_OK;
 }
@@ -637,7 +643,7 @@ int rb_enqueue_jacobian(pda_ctx* ctx, RbState& r, hipStream_t stream) {
     const int n = kGradLen * r.B;
     if (int rc = enqueue_derivative(ctx, r, 2, r.d_jac, uint32_t(n) * kRbJacRows, stream))
         return rc;
-    HIP_TRY(launch_rb_rows(r.d_jac, n, kRbJacRows, r.d_hjac, r.d_times + 1, stream));
+    HIP_TRY(launch_rb_rows(r.d_jac, n, kRbJacRows, r.d_hjac, rb_ended(r), r.d_times + 1, stream));
     r.adj_ran = true;
     return PDA_OK;
 }

@@ -142,8 +142,9 @@ int pda_get_samples(pda_ctx *ctx, int sid, float *E, int32_t *acc, float *F, int
  * completed, NULL before. */
 float *pda_samples_host(pda_ctx *ctx, int sid);
 
-/* Milliseconds spent by the slot's last run on the GPU (from the kernels' clock
- * readings). */
+/* Milliseconds spent by the slot's last run on the GPU, from the kernels' own
+ * clock readings: from the walk's first workgroup to the end of the last, so
+ * without the launches before and behind them. */
 int pda_last_run_ms(pda_ctx *ctx, int sid, float *ms);
 /* The same split into the walk pass over every unit and the finishing pass
  * (replayed units, histogram reduction, chi2). */
@@ -163,7 +164,7 @@ int pda_get_launch_shape(const pda_ctx *ctx, int *batch_tiles, int *waves_per_cu
  * shape (batch size, then waves per CU, then work counters) on the slot's
  * current work -- its parameter set (population = 0) or its population
  * (population = 1) -- with R resamples, each candidate timed `reps` times
- * with HIP events after one untimed run; keeps the fastest shape in the
+ * on the GPU after one untimed run; keeps the fastest shape in the
  * context and returns it (outputs may be NULL).  Overwrites the slot's last
  * results. */
 int pda_autotune(pda_ctx *ctx, int sid, int population, int R, int reps, int *batch_tiles,
@@ -271,8 +272,9 @@ int pda_rb_adjoint_population(pda_ctx *ctx, int sid, const double *g, int nbins,
 int pda_rb_jacobian_population(pda_ctx *ctx, int sid, const int32_t *which, double *J, int nbins,
                                int nargs);
 
-/* GPU milliseconds of the slot's last RB runs: the walk, the whole forward
- * sequence, the last adjoint or Jacobian kernel (0 before the first).
+/* GPU milliseconds of the slot's last RB runs, from the kernels' clock
+ * readings: the walk with the tables before it, the whole forward sequence, the
+ * last adjoint or Jacobian pass up to its summed result (0 before the first).
  * Outputs may be NULL. */
 int pda_rb_stats(pda_ctx *ctx, int sid, float *walk_ms, float *forward_ms, float *adjoint_ms);
 
