@@ -272,11 +272,15 @@ int pass_shape(pda_ctx* ctx, int mode, int n, bool wide, int B, int cap, uint32_
                PassShape& ps) {
     static const char* names[] = {"forward", "adjoint", "Jacobian"};
     constexpr size_t kStatic = sizeof(RbModel) + 64;  // the kernels' static LDS
-    // the bins a pass supports: rows of an odd number of doubles and the score
-    // differences of four waves
+    // The bins a pass takes: the limit stays where rows of an odd number of
+    // doubles and the score differences of four waves had put it (1,021 bins for
+    // the Jacobian of 4 states, every other pass all 1,024), though the layout
+    // launched is smaller; that has to fit too.
     const size_t rows = sizeof(double) * size_t(mode == 2 ? B * ((n * n) | 1) : B);
+    const size_t least = rb_unit_lds_bytes(B, mode, n, 1, false);
     if (rows + (mode ? sizeof(double) * 4u * kWave * size_t(n * (n - 1)) : 0) + kStatic >
-        ctx->lds_per_block)
+            ctx->lds_per_block ||
+        least + kStatic > ctx->lds_per_block)
         return fail(PDA_E_DATA, "%d bins exceed the LDS of the RB %s pass", B, names[mode]);
     // The adjoint keeps the pool's first floats in LDS (3 states, 6.4e6 units:
     // 155 us, 174 without), unless the run is too small to repay the copy;
