@@ -244,11 +244,21 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(
             if (start_next == started) {  // start 64 units
                 if (pool_next >= pool_end) {
                     if (drained) break;
-                    uint32_t k = 0;
-                    if (lane == 0)
+                    uint32_t k = 0, listed = 0;
+                    if (lane == 0) {
                         k = atomicAdd(&io.work[queue * kCounterStride], kPop ? 1u : a.batch);
+                        if (kPop)
+                            listed = __hip_atomic_load(io.replay_count, __ATOMIC_RELAXED,
+                                                       __HIP_MEMORY_SCOPE_AGENT);
+                    }
                     k = __builtin_amdgcn_readfirstlane(k);
                     if (kPop) k = k * a.queues + queue;
+                    // more than the list holds: the run is repeated as a whole
+                    // (pda_get_population_result), what is left of it is not walked
+                    if (kPop && __builtin_amdgcn_readfirstlane(listed) > a.replay_cap) {
+                        drained = true;
+                        break;
+                    }
                     if (k >= (kPop ? batches : q.end - q.begin)) {
                         drained = true;
                         break;
@@ -814,7 +824,8 @@ __global__ __launch_bounds__(kWave) void pop_replay_kernel(
     const uint2* __restrict__ links, const PopControl* __restrict__ ctl,
     const Model* __restrict__ models, const RunArgs a, int32_t* __restrict__ hist_acc,
     const uint64_t* __restrict__ replay, const uint32_t* __restrict__ replay_count) {
-    const uint32_t count = *replay_count < a.replay_cap ? *replay_count : a.replay_cap;
+    const uint32_t count = *replay_count;
+    if (count > a.replay_cap) return;  // the run is repeated as a whole
     const uint32_t stride = gridDim.x * blockDim.x;
     for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < count; i += stride) {
         const uint64_t e = replay[i];
