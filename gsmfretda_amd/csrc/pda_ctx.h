@@ -316,6 +316,7 @@ hipError_t launch_model(const Model& M, Model* model, ThrPair* thr, uint8_t* gui
                         hipStream_t stream);
 hipError_t launch_guide(const Model* models, int nsets, int max_states, ThrPair* thr,
                         uint8_t* guide, hipStream_t stream);
+hipError_t launch_tables(const Model* models, int nsets, BinomTable* tabs, hipStream_t stream);
 hipError_t launch_pop_walk(int pass, uint32_t grid, const BurstDesc* bursts,
                            const WalkBurst* order, const uint32_t* ticks, const uint2* links, const PopControl* ctl,
                            const Model* models, const BinomTable* tabs,

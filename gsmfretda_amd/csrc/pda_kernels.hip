@@ -708,6 +708,19 @@ __global__ __launch_bounds__(kWave) void guide_kernel(const Model* __restrict__ 
     guide_row(M, s, int(blockIdx.x) % kBinomTable, thr, guide);
 }
 
+// The inversion tables of a population's sets (kPassTable), one workgroup per
+// set, a thread per count: build_binom_table's values.  (Formed on the host and
+// copied with every set_population, 49 MB for 4,000 sets, they took 28.5 ms of
+// a generation of 500 bursts x 4; here 2.4.)
+__global__ __launch_bounds__(kBinomTable) void table_kernel(const Model* __restrict__ models,
+                                                            BinomTable* __restrict__ tabs) {
+    const Model& M = models[blockIdx.x];
+    BinomTable& T = tabs[blockIdx.x];
+    const int m = int(threadIdx.x);
+    for (int s = 0; s < M.n; ++s)
+        inversion_constants(m, M.pp[s], M.qq[s], M.lq[s], &T.qn[s][m], &T.bound[s][m]);
+}
+
 // ---- population runs ---------------------------------------------------------
 //
 // A population of parameter sets (an optimiser generation) over the same
@@ -1195,6 +1208,12 @@ hipError_t launch_guide(const Model* models, int nsets, int max_states, ThrPair*
                         uint8_t* guide, hipStream_t stream) {
     hipLaunchKernelGGL(guide_kernel, dim3(uint32_t(max_states) * kBinomTable, uint32_t(nsets)),
                        dim3(kWave), 0, stream, models, thr, guide);
+    return hipGetLastError();
+}
+
+hipError_t launch_tables(const Model* models, int nsets, BinomTable* tabs, hipStream_t stream) {
+    hipLaunchKernelGGL(table_kernel, dim3(uint32_t(nsets)), dim3(kBinomTable), 0, stream, models,
+                       tabs);
     return hipGetLastError();
 }
 

@@ -6,7 +6,8 @@
 // src/streamWorker.cpp:83-182).  A population run evaluates a whole
 // generation -- sets of uneven state counts over the same resident bursts --
 // in one launch sequence that is captured once into a hipGraph and replayed:
-//   H2D copy of the generation's model tables and stream keys
+//   H2D copy of the generation's models and stream keys
+//   -> guide_kernel or table_kernel (the acceptor draws' rows or tables)
 //   -> fast_walk_kernel (persistent grid)
 //   -> pop_replay_kernel (abandoned units, general form)
 //   -> pop_finish_kernel (one workgroup per set: histogram and chi2, into the
@@ -145,6 +146,8 @@ int enqueue_population(pda_ctx* ctx, Slot& s, int pass, uint32_t grid, const Run
     if (pass == kPassGuided) {
         HIP_TRY(launch_guide(models, p.nsets, p.max_states, p.d_thr, p.d_guide, s.stream));
         guide = BinomGuide{p.d_thr, p.d_guide};
+    } else if (pass == kPassTable) {
+        HIP_TRY(launch_tables(models, p.nsets, p.d_tabs, s.stream));
     }
     HIP_TRY(launch_pop_walk(pass, grid, ctx->d_bursts,
                             ctx->d_plain, ctx->d_ticks, ctx->d_links, ctl, models,
@@ -372,20 +375,13 @@ int pda_set_population(pda_ctx* ctx, int sid, int nsets, const int32_t* nstates,
         HIP_TRY(hipMalloc(&p.d_guide, states * size_t(kBinomTable) * kGuideBuckets));
         p.cap_guide_states = states;
     }
-    if (!guided && !any_v) {
-        if (size_t(nsets) > p.cap_tabs) {
-            drop_graph(p);
-            (void)hipFree(p.d_tabs);
-            p.d_tabs = nullptr;
-            p.cap_tabs = 0;
-            HIP_TRY(hipMalloc(&p.d_tabs, sizeof(BinomTable) * size_t(nsets)));
-            p.cap_tabs = size_t(nsets);
-        }
-        std::vector<BinomTable> tabs(static_cast<size_t>(nsets));
-        for (int i = 0; i < nsets; ++i) build_binom_table(models[size_t(i)], tabs[size_t(i)]);
-        HIP_TRY(hipMemcpyAsync(p.d_tabs, tabs.data(), sizeof(BinomTable) * size_t(nsets),
-                               hipMemcpyHostToDevice, s->stream));
-        HIP_TRY(hipStreamSynchronize(s->stream));
+    if (!guided && !any_v && size_t(nsets) > p.cap_tabs) {
+        drop_graph(p);
+        (void)hipFree(p.d_tabs);
+        p.d_tabs = nullptr;
+        p.cap_tabs = 0;
+        HIP_TRY(hipMalloc(&p.d_tabs, sizeof(BinomTable) * size_t(nsets)));
+        p.cap_tabs = size_t(nsets);
     }
     p.guided = guided;
     p.max_states = max_states;
