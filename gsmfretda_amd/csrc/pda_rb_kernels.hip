@@ -556,17 +556,17 @@ __host__ __device__ constexpr int rb_lds_floats(int n) {
     return (n == 2 ? 4900 : n == 3 ? 6020 : 5863) + 3;
 }
 // Accumulators of a workgroup per copy, in 8-byte entries: the forward's bins;
-// the Jacobian's rows of n efficiency and n (n - 1) rate columns.  (The
-// adjoint's cotangent is not an accumulator: one copy, and a 0 for the
-// outcomes outside the histogram.)
-__host__ __device__ inline int rb_unit_acc(int B, int mode, int n) {
-    return mode == kRbJac ? B * n * n : mode == kRbGrad ? B + 1 : B;
+// the Jacobian's rows of n efficiency and n (n - 1) rate columns, `stride`
+// apart.  (The adjoint's cotangent is not an accumulator: one copy, and a 0 for
+// the outcomes outside the histogram.)
+__host__ __device__ inline int rb_unit_acc(int B, int mode, int stride) {
+    return mode == kRbJac ? B * stride : mode == kRbGrad ? B + 1 : B;
 }
 // Dynamic LDS: the accumulators, the pool's first floats, the tile's order
 // and its 64 counters (one per total, one for the group to take next).
-__host__ __device__ inline size_t rb_unit_lds(int B, int mode, int n, int copies, int threads,
-                                              bool pool) {
-    return sizeof(double) * size_t(rb_unit_acc(B, mode, n)) * size_t(copies) +
+__host__ __device__ inline size_t rb_unit_lds(int B, int mode, int n, int stride, int copies,
+                                              int threads, bool pool) {
+    return sizeof(double) * size_t(rb_unit_acc(B, mode, stride)) * size_t(copies) +
            (pool ? sizeof(float) * size_t(rb_lds_floats(n)) : 0) +
            sizeof(uint16_t) * size_t(threads) * kRbUnitPer + sizeof(uint32_t) * 64u;
 }
@@ -585,10 +585,22 @@ struct RbUnitArgs {
     double* grad;
     uint32_t* work;
     int32_t copies;  // accumulator copies, a power of two
+    int32_t stride;  // Jacobian: from row to row, n^2 or, odd, one more
     int32_t tile;    // units a workgroup takes at a time
     int32_t pool;    // the pool's first floats are kept in LDS
     RunTimes* times;  // forward: where the walk's end goes, or null
 };
+
+// Entry j becomes entry (j + turn) & 3, turn 0 .. 3.
+__device__ __forceinline__ void turn_by(float (&v)[4], int turn) {
+    const bool one = turn & 1, two = turn & 2;
+    const float a = one ? v[1] : v[0], b = one ? v[2] : v[1], c = one ? v[3] : v[2],
+                d = one ? v[0] : v[3];
+    v[0] = two ? c : a;
+    v[1] = two ? d : b;
+    v[2] = two ? a : c;
+    v[3] = two ? b : d;
+}
 
 // rb_bin() for F in quotient_range and its reciprocal rF rounded to float; B
 // for outcomes outside the histogram.  floor(E B) from the float product: one
@@ -603,7 +615,9 @@ __device__ __forceinline__ int rb_bin_quick(int a, float F, float rF, float Bf, 
 
 constexpr int rb_unit_threads_of(int mode) { return mode == kRbJac ? 1024 : 256; }
 
-template <int kMode, int kN>
+// kTurn (Jacobian): the lanes of a wave go through their outcomes from different
+// places, see pass_shape.
+template <int kMode, int kN, bool kTurn>
 __global__ __launch_bounds__(rb_unit_threads_of(kMode)) void rb_unit_kernel(const RunArgs a,
                                                                             const RbUnitArgs p) {
     constexpr bool kDeriv = kMode != kRbFwd;
@@ -613,7 +627,7 @@ __global__ __launch_bounds__(rb_unit_threads_of(kMode)) void rb_unit_kernel(cons
     const int tid = int(threadIdx.x), lane = tid % kWave;
     if (kMode == kRbFwd && p.times && blockIdx.x == 0 && tid == 0) stamp(&p.times->walked);
     const int B = a.B;
-    const int nacc = rb_unit_acc(B, kMode, kN) * p.copies;
+    const int nacc = rb_unit_acc(B, kMode, p.stride) * p.copies;
     float* s_pool = reinterpret_cast<float*>(s_acc + nacc);
     uint16_t* s_order = reinterpret_cast<uint16_t*>(s_pool + (p.pool ? rb_lds_floats(kN) : 0));
     uint32_t* s_count = reinterpret_cast<uint32_t*>(s_order + kThreads * kRbUnitPer);
@@ -722,16 +736,30 @@ __global__ __launch_bounds__(rb_unit_threads_of(kMode)) void rb_unit_kernel(cons
             // offset + 3.  Lanes past their unit's outcomes read on into the
             // blocks that follow.
             auto outcomes = [&](auto&& four) {
+                const int turn = kTurn ? lane & 3 : 0;
+                int at = kTurn ? (lane >> 2) % (longest / 4 + 1) * 4 : 0;
                 for (int q0 = 0; q0 <= longest; q0 += 4) {
-                    float P4[4], D4[kN][4];
-                    four(offP + uint32_t(q0), P4);
+                    float P4[4], D4[kN][4], L4[kTurn ? kN : 1][4];
+                    if (!kTurn) at = q0;
+                    four(offP + uint32_t(at), P4);
                     if (kDeriv) {
 #pragma unroll
-                        for (int s = 0; s < kN; ++s) four(offD[s] + uint32_t(q0), D4[s]);
+                        for (int s = 0; s < kN; ++s) four(offD[s] + uint32_t(at), D4[s]);
+                    }
+                    if constexpr (kTurn) {
+                        turn_by(P4, turn);
+#pragma unroll
+                        for (int s = 0; s < kN; ++s) {  // L4: the entries one before D4's
+                            L4[s][0] = at > 0 ? p.poolP[offD[s] + uint32_t(at) - 1u] : 0.0f;
+#pragma unroll
+                            for (int j = 1; j < 4; ++j) L4[s][j] = D4[s][j - 1];
+                            turn_by(D4[s], turn);
+                            turn_by(L4[s], turn);
+                        }
                     }
 #pragma unroll
                     for (int j = 0; j < 4; ++j) {
-                        const int q = q0 + j;
+                        const int q = kTurn ? at + ((j + turn) & 3) : q0 + j;
                         const bool act = q <= Mt;
                         const float P = P4[j];
                         int b = 0;
@@ -764,11 +792,12 @@ __global__ __launch_bounds__(rb_unit_threads_of(kMode)) void rb_unit_kernel(cons
 #pragma unroll
                             for (int s = 0; s < kN; ++s) {
                                 const float pd = q < Mt ? D4[s][j] : 0.0f;
-                                e[s] = double(mm[s]) * (double(pd_last[s]) - double(pd));
+                                const float before = kTurn ? L4[kTurn ? s : 0][j] : pd_last[s];
+                                e[s] = double(mm[s]) * (double(before) - double(pd));
                                 pd_last[s] = pd;
                             }
                             if (act && b < B) {
-                                double* row = s_acc + size_t(b * kCols) * size_t(p.copies) + copy;
+                                double* row = s_acc + size_t(b * p.stride) * size_t(p.copies) + copy;
 #pragma unroll
                                 for (int s = 0; s < kN; ++s) atomicAdd(&row[s * p.copies], e[s]);
 #pragma unroll
@@ -777,6 +806,7 @@ __global__ __launch_bounds__(rb_unit_threads_of(kMode)) void rb_unit_kernel(cons
                             }
                         }
                     }
+                    if (kTurn) at = at + 4 > longest ? 0 : at + 4;
                 }
             };
             if (p.pool && longest < rb_lds_totals(kN))
@@ -832,7 +862,8 @@ __global__ __launch_bounds__(rb_unit_threads_of(kMode)) void rb_unit_kernel(cons
         for (int i = tid; i < B * kCols; i += kThreads) {
             const int b = i / kCols, col = i - b * kCols;
             double v = 0.0;
-            for (int x = 0; x < p.copies; ++x) v += s_acc[size_t(i) * size_t(p.copies) + size_t(x)];
+            const double* from = s_acc + size_t(b * p.stride + col) * size_t(p.copies);
+            for (int x = 0; x < p.copies; ++x) v += from[x];
             if (col >= kN) v *= f;
             if (v != 0.0) atomicAdd(&J[size_t(b) * kRbGradLen + size_t(col)], v);
         }
@@ -1218,19 +1249,21 @@ hipError_t rb_walk_occupancy(bool scores, int n, int* per_cu) {
 #undef PDA_RB_OCC
 }
 
-template <int kMode>
+template <int kMode, bool kTurn>
 static hipError_t rb_unit_occupancy_m(int n, size_t l, int* per_cu) {
     const int tu = rb_unit_threads_of(kMode);
-    if (n == 2) return hipOccupancyMaxActiveBlocksPerMultiprocessor(per_cu, rb_unit_kernel<kMode, 2>, tu, l);
-    if (n == 3) return hipOccupancyMaxActiveBlocksPerMultiprocessor(per_cu, rb_unit_kernel<kMode, 3>, tu, l);
-    return hipOccupancyMaxActiveBlocksPerMultiprocessor(per_cu, rb_unit_kernel<kMode, 4>, tu, l);
+    if (n == 2) return hipOccupancyMaxActiveBlocksPerMultiprocessor(per_cu, rb_unit_kernel<kMode, 2, kTurn>, tu, l);
+    if (n == 3) return hipOccupancyMaxActiveBlocksPerMultiprocessor(per_cu, rb_unit_kernel<kMode, 3, kTurn>, tu, l);
+    return hipOccupancyMaxActiveBlocksPerMultiprocessor(per_cu, rb_unit_kernel<kMode, 4, kTurn>, tu, l);
 }
 
-hipError_t rb_unit_occupancy(int mode, int n, int dyn_lds, int* per_cu) {
+hipError_t rb_unit_occupancy(int mode, int n, bool turn, int dyn_lds, int* per_cu) {
     const size_t l = size_t(dyn_lds);
-    if (mode == kRbGrad) return rb_unit_occupancy_m<kRbGrad>(n, l, per_cu);
-    if (mode == kRbJac) return rb_unit_occupancy_m<kRbJac>(n, l, per_cu);
-    return rb_unit_occupancy_m<kRbFwd>(n, l, per_cu);
+    if (mode == kRbGrad) return rb_unit_occupancy_m<kRbGrad, false>(n, l, per_cu);
+    if (mode == kRbJac)
+        return turn ? rb_unit_occupancy_m<kRbJac, true>(n, l, per_cu)
+                    : rb_unit_occupancy_m<kRbJac, false>(n, l, per_cu);
+    return rb_unit_occupancy_m<kRbFwd, false>(n, l, per_cu);
 }
 
 hipError_t rb_big_occupancy(int mode, bool wide, int dyn_lds, int* per_cu) {
@@ -1282,8 +1315,8 @@ hipError_t launch_rb_walk(bool scores, int n, uint32_t grid, uint32_t replay_gri
 }
 
 int rb_unit_threads(int mode) { return rb_unit_threads_of(mode); }
-size_t rb_unit_lds_bytes(int B, int mode, int n, int copies, bool pool) {
-    return rb_unit_lds(B, mode, n, copies, rb_unit_threads_of(mode), pool);
+size_t rb_unit_lds_bytes(int B, int mode, int n, int stride, int copies, bool pool) {
+    return rb_unit_lds(B, mode, n, stride, copies, rb_unit_threads_of(mode), pool);
 }
 size_t rb_big_lds_bytes(int B, int cap, int mode, bool wide) { return rb_big_lds(B, cap, mode, wide); }
 
@@ -1320,33 +1353,36 @@ hipError_t launch_rb_memo(int n, const float* pmf_tab, const uint4* items, uint3
     return hipGetLastError();
 }
 
-template <int kMode, int kN>
+template <int kMode, int kN, bool kTurn>
 static void launch_rb_unit_n(uint32_t grid, const RunArgs& a, const RbUnitArgs& p,
                              hipStream_t stream) {
     const int threads = rb_unit_threads_of(kMode);
-    hipLaunchKernelGGL((rb_unit_kernel<kMode, kN>), dim3(grid), dim3(uint32_t(threads)),
-                       rb_unit_lds(a.B, kMode, kN, p.copies, threads, p.pool != 0), stream, a, p);
+    hipLaunchKernelGGL((rb_unit_kernel<kMode, kN, kTurn>), dim3(grid), dim3(uint32_t(threads)),
+                       rb_unit_lds(a.B, kMode, kN, p.stride, p.copies, threads, p.pool != 0),
+                       stream, a, p);
 }
 
-hipError_t launch_rb_unit(int mode, int n, uint32_t grid, int copies, int tile, bool pool,
-                          const RunArgs& a, const uint2* cnt, const float* F, const float* S,
+hipError_t launch_rb_unit(int mode, int n, uint32_t grid, int copies, int stride, bool turn,
+                          int tile, bool pool, const RunArgs& a, const uint2* cnt, const float* F, const float* S,
                           const double* Sbar, const double* g, const uint32_t* rank_offP,
                           const uint4* rank_offD, const float* poolP,
                           unsigned long long* hist_acc, double* grad, uint32_t* work,
                           RunTimes* times, hipStream_t stream) {
     if (n < 2 || n > kRbMaxStates) return hipErrorInvalidValue;
     const RbUnitArgs p{cnt,      F,    S,    Sbar,   g,    rank_offP, rank_offD, poolP,
-                       hist_acc, grad, work, copies, tile, pool ? 1 : 0, times};
-#define PDA_RB_UNIT_M(M)                                       \
-    if (n == 2) launch_rb_unit_n<M, 2>(grid, a, p, stream);    \
-    else if (n == 3) launch_rb_unit_n<M, 3>(grid, a, p, stream); \
-    else launch_rb_unit_n<M, 4>(grid, a, p, stream)
+                       hist_acc, grad, work, copies, stride, tile, pool ? 1 : 0, times};
+#define PDA_RB_UNIT_M(M, T)                                         \
+    if (n == 2) launch_rb_unit_n<M, 2, T>(grid, a, p, stream);      \
+    else if (n == 3) launch_rb_unit_n<M, 3, T>(grid, a, p, stream); \
+    else launch_rb_unit_n<M, 4, T>(grid, a, p, stream)
     if (mode == kRbGrad) {
-        PDA_RB_UNIT_M(kRbGrad);
+        PDA_RB_UNIT_M(kRbGrad, false);
+    } else if (mode == kRbJac && turn) {
+        PDA_RB_UNIT_M(kRbJac, true);
     } else if (mode == kRbJac) {
-        PDA_RB_UNIT_M(kRbJac);
+        PDA_RB_UNIT_M(kRbJac, false);
     } else {
-        PDA_RB_UNIT_M(kRbFwd);
+        PDA_RB_UNIT_M(kRbFwd, false);
     }
 #undef PDA_RB_UNIT_M
     return hipGetLastError();
