@@ -1074,10 +1074,12 @@ __global__ __launch_bounds__(kWave) void rb_big_kernel(
 // Per burst bl and rate k: Sbar[bl K + k] = (1 / R) sum_r S[(bl R + r) K + k],
 // summed r ascending in double.  A workgroup stages the scores of a run of
 // whole bursts in LDS with coalesced loads, then one thread per (burst,
-// rate) sums them; bursts whose R K scores exceed the stage are summed
-// straight from global memory.  Bound by the scores' 154 MB (100,000 bursts x 64
+// rate) sums them; a burst whose R K scores exceed the stage is taken a part of
+// its resamples at a time.  Bound by the scores' 154 MB (100,000 bursts x 64
 // of 3 states): 33 us, 82 with single-float loads and half as many workgroups
-// of twice the stage.
+// of twice the stage.  (Bursts beyond the stage had been summed straight from
+// memory, a thread per burst and rate: 200 bursts x 1,000 of 3 states 182 us,
+// now 21.)
 constexpr uint32_t kRbSbarStage = 4096;  // floats
 __global__ __launch_bounds__(256) void rb_score_mean_kernel(const RunArgs a, int K,
                                                             const float* __restrict__ S,
@@ -1085,35 +1087,32 @@ __global__ __launch_bounds__(256) void rb_score_mean_kernel(const RunArgs a, int
     __shared__ __align__(8) float st[kRbSbarStage];
     const uint64_t nb = a.nunits / a.R;
     const uint32_t per = a.R * uint32_t(K);  // scores per burst
-    const uint32_t bpb = per <= kRbSbarStage ? kRbSbarStage / per : 0u;
-    if (bpb == 0) {
-        for (uint64_t i = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x; i < nb * uint64_t(K);
-             i += uint64_t(gridDim.x) * blockDim.x) {
-            const uint64_t bl = i / uint64_t(K), k = i - bl * uint64_t(K);
-            const float* src = S + bl * per + k;
-            double sum = 0.0;
-            for (uint32_t r = 0; r < a.R; ++r) sum += double(src[uint64_t(r) * uint64_t(K)]);
-            Sbar[i] = sum / double(a.R);
-        }
-        return;
-    }
+    // bursts at a time, or resamples of one burst
+    const uint32_t bpb = per <= kRbSbarStage ? kRbSbarStage / per : 1u;
+    const uint32_t rpb = per <= kRbSbarStage ? a.R : kRbSbarStage / uint32_t(K);
     for (uint64_t b0 = uint64_t(blockIdx.x) * bpb; b0 < nb; b0 += uint64_t(gridDim.x) * bpb) {
         const uint32_t nbh = uint32_t(nb - b0 < bpb ? nb - b0 : bpb);
-        const float* src = S + b0 * per;
-        __syncthreads();
-        // K is even: whole pairs, 8-byte aligned
-        const float2* src2 = reinterpret_cast<const float2*>(src);
-        float2* st2 = reinterpret_cast<float2*>(st);
+        double part = 0.0;  // of thread k < K, where the burst is taken in parts
+        for (uint32_t r0 = 0; r0 < a.R; r0 += rpb) {
+            const uint32_t rh = a.R - r0 < rpb ? a.R - r0 : rpb;
+            const uint32_t len = per <= kRbSbarStage ? nbh * per : rh * uint32_t(K);
+            const float* src = S + b0 * per + uint64_t(r0) * uint64_t(K);
+            __syncthreads();
+            // K is even: whole pairs, 8-byte aligned
+            const float2* src2 = reinterpret_cast<const float2*>(src);
+            float2* st2 = reinterpret_cast<float2*>(st);
 #pragma unroll 8
-        for (uint32_t i = threadIdx.x; i < nbh * per / 2u; i += 256u) st2[i] = src2[i];
-        __syncthreads();
-        for (uint32_t t = threadIdx.x; t < nbh * uint32_t(K); t += blockDim.x) {
-            const uint32_t bl = t / uint32_t(K), k = t - bl * uint32_t(K);
-            const float* x = st + bl * per + k;
-            double sum = 0.0;
+            for (uint32_t i = threadIdx.x; i < len / 2u; i += 256u) st2[i] = src2[i];
+            __syncthreads();
+            for (uint32_t t = threadIdx.x; t < nbh * uint32_t(K); t += blockDim.x) {
+                const uint32_t bl = t / uint32_t(K), k = t - bl * uint32_t(K);
+                const float* x = st + bl * per + k;
+                double sum = part;
 #pragma unroll 8
-            for (uint32_t r = 0; r < a.R; ++r) sum += double(x[r * uint32_t(K)]);
-            Sbar[(b0 + bl) * uint64_t(K) + k] = sum / double(a.R);
+                for (uint32_t r = 0; r < rh; ++r) sum += double(x[r * uint32_t(K)]);
+                if (r0 + rh == a.R) Sbar[(b0 + bl) * uint64_t(K) + k] = sum / double(a.R);
+                else part = sum;
+            }
         }
     }
 }
@@ -1424,8 +1423,8 @@ hipError_t launch_rb_score_mean(const RunArgs& a, int K, const float* S, double*
                                 int num_cu, hipStream_t stream) {
     const uint64_t nb = a.nunits / a.R;
     const uint64_t per = uint64_t(a.R) * uint64_t(K);
-    const uint64_t bpb = per <= kRbSbarStage ? kRbSbarStage / per : 0;
-    const uint64_t want = bpb ? (nb + bpb - 1) / bpb : (nb * uint64_t(K) + 255) / 256;
+    const uint64_t bpb = per <= kRbSbarStage ? kRbSbarStage / per : 1;
+    const uint64_t want = (nb + bpb - 1) / bpb;
     // a few workgroups per CU, each looping over its share
     const uint64_t cap = uint64_t(num_cu > 0 ? num_cu : 1) * 8u;
     const uint32_t grid = uint32_t(std::max<uint64_t>(1, std::min<uint64_t>(want, cap)));
