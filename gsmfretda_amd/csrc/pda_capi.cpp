@@ -177,13 +177,20 @@ int load_common(pda_ctx* ctx, const int64_t* start, const int64_t* stop, const i
         HIP_TRY(hipMalloc(&ctx->d_bursts, sizeof(BurstDesc) * size_t(nbursts)));
         HIP_TRY(hipMemcpy(ctx->d_bursts, bursts.data(), sizeof(BurstDesc) * size_t(nbursts),
                           hipMemcpyHostToDevice));
-        std::vector<WalkBurst> plain, order;
-        burst_order(bursts, plain, order);
+        const std::vector<uint32_t> order = burst_order(bursts);
         const size_t bytes = sizeof(WalkBurst) * size_t(nbursts);
         HIP_TRY(hipMalloc(&ctx->d_plain, bytes));
-        HIP_TRY(hipMemcpy(ctx->d_plain, plain.data(), bytes, hipMemcpyHostToDevice));
         HIP_TRY(hipMalloc(&ctx->d_order, bytes));
-        HIP_TRY(hipMemcpy(ctx->d_order, order.data(), bytes, hipMemcpyHostToDevice));
+        uint32_t* d_idx = nullptr;
+        HIP_TRY(hipMalloc(&d_idx, sizeof(uint32_t) * size_t(nbursts)));
+        hipError_t e = hipMemcpy(d_idx, order.data(), sizeof(uint32_t) * size_t(nbursts),
+                                 hipMemcpyHostToDevice);
+        if (e == hipSuccess)
+            e = launch_order(ctx->d_bursts, d_idx, uint32_t(nbursts), ctx->d_plain, ctx->d_order,
+                             nullptr);
+        if (e == hipSuccess) e = hipStreamSynchronize(nullptr);
+        (void)hipFree(d_idx);
+        HIP_TRY(e);
     }
     if (total > 0) {
         HIP_TRY(hipMalloc(&ctx->d_ticks, sizeof(uint32_t) * size_t(total)));

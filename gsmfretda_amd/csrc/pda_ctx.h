@@ -311,6 +311,9 @@ hipError_t launch_walk(int pass, uint32_t grid, const BurstDesc* bursts, const W
                        uint32_t* replay_count, uint32_t* work, float* outE, int32_t* outAcc,
                        float* outF, const float* obs, ResultHeader* result, RunTimes* times,
                        hipStream_t stream);
+// plain[i] = burst i, order[i] = burst idx[i]
+hipError_t launch_order(const BurstDesc* bursts, const uint32_t* idx, uint32_t n, WalkBurst* plain,
+                        WalkBurst* order, hipStream_t stream);
 // stores the model of a parameter set and builds its threshold rows
 hipError_t launch_model(const Model& M, Model* model, ThrPair* thr, uint8_t* guide,
                         hipStream_t stream);

@@ -393,6 +393,19 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(
     }
 }
 
+// The bursts as the walks start them, formed here from their indices: the two
+// arrays made on the host and copied were a twentieth of a load's time.
+__global__ __launch_bounds__(256) void order_kernel(const BurstDesc* __restrict__ bursts,
+                                                    const uint32_t* __restrict__ idx, uint32_t n,
+                                                    WalkBurst* __restrict__ plain,
+                                                    WalkBurst* __restrict__ order) {
+    const uint32_t i = blockIdx.x * 256u + threadIdx.x;
+    if (i >= n) return;
+    const uint32_t b = idx[i];
+    plain[i] = WalkBurst{bursts[i], i, {0u, 0u, 0u}};
+    order[i] = WalkBurst{bursts[b], b, {0u, 0u, 0u}};
+}
+
 // chi2 of one histogram by one wave, as src/streamWorker.cpp:194-206: the
 // reference's float accumulation and FP64.  Reads the 8 accumulator rows
 // (`pitch` apart, left zero for the next run) and writes their sum.
@@ -1194,6 +1207,13 @@ hipError_t launch_walk(int pass, uint32_t grid, const BurstDesc* bursts, const W
         launch_fast<false, kPassGuided, true>(grid, lds, io, a, fa, stream);
     else
         launch_fast<false, kPassGuided, false>(grid, lds, io, a, fa, stream);
+    return hipGetLastError();
+}
+
+hipError_t launch_order(const BurstDesc* bursts, const uint32_t* idx, uint32_t n, WalkBurst* plain,
+                        WalkBurst* order, hipStream_t stream) {
+    hipLaunchKernelGGL(order_kernel, dim3((n + 255u) / 256u), dim3(256), 0, stream, bursts, idx, n,
+                       plain, order);
     return hipGetLastError();
 }
 

@@ -264,34 +264,31 @@ bool draws_in_place(const LongRuns& r, int64_t nbursts, int64_t nphotons, int64_
 
 // A counting sort of each part.  A unit's windows grow with its burst's duration:
 // the walk starts a part's long ones first, and a run ends with short ones.
-void burst_order(const std::vector<BurstDesc>& bursts, std::vector<WalkBurst>& plain,
-                 std::vector<WalkBurst>& order) {
+std::vector<uint32_t> burst_order(const std::vector<BurstDesc>& bursts) {
     constexpr uint32_t kOrderBuckets = 256;
     constexpr size_t kOrderParts = 4u * kDefaultQueues;
     float longest = 0.0f;
     for (const BurstDesc& d : bursts)
         if (d.T < INFINITY && d.T > longest) longest = d.T;
     const float scale = longest > 0.0f ? float(kOrderBuckets - 1) / longest : 0.0f;
-    auto bucket = [&](const BurstDesc& d) {  // 0: the longest
-        const float x = d.T * scale;
-        return x >= 1.0f ? kOrderBuckets - 1u - std::min(uint32_t(std::min(x, float(kOrderBuckets))),
-                                                         kOrderBuckets - 1u)
-                         : kOrderBuckets - 1u;
-    };
     const size_t n = bursts.size();
-    plain.resize(n);
-    order.resize(n);
-    for (size_t i = 0; i < n; ++i) plain[i] = WalkBurst{bursts[i], uint32_t(i), {0u, 0u, 0u}};
+    std::vector<uint8_t> bucket(n);  // 0: the longest
+    for (size_t i = 0; i < n; ++i) {
+        const float x = std::min(bursts[i].T * scale, float(kOrderBuckets - 1));
+        bucket[i] = uint8_t(x >= 1.0f ? kOrderBuckets - 1u - uint32_t(x) : kOrderBuckets - 1u);
+    }
+    std::vector<uint32_t> order(n);
     // a queue's share stays one region of the photon arrays, and has long and
     // short bursts under way together
     const size_t part = std::max<size_t>((n + kOrderParts - 1) / kOrderParts, 1);
     for (size_t b0 = 0; b0 < n; b0 += part) {
         const size_t b1 = std::min(n, b0 + part);
         uint32_t next[kOrderBuckets + 1] = {};
-        for (size_t i = b0; i < b1; ++i) ++next[bucket(bursts[i]) + 1];
+        for (size_t i = b0; i < b1; ++i) ++next[bucket[i] + 1];
         for (uint32_t i = 0; i < kOrderBuckets; ++i) next[i + 1] += next[i];
-        for (size_t i = b0; i < b1; ++i) order[b0 + next[bucket(bursts[i])]++] = plain[i];
+        for (size_t i = b0; i < b1; ++i) order[b0 + next[bucket[i]]++] = uint32_t(i);
     }
+    return order;
 }
 
 // Inversion constants of binomial_inversion() (pda_math.h) per state and count.

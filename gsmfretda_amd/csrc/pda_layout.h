@@ -68,11 +68,10 @@ int build_model(const Photophysics& ph, int n, const float* args, int nargs, Mod
 bool draws_in_place(const LongRuns& r, int64_t nbursts, int64_t nphotons, int64_t range,
                     const Photophysics& ph, bool bg_on, bool population);
 
-// The bursts as a walk starts them: as they come, and by falling duration (in
-// 256 steps of the longest, a step's bursts in their order) within each of equal
-// parts, four to a default queue's share.
-void burst_order(const std::vector<BurstDesc>& bursts, std::vector<WalkBurst>& plain,
-                 std::vector<WalkBurst>& order);
+// The bursts in the order in which a walk over all of them starts them: by
+// falling duration (in 256 steps of the longest, a step's bursts in their order)
+// within each of equal parts, four to a default queue's share.
+std::vector<uint32_t> burst_order(const std::vector<BurstDesc>& bursts);
 // Tabulated inversion constants for the fast walk (needs M from build_model).
 void build_binom_table(const Model& M, BinomTable& T);
 
