@@ -386,10 +386,9 @@ hipError_t launch_rb_big(int mode, bool wide, uint32_t grid, int cap, const RbMo
                          unsigned long long* hist_acc, double* grad, hipStream_t stream);
 hipError_t launch_rb_score_mean(const RunArgs& a, int K, const float* S, double* Sbar,
                                 int num_cu, hipStream_t stream);
-// out[i] = sum of the nrows rows of n doubles; ended: a counter that rb_begin
-// zeroed
-hipError_t launch_rb_rows(const double* rows, int n, int nrows, double* out, uint32_t* ended,
-                          RunTimes* times, hipStream_t stream);
+// out[i] = sum of the nrows rows of n doubles
+hipError_t launch_rb_rows(const double* rows, int n, int nrows, double* out, RunTimes* times,
+                          hipStream_t stream);
 hipError_t launch_rb_finish(const RunArgs& a, const float* obs, unsigned long long* hist_acc,
                             void* res, RunTimes* times, hipStream_t stream);
 

@@ -192,7 +192,6 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(
     __shared__ float2 s_done[2 * kWave];      // (acc, F) of units not yet binned
     extern __shared__ int32_t s_hist[];       // [kSlots][a.B]
     const uint32_t lane = threadIdx.x;
-    if (!kPop && io.times && blockIdx.x == 0 && lane == 0) stamp(&io.times->start);
     for (uint32_t i = lane; i < uint32_t(kSlots) * uint32_t(a.B); i += kWave) s_hist[i] = 0;
     auto load_model = [&](uint32_t into, uint32_t set) {
         const uint32_t* src = reinterpret_cast<const uint32_t*>(&io.models[set]);
@@ -210,6 +209,9 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(
                           bitsf(__builtin_amdgcn_readfirstlane(fbits(M.r0_r))));
         load_model(0u, 0u);
     }
+
+    // (as the first instruction it cost broadened runs of 50 us 0.6)
+    if (!kPop && io.times && blockIdx.x == 0 && lane == 0) stamp(&io.times->start);
 
     const uint32_t seed = kPop ? io.ctl->seed : a.seed;
     const uint32_t queue = blockIdx.x % a.queues;

@@ -297,7 +297,9 @@ int pass_shape(pda_ctx* ctx, int mode, int n, bool wide, int B, int cap, uint32_
     // same bank.  4 states, 2,000,000 units of 2,000 bursts: 1,000 bins 1586 -> 442
     // us, 200 bins 484 -> 359; 3 states, 1,000 bins 790 -> 337.  (A wave per 64
     // outcomes of the units in turn had taken 790, 426 and 600.)  With more
-    // copies the turning costs more than it saves: 3 states, 50 bins 125 -> 148.
+    // copies the turning costs more than it saves (3 states, 50 bins 125 -> 148),
+    // and with two to four in a small run (4 states, 20,000 units, 200 bins 75 ->
+    // 79).
     const size_t threads = size_t(rb_unit_threads(mode));
     const size_t budget = std::min<size_t>(ctx->lds_per_block, mode == 2 ? 131072 : 40960);
     const int most = mode == 1 ? 1 : mode == 2 ? 32 : 16;
@@ -308,7 +310,7 @@ int pass_shape(pda_ctx* ctx, int mode, int n, bool wide, int B, int cap, uint32_
     ps.pool = mode == 1 && nunits >= 65536u && lds_of(ps.stride, 1, true) <= budget;
     ps.copies = 1;
     while (ps.copies < most && lds_of(ps.stride, 2 * ps.copies, ps.pool) <= budget) ps.copies *= 2;
-    ps.turn = mode == 2 && ps.copies <= 4;
+    ps.turn = mode == 2 && ps.copies <= (nunits >= 65536u ? 4 : 1);
     if (ps.turn && lds_of(ps.stride | 1, ps.copies, false) + kStatic <= ctx->lds_per_block)
         ps.stride |= 1;
     const size_t lds = lds_of(ps.stride, ps.copies, ps.pool);
@@ -624,11 +626,6 @@ int enqueue_derivative(pda_ctx* ctx, RbState& r, int mode, double* out, uint32_t
     return PDA_OK;
 }
 
-// The counter of the pass's last launch: the line after the unit pass's.
-uint32_t* rb_ended(const RbState& r) {
-    return r.d_work + size_t(kMaxQueues + kAuxQueues) * kCounterStride;
-}
-
 // Enqueues the adjoint pass of state r's last forward for the cotangent g
 // (nbins entries; r's pinned buffers must be free: the caller waited for the
 // stream), its gradient written to r.h_grad.
@@ -637,8 +634,7 @@ int rb_enqueue_adjoint(pda_ctx* ctx, RbState& r, const double* g,
     std::memcpy(r.h_g, g, sizeof(double) * size_t(r.B));
     if (int rc = enqueue_derivative(ctx, r, 1, r.d_grad, uint32_t(kGradLen * kRbGradRows), stream))
         return rc;
-    HIP_TRY(launch_rb_rows(r.d_grad, kGradLen, kRbGradRows, r.d_hgrad, rb_ended(r), r.d_times + 1,
-                           stream));
+    HIP_TRY(launch_rb_rows(r.d_grad, kGradLen, kRbGradRows, r.d_hgrad, r.d_times + 1, stream));
     r.adj_ran = true;
     return PDA_OK;
 }
@@ -663,7 +659,7 @@ int rb_enqueue_jacobian(pda_ctx* ctx, RbState& r, hipStream_t stream) {
     const int n = kGradLen * r.B;
     if (int rc = enqueue_derivative(ctx, r, 2, r.d_jac, uint32_t(n) * kRbJacRows, stream))
         return rc;
-    HIP_TRY(launch_rb_rows(r.d_jac, n, kRbJacRows, r.d_hjac, rb_ended(r), r.d_times + 1, stream));
+    HIP_TRY(launch_rb_rows(r.d_jac, n, kRbJacRows, r.d_hjac, r.d_times + 1, stream));
     r.adj_ran = true;
     return PDA_OK;
 }

@@ -143,8 +143,8 @@ int pda_get_samples(pda_ctx *ctx, int sid, float *E, int32_t *acc, float *F, int
 float *pda_samples_host(pda_ctx *ctx, int sid);
 
 /* Milliseconds spent by the slot's last run on the GPU, from the kernels' own
- * clock readings: from the walk's first workgroup to the end of the last, so
- * without the launches before and behind them. */
+ * clock readings: from the walk's first workgroup, its model loaded, to the end
+ * of the run's last, so without the launches before, between and behind them. */
 int pda_last_run_ms(pda_ctx *ctx, int sid, float *ms);
 /* The same split into the walk pass over every unit and the finishing pass
  * (replayed units, histogram reduction, chi2). */
