@@ -358,7 +358,7 @@ hipError_t launch_rb_walk(bool scores, int n, uint32_t grid, uint32_t replay_gri
                           hipStream_t stream);
 // dynamic LDS bytes (mode: 0 forward, 1 adjoint, 2 Jacobian)
 int rb_unit_threads(int mode);
-size_t rb_unit_lds_bytes(int B, int mode, int n, int stride, int copies, bool pool);
+size_t rb_unit_lds_bytes(int B, int mode, int n, bool turn, int copies, bool pool);
 size_t rb_big_lds_bytes(int B, int cap, int mode, bool wide);
 // times (or null): where the launches of a run put their clock readings
 hipError_t launch_rb_table(const RbModel& R, const Model& M, RbModel* rbm, Model* model,
@@ -369,11 +369,11 @@ hipError_t launch_rb_begin(double* rows, uint32_t n, uint32_t* work, const doubl
                            double* g, int B, RunTimes* times, hipStream_t stream);
 hipError_t launch_rb_memo(int n, const float* pmf_tab, const uint4* items, uint32_t nitems,
                           const uint32_t* rank_offP, float* poolP, hipStream_t stream);
-// copies: of the LDS accumulators; stride: between the Jacobian's rows there;
-// turn: its lanes' outcomes in different orders; tile: units a workgroup takes
-// at a time; pool: the smallest totals' pmfs kept in LDS
-hipError_t launch_rb_unit(int mode, int n, uint32_t grid, int copies, int stride, bool turn,
-                          int tile, bool pool, const RunArgs& a, const uint2* cnt, const float* F, const float* S,
+// copies: of the LDS accumulators; turn: the Jacobian's lanes take their
+// outcomes in different orders; tile: units a workgroup takes at a time; pool:
+// the smallest totals' pmfs kept in LDS
+hipError_t launch_rb_unit(int mode, int n, uint32_t grid, int copies, bool turn, int tile,
+                          bool pool, const RunArgs& a, const uint2* cnt, const float* F, const float* S,
                           const double* Sbar, const double* g, const uint32_t* rank_offP,
                           const uint4* rank_offD, const float* poolP,
                           unsigned long long* hist_acc, double* grad, uint32_t* work,

@@ -183,6 +183,9 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(
     fast_waves_per_eu(kPop, kPass)))) void fast_walk_kernel(const FastIO io, const RunArgs a,
                                                             const FastArgs launch) {
     constexpr int kSlots = kPop ? 2 : 1;
+    // broadened walks choose their form so that the list suffices, and the look
+    // at its count takes 1 % of the 64 sets below
+    constexpr bool kStops = kPop && !is_broad(kPass);
     using Mod = typename std::conditional<
         kPass == kPassGuided, FastModel,
         typename std::conditional<is_broad(kPass), BroadModel, Model>::type>::type;
@@ -249,7 +252,7 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(
                     uint32_t k = 0, listed = 0;
                     if (lane == 0) {
                         k = atomicAdd(&io.work[queue * kCounterStride], kPop ? 1u : a.batch);
-                        if (kPop)
+                        if (kStops)
                             listed = __hip_atomic_load(io.replay_count, __ATOMIC_RELAXED,
                                                        __HIP_MEMORY_SCOPE_AGENT);
                     }
@@ -257,7 +260,7 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(
                     if (kPop) k = k * a.queues + queue;
                     // more than the list holds: the run is repeated as a whole
                     // (pda_get_population_result), what is left of it is not walked
-                    if (kPop && __builtin_amdgcn_readfirstlane(listed) > a.replay_cap) {
+                    if (kStops && __builtin_amdgcn_readfirstlane(listed) > a.replay_cap) {
                         drained = true;
                         break;
                     }

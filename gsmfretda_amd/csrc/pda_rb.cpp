@@ -263,7 +263,7 @@ int ensure_memo_layout(pda_ctx* ctx, int n) {
 // units exit at once).
 struct PassShape {
     uint32_t unit_grid = 1, big_grid = 1, huge_grid = 1;
-    int copies = 1, stride = 1, tile = kWave;
+    int copies = 1, tile = kWave;
     bool turn = false, pool = false;
     int big_cap = 1;    // rb_big_kernel's buffers for the big list (the huge list: the run's cap)
     bool wide = false;  // rb_big_kernel's derivative buffers in double
@@ -277,7 +277,7 @@ int pass_shape(pda_ctx* ctx, int mode, int n, bool wide, int B, int cap, uint32_
     // the Jacobian of 4 states, every other pass all 1,024), though the layout
     // launched is smaller; that has to fit too.
     const size_t rows = sizeof(double) * size_t(mode == 2 ? B * ((n * n) | 1) : B);
-    const size_t least = rb_unit_lds_bytes(B, mode, n, n * n, 1, false);
+    const size_t least = rb_unit_lds_bytes(B, mode, n, false, 1, false);
     if (rows + (mode ? sizeof(double) * 4u * kWave * size_t(n * (n - 1)) : 0) + kStatic >
             ctx->lds_per_block ||
         least + kStatic > ctx->lds_per_block)
@@ -293,8 +293,7 @@ int pass_shape(pda_ctx* ctx, int mode, int n, bool wide, int B, int cap, uint32_
     // one burst often have one F: 64 lanes at the same outcome then add to the
     // same row, one after the other.  With up to four copies the lanes go
     // through their outcomes in different orders (turn), and rows are an odd
-    // number of doubles apart where that takes no copy: even ones begin in the
-    // same bank.  4 states, 2,000,000 units of 2,000 bursts: 1,000 bins 1586 -> 442
+    // number of doubles apart: even ones begin in the same bank.  4 states, 2,000,000 units of 2,000 bursts: 1,000 bins 1586 -> 442
     // us, 200 bins 484 -> 359; 3 states, 1,000 bins 790 -> 337.  (A wave per 64
     // outcomes of the units in turn had taken 790, 426 and 600.)  With more
     // copies the turning costs more than it saves (3 states, 50 bins 125 -> 148),
@@ -303,17 +302,15 @@ int pass_shape(pda_ctx* ctx, int mode, int n, bool wide, int B, int cap, uint32_
     const size_t threads = size_t(rb_unit_threads(mode));
     const size_t budget = std::min<size_t>(ctx->lds_per_block, mode == 2 ? 131072 : 40960);
     const int most = mode == 1 ? 1 : mode == 2 ? 32 : 16;
-    ps.stride = n * n;
-    auto lds_of = [&](int stride, int copies, bool pool) {
-        return rb_unit_lds_bytes(B, mode, n, stride, copies, pool);
+    auto lds_of = [&](bool turn, int copies, bool pool) {
+        return rb_unit_lds_bytes(B, mode, n, turn, copies, pool);
     };
-    ps.pool = mode == 1 && nunits >= 65536u && lds_of(ps.stride, 1, true) <= budget;
+    ps.pool = mode == 1 && nunits >= 65536u && lds_of(false, 1, true) <= budget;
     ps.copies = 1;
-    while (ps.copies < most && lds_of(ps.stride, 2 * ps.copies, ps.pool) <= budget) ps.copies *= 2;
-    ps.turn = mode == 2 && ps.copies <= (nunits >= 65536u ? 4 : 1);
-    if (ps.turn && lds_of(ps.stride | 1, ps.copies, false) + kStatic <= ctx->lds_per_block)
-        ps.stride |= 1;
-    const size_t lds = lds_of(ps.stride, ps.copies, ps.pool);
+    while (ps.copies < most && lds_of(false, 2 * ps.copies, ps.pool) <= budget) ps.copies *= 2;
+    ps.turn = mode == 2 && ps.copies <= (nunits >= 65536u ? 4 : 1) &&
+              lds_of(true, ps.copies, false) + kStatic <= ctx->lds_per_block;
+    const size_t lds = lds_of(ps.turn, ps.copies, ps.pool);
     int per = 0;
     HIP_TRY(rb_unit_occupancy(mode, n, ps.turn, int(lds), &per));
     const uint64_t slots = uint64_t(ctx->num_cu) * uint64_t(std::max(per, 1));
@@ -484,7 +481,7 @@ int rb_enqueue_forward(pda_ctx* ctx, Slot& s, RbState& r, const Model& M,
                            r.d_big, r.d_huge, r.d_big_count, r.d_replay, r.d_replay_count,
                            stream));
     if (aux) HIP_TRY(hipStreamWaitEvent(stream, s.rb_join, 0));
-    HIP_TRY(launch_rb_unit(0, n, ps.unit_grid, ps.copies, ps.stride, ps.turn, ps.tile, ps.pool, a,
+    HIP_TRY(launch_rb_unit(0, n, ps.unit_grid, ps.copies, ps.turn, ps.tile, ps.pool, a,
                            r.d_cnt, r.d_F, nullptr, nullptr, nullptr, ML.d_rank_offP, ML.d_rank_offD, r.d_poolP,
                            r.d_hist, nullptr, r.d_work, r.d_times, stream));
     HIP_TRY(launch_rb_big(0, false, ps.big_grid, ps.big_cap, d_rbm, ctx->d_lf, r.d_pmf_tab, a, r.d_cnt,
@@ -613,7 +610,7 @@ int enqueue_derivative(pda_ctx* ctx, RbState& r, int mode, double* out, uint32_t
         HIP_TRY(launch_rb_score_mean(a, r.K, r.d_S, r.d_Sbar, ctx->num_cu, stream));
         r.sbar_valid = true;
     }
-    HIP_TRY(launch_rb_unit(mode, r.n, ps.unit_grid, ps.copies, ps.stride, ps.turn, ps.tile, ps.pool,
+    HIP_TRY(launch_rb_unit(mode, r.n, ps.unit_grid, ps.copies, ps.turn, ps.tile, ps.pool,
                            a, r.d_cnt, r.d_F, r.d_S, r.d_Sbar, g, ML.d_rank_offP, ML.d_rank_offD, r.d_poolP,
                            nullptr, out, r.d_work, nullptr, stream));
     HIP_TRY(launch_rb_big(mode, ps.wide, ps.big_grid, ps.big_cap, d_rbm, ctx->d_lf, r.d_pmf_tab, a,

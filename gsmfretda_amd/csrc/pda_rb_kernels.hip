@@ -556,17 +556,21 @@ __host__ __device__ constexpr int rb_lds_floats(int n) {
     return (n == 2 ? 4900 : n == 3 ? 6020 : 5863) + 3;
 }
 // Accumulators of a workgroup per copy, in 8-byte entries: the forward's bins;
-// the Jacobian's rows of n efficiency and n (n - 1) rate columns, `stride`
-// apart.  (The adjoint's cotangent is not an accumulator: one copy, and a 0 for
-// the outcomes outside the histogram.)
-__host__ __device__ inline int rb_unit_acc(int B, int mode, int stride) {
-    return mode == kRbJac ? B * stride : mode == kRbGrad ? B + 1 : B;
+// the Jacobian's rows of n efficiency and n (n - 1) rate columns, where its
+// lanes are turned (kTurn) an odd number of entries apart.  (The adjoint's
+// cotangent is not an accumulator: one copy, and a 0 for the outcomes outside
+// the histogram.)
+__host__ __device__ constexpr int rb_jac_stride(int n, bool turn) {
+    return turn ? n * n | 1 : n * n;
+}
+__host__ __device__ inline int rb_unit_acc(int B, int mode, int n, bool turn) {
+    return mode == kRbJac ? B * rb_jac_stride(n, turn) : mode == kRbGrad ? B + 1 : B;
 }
 // Dynamic LDS: the accumulators, the pool's first floats, the tile's order
 // and its 64 counters (one per total, one for the group to take next).
-__host__ __device__ inline size_t rb_unit_lds(int B, int mode, int n, int stride, int copies,
+__host__ __device__ inline size_t rb_unit_lds(int B, int mode, int n, bool turn, int copies,
                                               int threads, bool pool) {
-    return sizeof(double) * size_t(rb_unit_acc(B, mode, stride)) * size_t(copies) +
+    return sizeof(double) * size_t(rb_unit_acc(B, mode, n, turn)) * size_t(copies) +
            (pool ? sizeof(float) * size_t(rb_lds_floats(n)) : 0) +
            sizeof(uint16_t) * size_t(threads) * kRbUnitPer + sizeof(uint32_t) * 64u;
 }
@@ -585,7 +589,6 @@ struct RbUnitArgs {
     double* grad;
     uint32_t* work;
     int32_t copies;  // accumulator copies, a power of two
-    int32_t stride;  // Jacobian: from row to row, n^2 or, odd, one more
     int32_t tile;    // units a workgroup takes at a time
     int32_t pool;    // the pool's first floats are kept in LDS
     RunTimes* times;  // forward: where the walk's end goes, or null
@@ -621,13 +624,13 @@ template <int kMode, int kN, bool kTurn>
 __global__ __launch_bounds__(rb_unit_threads_of(kMode)) void rb_unit_kernel(const RunArgs a,
                                                                             const RbUnitArgs p) {
     constexpr bool kDeriv = kMode != kRbFwd;
-    constexpr int K = kN * (kN - 1), kCols = kN * kN;
+    constexpr int K = kN * (kN - 1), kCols = kN * kN, kStride = rb_jac_stride(kN, kTurn);
     constexpr int kThreads = rb_unit_threads_of(kMode);
     extern __shared__ __align__(16) double s_acc[];
     const int tid = int(threadIdx.x), lane = tid % kWave;
     if (kMode == kRbFwd && p.times && blockIdx.x == 0 && tid == 0) stamp(&p.times->walked);
     const int B = a.B;
-    const int nacc = rb_unit_acc(B, kMode, p.stride) * p.copies;
+    const int nacc = rb_unit_acc(B, kMode, kN, kTurn) * p.copies;
     float* s_pool = reinterpret_cast<float*>(s_acc + nacc);
     uint16_t* s_order = reinterpret_cast<uint16_t*>(s_pool + (p.pool ? rb_lds_floats(kN) : 0));
     uint32_t* s_count = reinterpret_cast<uint32_t*>(s_order + kThreads * kRbUnitPer);
@@ -797,7 +800,7 @@ __global__ __launch_bounds__(rb_unit_threads_of(kMode)) void rb_unit_kernel(cons
                                 pd_last[s] = pd;
                             }
                             if (act && b < B) {
-                                double* row = s_acc + size_t(b * p.stride) * size_t(p.copies) + copy;
+                                double* row = s_acc + size_t(b * kStride) * size_t(p.copies) + copy;
 #pragma unroll
                                 for (int s = 0; s < kN; ++s) atomicAdd(&row[s * p.copies], e[s]);
 #pragma unroll
@@ -862,7 +865,7 @@ __global__ __launch_bounds__(rb_unit_threads_of(kMode)) void rb_unit_kernel(cons
         for (int i = tid; i < B * kCols; i += kThreads) {
             const int b = i / kCols, col = i - b * kCols;
             double v = 0.0;
-            const double* from = s_acc + size_t(b * p.stride + col) * size_t(p.copies);
+            const double* from = s_acc + size_t(b * kStride + col) * size_t(p.copies);
             for (int x = 0; x < p.copies; ++x) v += from[x];
             if (col >= kN) v *= f;
             if (v != 0.0) atomicAdd(&J[size_t(b) * kRbGradLen + size_t(col)], v);
@@ -1315,8 +1318,8 @@ hipError_t launch_rb_walk(bool scores, int n, uint32_t grid, uint32_t replay_gri
 }
 
 int rb_unit_threads(int mode) { return rb_unit_threads_of(mode); }
-size_t rb_unit_lds_bytes(int B, int mode, int n, int stride, int copies, bool pool) {
-    return rb_unit_lds(B, mode, n, stride, copies, rb_unit_threads_of(mode), pool);
+size_t rb_unit_lds_bytes(int B, int mode, int n, bool turn, int copies, bool pool) {
+    return rb_unit_lds(B, mode, n, turn, copies, rb_unit_threads_of(mode), pool);
 }
 size_t rb_big_lds_bytes(int B, int cap, int mode, bool wide) { return rb_big_lds(B, cap, mode, wide); }
 
@@ -1358,19 +1361,19 @@ static void launch_rb_unit_n(uint32_t grid, const RunArgs& a, const RbUnitArgs& 
                              hipStream_t stream) {
     const int threads = rb_unit_threads_of(kMode);
     hipLaunchKernelGGL((rb_unit_kernel<kMode, kN, kTurn>), dim3(grid), dim3(uint32_t(threads)),
-                       rb_unit_lds(a.B, kMode, kN, p.stride, p.copies, threads, p.pool != 0),
+                       rb_unit_lds(a.B, kMode, kN, kTurn, p.copies, threads, p.pool != 0),
                        stream, a, p);
 }
 
-hipError_t launch_rb_unit(int mode, int n, uint32_t grid, int copies, int stride, bool turn,
-                          int tile, bool pool, const RunArgs& a, const uint2* cnt, const float* F, const float* S,
+hipError_t launch_rb_unit(int mode, int n, uint32_t grid, int copies, bool turn, int tile,
+                          bool pool, const RunArgs& a, const uint2* cnt, const float* F, const float* S,
                           const double* Sbar, const double* g, const uint32_t* rank_offP,
                           const uint4* rank_offD, const float* poolP,
                           unsigned long long* hist_acc, double* grad, uint32_t* work,
                           RunTimes* times, hipStream_t stream) {
     if (n < 2 || n > kRbMaxStates) return hipErrorInvalidValue;
     const RbUnitArgs p{cnt,      F,    S,    Sbar,   g,    rank_offP, rank_offD, poolP,
-                       hist_acc, grad, work, copies, stride, tile, pool ? 1 : 0, times};
+                       hist_acc, grad, work, copies, tile, pool ? 1 : 0, times};
 #define PDA_RB_UNIT_M(M, T)                                         \
     if (n == 2) launch_rb_unit_n<M, 2, T>(grid, a, p, stream);      \
     else if (n == 3) launch_rb_unit_n<M, 3, T>(grid, a, p, stream); \
