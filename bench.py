@@ -120,7 +120,7 @@ def roofline(units, walk_ms):
     counter = {"bound": "valu", "achieved": achieved, "peak": peak, "unit": "TOP/s",
                "frac": achieved / peak, "traffic": traffic, "kernel": "fast_walk_kernel",
                "kernel_ms_avg": walk_ms, "ops_per_unit": cm["valu_lane_ops_per_unit"],
-               "basis": "SQ_THREAD_CYCLES_VALU per unit of an earlier build, frozen"}
+               "basis": "SQ_THREAD_CYCLES_VALU per unit, measured once and frozen"}
     hb = cm["hbm_algorithmic_bytes_per_unit"] * units / t / 1e9
     hbm = {"bound": "hbm", "achieved": hb, "peak": cm["hbm_peak_bytes_per_s"] / 1e9,
            "unit": "GB/s", "frac": hb * 1e9 / cm["hbm_peak_bytes_per_s"], "traffic": traffic}

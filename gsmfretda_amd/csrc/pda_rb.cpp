@@ -282,20 +282,22 @@ int pass_shape(pda_ctx* ctx, int mode, int n, bool wide, int B, int cap, uint32_
             ctx->lds_per_block ||
         least + kStatic > ctx->lds_per_block)
         return fail(PDA_E_DATA, "%d bins exceed the LDS of the RB %s pass", B, names[mode]);
-    // The adjoint keeps the pool's first floats in LDS (3 states, 6.4e6 units:
-    // 155 us, 174 without), unless the run is too small to repay the copy;
-    // the forward reads each entry once and is faster with the LDS left to
-    // more workgroups (forward 451 us, 470 with), as is the Jacobian with it
-    // left to copies.  Copies: the Jacobian's rows of 3 states take 246 us
+    // The adjoint keeps the pool's first floats in LDS where the run repays the
+    // copy: whole calls with 2, 3 and 4 states and 2,097,152 units 96, 105 and 135
+    // us, 99, 107 and 137 without; 524,288 units 62, 65 and 72, 60, 63 and 69
+    // without; 65,536 46, 47 and 50, 44, 45 and 48 without.  The forward reads
+    // each entry once and is faster with the LDS left to more workgroups
+    // (forward 451 us, 470 with), as is the Jacobian with it left to copies.  Copies: the Jacobian's rows of 3 states take 246 us
     // with 8, 227 with 16, 215 with 32; the forward's gain nothing past 16.
     //
     // Many bins leave room for few copies of the Jacobian's rows, and units of
     // one burst often have one F: 64 lanes at the same outcome then add to the
     // same row, one after the other.  With up to four copies the lanes go
     // through their outcomes in different orders (turn), and rows are an odd
-    // number of doubles apart: even ones begin in the same bank.  4 states, 2,000,000 units of 2,000 bursts: 1,000 bins 1586 -> 442
-    // us, 200 bins 484 -> 359; 3 states, 1,000 bins 790 -> 337.  (A wave per 64
-    // outcomes of the units in turn had taken 790, 426 and 600.)  With more
+    // number of doubles apart: even ones begin in the same bank.  4 states, 2,000
+    // bursts x 1,000: 1,000 bins 1586 -> 442 us, 200 bins 484 -> 359; 3 states,
+    // 1,000 bins 790 -> 337.  (A wave per 64 outcomes of the units in turn had
+    // taken 790, 426 and 600.)  With more
     // copies the turning costs more than it saves (3 states, 50 bins 125 -> 148),
     // and with two to four in a small run (4 states, 20,000 units, 200 bins 75 ->
     // 79).
@@ -305,7 +307,7 @@ int pass_shape(pda_ctx* ctx, int mode, int n, bool wide, int B, int cap, uint32_
     auto lds_of = [&](bool turn, int copies, bool pool) {
         return rb_unit_lds_bytes(B, mode, n, turn, copies, pool);
     };
-    ps.pool = mode == 1 && nunits >= 65536u && lds_of(false, 1, true) <= budget;
+    ps.pool = mode == 1 && nunits >= (1u << 20) && lds_of(false, 1, true) <= budget;
     ps.copies = 1;
     while (ps.copies < most && lds_of(false, 2 * ps.copies, ps.pool) <= budget) ps.copies *= 2;
     ps.turn = mode == 2 && ps.copies <= (nunits >= 65536u ? 4 : 1) &&
