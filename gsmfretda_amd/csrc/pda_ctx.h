@@ -109,8 +109,12 @@ struct Population {
 
 // Sets of an RB population that run beside each other, less one: with 1, 2, 3
 // and 5 a Jacobian step of four sets of 4 states (50,000 bursts x 8, fast
-// dynamics) takes 1.21, 1.12, 1.26 and 1.26 ms (1.38 without), the runtime's
-// four hardware queues also serving the process's other streams.
+// dynamics) takes 1.21, 1.12, 1.26 and 1.26 ms (1.38 without) in a process with
+// one context, the runtime's four hardware queues serving all its streams.  The
+// step's time depends on the data and on what else the process keeps: over
+// three contexts taking turns, each with other data, 1.7, 2.0 and 1.6 ms with
+// two and 2.0, 2.5 and 1.9 without; beside 7 other streams 1.11 and 1.44, a
+// context of 16 slots besides 1.10 and 1.42.
 constexpr int kRbParallel = 2;
 
 struct RbModel;

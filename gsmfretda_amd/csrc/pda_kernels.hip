@@ -12,11 +12,12 @@
 //     (seed, set, window, sub-stream, resample, burst) -- no RNG state in
 //     memory, nothing to initialise (replaces setup_kernel,
 //     src/gen_rand.cuh:7-25);
-//   * the common case runs in a lean form (fast_walk_kernel, at most 72
-//     VGPRs); the rare units that need BTPE draws, inversion restarts or
-//     large background means are listed and replayed in full by walk_kernel
-//     over the whole grid, whose last workgroup sums the accumulator rows,
-//     computes chi2 and writes both to the host's result buffer.
+//   * the common case runs in a lean form (fast_walk_kernel, at most 64 VGPRs,
+//     with distance broadening 69 or 72, 80 where its rare draws are made in
+//     place); the units that need more are listed and replayed in full by
+//     walk_kernel over the whole grid, whose last workgroup sums the
+//     accumulator rows, computes chi2 and writes both to the host's result
+//     buffer.
 #include <hip/hip_runtime.h>
 
 #include "pda_math.h"
@@ -89,9 +90,9 @@ __device__ __forceinline__ void flush_hist(int32_t* h, int32_t* __restrict__ row
 // scope atomics to one line serialise); workgroup g draws from queue
 // g % a.queues, so with a multiple of 8 queues each queue is served by
 // one XCD and its bursts stay in that XCD's L2.  Batches are small
-// (about six grabs per wave): the wave that grabs last still walks a
-// whole batch, so the batch sets the grid's tail.  Photons are read
-// through L1/L2.
+// (about six grabs per wave, 32 for a population): the wave that grabs
+// last still walks a whole batch, so the batch sets the grid's tail.
+// Photons are read through L1/L2.
 //
 // A population's work is a flat list of batches: set s owns batches
 // [s * bps, (s + 1) * bps), each covering up to a.batch consecutive units of
@@ -105,27 +106,28 @@ __device__ __forceinline__ void flush_hist(int32_t* h, int32_t* __restrict__ row
 // change sets.
 //
 // kPop: population (two LDS model slots with a histogram each); kPass: the
-// acceptor draw (kPassGuided, kPassTable, kPassBroad, kPassBroadAll); kSamples: per-unit
-// outputs.
+// acceptor draw (kPassGuided, kPassTable, kPassBroad, kPassBroadAll); kSamples:
+// per-unit outputs.
 //
-// Bound by VALU issue (at or above 95 % of the cycles), so what counts is the
-// instructions of fast_window: the window's arithmetic without the cases its
-// arguments cannot have, correctly rounded quotients from reciprocals kept
-// per model, and the launch's divisions done on the host (unit / R, the
-// queues' shares) took a 3-state evaluation of 100,000 bursts x 100 from 459
-// to 407 us and the 256-set generation from 16.7 to 14.7 ms; a search in
-// uniform steps, 32-bit draws and windows without early returns from there to
-// 387 us and 13.2 ms.  The register limit
-// keeps 8 waves on a SIMD: the window loop waits on dependent loads, which the
+// Bound by VALU issue on large runs (90 % of the cycles for 100,000 bursts x 100
+// of 3 states, all of them for 256 sets; 68 % for 50,000 x 32 alone, whose end
+// has idle lanes), so what counts is the instructions of fast_window: the
+// window's arithmetic without the cases its arguments cannot have, correctly
+// rounded quotients from reciprocals kept per model, and the launch's divisions
+// done on the host (unit / R, the queues' shares) took a 3-state evaluation of
+// 100,000 bursts x 100 from 459 to 407 us and the 256-set generation from 16.7
+// to 14.7 ms; a search in uniform steps, 32-bit draws and windows without early
+// returns from there to 387 us and 13.2 ms.  The register limit keeps 8 waves
+// on a SIMD: the window loop waits on dependent loads, which the
 // other waves hide (the 256-set generation 11.3 ms on the GPU with 7 and 10.6
 // with 8, 64 sets of fast dynamics 12.1 and 11.3).
 // A single set's bursts are started by falling duration within each quarter of
 // a queue's share (burst_order in pda_layout.cpp), so that a run ends with units
 // of few windows and not with some lane's thirtieth: 50,000 bursts x 50 of 3
 // states under a 30 kHz background 272 -> 223 us, 100,000 x 100 of 3 states
-// 315 -> 304.  With whole shares sorted those take 244 and 313, with all bursts
-// sorted and dealt out to the queues 248 and 318, and a population 6 % more;
-// populations, whose other sets fill the end of each, and the RB walk, which
+// 315 -> 304 (one data set, its photons cached; 327 where three take turns).
+// With whole shares sorted those take 244 and 313, with all bursts sorted and
+// dealt out to the queues 248 and 318, and a population 6 % more; populations, whose other sets fill the end of each, and the RB walk, which
 // writes per burst, start them as they come.
 // Units are started 64 at a time into LDS and taken from there one lane at a
 // time as lanes fall idle, and ended ones wait in LDS until 64 can be binned:
@@ -135,15 +137,17 @@ __device__ __forceinline__ void flush_hist(int32_t* h, int32_t* __restrict__ row
 // 100,000 x 100 of 3 states 293 -> 288 us; 256 sets of slow dynamics the same
 // (10.62).  The population's workgroup has to stay within 5,120 bytes of LDS
 // for 32 of them on a CU (LDS is handed out in 1,280), which is why the models
-// come in parts; at 6,400 the 256 sets took 12.9 ms.  (Starting units together
-// with their first windows was slower: 14 % more instructions, the first
-// window's close running for half of the lanes.)
+// come in parts.  That holds up to 96 bins (broadened 72); beyond, 25 share a CU
+// and the 256 sets take 12.9 ms at 100 or 200 bins for 10.7 at 50, the 64 of
+// fast dynamics 12.1 for 10.5 and the broadened ones 1.04 for 0.97.  (Starting
+// units together with their first windows was slower: 14 % more instructions,
+// the first window's close running for half of the lanes.)
 // The draw of a broadened efficiency and its binomial (kPassBroad) need up to
-// 74 registers (7 waves for populations: 0.94 ms against 0.98 with 6 on the
+// 72 registers (7 waves for populations: 0.94 ms against 0.98 with 6 on the
 // 64 sets below; no difference for single sets).  They had been the general
 // form's, at 186 registers and two waves per SIMD with logarithms,
-// exponentials and divisions in double per window: 50,000 bursts x 50 of a 3-state model 371 -> 197 us, 64 sets x
-// 20,000 x 16 2.74 -> 1.41 ms.
+// exponentials and divisions in double per window: 50,000 bursts x 50 of a
+// 3-state model 371 -> 197 us, 64 sets x 20,000 x 16 2.74 -> 1.41 ms.
 //
 // kPassBroadAll: counts beyond the table and background means above 64 are
 // drawn in the window.  A broadened unit had not been abandoned for them before
@@ -152,7 +156,7 @@ __device__ __forceinline__ void flush_hist(int32_t* h, int32_t* __restrict__ row
 // bursts x 64 at efficiencies near 0.99, 17 % of their units abandoned, took
 // 8.5 ms where the general form had taken 3.5, and under a 60 kHz background
 // 17.0 against 8.3; with the draws in place 1.9 and 2.1.  The draws spill up to
-// 300 bytes where they are made; with 6 waves the 64 sets below take 1.06 ms,
+// 392 bytes where they are made; with 6 waves the 64 sets below take 1.06 ms,
 // with 5 1.09, 4 1.23 and 3 1.44, against kPassBroad's 0.95: which of the two
 // a run takes is decided by its bursts (draws_in_place in pda_layout.cpp).
 constexpr bool is_broad(int pass) { return pass == kPassBroad || pass == kPassBroadAll; }
@@ -742,9 +746,10 @@ __global__ __launch_bounds__(kBinomTable) void table_kernel(const Model* __restr
 // ---- population runs ---------------------------------------------------------
 //
 // A population of parameter sets (an optimiser generation) over the same
-// resident bursts in one launch sequence: pop_walk_kernel walks every
-// (set, burst, resample) unit, pop_replay_kernel recomputes the units the
-// fast form abandoned, pop_finish_kernel computes each set's histogram and
+// resident bursts in one launch sequence: fast_walk_kernel walks every
+// (set, burst, resample) unit, pop_replay_kernel recomputes the units it
+// abandoned (where they are more than the list holds, pop_walk_kernel walks
+// all of them again), pop_finish_kernel computes each set's histogram and
 // chi2.  The reference evaluates one set per stream and per mc::run_kernel
 // call (src/gpuWorker.cpp:71-80); the units and their random streams are the
 // same as a single-set run with set id set_base + s * set_stride.

@@ -7,12 +7,14 @@
 // Two forms of the same computation:
 //   * general: every branch of the reference (distance broadening, BTPE,
 //     inversion restarts, Poisson chunking for large background means);
-//   * fast: the common case only -- no broadening (v == 0, so the broadened
-//     efficiency and its binomial inversion constants are per-state tables),
-//     inversion without restarts, background means <= 64.  A unit that would
-//     leave the common case is abandoned (replay = true) and recomputed from
-//     scratch by the general form; the keyed random streams make the replay
-//     produce exactly the draws the fast form would have consumed.
+//   * fast: the common case -- counts below 128, inversion without restarts,
+//     background means <= 64.  The acceptor draw is by thresholds or tables of
+//     the states' efficiencies (v == 0), or of an efficiency drawn per window
+//     (broadening), where larger counts and means may be drawn in place
+//     (BroadAll).  A unit that would leave the common case is abandoned
+//     (replay = true) and recomputed from scratch by the general form; the
+//     keyed random streams make the replay produce exactly the draws the fast
+//     form would have consumed.
 #pragma once
 #include <type_traits>
 
@@ -247,7 +249,8 @@ PDA_HD int binomial_broad(int n, float p, uint32_t hi, uint32_t lo) {
 // (< 2^32), floor(u m / 2^(31+l)) = floor(u / d) for every u < 2^31 (m d =
 // 2^(31+l) + e with 0 <= e < d, so u m / 2^(31+l) exceeds u / d by less than
 // u / 2^(31+l) * e / d < 2^-l <= 1 / d, which cannot reach the next integer).
-// Unit indices stay below 2^31 (every run checks it).  Built once per wave.
+// Unit indices stay below 2^31 (every run checks it).  Built on the host, an
+// argument of the launch.
 struct UnitDiv {
     uint32_t m, sh;
 };
