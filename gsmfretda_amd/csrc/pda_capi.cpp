@@ -178,23 +178,20 @@ int load_common(pda_ctx* ctx, const int64_t* start, const int64_t* stop, const i
         HIP_TRY(hipMemcpy(ctx->d_bursts, bursts.data(), sizeof(BurstDesc) * size_t(nbursts),
                           hipMemcpyHostToDevice));
         const std::vector<uint32_t> order = burst_order(bursts);
+        const size_t idx_bytes = sizeof(uint32_t) * size_t(nbursts);
         const size_t bytes = sizeof(WalkBurst) * size_t(nbursts);
         HIP_TRY(hipMalloc(&ctx->d_plain, bytes));
         HIP_TRY(hipMalloc(&ctx->d_order, bytes));
-        uint32_t* d_idx = nullptr;
-        HIP_TRY(hipMalloc(&d_idx, sizeof(uint32_t) * size_t(nbursts)));
-        hipError_t e = hipMemcpy(d_idx, order.data(), sizeof(uint32_t) * size_t(nbursts),
-                                 hipMemcpyHostToDevice);
-        if (e == hipSuccess)
-            e = launch_order(ctx->d_bursts, d_idx, uint32_t(nbursts), ctx->d_plain, ctx->d_order,
-                             nullptr);
-        if (e == hipSuccess) e = hipStreamSynchronize(nullptr);
-        (void)hipFree(d_idx);
-        HIP_TRY(e);
+        // the links' buffer holds the order until the links overwrite it
+        HIP_TRY(hipMalloc(&ctx->d_links, std::max(sizeof(uint2) * size_t(total), idx_bytes)));
+        uint32_t* idx = reinterpret_cast<uint32_t*>(ctx->d_links);
+        HIP_TRY(hipMemcpy(idx, order.data(), idx_bytes, hipMemcpyHostToDevice));
+        HIP_TRY(launch_order(ctx->d_bursts, idx, uint32_t(nbursts), ctx->d_plain, ctx->d_order,
+                             nullptr));
+        HIP_TRY(hipStreamSynchronize(nullptr));
     }
     if (total > 0) {
         HIP_TRY(hipMalloc(&ctx->d_ticks, sizeof(uint32_t) * size_t(total)));
-        HIP_TRY(hipMalloc(&ctx->d_links, sizeof(uint2) * size_t(total)));
         HIP_TRY(hipMemcpy(ctx->d_ticks, ticks.data(), sizeof(uint32_t) * size_t(total),
                           hipMemcpyHostToDevice));
         HIP_TRY(hipMemcpy(ctx->d_links, links.data(), sizeof(uint2) * size_t(total),

@@ -28,8 +28,8 @@ int fail_to(std::string& err, int code, const char* fmt, ...) {
 
 // The runs a burst's photons start, its links at lk.
 static void add_runs(const BurstDesc& d, const uint2* lk, LongRuns& out) {
+    out.starts += (d.P + LongRuns::kEvery - 1u) / LongRuns::kEvery;
     for (uint32_t i = 0; i < d.P; i += LongRuns::kEvery) {
-        ++out.starts;
         const uint32_t f = lk[i].x & kIndexMask, colour = lk[i].x >> 30;
         if (f >= d.P || colour == 3u) continue;  // (one in both channels counts nothing)
         std::vector<uint64_t>& h = out.at_least[colour - 1u];
@@ -89,11 +89,6 @@ int encode_bursts(const int64_t* start, const int64_t* stop, const int64_t* ista
         uint32_t* tk = ticks.data() + d.off;
         uint2* lk = links.data() + d.off;
         col.resize(P);
-        for (uint32_t i = 0; i < P; ++i) {
-            tk[i] = kTickSentinel;
-            lk[i].x = P;
-            lk[i].y = P;
-        }
         int64_t prev = -1;
         for (uint32_t i = 0; i < P; ++i) {
             col[i] = src.colour(base + i);
